@@ -350,16 +350,17 @@ rxm_status rxm_symdir_grad(rxm_mesh* mesh, const float* Mr, const float* uv, con
  * synchronisation; when any of iters / start_residual / final_residual is
  * non-NULL the call waits for the stream and reports the iterations taken and
  * the squared residual norms, as the reference's solver does. Work vectors
- * (4 x 3V floats) are allocated by the mesh on first use. */
+ * (4 x 3V floats, shared by the solves of the mesh) are allocated by the mesh
+ * on first use. */
 rxm_status rxm_mcf_implicit_cg(rxm_mesh* mesh, const int32_t* row_ptr, const int32_t* col,
                                const float* val, const float* mass, const float* x, float* out,
                                int max_iter, float abs_tol, float rel_tol, int* iters,
                                float* start_residual, float* final_residual, void* stream);
 
-/* Implicit MCF step with the system never assembled: CG (precond = 0) or
- * Jacobi-preconditioned CG (precond = 1) on A X = B, where every product
- * recomputes the weights from the fixed input coordinates `coords` (3 x V
- * SoA): A = M + dt L with cotangent weights max(0, cot + cot) and Voronoi
+/* Implicit MCF step without a system from the caller: CG (precond = 0) or
+ * Jacobi-preconditioned CG (precond = 1) on A X = B with the weights of the
+ * fixed input coordinates `coords` (3 x V SoA), evaluated once per call into
+ * mesh-owned scratch (cotangent weights: rxm_cot_nnz floats; no CSR): A = M + dt L with cotangent weights max(0, cot + cot) and Voronoi
  * mass (uniform = 0), or unit weights and mass = valence (uniform = 1); B =
  * M x (the reference's init_B). x is the initial X (3 x V SoA; the reference
  * starts from the input coordinates), the solution goes to `out`. Stopping

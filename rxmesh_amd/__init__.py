@@ -526,8 +526,8 @@ class Mesh:
 
     def mcf_matfree_cg(self, coords, x, dt, uniform=False, precond=False, max_iter=100, abs_tol=1e-6, rel_tol=0.0,
                        out=None, stats=True, stream=None):
-        """Implicit MCF step with the system never assembled (weights recomputed
-        from `coords` in every product): CG, or Jacobi-preconditioned CG, on
+        """Implicit MCF step without an assembled CSR (the weights of `coords`
+        are evaluated once per call): CG, or Jacobi-preconditioned CG, on
         A X = M x from X = x. Returns (X, iterations, start residual, final
         residual) -- the last three None when stats is False."""
         import torch

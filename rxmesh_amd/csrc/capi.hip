@@ -11,6 +11,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <atomic>
 #include <vector>
 
@@ -63,9 +64,9 @@ struct rxm_mesh
     const uint32_t*   d_vvk_xlin  = nullptr;
     uint32_t          smooth_steps = 0;  // > 0: Jacobi steps per launch over the K-level plan
     uint32_t          smooth_g4    = 1;  // two-step launches pass float4 iterates between them
-    float*            d_cg         = nullptr;  // CG work vectors: r, p (two), s (3 V floats each), partials
-    CgState*          d_cg_state   = nullptr;
-    float*            d_mf         = nullptr;  // matrix-free CG: r, p (two), s (3 V each), mass, diag (V), partials
+    float*            d_cg         = nullptr;  // CG work arrays (CgWork)
+    float*            d_mf         = nullptr;  // matrix-free CG: mass, diag (V each), weights (one per row entry)
+    size_t            mf_floats    = 0;        // size of d_mf
     float*            d_iter4      = nullptr;  // two float4 iterates (8 V floats), allocated on first use
     uint32_t          smooth_fused = 0;  // 1: two Jacobi steps per launch
     uint32_t          spmv_lanes   = 8;  // lanes per CSR row in the SpMV-3 kernels
@@ -348,7 +349,7 @@ int ensure_vv_plan(rxm_mesh* m, void* stream)
     m->allocs.push_back(m->d_vv_nbr);
     m->device_bytes += 2ull * (rb[h.P] + nb[h.P]);
     Bump b(nullptr);
-    plan_q2(b, 0, h.max_nv, h.max_ne, h.max_nf);
+    plan_vvl(b, h.max_ne, h.max_nvo);
     rc = launch_patches(k_query2_vv_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm,
                         m->d_vv_rbase, m->d_vv_nbase, m->d_vv_roff, m->d_vv_nbr);
     if (rc) {
@@ -1322,6 +1323,25 @@ rxm_status rxm_to_global(rxm_mesh* m, int kind, int ncomp, const float* l, float
     return permute(m, kind, ncomp, l, g, false, stream);
 }
 
+}  // extern "C"
+
+// One launch over the cached pattern (ensure_cot_plan done): the system's
+// rows (CSR), or values, mass and diagonal only.
+template <bool CSR>
+static int launch_cot_assemble(rxm_mesh* m, const uint32_t* vv_base, const float* pos, float dt, int32_t* row_ptr,
+                               int32_t* col, float* val, float* mass, float* diag, void* stream)
+{
+    Bump b(nullptr);
+    plan_cot(b, m->h.max_nv, m->h.max_ne, m->h.max_nvo, op_max_patch(m, RXM_OP_VV));
+    auto go = [&](auto kernel, uint32_t threads) {
+        return launch_patches_xcd(kernel, threads, b.bytes(), stream, m, m->dm, vv_base, m->d_cot_rs, m->d_cot_ent,
+                                  pos, dt, row_ptr, col, val, mass, diag);
+    };
+    return (m->cot_threads == 512) ? go(k_cot_assemble<512, CSR>, 512) : go(k_cot_assemble<256, CSR>, 256);
+}
+
+extern "C" {
+
 rxm_status rxm_cot_nnz(rxm_mesh* m, int64_t* nnz)
 {
     if (!m || !nnz) return RXM_ERR_INVALID_ARG;
@@ -1342,13 +1362,7 @@ rxm_status rxm_cot_csr_assemble(rxm_mesh* m, const float* pos, float dt, int32_t
     if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
     if ((rc = ensure_cot_plan(m))) return rc;
     const uint32_t maxrow = op_max_patch(m, kOpCot);
-    Bump           b(nullptr);
-    plan_cot(b, m->h.max_nv, m->h.max_ne, m->h.max_nvo, op_max_patch(m, RXM_OP_VV));
-    auto go = [&](auto kernel, uint32_t threads) {
-        return launch_patches_xcd(kernel, threads, b.bytes(), stream, m, m->dm, vv_base, m->d_cot_rs, m->d_cot_ent,
-                                  pos, dt, row_ptr, col, val, mass);
-    };
-    rc = (m->cot_threads == 512) ? go(k_cot_assemble<512>, 512) : go(k_cot_assemble<256>, 256);
+    rc = launch_cot_assemble<true>(m, vv_base, pos, dt, row_ptr, col, val, mass, nullptr, stream);
     if (rc || m->cot_nplist == 0) return rc;
     Bump br(nullptr);
     plan_cot_ring(br, m->h.max_nv, m->h.max_ne, m->h.max_nf, m->h.max_nv, maxrow);
@@ -1414,6 +1428,105 @@ rxm_status rxm_mcf_explicit(rxm_mesh* m, const int32_t* row_ptr, const int32_t* 
     return rc;
 }
 
+}  // extern "C"
+
+namespace {
+// Work arrays of the CG solves, allocated by the mesh on first use: r, two
+// directions and s (3 components of cg_stride each), per-patch partials, the
+// update's partials and the two scalar states.
+struct CgWork
+{
+    float *  r, *p[2], *s, *part;
+    double*  rpart;
+    CgState *upd, *app;
+    uint32_t groups;  // workgroups of the update
+};
+int cg_work(rxm_mesh* m, CgWork& w)
+{
+    const size_t   v3 = 3 * cg_stride(m->h.nV), np = (size_t(m->h.P) + 63u) & ~size_t(63);
+    const size_t   nd = kCgUpdateGroups * sizeof(double) + 2 * sizeof(CgState), bytes = (4 * v3 + np) * sizeof(float) + nd;
+    if (!m->d_cg) {
+        float* p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
+        m->allocs.push_back(p);
+        m->device_bytes += bytes;
+        m->d_cg = p;
+    }
+    w.r    = m->d_cg;
+    w.p[0] = w.r + v3;
+    w.p[1] = w.p[0] + v3;
+    w.s    = w.p[1] + v3;
+    w.part = w.s + v3;
+    w.rpart = reinterpret_cast<double*>(w.part + np);
+    w.upd   = reinterpret_cast<CgState*>(w.rpart + kCgUpdateGroups);
+    w.app   = w.upd + 1;
+    // one quad per thread and round; at most kCgUpdateGroups workgroups, so
+    // the product's workgroups sum at most that many partials
+    const size_t quads = v3 / 4;
+    w.groups = static_cast<uint32_t>(std::min<size_t>(kCgUpdateGroups, (quads + kCgUpdateThreads - 1) / kCgUpdateThreads));
+    return RXM_OK;
+}
+
+// A X = M x from X = x over the mesh's cotangent system (val) or, UNI, the
+// uniform-weight system; diag: Jacobi preconditioner (null: none).
+template <bool PRE, bool UNI>
+int cg_solve(rxm_mesh* m, const float* val, float dt, const float* mass, const float* diag, const float* x, float* out,
+             int max_iter, float abs_tol, float rel_tol, int* iters, float* start_residual, float* final_residual,
+             void* stream)
+{
+    CgWork w{};
+    int    rc = cg_work(m, w);
+    if (rc) return rc;
+    const uint32_t* vv_base = nullptr;
+    if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
+    constexpr uint32_t T = 256;
+    const uint32_t     n = m->h.nV, P = m->h.P;
+    hipStream_t        hs = static_cast<hipStream_t>(stream);
+    Bump               b(nullptr);
+    plan_cg(b, m->h.max_nv, m->h.max_nvo, m->vv_max_nent, UNI, T);
+    auto apply = [&](auto kernel, const float* xin, float* pnew, const CgState* upd) {
+        return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
+                                  static_cast<const uint16_t*>(m->d_vv_roff), static_cast<const uint16_t*>(m->d_vv_nbr),
+                                  val, dt, xin, static_cast<const float*>(w.r), diag, out, pnew, w.s, w.part,
+                                  static_cast<const double*>(w.rpart), w.groups, upd, w.app, abs_tol, rel_tol);
+    };
+    auto update = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(w.groups), dim3(kCgUpdateThreads), 0, hs, n, mass, x, out, w.r,
+                           static_cast<const float*>(w.s), diag, static_cast<const float*>(w.part), P, w.rpart,
+                           static_cast<const CgState*>(w.app), w.upd);
+    };
+    auto finish = [&](auto kernel, uint32_t grid, const float* pv) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, hs, n, static_cast<const double*>(w.rpart), w.groups, pv,
+                           out, static_cast<const CgState*>(w.upd), w.app, abs_tol, rel_tol);
+    };
+    // set-up: s = A x0, r = M x0 - s, x = x0
+    if ((rc = apply(k_cg_apply<T, 0, PRE, UNI>, x, nullptr, w.upd))) return rc;
+    update(k_cg_update<0>);
+    for (int it = 0; it < max_iter; ++it) {
+        // the first iteration takes p = z (p_old unread), later ones z + beta p_old
+        float* pnew = w.p[(it + 1) & 1];
+        rc = it == 0 ? apply(k_cg_apply<T, 1, PRE, UNI>, w.p[it & 1], pnew, w.upd)
+                     : apply(k_cg_apply<T, 2, PRE, UNI>, w.p[it & 1], pnew, w.upd);
+        if (rc) return rc;
+        update(k_cg_update<1>);
+    }
+    if (max_iter == 0) finish(k_cg_finish<true>, 1, nullptr);
+    else finish(k_cg_finish<false>, (n + 255u) / 256u, w.p[max_iter & 1]);
+    RXM_HIP(hipGetLastError());
+    if (iters || start_residual || final_residual) {
+        CgState h{};
+        RXM_HIP(hipMemcpyAsync(&h, w.app, sizeof(CgState), hipMemcpyDeviceToHost, hs));
+        RXM_HIP(hipStreamSynchronize(hs));
+        if (iters) *iters = static_cast<int>(h.iters);
+        if (start_residual) *start_residual = h.start;
+        if (final_residual) *final_residual = h.delta;
+    }
+    return RXM_OK;
+}
+}  // namespace
+
+extern "C" {
+
 rxm_status rxm_mcf_implicit_cg(rxm_mesh* m, const int32_t* row_ptr, const int32_t* col, const float* val,
                                const float* mass, const float* x, float* out, int max_iter, float abs_tol,
                                float rel_tol, int* iters, float* start_residual, float* final_residual,
@@ -1425,58 +1538,8 @@ rxm_status rxm_mcf_implicit_cg(rxm_mesh* m, const int32_t* row_ptr, const int32_
     int rc = check_system_runs(m);
     if (!rc) rc = ensure_vv_plan(m, stream);
     if (rc) return rc;
-    const uint32_t* vv_base = nullptr;
-    if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
-    const uint32_t n = m->h.nV, P = m->h.P, nb = (n + 255u) / 256u;
-    const size_t   v3 = size_t(3) * n, npart = std::max<size_t>(P, nb);
-    if (!m->d_cg) {
-        float* p = nullptr;
-        if (hipMalloc(&p, (4 * v3 + npart) * sizeof(float)) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(p);
-        m->device_bytes += (4 * v3 + npart) * sizeof(float);
-        CgState* st = nullptr;
-        if (hipMalloc(&st, sizeof(CgState)) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(st);
-        m->d_cg       = p;
-        m->d_cg_state = st;
-    }
-    float *    r = m->d_cg, *pv[2] = {m->d_cg + v3, m->d_cg + 2 * v3}, *s = m->d_cg + 3 * v3, *part = m->d_cg + 4 * v3;
-    CgState*   st = m->d_cg_state;
-    hipStream_t hs = static_cast<hipStream_t>(stream);
-    Bump b(nullptr);
-    plan_sl(b, m->h.max_nv, m->h.max_nvo, m->vv_max_nent, false);
-    b.alloc<float>(m->vv_max_nent + m->h.max_nvo);
-    b.alloc<float>(256 / 64);
-    const uint32_t lds = b.bytes();
-    auto apply = [&](auto kernel, const float* xin, float* pnew, float* y) {
-        return launch_patches_xcd(kernel, 256, lds, stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
-                                  m->d_vv_roff, m->d_vv_nbr, val, xin, static_cast<const float*>(r), pnew, y, part,
-                                  static_cast<const CgState*>(st));
-    };
-    // set-up: s = A x0, r = M x0 - s, x = x0, delta = <r, r>
-    if ((rc = apply(k_cg_apply<256, 0>, x, nullptr, s))) return rc;
-    hipLaunchKernelGGL((k_cg_update<0>), dim3(nb), dim3(256), 0, hs, n, mass, x, out, r, nullptr, s, part, st);
-    hipLaunchKernelGGL((k_cg_scalar<0>), dim3(1), dim3(1024), 0, hs, nb, part, st, abs_tol, rel_tol);
-    for (int it = 0; it < max_iter; ++it) {
-        float* pold = pv[it & 1];
-        float* pnew = pv[(it + 1) & 1];
-        // the first iteration stages p = r (p_old unread), later ones r + beta p_old
-        rc = it == 0 ? apply(k_cg_apply<256, 1>, pold, pnew, s) : apply(k_cg_apply<256, 2>, pold, pnew, s);
-        if (rc) return rc;
-        hipLaunchKernelGGL((k_cg_scalar<1>), dim3(1), dim3(1024), 0, hs, P, part, st, abs_tol, rel_tol);
-        hipLaunchKernelGGL((k_cg_update<1>), dim3(nb), dim3(256), 0, hs, n, mass, x, out, r, pnew, s, part, st);
-        hipLaunchKernelGGL((k_cg_scalar<2>), dim3(1), dim3(1024), 0, hs, nb, part, st, abs_tol, rel_tol);
-    }
-    RXM_HIP(hipGetLastError());
-    if (iters || start_residual || final_residual) {
-        CgState h{};
-        RXM_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, hs));
-        RXM_HIP(hipStreamSynchronize(hs));
-        if (iters) *iters = static_cast<int>(h.iters);
-        if (start_residual) *start_residual = h.start;
-        if (final_residual) *final_residual = h.delta;
-    }
-    return RXM_OK;
+    return cg_solve<false, false>(m, val, 0.f, mass, nullptr, x, out, max_iter, abs_tol, rel_tol, iters,
+                                  start_residual, final_residual, stream);
 }
 
 rxm_status rxm_mcf_matfree_cg(rxm_mesh* m, const float* coords, const float* x, float* out, float dt, int uniform,
@@ -1493,75 +1556,37 @@ rxm_status rxm_mcf_matfree_cg(rxm_mesh* m, const float* coords, const float* x, 
         // the face pass gives a vertex its reference weights only when its
         // ring is one closed fan (a closed vertex-manifold mesh)
         if (m->cot_nplist != 0) return RXM_ERR_UNSUPPORTED;
-    } else if ((rc = ensure_cot_plan(m))) {
-        return rc;
+        if ((rc = check_system_runs(m))) return rc;
     }
-    const uint32_t* vv_base = nullptr;
-    if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
-    const uint32_t n = m->h.nV, P = m->h.P, nb = (n + 255u) / 256u;
-    const size_t   v3 = size_t(3) * n, npart = std::max<size_t>(P, nb);
-    if (!m->d_mf) {
+    if ((rc = ensure_vv_plan(m, stream))) return rc;
+    // mass and diagonal per vertex; the weights, one float per row entry
+    const size_t n = cg_stride(m->h.nV), cnt = 2 * n + (uni ? 0 : size_t(op_base(m, kOpCot).back()));
+    if (cnt > m->mf_floats) {
         float* p = nullptr;
-        const size_t cnt = 4 * v3 + 2 * size_t(n) + npart;
         if (hipMalloc(&p, cnt * sizeof(float)) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
         m->allocs.push_back(p);
         m->device_bytes += cnt * sizeof(float);
-        m->d_mf = p;
+        m->d_mf      = p;
+        m->mf_floats = cnt;
     }
-    if (!m->d_cg_state) {
-        CgState* st = nullptr;
-        if (hipMalloc(&st, sizeof(CgState)) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(st);
-        m->d_cg_state = st;
+    float *mass = m->d_mf, *diag = mass + n, *val = diag + n;
+    if (uni) {
+        rc = launch_patches(k_uniform_diag, 256, 0, stream, m, m->dm, m->d_vv_rbase,
+                            static_cast<const uint16_t*>(m->d_vv_roff), dt, mass, diag);
+    } else {
+        const uint32_t* vv_base = nullptr;
+        if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
+        rc = launch_cot_assemble<false>(m, vv_base, coords, dt, nullptr, nullptr, val, mass, diag, stream);
     }
-    float *r = m->d_mf, *pv[2] = {m->d_mf + v3, m->d_mf + 2 * v3}, *s = m->d_mf + 3 * v3;
-    float *mass = m->d_mf + 4 * v3, *diag = mass + n, *part = diag + n;
-    CgState*    st = m->d_cg_state;
-    hipStream_t hs = static_cast<hipStream_t>(stream);
-    constexpr uint32_t T = 256;
-    Bump b(nullptr);
-    plan_mf(b, m->h.max_nv, m->h.max_ne, m->h.max_nvo, op_max_patch(m, RXM_OP_VV), uni, T);
-    const uint32_t lds = b.bytes();
-    float* dg = pre ? diag : nullptr;
-    auto apply = [&](auto kernel, const float* xin, float* pnew, float* y) {
-        return launch_patches_xcd(kernel, T, lds, stream, m, m->dm, vv_base, m->d_cot_rs, m->d_cot_ent, coords, dt,
-                                  xin, static_cast<const float*>(r), dg, mass, pnew, y, part,
-                                  static_cast<const CgState*>(st));
+    if (rc) return rc;
+    auto solve = [&](auto pre_c, auto uni_c) {
+        constexpr bool PRE = decltype(pre_c)::value, UNI = decltype(uni_c)::value;
+        return cg_solve<PRE, UNI>(m, UNI ? nullptr : val, dt, mass, PRE ? diag : nullptr, x, out, max_iter, abs_tol,
+                                  rel_tol, iters, start_residual, final_residual, stream);
     };
-    // the kernel for (mode, weights, preconditioner)
-    auto launch = [&](int mode, const float* xin, float* pnew, float* y) {
-#define RXM_MF(MODE)                                                                         \
-    (uni ? (pre ? apply(k_mf_apply<T, MODE, true, true>, xin, pnew, y)                       \
-                : apply(k_mf_apply<T, MODE, true, false>, xin, pnew, y))                     \
-         : (pre ? apply(k_mf_apply<T, MODE, false, true>, xin, pnew, y)                      \
-                : apply(k_mf_apply<T, MODE, false, false>, xin, pnew, y)))
-        return mode == 0 ? RXM_MF(0) : (mode == 1 ? RXM_MF(1) : RXM_MF(2));
-#undef RXM_MF
-    };
-    // set-up: s = A x0, mass (and diag), r = B - s with B = mass * x0, x = x0, delta
-    if ((rc = launch(0, x, nullptr, s))) return rc;
-    hipLaunchKernelGGL((k_cg_update<0>), dim3(nb), dim3(256), 0, hs, n, static_cast<const float*>(mass), x, out, r,
-                       nullptr, s, part, st, static_cast<const float*>(dg));
-    hipLaunchKernelGGL((k_cg_scalar<0>), dim3(1), dim3(1024), 0, hs, nb, part, st, abs_tol, rel_tol);
-    for (int it = 0; it < max_iter; ++it) {
-        float* pold = pv[it & 1];
-        float* pnew = pv[(it + 1) & 1];
-        if ((rc = launch(it == 0 ? 1 : 2, pold, pnew, s))) return rc;
-        hipLaunchKernelGGL((k_cg_scalar<1>), dim3(1), dim3(1024), 0, hs, P, part, st, abs_tol, rel_tol);
-        hipLaunchKernelGGL((k_cg_update<1>), dim3(nb), dim3(256), 0, hs, n, static_cast<const float*>(mass), x, out,
-                           r, pnew, s, part, st, static_cast<const float*>(dg));
-        hipLaunchKernelGGL((k_cg_scalar<2>), dim3(1), dim3(1024), 0, hs, nb, part, st, abs_tol, rel_tol);
-    }
-    RXM_HIP(hipGetLastError());
-    if (iters || start_residual || final_residual) {
-        CgState h{};
-        RXM_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, hs));
-        RXM_HIP(hipStreamSynchronize(hs));
-        if (iters) *iters = static_cast<int>(h.iters);
-        if (start_residual) *start_residual = h.start;
-        if (final_residual) *final_residual = h.delta;
-    }
-    return RXM_OK;
+    using yes = std::true_type;
+    using no  = std::false_type;
+    return pre ? (uni ? solve(yes{}, yes{}) : solve(yes{}, no{})) : (uni ? solve(no{}, yes{}) : solve(no{}, no{}));
 }
 
 rxm_status rxm_symdir_rest(rxm_mesh* m, const float* rest_pos, float* Mr, void* stream)

@@ -3,6 +3,7 @@
 // and the symmetric Dirichlet energy with its hand-written adjoint.
 #pragma once
 #include <cfloat>
+#include <type_traits>
 
 #include "k_geometry.hpp"
 
@@ -245,13 +246,15 @@ __device__ __forceinline__ void stage_vertices(const DevMesh& m, const PatchDesc
 // ring is one closed fan; the rows of other vertices (boundary, several
 // fans) take wedges across the ring's gaps, as the reference's cyclic walk
 // does, and are rewritten afterwards by k_cot_ring_rows.
-template <uint32_t T>
+// CSR false: values, mass and, by vertex, the diagonal only (the weights of the
+// matrix-free solve); row_ptr and col are not written.
+template <uint32_t T, bool CSR = true>
 __global__ __launch_bounds__(T) void k_cot_assemble(DevMesh m, const uint32_t* __restrict__ vv_base,
                                                     const uint32_t* __restrict__ rs,
                                                     const uint16_t* __restrict__ ent, const float* __restrict__ pos,
                                                     float dt, int32_t* __restrict__ row_ptr,
                                                     int32_t* __restrict__ col, float* __restrict__ val,
-                                                    float* __restrict__ mass)
+                                                    float* __restrict__ mass, float* __restrict__ diag)
 {
     extern __shared__ uint4 smem[];
     const uint32_t p = patch_of_block(m.P);  // XCD-contiguous patch ranges
@@ -319,20 +322,24 @@ __global__ __launch_bounds__(T) void k_cot_assemble(DevMesh m, const uint32_t* _
         }
         const float    ms = 1.0f / (0.5f / vw);
         const uint32_t o  = bse + k0 + v;
-        row_ptr[d.vp + v] = static_cast<int32_t>(o);
-        mass[d.vp + v]    = ms;
-        col[o]            = static_cast<int32_t>(d.vp + v);
-        val[o]            = ms + sum_w;
+        if constexpr (CSR) {
+            row_ptr[d.vp + v] = static_cast<int32_t>(o);
+            col[o]            = static_cast<int32_t>(d.vp + v);
+        } else {
+            diag[d.vp + v] = ms + sum_w;
+        }
+        mass[d.vp + v] = ms;
+        val[o]         = ms + sum_w;
     }
-    if (threadIdx.x == 0) row_ptr[d.vp + d.nvo] = static_cast<int32_t>(bse + nent + d.nvo);
+    if (CSR && threadIdx.x == 0) row_ptr[d.vp + d.nvo] = static_cast<int32_t>(bse + nent + d.nvo);
     // off-diagonal entries, contiguous over the patch's output range
     for (uint32_t k = threadIdx.x; k < nent; k += T) {
         const uint32_t u = L.ent[k], e = u >> 1, x = L.ev[e], v = (u & 1u) ? hi16(x) : lo16(x);
         const float2   c = L.cot[e];
         const float    w = c.x + c.y;
         const uint32_t o = bse + k + v + 1;
-        col[o]           = static_cast<int32_t>(L.lin[(u & 1u) ? lo16(x) : hi16(x)]);
-        val[o]           = -(((w >= 0.f) ? w : 0.f) * dt);
+        if constexpr (CSR) col[o] = static_cast<int32_t>(L.lin[(u & 1u) ? lo16(x) : hi16(x)]);
+        val[o] = -(((w >= 0.f) ? w : 0.f) * dt);
     }
 }
 
@@ -560,356 +567,436 @@ __global__ __launch_bounds__(T) void k_mcf_patch(DevMesh m, const uint32_t* __re
 // on A X = B with B = M x (apps/MCF/mcf_kernels.cuh:302-352, mcf_B_setup) for
 // the three coordinate columns at once: dot products and norms run over all
 // 3V entries, as the reference's cuBLAS calls over the whole V x 3 matrix do.
-// The loop runs on the device: the scalars live in CgState, every kernel
-// returns at once when `done` is set, and the host launches max_iter
-// iterations without reading anything back. Partial sums are per workgroup
-// in a fixed order and reduced by one workgroup in a fixed order, so a solve
-// is deterministic.
+// The loop runs on the device and the host enqueues max_iter iterations of two
+// launches without reading anything back:
+//   k_cg_apply   sums the update's partials (<r, r>), takes beta and the
+//                stopping decision from them, adds the last alpha p to x,
+//                forms p = r + beta p and s = A p, partial <s, p> per patch;
+//   k_cg_update  sums those partials, takes alpha, r -= alpha s, partial
+//                <r, r> per workgroup.
+// Every workgroup sums the partials itself, in the same fixed order and in
+// FP64, so all of them hold the same scalar, two solves are bit-identical and
+// no launch of its own (a single workgroup, 2.5-4.4 us each, twice per
+// iteration) stands between the passes. The update runs in at most
+// kCgUpdateGroups workgroups so that the product's workgroups have few
+// partials to sum. Adding alpha p to x in the product, which has p in
+// registers, instead of in the update saves one read of p (12 V bytes).
+// Bound: 160 V bytes of vectors and values per iteration from the Infinity
+// Cache, and the product's four dependent round trips (descriptor, ids and
+// plan, ribbon words, stores). Assembly + 20 iterations, 1201 x 401 torus
+// (482k vertices): 647 -> 494 us; an iteration 15.5 + 8.8 and two sums of 4.3 +
+// 3.6 us -> 14.5 + 7.7 us.
+// Scalars pass through two states: the product reads `upd` and writes `app`,
+// the update reads `app` and writes `upd`, so no launch reads what it writes.
 struct CgState
 {
-    float    delta, delta_old, alpha, beta, start;
-    uint32_t iters, done, pad;
+    float    delta, alpha, beta, start;
+    uint32_t iters, done;
 };
+constexpr uint32_t kCgUpdateThreads = 1024, kCgUpdateGroups = 512;
 
-// y = A x (MODE 0, the set-up), or, for a CG iteration, p_new = r (MODE 1,
-// the first) or r + beta p_old (MODE 2) staged for the patch's local
-// vertices, y = A p_new, p_new written for the owned rows and <y, p_new>
-// summed per workgroup into partial[p]. The pattern is the patch-local VV
-// plan (the system's pattern; col is unused).
-template <uint32_t T, int MODE>
+// component stride of the solver's vectors: whole 256-byte lines
+__host__ __device__ inline size_t cg_stride(uint32_t n) { return (size_t(n) + 63u) & ~size_t(63); }
+
+// Sum over the wave, in lane 63: rows of 16 lanes by DPP shifts, then the row
+// totals broadcast upwards (a fixed order; no LDS round trip per step).
+__device__ __forceinline__ double wave_sum63(double v)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        const uint64_t u = __double_as_longlong(v);
+        const uint32_t lo = __builtin_amdgcn_update_dpp(0u, uint32_t(u), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        const uint32_t hi = __builtin_amdgcn_update_dpp(0u, uint32_t(u >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        v += __longlong_as_double(static_cast<long long>((uint64_t(hi) << 32) | lo));
+    };
+    using r1 = std::integral_constant<int, 0x111>;  // row_shr 1, 2, 4, 8
+    using r2 = std::integral_constant<int, 0x112>;
+    using r4 = std::integral_constant<int, 0x114>;
+    using r8 = std::integral_constant<int, 0x118>;
+    using b15 = std::integral_constant<int, 0x142>;  // row_bcast 15, 31
+    using b31 = std::integral_constant<int, 0x143>;
+    using all = std::integral_constant<int, 0xf>;
+    step(r1{}, all{});
+    step(r2{}, all{});
+    step(r4{}, all{});
+    step(r8{}, all{});
+    step(b15{}, std::integral_constant<int, 0xa>{});
+    step(b31{}, std::integral_constant<int, 0xc>{});
+    return v;
+}
+
+// Sum over the workgroup, the same value in every thread: wave sums, then the
+// wave totals in order. red: T / 64 doubles, used once per kernel.
+template <uint32_t T>
+__device__ __forceinline__ double block_sum(double v, double* red)
+{
+    v = wave_sum63(v);
+    if ((threadIdx.x & 63u) == 63u) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (uint32_t i = 0; i < T / 64u; ++i) t += red[i];
+    return t;
+}
+
+// States are read and written field by field: a struct copied whole under a
+// branch became a private array, which the compiler placed in LDS with the
+// workgroup size read from the dispatch packet in host memory by every
+// workgroup (the update took 17-20 us instead of 8).
+__device__ __forceinline__ CgState cg_load(const CgState* __restrict__ q)
+{
+    CgState s;
+    s.delta = q->delta;
+    s.alpha = q->alpha;
+    s.beta  = q->beta;
+    s.start = q->start;
+    s.iters = q->iters;
+    s.done  = q->done;
+    return s;
+}
+__device__ __forceinline__ void cg_store(CgState* __restrict__ q, const CgState& s)
+{
+    q->delta = s.delta;
+    q->alpha = s.alpha;
+    q->beta  = s.beta;
+    q->start = s.start;
+    q->iters = s.iters;
+    q->done  = s.done;
+}
+
+// Scalar step on sum = <r, r> (<r, r / diag> with the preconditioner) after the
+// set-up (FIRST) or an update: stop when it is below abs_tol or, relative to
+// the start, below rel_tol; else beta = delta / delta_old and one more
+// iteration taken.
+template <bool FIRST>
+__device__ __forceinline__ CgState cg_next(CgState s, double total, float abs_tol, float rel_tol)
+{
+    const float sum = static_cast<float>(total);
+    if constexpr (FIRST) {
+        s.start = sum;
+        s.iters = 0;
+        s.alpha = s.beta = 0.f;
+        s.done = (sum < abs_tol || sum / sum < rel_tol) ? 1u : 0u;
+    } else if (sum < abs_tol || sum / s.start < rel_tol) {
+        s.done = 1u;
+    } else {
+        s.beta = sum / s.delta;
+        s.iters += 1u;
+        s.done = 0u;
+    }
+    s.delta = sum;
+    return s;
+}
+
+// LDS carve of the product: the plan rows and direction (plan_sl), the values
+// (none with uniform weights) and the wave totals.
+struct PlanCG
+{
+    PlanSL  sl;
+    float*  w;
+    double* red;
+};
+__host__ __device__ inline PlanCG plan_cg(Bump& b, uint32_t nv, uint32_t nvo, uint32_t nent, bool uniform,
+                                          uint32_t threads)
+{
+    PlanCG p{};
+    p.sl  = plan_sl(b, nv, nvo, nent, false);
+    p.w   = uniform ? nullptr : b.alloc<float>(nent + nvo + 3u);
+    p.red = b.alloc<double>(threads / 64u);
+    return p;
+}
+
+// MODE 0 (set-up): y = A x, x the caller's start vector (component stride nV).
+// MODE 1 (first iteration) / 2: p = z, or z + beta p_old, z = r, or r / diag
+// with the Jacobi preconditioner (PRE, the reference's precond_matvec,
+// mcf_kernels.cuh:219-299); p written for the owned rows, y = A p, <y, p>
+// into partial[patch], and (MODE 2) sol += alpha p_old of the iteration
+// before. UNI: uniform weights (off-diagonals -dt, diagonal valence + the
+// row's dt), val unread. The pattern is the patch-local VV plan.
+template <uint32_t T, int MODE, bool PRE, bool UNI>
 __global__ __launch_bounds__(T) void k_cg_apply(DevMesh m, const uint32_t* __restrict__ vv_base,
                                                 const uint32_t* __restrict__ rbase,
                                                 const uint32_t* __restrict__ nbase,
                                                 const uint16_t* __restrict__ roff, const uint16_t* __restrict__ nbr,
-                                                const float* __restrict__ val, const float* __restrict__ x,
-                                                const float* __restrict__ r, float* __restrict__ p_new,
+                                                const float* __restrict__ val, float dt, const float* __restrict__ x,
+                                                const float* __restrict__ r, const float* __restrict__ diag,
+                                                float* __restrict__ sol, float* __restrict__ p_new,
                                                 float* __restrict__ y, float* __restrict__ partial,
-                                                const CgState* __restrict__ st)
+                                                const double* __restrict__ part_in, uint32_t nin,
+                                                const CgState* __restrict__ upd, CgState* __restrict__ app,
+                                                float abs_tol, float rel_tol)
 {
     extern __shared__ uint4 smem[];
     const uint32_t p = patch_of_block(m.P);  // XCD-contiguous patch ranges
     if (p >= m.P) return;
-    if (MODE != 0 && st->done) return;
-    const PatchDesc d   = load_desc(m.patch, p);
+    CgState         st{};
+    const PatchDesc d = load_desc(m.patch, p);
     // true VV entry count (nbase runs are padded to 8; the system's run is not)
-    const uint32_t  rb  = rbase[p], nbb = nbase[p], nent = vv_base[p + 1] - vv_base[p];
-    const uint32_t  bse = vv_base[p] + d.vp;
-    const uint32_t  N   = m.nV;
-    Bump            b(reinterpret_cast<char*>(smem));
-    const PlanSL    L = plan_sl(b, d.nv, d.nvo, nent, false);
-    float*          w = b.alloc<float>(nent + d.nvo);
-    float*          red = b.alloc<float>(T / 64u);
-    stage_u16x8<T>(L.ro, roff + rb, d.nvo + 1);
-    stage_u16x8<T>(L.nb, nbr + nbb, nent);
-    stage_words<T, 8>(reinterpret_cast<uint32_t*>(w), reinterpret_cast<const uint32_t*>(val) + bse, nent + d.nvo);
-    if constexpr (MODE == 0) {
-        stage_positions_batched<T, 512u / T, false>(L.x, L.y, L.z, nullptr, x, N, d, m.v_lin);
-    } else {
-        // x holds p_old here (unread in the first iteration)
-        const float     beta = MODE == 2 ? st->beta : 0.f;
-        const uint32_t* vl   = m.v_lin + d.v_off;
-        for (uint32_t l = threadIdx.x; l < d.nv; l += T) {
-            const uint32_t g = lin_of(l, d.nvo, d.vp, vl);
-            if constexpr (MODE == 1) {
-                L.x[l] = r[g];
-                L.y[l] = r[N + g];
-                L.z[l] = r[2 * N + g];
-            } else {
-                L.x[l] = r[g] + beta * x[g];
-                L.y[l] = r[N + g] + beta * x[N + g];
-                L.z[l] = r[2 * N + g] + beta * x[2 * N + g];
+    const uint32_t rb = rbase[p], nbb = nbase[p], vb = vv_base[p], nent = vv_base[p + 1] - vb;
+    if constexpr (MODE == 2) st = cg_load(upd);
+    if (MODE == 2 && st.done) return;
+    const size_t   N = m.nV, S = cg_stride(m.nV);
+    Bump           b(reinterpret_cast<char*>(smem));
+    const PlanCG   L  = plan_cg(b, d.nv, d.nvo, nent, UNI, T);
+    const uint32_t  t = threadIdx.x, nvo = d.nvo, nr = d.nv - nvo;  // nr: ribbon vertices
+    const uint32_t* vl   = m.v_lin + d.v_off;
+    const float*    vsrc = UNI ? nullptr : val + vb + d.vp;
+    // first round trip: ribbon ids, plan rows, values, partials and the owned
+    // vertices' words; second: the ribbon's words. Clamped indices read a
+    // valid element whose value is not used.
+    constexpr uint32_t         RO = (512u + T - 1u) / T;
+    HeldFloats<T, UNI ? 1 : 2> hw;
+    Held<T, 1, u32x4>          hro, hnb;
+    const uint32_t             nro = (nvo + 1u + 7u) >> 3, nnb = (nent + 7u) >> 3;
+    const u32x4 *ros = reinterpret_cast<const u32x4*>(roff + rb), *nbs = reinterpret_cast<const u32x4*>(nbr + nbb);
+    const uint32_t gr = vl[min(nvo + t, d.nv - 1u)];
+    hro.load(ros, nro);
+    hnb.load(nbs, nnb);
+    if constexpr (!UNI) hw.load(vsrc, nent + nvo);
+    double acc0 = 0.0, acc1 = 0.0;
+    if constexpr (MODE != 0) {
+        static_assert(2 * T >= kCgUpdateGroups, "two rounds hold every partial");
+        acc0 = part_in[min(t, nin - 1u)];
+        acc1 = part_in[min(t + T, nin - 1u)];
+    }
+    float a[RO][3], po[RO][3], xs[RO][3], dg[RO];
+#pragma unroll
+    for (uint32_t k = 0; k < RO; ++k) {
+        if (k * T >= nvo && k) continue;
+        const size_t gg = min(d.vp + t + k * T, m.nV - 1u);
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            a[k][c] = (MODE == 0) ? x[c * N + gg] : r[c * S + gg];
+            if constexpr (MODE == 2) {
+                po[k][c] = x[c * S + gg];  // x holds p_old
+                xs[k][c] = sol[c * N + gg];
             }
         }
+        if constexpr (MODE != 0 && PRE) dg[k] = diag[gg];
     }
+    float ar[3], pr[3], dr = 1.f;
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+        ar[c] = (MODE == 0) ? x[c * N + gr] : r[c * S + gr];
+        if constexpr (MODE == 2) pr[c] = x[c * S + gr];
+    }
+    if constexpr (MODE != 0 && PRE) dr = diag[gr];
+    hro.store(reinterpret_cast<u32x4*>(L.sl.ro), ros, nro);
+    hnb.store(reinterpret_cast<u32x4*>(L.sl.nb), nbs, nnb);
+    uint32_t mis = 0;
+    if constexpr (!UNI) {
+        hw.store(L.w, vsrc, nent + nvo);
+        mis = hw.shift(vsrc);
+    }
+    if constexpr (MODE != 0) {
+        const double acc = (t < nin ? acc0 : 0.0) + (t + T < nin ? acc1 : 0.0);
+        st = cg_next<MODE == 1>(st, block_sum<T>(acc, L.red), abs_tol, rel_tol);
+        if (p == 0 && t == 0) cg_store(app, st);
+    }
+    // direction of a vertex from its words into LDS
+    const float alpha = st.alpha, beta = st.beta;
+    auto        put   = [&](uint32_t l, const float (&av)[3], const float (&pv)[3], float dv) {
+        float* const o[3] = {L.sl.x, L.sl.y, L.sl.z};
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            const float z = (MODE != 0 && PRE) ? av[c] / dv : av[c];
+            o[c][l]       = (MODE == 2) ? z + beta * pv[c] : z;
+        }
+    };
+    auto finish = [&](size_t gg, const float (&pv)[3], const float (&xv)[3]) {  // the last iteration's step of x
+        if constexpr (MODE == 2)
+#pragma unroll
+            for (uint32_t c = 0; c < 3; ++c) sol[c * N + gg] = xv[c] + alpha * pv[c];
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < RO; ++k)
+        if (t + k * T < nvo) {
+            finish(d.vp + t + k * T, po[k], xs[k]);
+            put(t + k * T, a[k], po[k], dg[k]);
+        }
+    if (t < nr) put(nvo + t, ar, pr, dr);
+    auto direct = [&](uint32_t l, size_t gg, bool owned) {  // vertices beyond the register rounds
+        float av[3], pv[3] = {}, xv[3] = {};
+        for (uint32_t c = 0; c < 3; ++c) {
+            av[c] = (MODE == 0) ? x[c * N + gg] : r[c * S + gg];
+            if constexpr (MODE == 2) {
+                pv[c] = x[c * S + gg];
+                if (owned) xv[c] = sol[c * N + gg];
+            }
+        }
+        if (owned) finish(gg, pv, xv);
+        put(l, av, pv, (MODE != 0 && PRE) ? diag[gg] : 1.f);
+    };
+    for (uint32_t l = t + RO * T; l < nvo; l += T) direct(l, d.vp + l, true);
+    for (uint32_t l = nvo + t + T; l < d.nv; l += T) direct(l, vl[l], false);
+    if (MODE != 0 && st.done) return;  // converged: x is complete (the same decision in every workgroup)
     __syncthreads();
     float dotp = 0.f;
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
-        const uint32_t k0 = L.ro[v], k1 = L.ro[v + 1];
-        const float*   wr = w + k0 + v;  // diagonal, then the row's neighbours
-        const float    px = L.x[v], py = L.y[v], pz = L.z[v];
-        float          ax = wr[0] * px, ay = wr[0] * py, az = wr[0] * pz;
-        for (uint32_t k = k0; k < k1; ++k) {
-            const uint32_t q = L.nb[k];
-            const float    c = wr[1 + k - k0];
-            ax += c * L.x[q];
-            ay += c * L.y[q];
-            az += c * L.z[q];
+    for (uint32_t v = t; v < d.nvo; v += T) {
+        const uint32_t k0 = L.sl.ro[v], k1 = L.sl.ro[v + 1];
+        const float*   wr = L.w + mis + k0 + v;  // diagonal, then the row's neighbours
+        const float    px = L.sl.x[v], py = L.sl.y[v], pz = L.sl.z[v];
+        float          w0;
+        if constexpr (UNI) {
+            float sum_w = 0.f;
+            for (uint32_t k = k0; k < k1; ++k) sum_w += dt;
+            w0 = static_cast<float>(k1 - k0) + sum_w;
+        } else {
+            w0 = wr[0];
         }
-        const uint32_t g = d.vp + v;
-        y[g]             = ax;
-        y[N + g]         = ay;
-        y[2 * N + g]     = az;
+        float ax = w0 * px, ay = w0 * py, az = w0 * pz;
+        for (uint32_t k = k0; k < k1; ++k) {
+            const uint32_t q = L.sl.nb[k];
+            const float    c = UNI ? -dt : wr[1 + k - k0];
+            ax += c * L.sl.x[q];
+            ay += c * L.sl.y[q];
+            az += c * L.sl.z[q];
+        }
+        const size_t gg = d.vp + v;
+        y[gg]           = ax;
+        y[S + gg]       = ay;
+        y[2 * S + gg]   = az;
         if constexpr (MODE != 0) {
-            p_new[g]         = px;
-            p_new[N + g]     = py;
-            p_new[2 * N + g] = pz;
+            p_new[gg]         = px;
+            p_new[S + gg]     = py;
+            p_new[2 * S + gg] = pz;
             dotp += ax * px + ay * py + az * pz;
         }
     }
     if constexpr (MODE != 0) {
         // fixed-order workgroup sum: wave shuffles, then wave totals in order
+        // (every thread has read the first sum's totals: a barrier lies between)
+        float* red = reinterpret_cast<float*>(L.red);
         for (uint32_t o = 32; o > 0; o >>= 1) dotp += __shfl_xor(dotp, o, 64);
-        if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = dotp;
+        if ((t & 63u) == 0) red[t >> 6] = dotp;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            float t = 0.f;
-            for (uint32_t i = 0; i < T / 64u; ++i) t += red[i];
-            partial[p] = t;
+        if (t == 0) {
+            float s = 0.f;
+            for (uint32_t i = 0; i < T / 64u; ++i) s += red[i];
+            partial[p] = s;
         }
     }
 }
 
-// ---- matrix-free implicit MCF product -----------------------------------------
-// LDS carve of the matrix-free product: the assembly's carve (positions and
-// half-edge terms only for cotangent weights) plus the staged input vector.
-struct PlanMF
+// Set-up of the matrix-free solve with uniform weights: mass = valence (the
+// reference's init_B scale) and, for the preconditioner, the diagonal the
+// product uses.
+__global__ __launch_bounds__(256) void k_uniform_diag(DevMesh m, const uint32_t* __restrict__ rbase,
+                                                      const uint16_t* __restrict__ roff, float dt,
+                                                      float* __restrict__ mass, float* __restrict__ diag)
 {
-    float4*   pos;
-    float4*   he;
-    uint32_t *lin, *ev, *rs;
-    uint16_t* ent;
-    float *   vx, *vy, *vz, *red;
-};
-__host__ __device__ inline PlanMF plan_mf(Bump& b, uint32_t nv, uint32_t ne, uint32_t nvo, uint32_t nent,
-                                          bool uniform, uint32_t threads)
-{
-    PlanMF p{};
-    if (!uniform) {
-        p.pos = b.alloc<float4>(nv);
-        p.he  = b.alloc<float4>(ne);
-        p.lin = b.alloc<uint32_t>(nv);
-    }
-    p.ev  = b.alloc<uint32_t>(r4(ne));
-    p.rs  = b.alloc<uint32_t>(nvo + 1);
-    p.ent = b.alloc<uint16_t>(nent);
-    p.vx  = b.alloc<float>(nv);
-    p.vy  = b.alloc<float>(nv);
-    p.vz  = b.alloc<float>(nv);
-    p.red = b.alloc<float>(threads / 64u);
-    return p;
-}
-
-// y = A v for the implicit MCF system A = M + dt L with the weights
-// recomputed from the fixed coordinates in every product (the reference's
-// matvec, apps/MCF/mcf_kernels.cuh:114-213): per owned row, in the order of
-// the reference's ring loop, acc -= (dt w_e) v[r_e] over the row's edges,
-// then y = acc + diag v[p] with diag = 1 / v_weight + sum_e dt w_e.
-// Cotangent weights (UNIFORM false): w_e = max(0, cot + cot) of the edge and
-// v_weight = 0.5 / (the vertex's Voronoi area), from one evaluation of every
-// face of the patch (the terms k_cot_assemble computes); every vertex ring
-// must be one closed fan (checked on the host). Uniform weights: w_e = 1,
-// v_weight = 1 / valence, no orientation needed.
-// MODE 0 (set-up): v = x; also writes mass[g] = 1 / v_weight (the
-// reference's init_B scale: valence for uniform weights) and, if diag is not
-// null, diag[g] for the preconditioner. MODE 1 / 2 (CG iteration): v = the
-// new direction p = z (MODE 1) or z + beta p_old (MODE 2), z = r, or r / diag
-// (Jacobi, the reference's precond_matvec, :219-299) when PRECOND; p is
-// written for the owned rows and <y, p> summed per workgroup into partial[p].
-template <uint32_t T, int MODE, bool UNIFORM, bool PRECOND>
-__global__ __launch_bounds__(T) void k_mf_apply(DevMesh m, const uint32_t* __restrict__ vv_base,
-                                                const uint32_t* __restrict__ rs, const uint16_t* __restrict__ ent,
-                                                const float* __restrict__ coords, float dt,
-                                                const float* __restrict__ x, const float* __restrict__ r,
-                                                float* __restrict__ diag, float* __restrict__ mass,
-                                                float* __restrict__ p_new, float* __restrict__ y,
-                                                float* __restrict__ partial, const CgState* __restrict__ st)
-{
-    extern __shared__ uint4 smem[];
-    const uint32_t p = patch_of_block(m.P);  // XCD-contiguous patch ranges
-    if (p >= m.P) return;
-    if (MODE != 0 && st->done) return;
-    const PatchDesc d  = load_desc(m.patch, p);
-    const uint32_t  vb = vv_base[p], nent = vv_base[p + 1] - vb;
-    const uint32_t  N  = m.nV;
-    Bump            b(reinterpret_cast<char*>(smem));
-    const PlanMF    L = plan_mf(b, d.nv, d.ne, d.nvo, nent, UNIFORM, T);
-    stage_u32(L.ev, m.ev + d.e_off, d.ne);
-    stage_halves<T, 8>(L.ent, ent + vb, nent);
-    stage_words<T, 2>(L.rs, rs + d.vp, d.nvo + 1, vb);
-    if constexpr (!UNIFORM) {
-        stage_vertices<T>(m, d, coords, L.pos, L.lin);
-        for (uint32_t i = threadIdx.x; i < d.ne; i += T) L.he[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    {
-        const uint32_t* vl   = m.v_lin + d.v_off;
-        const float     beta = MODE == 2 ? st->beta : 0.f;
-        for (uint32_t l = threadIdx.x; l < d.nv; l += T) {
-            const uint32_t g = lin_of(l, d.nvo, d.vp, vl);
-            float          a[3];
-#pragma unroll
-            for (uint32_t c = 0; c < 3; ++c) {
-                if constexpr (MODE == 0) {
-                    a[c] = x[c * N + g];
-                } else {
-                    const float z = PRECOND ? r[c * N + g] / diag[g] : r[c * N + g];
-                    a[c]          = (MODE == 2) ? z + beta * x[c * N + g] : z;  // x holds p_old
-                }
-            }
-            L.vx[l] = a[0];
-            L.vy[l] = a[1];
-            L.vz[l] = a[2];
-        }
-    }
-    __syncthreads();
-    if constexpr (!UNIFORM) {
-        const uint16_t* fe = m.fe + 3u * d.f_off;
-        float2*         hh = reinterpret_cast<float2*>(L.he);  // hh[2e + dir]
-        for (uint32_t f = threadIdx.x; f < d.nf; f += T) {
-            uint32_t xs[3], a[3];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) xs[j] = fe[3 * f + j];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const uint32_t e = L.ev[xs[j] >> 1];
-                a[j]             = (xs[j] & 1u) ? hi16(e) : lo16(e);
-            }
-            const float4  q0 = L.pos[a[0]], q1 = L.pos[a[1]], q2 = L.pos[a[2]];
-            const FaceCot c  = face_cot(f3{q0.x, q0.y, q0.z}, f3{q1.x, q1.y, q1.z}, f3{q2.x, q2.y, q2.z});
-#pragma unroll
-            for (int j = 0; j < 3; ++j) hh[xs[j]] = make_float2(c.cot[(j + 2) % 3], c.vor[j]);
-        }
-        __syncthreads();
-    }
-    float dotp = 0.f;
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
-        const uint32_t k0 = L.rs[v], k1 = L.rs[v + 1];
-        float          sum_w = 0.f, vw = 0.f, ax = 0.f, ay = 0.f, az = 0.f;
-        for (uint32_t k = k0; k < k1; ++k) {
-            const uint32_t e = L.ent[k] >> 1, xe = L.ev[e];
-            const uint32_t q = (lo16(xe) == v) ? hi16(xe) : lo16(xe);
-            float          w = 1.f;
-            if constexpr (!UNIFORM) {
-                const float4 h = L.he[e];
-                w              = h.x + h.z;
-                w              = (w >= 0.f) ? w : 0.f;
-                vw += (lo16(xe) == v) ? h.y : h.w;
-            }
-            const float wd = w * dt;
-            sum_w += wd;
-            ax -= wd * L.vx[q];
-            ay -= wd * L.vy[q];
-            az -= wd * L.vz[q];
-        }
-        const float vwt = UNIFORM ? 1.0f / static_cast<float>(k1 - k0) : 0.5f / vw;
-        const float dg  = 1.0f / vwt + sum_w;
-        const float px = L.vx[v], py = L.vy[v], pz = L.vz[v];
-        ax += dg * px;
-        ay += dg * py;
-        az += dg * pz;
-        const uint32_t g = d.vp + v;
-        y[g]             = ax;
-        y[N + g]         = ay;
-        y[2 * N + g]     = az;
-        if constexpr (MODE == 0) {
-            // the reference's init_B: x * valence (uniform) or x / v_weight
-            mass[g] = UNIFORM ? static_cast<float>(k1 - k0) : 1.0f / vwt;
-            if (diag) diag[g] = dg;
-        } else {
-            p_new[g]         = px;
-            p_new[N + g]     = py;
-            p_new[2 * N + g] = pz;
-            dotp += ax * px + ay * py + az * pz;
-        }
-    }
-    if constexpr (MODE != 0) {
-        for (uint32_t o = 32; o > 0; o >>= 1) dotp += __shfl_xor(dotp, o, 64);
-        if ((threadIdx.x & 63u) == 0) L.red[threadIdx.x >> 6] = dotp;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            float t = 0.f;
-            for (uint32_t i = 0; i < T / 64u; ++i) t += L.red[i];
-            partial[p] = t;
-        }
+    const uint32_t  p = blockIdx.x;
+    const PatchDesc d = load_desc(m.patch, p);
+    const uint16_t* ro = roff + rbase[p];
+    for (uint32_t v = threadIdx.x; v < d.nvo; v += 256u) {
+        const uint32_t k = ro[v + 1] - ro[v];
+        float          sum_w = 0.f;
+        for (uint32_t i = 0; i < k; ++i) sum_w += dt;
+        mass[d.vp + v] = static_cast<float>(k);
+        diag[d.vp + v] = static_cast<float>(k) + sum_w;
     }
 }
 
-// Per linear vertex (MODE 0, set-up): r = b - s with b = mass * x0, and the
-// workgroup's partial <r, r> (<r, r / diag> with the Jacobi preconditioner,
-// diag non-null). MODE 1 (iteration): x += alpha p, r -= alpha s and the
-// partial <r, r> (<r, r / diag>).
+// MODE 0 (set-up): r = b - s with b = mass * x0, x = x0 and the workgroup's
+// partial <r, r> (<r, r / diag> with the Jacobi preconditioner, diag
+// non-null). MODE 1 (iteration): alpha = delta / <s, p> from the product's
+// npart partials, r -= alpha s, partial <r, r>. r and s are the solver's own
+// (stride cg_stride, 16-byte quads); the pad past n is masked out.
 template <int MODE>
-__global__ __launch_bounds__(256) void k_cg_update(uint32_t n, const float* __restrict__ mass,
-                                                   const float* __restrict__ x0, float* __restrict__ x,
-                                                   float* __restrict__ r, const float* __restrict__ pvec,
-                                                   const float* __restrict__ s, float* __restrict__ partial,
-                                                   const CgState* __restrict__ st,
-                                                   const float* __restrict__ diag = nullptr)
+__global__ __launch_bounds__(kCgUpdateThreads) void k_cg_update(uint32_t n, const float* __restrict__ mass,
+                                                                const float* __restrict__ x0, float* __restrict__ x,
+                                                                float* __restrict__ r, const float* __restrict__ s,
+                                                                const float* __restrict__ diag,
+                                                                const float* __restrict__ part_in, uint32_t npart,
+                                                                double* __restrict__ partial,
+                                                                const CgState* __restrict__ app,
+                                                                CgState* __restrict__ upd)
 {
-    __shared__ float red[4];
-    if (MODE == 1 && st->done) return;
-    const uint32_t i   = blockIdx.x * 256u + threadIdx.x;
-    float          acc = 0.f;
-    if (i < n) {
-        if constexpr (MODE == 0) {
-            // b = M x0 rounded on its own (the reference stores B, then forms
-            // B - A x): no fused multiply-subtract here
+    constexpr uint32_t T = kCgUpdateThreads;
+    __shared__ double  red[2][T / 64u];
+    const size_t       S  = cg_stride(n);
+    const uint32_t     t0 = blockIdx.x * T + threadIdx.x, step = gridDim.x * T;
+    double             acc = 0.0;
+    if constexpr (MODE == 0) {
+        // b = M x0 rounded on its own (the reference stores B, then forms
+        // B - A x): no fused multiply-subtract here
 #pragma clang fp contract(off)
-            const float M = mass[i];
-            const float D = diag ? diag[i] : 1.f;
+        for (uint32_t i = t0; i < n; i += step) {
+            const float M = mass[i], D = diag ? diag[i] : 1.f;
 #pragma unroll
             for (uint32_t c = 0; c < 3; ++c) {
-                const float v = M * x0[c * n + i] - s[c * n + i];
-                r[c * n + i]  = v;
-                x[c * n + i]  = x0[c * n + i];
-                acc += diag ? v * (v / D) : v * v;
-            }
-        } else {
-            const float a = st->alpha;
-            const float D = diag ? diag[i] : 1.f;
-#pragma unroll
-            for (uint32_t c = 0; c < 3; ++c) {
-                x[c * n + i] += a * pvec[c * n + i];
-                const float v = r[c * n + i] - a * s[c * n + i];
-                r[c * n + i]  = v;
-                acc += diag ? v * (v / D) : v * v;
+                const float x0v = x0[c * size_t(n) + i];
+                const float v   = M * x0v - s[c * S + i];
+                r[c * S + i]    = v;
+                x[c * size_t(n) + i] = x0v;
+                acc += static_cast<double>(diag ? v * (v / D) : v * v);
             }
         }
+    } else {
+        CgState st = cg_load(app);
+        if (st.done) {  // the product has finished x; pass the decision on
+            if (blockIdx.x == 0 && threadIdx.x == 0) cg_store(upd, st);
+            return;
+        }
+        const uint32_t nq = static_cast<uint32_t>(S >> 2);  // quads per component
+        float4*        r4 = reinterpret_cast<float4*>(r);
+        const float4*  s4 = reinterpret_cast<const float4*>(s);
+        // the first quad's loads go out before the partials are summed
+        uint32_t     q  = t0;
+        const bool   on = q < 3u * nq;
+        float4       rv = on ? r4[q] : float4{}, sv = on ? s4[q] : float4{};
+        double       sp = 0.0;
+        for (uint32_t i = threadIdx.x; i < npart; i += T) sp += static_cast<double>(part_in[i]);
+        sp       = block_sum<T>(sp, red[0]);
+        st.alpha = st.delta / static_cast<float>(sp);
+        if (t0 == 0) cg_store(upd, st);
+        const float alpha = st.alpha;
+        while (q < 3u * nq) {
+            const uint32_t qn = q + step;
+            float4         rn{}, sn{};
+            if (qn < 3u * nq) {
+                rn = r4[qn];
+                sn = s4[qn];
+            }
+            const uint32_t c = (q >= nq ? 1u : 0u) + (q >= 2u * nq ? 1u : 0u), i = 4u * (q - c * nq);
+            float          v[4] = {rv.x - alpha * sv.x, rv.y - alpha * sv.y, rv.z - alpha * sv.z, rv.w - alpha * sv.w};
+            r4[q]               = make_float4(v[0], v[1], v[2], v[3]);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if (i + j < n) acc += static_cast<double>(diag ? v[j] * (v[j] / diag[i + j]) : v[j] * v[j]);
+            q  = qn;
+            rv = rn;
+            sv = sn;
+        }
     }
-    for (uint32_t o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+    acc = block_sum<T>(acc, red[1]);
+    if (threadIdx.x == 0) partial[blockIdx.x] = acc;
 }
 
-// One workgroup: fixed-order sum of the partials, then the scalar step.
-//   STEP 0 (set-up): delta = start = sum; done if already converged.
-//   STEP 1 (after the SpMV): alpha = delta / sum.
-//   STEP 2 (after the update): delta_old = delta, delta = sum; done when
-//          delta < abs_tol or delta / start < rel_tol, else beta =
-//          delta / delta_old and one more iteration taken.
-template <int STEP>
-__global__ __launch_bounds__(1024) void k_cg_scalar(uint32_t n, const float* __restrict__ partial,
-                                                    CgState* __restrict__ st, float abs_tol, float rel_tol)
+// After the last iteration (FIRST: none was asked for): the scalar step on the
+// update's partials and, unless an earlier product found the solve converged,
+// x += alpha p.
+template <bool FIRST>
+__global__ __launch_bounds__(256) void k_cg_finish(uint32_t n, const double* __restrict__ part_in, uint32_t nin,
+                                                   const float* __restrict__ pvec, float* __restrict__ x,
+                                                   const CgState* __restrict__ upd, CgState* __restrict__ app,
+                                                   float abs_tol, float rel_tol)
 {
-    __shared__ double s[1024];
-    if (STEP != 0 && st->done) return;
-    double acc = 0.0;
-    for (uint32_t i = threadIdx.x; i < n; i += 1024) acc += static_cast<double>(partial[i]);
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (uint32_t k = 512; k > 0; k >>= 1) {
-        if (threadIdx.x < k) s[threadIdx.x] += s[threadIdx.x + k];
-        __syncthreads();
+    __shared__ double red[4];
+    CgState           st{};
+    if constexpr (!FIRST) st = cg_load(upd);
+    if (!FIRST && st.done) return;
+    if (blockIdx.x == 0) {
+        double acc = 0.0;
+        for (uint32_t i = threadIdx.x; i < nin; i += 256u) acc += part_in[i];
+        const CgState e = cg_next<FIRST>(st, block_sum<256>(acc, red), abs_tol, rel_tol);
+        if (threadIdx.x == 0) cg_store(app, e);
     }
-    if (threadIdx.x != 0) return;
-    const float sum = static_cast<float>(s[0]);
-    if constexpr (STEP == 0) {
-        st->delta = st->start = sum;
-        st->delta_old = 0.f;
-        st->alpha = st->beta = 0.f;
-        st->iters = 0;
-        st->done  = (sum < abs_tol || sum / sum < rel_tol) ? 1u : 0u;
-    } else if constexpr (STEP == 1) {
-        st->alpha = st->delta / sum;
-    } else {
-        st->delta_old = st->delta;
-        st->delta     = sum;
-        if (sum < abs_tol || sum / st->start < rel_tol) {
-            st->done = 1u;
-        } else {
-            st->beta = sum / st->delta_old;
-            st->iters += 1u;
-        }
+    if constexpr (!FIRST) {
+        const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+        const size_t   S = cg_stride(n);
+        if (i < n)
+#pragma unroll
+            for (uint32_t c = 0; c < 3; ++c) x[c * size_t(n) + i] += st.alpha * pvec[c * S + i];
     }
 }
 

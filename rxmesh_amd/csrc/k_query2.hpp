@@ -175,6 +175,23 @@ __global__ __launch_bounds__(T) void k_query2_vx(DevMesh m, const uint32_t* __re
 // local neighbour ids at nbr + nbase[p], rows in ascending local-edge order.
 // This is the query engine's native (RXMesh-style) encoding of the relation;
 // iterative kernels consume it with half the index bytes of an int32 CSR.
+// Slots are u16, EV's index of the row's other endpoint (2 e + 1 - end: sorts
+// like e, and needs ne <= 2^15, beyond which EV alone fills a CU's LDS).
+struct PlanVVL
+{
+    uint32_t *ev, *off, *wave;
+    uint16_t* slots;
+};
+__host__ __device__ inline PlanVVL plan_vvl(Bump& b, uint32_t ne, uint32_t nvo)
+{
+    PlanVVL p{};
+    p.ev    = b.alloc<uint32_t>(r4(ne));
+    p.off   = b.alloc<uint32_t>(nvo + 1);
+    p.wave  = b.alloc<uint32_t>(20);
+    p.slots = b.alloc<uint16_t>(2 * ne);
+    return p;
+}
+
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_query2_vv_local(DevMesh m, const uint32_t* __restrict__ rbase,
                                                        const uint32_t* __restrict__ nbase,
@@ -184,27 +201,20 @@ __global__ __launch_bounds__(T) void k_query2_vv_local(DevMesh m, const uint32_t
     const uint32_t  p = blockIdx.x;
     const PatchDesc d = load_desc(m.patch, p);
     Bump            b(reinterpret_cast<char*>(smem));
-    const PlanQ2    L = plan_q2(b, 0, d.nv, d.ne, d.nf);
+    const PlanVVL   L = plan_vvl(b, d.ne, d.nvo);
     stage_u32(L.ev, m.ev + d.e_off, d.ne);
     for (uint32_t c = threadIdx.x; c <= d.nvo; c += T) L.off[c] = 0;
     __syncthreads();
+    const uint16_t* ev16 = reinterpret_cast<const uint16_t*>(L.ev);
     fill_columns<T, true>(
-        2 * d.ne, d.nvo,
-        [&](uint32_t i) {
-            const uint32_t x = L.ev[i >> 1];
-            return (i & 1u) ? hi16(x) : lo16(x);
-        },
-        [&](uint32_t i) {
-            const uint32_t x = L.ev[i >> 1];
-            return ((i >> 1) << 16) | ((i & 1u) ? lo16(x) : hi16(x));
-        },
+        2 * d.ne, d.nvo, [&](uint32_t i) { return static_cast<uint32_t>(ev16[i]); }, [&](uint32_t i) { return i ^ 1u; },
         L.off, L.slots, L.wave);
     uint16_t* ro = roff + rbase[p];
     uint16_t* nb = nbr + nbase[p];
     for (uint32_t v = threadIdx.x; v <= d.nvo; v += T) ro[v] = static_cast<uint16_t>(L.off[v]);
     for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
         const uint32_t o = L.off[v], k = L.off[v + 1] - o;
-        sort_row(L.slots + o, k, [&](uint32_t j, uint32_t s) { nb[o + j] = static_cast<uint16_t>(lo16(s)); });
+        sort_row(L.slots + o, k, [&](uint32_t j, uint32_t s) { nb[o + j] = ev16[s]; });
     }
 }
 

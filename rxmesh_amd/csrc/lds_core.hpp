@@ -69,6 +69,85 @@ __device__ __forceinline__ void stage_u32(uint32_t* __restrict__ dst, const uint
     stage_vec2(reinterpret_cast<uint4*>(dst), reinterpret_cast<const uint4*>(src), (n + 3u) >> 2);
 }
 
+// 16-byte words held in registers between a load and an LDS store (vector
+// types: arrays of the float4 / uint4 classes went to scratch)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float    f32x4 __attribute__((ext_vector_type(4)));
+
+// Copies of n elements global -> LDS in two halves, so that a workgroup can
+// issue the loads of several arrays before it waits for any of them. A load
+// under a per-lane branch makes the compiler wait for it at the branch's end,
+// one memory round trip per array; here every lane loads, from an address
+// clamped to the last element, and only whole rounds are skipped, by a
+// uniform branch. T threads, R rounds in registers; store() copies what larger
+// patches have beyond them.
+template <uint32_t T, uint32_t R, typename V>
+struct Held
+{
+    V                          a[R];
+    __device__ __forceinline__ void load(const V* __restrict__ s, uint32_t n)
+    {
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r)
+            if (r * T < n) a[r] = s[min(threadIdx.x + r * T, n - 1u)];
+    }
+    __device__ __forceinline__ void store(V* __restrict__ d, const V* __restrict__ s, uint32_t n) const
+    {
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r)
+            if (threadIdx.x + r * T < n) d[threadIdx.x + r * T] = a[r];
+        for (uint32_t i = threadIdx.x + R * T; i < n; i += T) d[i] = s[i];
+    }
+};
+
+// The same for n floats from a source of any 4-byte alignment, with 16-byte
+// loads: word i lands in d[shift(src) + i] (d 16-byte aligned, n + 3 words), so
+// the quads of the source that are whole and aligned stay aligned. The at most
+// three words before and after them are one load of a few lanes; nothing
+// outside [src, src + n) is read.
+template <uint32_t T, uint32_t R>
+struct HeldFloats
+{
+    f32x4 a[R];
+    float e;
+    __device__ static __forceinline__ uint32_t shift(const float* src)
+    {
+        return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(src) >> 2) & 3u;
+    }
+    // words before the first whole quad
+    __device__ static __forceinline__ uint32_t head(const float* src, uint32_t n)
+    {
+        return min((4u - shift(src)) & 3u, n);
+    }
+    // source word of end lane t (0..2 before the quads, 4..6 after), n if none
+    __device__ static __forceinline__ uint32_t end_word(uint32_t t, uint32_t h, uint32_t nq, uint32_t n)
+    {
+        const uint32_t i = (t < 3u) ? t : h + 4u * nq + t - 4u;
+        return (t < 3u ? t < h : (t >= 4u && t < 7u)) ? min(i, n) : n;
+    }
+    __device__ __forceinline__ void load(const float* __restrict__ src, uint32_t n)
+    {
+        const uint32_t h = head(src, n), nq = (n - h) >> 2;
+        const f32x4*   q = reinterpret_cast<const f32x4*>(src + h);
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r)
+            if (r * T < nq) a[r] = q[min(threadIdx.x + r * T, nq - 1u)];
+        if (n) e = src[min(end_word(threadIdx.x, h, nq, n), n - 1u)];
+    }
+    __device__ __forceinline__ void store(float* __restrict__ d, const float* __restrict__ src, uint32_t n) const
+    {
+        const uint32_t h = head(src, n), nq = (n - h) >> 2, s = shift(src);
+        const f32x4*   q = reinterpret_cast<const f32x4*>(src + h);
+        f32x4*         o = reinterpret_cast<f32x4*>(d) + (s ? 1u : 0u);  // first whole quad
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r)
+            if (threadIdx.x + r * T < nq) o[threadIdx.x + r * T] = a[r];
+        for (uint32_t i = threadIdx.x + R * T; i < nq; i += T) o[i] = q[i];
+        const uint32_t i = end_word(threadIdx.x, h, nq, n);
+        if (i < n) d[s + i] = e;
+    }
+};
+
 // Copy 3*nf u16 of a face row (8-byte aligned, padded to 4 faces) into LDS.
 __device__ __forceinline__ void stage_fe(uint16_t* __restrict__ dst, const uint16_t* __restrict__ src,
                                          uint32_t nf)

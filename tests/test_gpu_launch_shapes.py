@@ -1,0 +1,91 @@
+"""Kernels at the sizes where their launch shape or staging can go wrong:
+patches below and above the rounds a workgroup holds in registers, sources of
+every word alignment, empty owned sets, meshes of one to a few patches. Each
+against a plain FP64 restatement."""
+import numpy as np
+import pytest
+
+from rxmesh_amd import meshgen as mg
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(V, F, patch_size):
+    import rxmesh_amd as rx
+    import torch
+    m = rx.Mesh(F, patch_size=patch_size)
+    x = torch.from_numpy(np.ascontiguousarray(V[m.array("v_l2g")].T.astype(np.float32))).cuda()
+    return m, x
+
+
+def _cg64(rp, col, val, b, x, diag, iters):
+    """`iters` (preconditioned) CG iterations on the CSR system, FP64."""
+    rows = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+
+    def prod(v):
+        y = np.zeros_like(v)
+        np.add.at(y, rows, val[:, None] * v[col])
+        return y
+    x = x.copy()
+    r = b - prod(x)
+    z = r / diag
+    p, delta = z.copy(), (r * z).sum()
+    for _ in range(iters):
+        s = prod(p)
+        a = delta / (p * s).sum()
+        x += a * p
+        r -= a * s
+        z = r / diag
+        new = (r * z).sum()
+        p, delta = z + (new / delta) * p, new
+    return x
+
+
+@pytest.mark.parametrize("patch_size", [16, 64, 512, 2048])
+@pytest.mark.parametrize("mis", [0, 1, 2, 3])
+def test_cg_patch_sizes_and_alignment(patch_size, mis):
+    """Both implicit solves, six iterations, against the FP64 CG on the same
+    fp32 system; the value array starts at every word of a 16-byte line.
+    Tolerance 1e-5 of the largest coordinate, the forward error the solves
+    keep at dt = 1e-2."""
+    import torch
+    V, F = mg.permute_mesh(*mg.icosphere(4, seed=3, sigma=0.01), seed=3)
+    m, x = _mesh(V, F, patch_size)
+    dt, iters = 1e-2, 6
+    nnz = m.cot_nnz()
+    val = torch.empty(nnz + 4, dtype=torch.float32, device="cuda")[mis:mis + nnz]
+    A = m.cot_assemble(x, dt, out=(torch.empty(m.nV + 1, dtype=torch.int32, device="cuda"),
+                                   torch.empty(nnz, dtype=torch.int32, device="cuda"), val,
+                                   torch.empty(m.nV, dtype=torch.float32, device="cuda")))
+    rp, col, v64, mass = (t.cpu().numpy() for t in A)
+    v64, x64 = v64.astype(np.float64), x.cpu().numpy().T.astype(np.float64)
+    b = mass.astype(np.float64)[:, None] * x64
+    X, it, _, _ = m.mcf_implicit_cg(A, x, max_iter=iters, abs_tol=0.0)
+    ref = _cg64(rp, col, v64, b, x64, np.ones((m.nV, 1)), iters)
+    assert it == iters
+    assert np.abs(X.cpu().numpy().T - ref).max() <= 1e-5 * np.abs(ref).max()
+    Y, it, _, _ = m.mcf_matfree_cg(x, x, dt, precond=True, max_iter=iters, abs_tol=0.0)
+    ref = _cg64(rp, col, v64, b, x64, v64[rp[:-1]][:, None], iters)
+    assert it == iters
+    assert np.abs(Y.cpu().numpy().T - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+def test_cg_stops_inside_and_after_the_loop():
+    """A relative tolerance met by the last iteration allowed, by an earlier
+    one, and by the start itself: the solution and the counts are those of the
+    same number of unconditional iterations."""
+    import torch
+    V, F = mg.icosphere(4, seed=1, sigma=0.01)
+    m, x = _mesh(V, F, 128)
+    A = m.cot_assemble(x, 1e-2)
+    full = [m.mcf_implicit_cg(A, x, max_iter=k, abs_tol=0.0) for k in range(1, 7)]
+    start = full[0][2]
+    for k in range(1, 6):
+        tol = 1.001 * full[k - 1][3] / start  # met by the k-th update
+        assert all(f[3] / start >= tol for f in full[:k - 1])
+        for limit in (k, k + 3):
+            X, it, r0, r1 = m.mcf_implicit_cg(A, x, max_iter=limit, abs_tol=0.0, rel_tol=tol)
+            assert it == k - 1 and r0 == start and r1 == full[k - 1][3]
+            assert torch.equal(X, full[k - 1][0])
+    X, it, r0, r1 = m.mcf_implicit_cg(A, x, max_iter=3, abs_tol=2.0 * start)
+    assert it == 0 and r1 == start and torch.equal(X, x)
