@@ -89,7 +89,7 @@ struct rxm_mesh
     uint32_t        ring_threads   = 256;      // oriented VV, VE
     uint32_t        cot_threads    = 512;      // cotangent assembly
     uint32_t        smooth_aos4    = 0;        // 1: smoothing stages positions as float4
-    uint32_t        grad_threads   = 256;
+    uint32_t        grad_threads   = 512;
     uint32_t        grad_queue     = 0;        // 1: persistent work-queue launch
     uint32_t*       d_queue        = nullptr;  // work-queue ticket counter
     bool            system_runs_ok = false;    // check_system_runs passed
@@ -1228,7 +1228,7 @@ rxm_status rxm_set_launch_threads(rxm_mesh* m, int kernel, int threads)
         m->smooth_threads = static_cast<uint32_t>(threads);
         return RXM_OK;
     }
-    if (kernel == 1 && (threads == 128 || threads == 256)) {
+    if (kernel == 1 && (threads == 128 || threads == 256 || threads == 512)) {
         m->grad_threads = static_cast<uint32_t>(threads);
         return RXM_OK;
     }
@@ -1699,31 +1699,51 @@ rxm_status rxm_symdir3_energy(rxm_mesh* m, const float* Mr, const float* x, floa
     return launch_patches(k_symdir3_energy, kGeomThreads, b.bytes(), stream, m, m->dm, Mr, x, energy);
 }
 
+// LDS of the symmetric-Dirichlet gradient kernels. Patches whose corner
+// gradients do not fit a CU's LDS (beyond about 3,100 local faces) take the
+// lean form, which evaluates a face once per corner instead of once.
+static uint32_t symdir3_lds(const rxm_mesh* m, bool* lean)
+{
+    Bump b(nullptr), bl(nullptr);
+    plan_s3p(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
+    plan_s3p(bl, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent, true);
+    *lean = b.bytes() > kMaxLdsBytes;
+    return *lean ? bl.bytes() : b.bytes();
+}
+
 static int launch_symdir3_step(rxm_mesh* m, const float* Mr, float eta, const float* x, float* xo, void* stream)
 {
-    Bump b(nullptr);
-    plan_s3p(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
-    const uint32_t  lds = b.bytes();
-    const uint16_t* fvl = m->d_fp_fvl;
-    const uint16_t* ro  = m->d_fp_roff;
-    const uint16_t* vf  = m->d_fp_vf;
+    bool            lean = false;
+    const uint32_t  lds  = symdir3_lds(m, &lean);
+    const uint16_t* fvl  = m->d_fp_fvl;
+    const uint16_t* ro   = m->d_fp_roff;
+    const uint16_t* vf   = m->d_fp_vf;
+    auto            go   = [&](auto kernel, uint32_t T) {
+        return launch_patches_xcd(kernel, T, lds, stream, m, m->dm, m->d_fp_fbase, m->d_fp_rbase, m->d_fp_nbase, fvl, ro,
+                                  vf, Mr, eta, x, xo);
+    };
+    if (lean) return go(k_symdir3_step_plan<256, true>, 256);
     if (m->grad_queue) {
         hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, static_cast<hipStream_t>(stream), m->d_queue);
         RXM_HIP(hipGetLastError());
         // enough workgroups to fill the machine; LDS decides residency
         const uint32_t per_cu = std::max(1u, std::min(8u, (160u * 1024u) / std::max(lds, 1u)));
         const uint32_t grid   = std::min<uint32_t>(m->h.P, static_cast<uint32_t>(m->num_cus) * per_cu);
-        if (m->grad_threads == 128)
-            return launch_grid(k_symdir3_step_plan_queue<128>, grid, 128, lds, stream, m->dm, m->d_queue,
-                               m->d_fp_fbase, m->d_fp_rbase, m->d_fp_nbase, fvl, ro, vf, Mr, eta, x, xo);
-        return launch_grid(k_symdir3_step_plan_queue<256>, grid, 256, lds, stream, m->dm, m->d_queue, m->d_fp_fbase,
-                           m->d_fp_rbase, m->d_fp_nbase, fvl, ro, vf, Mr, eta, x, xo);
+        auto goq = [&](auto kernel, uint32_t T) {
+            return launch_grid(kernel, grid, T, lds, stream, m->dm, m->d_queue, m->d_fp_fbase, m->d_fp_rbase,
+                               m->d_fp_nbase, fvl, ro, vf, Mr, eta, x, xo);
+        };
+        switch (m->grad_threads) {
+            case 128: return goq(k_symdir3_step_plan_queue<128>, 128);
+            case 256: return goq(k_symdir3_step_plan_queue<256>, 256);
+            default: return goq(k_symdir3_step_plan_queue<512>, 512);
+        }
     }
-    if (m->grad_threads == 128)
-        return launch_patches(k_symdir3_step_plan<128>, 128, lds, stream, m, m->dm, m->d_fp_fbase, m->d_fp_rbase,
-                              m->d_fp_nbase, fvl, ro, vf, Mr, eta, x, xo);
-    return launch_patches(k_symdir3_step_plan<256>, 256, lds, stream, m, m->dm, m->d_fp_fbase, m->d_fp_rbase,
-                          m->d_fp_nbase, fvl, ro, vf, Mr, eta, x, xo);
+    switch (m->grad_threads) {
+        case 128: return go(k_symdir3_step_plan<128>, 128);
+        case 256: return go(k_symdir3_step_plan<256>, 256);
+        default: return go(k_symdir3_step_plan<512>, 512);
+    }
 }
 
 // Everything the step loop needs on the device before launching (or
@@ -1757,12 +1777,14 @@ rxm_status rxm_symdir3_grad(rxm_mesh* m, const float* Mr, const float* x, float*
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
     int rc = ensure_face_plan(m, stream);
     if (rc) return rc;
-    Bump b(nullptr);
-    plan_s3p(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
-    return launch_patches(k_symdir3_grad_plan<256>, 256, b.bytes(), stream, m, m->dm, m->d_fp_fbase, m->d_fp_rbase,
-                          m->d_fp_nbase, static_cast<const uint16_t*>(m->d_fp_fvl),
-                          static_cast<const uint16_t*>(m->d_fp_roff), static_cast<const uint16_t*>(m->d_fp_vf), Mr,
-                          x, grad);
+    bool           lean = false;
+    const uint32_t lds  = symdir3_lds(m, &lean);
+    auto           go   = [&](auto kernel, uint32_t T) {
+        return launch_patches_xcd(kernel, T, lds, stream, m, m->dm, m->d_fp_fbase, m->d_fp_rbase, m->d_fp_nbase,
+                                  static_cast<const uint16_t*>(m->d_fp_fvl), static_cast<const uint16_t*>(m->d_fp_roff),
+                                  static_cast<const uint16_t*>(m->d_fp_vf), Mr, x, grad);
+    };
+    return lean ? go(k_symdir3_grad_plan<256, true>, 256) : go(k_symdir3_grad_plan<512>, 512);
 }
 
 // The batched workload step: x1 = smooth(x), x = x1 - eta grad E_symdir3(x1).

@@ -76,6 +76,66 @@ __device__ __forceinline__ void stage_positions_batched(float* sx, float* sy, fl
     }
 }
 
+// C-component SoA vertex attribute of a patch (component stride N) on its way
+// into LDS, in the two halves of Held: ids() and owned() issue the loads that
+// depend on the descriptor alone, ribbon() those that need the ribbon's owner
+// ids, store() writes LDS (and copies what larger patches have beyond the
+// register rounds). o[k] keeps the words of owned vertex t + k T. Indices past
+// a range read a valid element whose value is not used.
+template <uint32_t T, uint32_t C>
+struct HeldVerts
+{
+    static constexpr uint32_t RO = (512u + T - 1u) / T, RR = (256u + T - 1u) / T;
+    float                     o[RO][C], q[RR][C];
+    uint32_t                  g[RR];
+    __device__ __forceinline__ void ids(const DevMesh& m, const PatchDesc& d)
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < RR; ++k)
+            if (k == 0 || d.nvo + k * T < d.nv) g[k] = m.v_lin[d.v_off + min(d.nvo + threadIdx.x + k * T, d.nv - 1u)];
+    }
+    __device__ __forceinline__ void owned(const float* __restrict__ src, const DevMesh& m, const PatchDesc& d)
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < RO; ++k)
+            if (k == 0 || k * T < d.nvo)
+#pragma unroll
+                for (uint32_t c = 0; c < C; ++c) o[k][c] = src[size_t(c) * m.nV + min(d.vp + threadIdx.x + k * T, m.nV - 1u)];
+    }
+    __device__ __forceinline__ void ribbon(const float* __restrict__ src, const DevMesh& m, const PatchDesc& d)
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < RR; ++k)
+            if (k == 0 || d.nvo + k * T < d.nv)
+#pragma unroll
+                for (uint32_t c = 0; c < C; ++c) q[k][c] = src[size_t(c) * m.nV + g[k]];
+    }
+    // put(l, words) for every local vertex
+    template <typename Put>
+    __device__ __forceinline__ void store(const float* __restrict__ src, const DevMesh& m, const PatchDesc& d, Put put) const
+    {
+        const uint32_t t = threadIdx.x;
+#pragma unroll
+        for (uint32_t k = 0; k < RO; ++k)
+            if (t + k * T < d.nvo) put(t + k * T, o[k]);
+#pragma unroll
+        for (uint32_t k = 0; k < RR; ++k)
+            if (d.nvo + t + k * T < d.nv) put(d.nvo + t + k * T, q[k]);
+        auto direct = [&](uint32_t l, uint32_t gg) {
+            float w[C];
+            for (uint32_t c = 0; c < C; ++c) w[c] = src[size_t(c) * m.nV + gg];
+            put(l, w);
+        };
+        for (uint32_t l = t + RO * T; l < d.nvo; l += T) direct(l, d.vp + l);
+        for (uint32_t l = d.nvo + t + RR * T; l < d.nv; l += T) direct(l, m.v_lin[d.v_off + l]);
+    }
+};
+
+// n u16 of a 16-byte aligned, 8-element padded run, in 16-byte words
+__host__ __device__ inline uint32_t words8(uint32_t n) { return (n + 7u) >> 3; }
+__device__ __forceinline__ const u32x4* as_words(const uint16_t* p) { return reinterpret_cast<const u32x4*>(p); }
+__device__ __forceinline__ u32x4*       as_words(uint16_t* p) { return reinterpret_cast<u32x4*>(p); }
+
 // ---- vertex normals -------------------------------------------------------
 struct PlanVN
 {

@@ -89,3 +89,46 @@ def test_cg_stops_inside_and_after_the_loop():
             assert torch.equal(X, full[k - 1][0])
     X, it, r0, r1 = m.mcf_implicit_cg(A, x, max_iter=3, abs_tol=2.0 * start)
     assert it == 0 and r1 == start and torch.equal(X, x)
+
+
+def _dirichlet_grad64(x, fv, rest):
+    """Gradient of sum A |J|^2 (1 + 1 / det(J^T J)) by FP64 autograd; x (V, 3), rest (4, F) m00 m10 m01 m11."""
+    import torch
+    x = torch.from_numpy(x).requires_grad_(True)
+    f = torch.from_numpy(fv.astype(np.int64))
+    m00, m10, m01, m11 = torch.from_numpy(rest)
+    det = m00 * m11 - m01 * m10
+    e1, e2 = x[f[:, 1]] - x[f[:, 0]], x[f[:, 2]] - x[f[:, 0]]
+    j0 = e1 * (m11 / det)[:, None] - e2 * (m10 / det)[:, None]
+    j1 = -e1 * (m01 / det)[:, None] + e2 * (m00 / det)[:, None]
+    a, b, c = (j0 * j0).sum(1), (j1 * j1).sum(1), (j0 * j1).sum(1)
+    (0.5 * det * (a + b) * (1 + 1 / (a * b - c * c))).sum().backward()
+    return x.grad.numpy()
+
+
+@pytest.mark.parametrize("patch_size", [16, 256, 512, 1024, 4096])
+def test_symdir3_patch_sizes(patch_size):
+    """The gradient and the step over patches from a few faces to more than a
+    workgroup's registers and (4096) LDS hold, every workgroup size: the same
+    bits, and within 1e-5 of the largest entry of the FP64 gradient (the bound
+    the gradient keeps elsewhere)."""
+    import torch
+    V, F = mg.permute_mesh(*mg.icosphere(5, seed=4, sigma=0.01), seed=4)
+    m, x = _mesh(V, F, patch_size)
+    Mr = m.symdir_rest(x)
+    y = (x * 1.1 + 0.01 * torch.sin(5.0 * x.flip(0))).contiguous()
+    g = m.symdir3_grad(Mr, y)
+    step = m.symdir3_grad_step(Mr, y, 1e-3)
+    for threads in (128, 256, 512):
+        m.set_launch_threads(1, threads)
+        for queue in (0, 1):
+            m.set_launch_threads(2, queue)
+            assert torch.equal(step, m.symdir3_grad_step(Mr, y, 1e-3))
+    l2g, f_l2g = m.array("v_l2g"), m.array("f_l2g")
+    yg = np.empty((m.nV, 3))
+    yg[l2g] = y.cpu().numpy().T
+    rest = np.empty((4, m.nF))
+    rest[:, f_l2g] = Mr.cpu().numpy()
+    ref = _dirichlet_grad64(yg, F, rest)[l2g].T
+    assert np.abs(g.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+    assert torch.allclose(step, y - 1e-3 * g, rtol=1e-6, atol=1e-7)
