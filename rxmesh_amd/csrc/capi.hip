@@ -85,7 +85,7 @@ struct rxm_mesh
     uint32_t        cot_nplist   = 0;
     const uint16_t* d_cot_ent    = nullptr;  // patch-local VV edge pattern (build_vv_edge_pattern)
     const uint32_t* d_cot_rs     = nullptr;
-    uint32_t        smooth_threads = 128;
+    uint32_t        smooth_threads = 0;        // 0: by the patch count (smooth_group)
     uint32_t        ring_threads   = 256;      // oriented VV, VE
     uint32_t        cot_threads    = 512;      // cotangent assembly
     uint32_t        smooth_aos4    = 0;        // 1: smoothing stages positions as float4
@@ -398,6 +398,17 @@ int ensure_face_plan(rxm_mesh* m, void* stream)
     return RXM_OK;
 }
 
+// Workgroup size of the smoothing kernels where the caller chose none. While
+// the patches are resident at about once (4 workgroups of 512 threads on each
+// of 256 CUs) a launch lasts as long as one workgroup's chain, which more
+// threads shorten; beyond that more, smaller workgroups hide each other's
+// latency. Ten single steps with 512 / 256 threads: 71 patches 35.4 / 43.5 us,
+// 491 42.6 / 48.1, 1279 61.8 / 64.3, 2015 80.9 / 78.6, 4249 143 / 124.
+uint32_t smooth_group(const rxm_mesh* m)
+{
+    return m->smooth_threads ? m->smooth_threads : (m->h.P <= 1500u ? 512u : 256u);
+}
+
 template <bool AOS4>
 int smooth_once_t(rxm_mesh* m, float lambda, const float* src, float* dst, void* stream)
 {
@@ -405,7 +416,7 @@ int smooth_once_t(rxm_mesh* m, float lambda, const float* src, float* dst, void*
     plan_sl(b, m->h.max_nv, m->h.max_nvo, m->vv_max_nent, AOS4);
     const uint16_t* ro = m->d_vv_roff;
     const uint16_t* nb = m->d_vv_nbr;
-    switch (m->smooth_threads) {
+    switch (smooth_group(m)) {
         case 64:
             return launch_patches_xcd(k_smooth_local<64, AOS4>, 64, b.bytes(), stream, m, m->dm, m->d_vv_rbase,
                                       m->d_vv_nbase, ro, nb, lambda, src, dst);
@@ -512,7 +523,7 @@ int smooth_steps(rxm_mesh* m, uint32_t steps, float lambda, const float* src, fl
                                   m->d_vvk_nbase, m->d_vvk_xbase, m->d_vvk_roff, m->d_vvk_nbr, m->d_vvk_xlin, steps,
                                   lambda, src, dst);
     };
-    switch (m->smooth_threads) {
+    switch (smooth_group(m)) {
         case 64: return go(k_smoothk<64>, 64);
         case 256: return go(k_smoothk<256>, 256);
         case 512: return go(k_smoothk<512>, 512);
@@ -531,7 +542,7 @@ int smooth_twice_t(rxm_mesh* m, float lambda, const float* src, float* dst, void
                                   m->d_vv2_xbase, m->d_vv2_xcnt, m->d_vv2_roff, m->d_vv2_nbr, m->d_vv2_xlin, lambda,
                                   src, dst);
     };
-    switch (m->smooth_threads) {
+    switch (smooth_group(m)) {
         case 64: return go(k_smooth2<64, AOS4>, 64);
         case 256: return go(k_smooth2<256, AOS4>, 256);
         case 512: return go(k_smooth2<512, AOS4>, 512);
@@ -551,7 +562,7 @@ int smooth_twice_g(rxm_mesh* m, float lambda, const float* src, float* dst, void
                                   m->d_vv2_xbase, m->d_vv2_xcnt, m->d_vv2_roff, m->d_vv2_nbr, m->d_vv2_xlin, lambda,
                                   src, dst);
     };
-    switch (m->smooth_threads) {
+    switch (smooth_group(m)) {
         case 64: return go(k_smooth2<64, false, GIN, GOUT>, 64);
         case 256: return go(k_smooth2<256, false, GIN, GOUT>, 256);
         case 512: return go(k_smooth2<512, false, GIN, GOUT>, 512);
