@@ -234,7 +234,10 @@ rxm_status rxm_build_edges_device(const uint32_t* fv, uint32_t num_faces, uint32
 /* Build (once; later calls return at once) the mesh's patch-local VV plan:
  * the VV query evaluated by the query engine and kept in its native
  * patch-local u16 encoding for iterative consumers. rxm_laplacian_smooth
- * builds it on first use; call this to keep the build out of a timed loop. */
+ * builds it on first use; call this to keep the build out of a timed loop.
+ * It also builds the multi-step smoothing plan (patch + rings of neighbours,
+ * three or five levels by the number of patches), which rxm_laplacian_smooth
+ * then uses for iters > 1; waits for the stream. */
 rxm_status rxm_vv_plan_build(rxm_mesh* mesh, void* stream);
 /* Launch configuration knobs (used by the autotuner):
  *   kernel 0: smoothing workgroup size 64 / 128 / 256 / 512 (default: by the
@@ -251,7 +254,8 @@ rxm_status rxm_vv_plan_build(rxm_mesh* mesh, void* stream);
  *   kernel 7: cotangent assembly workgroup size 256 / 512;
  *   kernel 8: smoothing, 1-6 = that many Jacobi steps per launch over the
  *             K-level plan (patch + rings of neighbours kept in LDS; overrides
- *             kernels 3 and 4), 0 = off;
+ *             kernels 3 and 4), 0 = off; until it is set, and while kernels 3
+ *             and 4 are 0, the steps rxm_vv_plan_build planned for;
  *   kernel 9: smoothing with two steps per launch (kernel 4 = 1, float
  *             arrays in LDS) and >= 4 iterations: 1 = the iterates between
  *             launches are one float4 per vertex in two buffers the mesh

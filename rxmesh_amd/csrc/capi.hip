@@ -25,6 +25,8 @@
 
 using namespace rxm;
 
+constexpr uint32_t kStepsAuto = 0xFFFFFFFFu;  // smooth_steps: by the patch count (auto_levels)
+
 struct rxm_mesh
 {
     HostMesh              h;
@@ -62,7 +64,9 @@ struct rxm_mesh
     const uint16_t*   d_vvk_roff  = nullptr;
     const uint16_t*   d_vvk_nbr   = nullptr;
     const uint32_t*   d_vvk_xlin  = nullptr;
-    uint32_t          smooth_steps = 0;  // > 0: Jacobi steps per launch over the K-level plan
+    uint32_t          smooth_steps = kStepsAuto;  // Jacobi steps per launch over the K-level plan; 0: off
+    bool              vvk_tried    = false;       // rxm_vv_plan_build has tried to make the plan of auto_levels rings,
+    bool              vvk_auto     = false;       // and has it
     uint32_t          smooth_g4    = 1;  // two-step launches pass float4 iterates between them
     float*            d_cg         = nullptr;  // CG work arrays (CgWork)
     float*            d_mf         = nullptr;  // matrix-free CG: mass, diag (V each), weights (one per row entry)
@@ -404,9 +408,11 @@ int ensure_face_plan(rxm_mesh* m, void* stream)
 // threads shorten; beyond that more, smaller workgroups hide each other's
 // latency. Ten single steps with 512 / 256 threads: 71 patches 35.4 / 43.5 us,
 // 491 42.6 / 48.1, 1279 61.8 / 64.3, 2015 80.9 / 78.6, 4249 143 / 124.
-uint32_t smooth_group(const rxm_mesh* m)
+// Several steps per launch have more to spread: three steps, ten iterations,
+// 2015 patches 55.1 / 57.2, 4249 102.8 / 100.7.
+uint32_t smooth_group(const rxm_mesh* m, bool multi = false)
 {
-    return m->smooth_threads ? m->smooth_threads : (m->h.P <= 1500u ? 512u : 256u);
+    return m->smooth_threads ? m->smooth_threads : (m->h.P <= (multi ? 3000u : 1500u) ? 512u : 256u);
 }
 
 template <bool AOS4>
@@ -496,21 +502,115 @@ int ensure_cot_plan(rxm_mesh* m)
 
 constexpr uint32_t kSmoothLevels = 6;  // rings of the K-level plan: up to 6 steps per launch
 
-int ensure_vvk_plan(rxm_mesh* m)
+// Uninitialised device array owned by the mesh.
+template <typename T>
+int device_array(rxm_mesh* m, size_t n, T** out)
 {
-    if (m->d_vvk_nbr) return RXM_OK;
-    int rc = build_vvk_plan(m->h, kSmoothLevels, m->vvk);
-    const VvkPlan& v = m->vvk;
-    if (!rc) rc = upload(m, v.lvl, m->d_vvk_lvl);
-    if (!rc) rc = upload(m, v.rbase, m->d_vvk_rbase);
-    if (!rc) rc = upload(m, v.nbase, m->d_vvk_nbase);
-    if (!rc) rc = upload(m, v.xbase, m->d_vvk_xbase);
-    if (!rc) rc = upload(m, v.roff, m->d_vvk_roff);
-    if (!rc) rc = upload(m, v.xlin, m->d_vvk_xlin);
-    if (!rc) rc = upload(m, v.nbr, m->d_vvk_nbr);  // last: marks the plan complete
-    if (rc) m->d_vvk_nbr = nullptr;
-    return rc;
+    const size_t bytes = std::max<size_t>(n * sizeof(T), 16);
+    T*           p     = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
+    m->allocs.push_back(p);
+    m->device_bytes += bytes;
+    *out = p;
+    return RXM_OK;
 }
+
+// The K-level plan over K rings, built by k_ring_plan from the VV plan (waits
+// for the stream to size it): 2 launches instead of a host walk with a map per
+// patch. Patches beyond the kernel's tables: RXM_ERR_PATCH_TOO_BIG.
+int build_ring_plan(rxm_mesh* m, uint32_t K, void* stream)
+{
+    const uint32_t P = m->h.P, W = 2 * K + 1;
+    hipStream_t    hs = static_cast<hipStream_t>(stream);
+    Bump           b(nullptr);
+    plan_rb(b);
+    uint32_t* lvl  = nullptr;  // counts, then the overflow flag
+    int       rc = device_array(m, size_t(P) * W + 1, &lvl);
+    if (rc) return rc;
+    uint32_t* flag = lvl + size_t(P) * W;
+    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, hs, flag);
+    auto go = [&](const uint32_t* rb, const uint32_t* nb, const uint32_t* xb, uint16_t* ro, uint16_t* nr, uint32_t* xl) {
+        return launch_patches(k_ring_plan<256>, 256, b.bytes(), stream, m, m->dm, K, m->d_vv_rbase, m->d_vv_nbase,
+                              static_cast<const uint16_t*>(m->d_vv_roff), static_cast<const uint16_t*>(m->d_vv_nbr), lvl,
+                              flag, rb, nb, xb, ro, nr, xl);
+    };
+    if ((rc = go(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr))) return rc;
+    VvkPlan v;
+    v.K = K;
+    v.lvl.resize(size_t(P) * W + 1);
+    RXM_HIP(hipMemcpyAsync(v.lvl.data(), lvl, v.lvl.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, hs));
+    RXM_HIP(hipStreamSynchronize(hs));
+    if (v.lvl.back()) return RXM_ERR_PATCH_TOO_BIG;
+    v.max_cnt.assign(K + 1, 0);
+    v.max_ent.assign(K, 0);
+    std::vector<uint32_t> base(3 * size_t(P + 1), 0);  // runs padded to 8 / 8 / 4 elements
+    uint32_t *rb = base.data(), *nb = rb + P + 1, *xb = nb + P + 1;
+    for (uint32_t p = 0; p < P; ++p) {
+        const uint32_t* c = &v.lvl[size_t(p) * W];
+        rb[p + 1] = rb[p] + ((c[K - 1] + 1u + 7u) & ~7u);
+        nb[p + 1] = nb[p] + ((c[2 * K] + 7u) & ~7u);
+        xb[p + 1] = xb[p] + ((c[K] - c[0] + 3u) & ~3u);
+        for (uint32_t k = 0; k <= K; ++k) v.max_cnt[k] = std::max(v.max_cnt[k], c[k]);
+        for (uint32_t k = 0; k < K; ++k) v.max_ent[k] = std::max(v.max_ent[k], c[K + 1 + k]);
+    }
+    const uint32_t* d_base = nullptr;
+    uint16_t *      ro = nullptr, *nr = nullptr;
+    uint32_t*       xl = nullptr;
+    if ((rc = upload(m, base, d_base)) || (rc = device_array(m, rb[P], &ro)) || (rc = device_array(m, nb[P], &nr)) ||
+        (rc = device_array(m, xb[P], &xl)))
+        return rc;
+    const uint32_t *drb = d_base, *dnb = d_base + P + 1, *dxb = d_base + 2 * (P + 1);
+    if ((rc = go(drb, dnb, dxb, ro, nr, xl))) return rc;
+    v.lvl.clear();
+    m->vvk         = std::move(v);
+    m->d_vvk_lvl   = lvl;
+    m->d_vvk_rbase = drb;
+    m->d_vvk_nbase = dnb;
+    m->d_vvk_xbase = dxb;
+    m->d_vvk_roff  = ro;
+    m->d_vvk_nbr   = nr;
+    m->d_vvk_xlin  = xl;
+    return RXM_OK;
+}
+
+// A K-level plan of at least K rings: on the device, or, for patches beyond
+// that kernel's tables, by the host walk.
+int ensure_vvk_plan(rxm_mesh* m, uint32_t K, void* stream)
+{
+    if (m->d_vvk_nbr && m->vvk.K >= K) return RXM_OK;
+    int rc = ensure_vv_plan(m, stream);
+    if (!rc) rc = build_ring_plan(m, K, stream);
+    if (rc != RXM_ERR_PATCH_TOO_BIG) return rc;
+    VvkPlan v;
+    rc = build_vvk_plan(m->h, K, v);
+    const uint32_t *lvl = nullptr, *rb = nullptr, *nb = nullptr, *xb = nullptr, *xl = nullptr;
+    const uint16_t *ro = nullptr, *nr = nullptr;
+    if (!rc) rc = upload(m, v.lvl, lvl);
+    if (!rc) rc = upload(m, v.rbase, rb);
+    if (!rc) rc = upload(m, v.nbase, nb);
+    if (!rc) rc = upload(m, v.xbase, xb);
+    if (!rc) rc = upload(m, v.roff, ro);
+    if (!rc) rc = upload(m, v.xlin, xl);
+    if (!rc) rc = upload(m, v.nbr, nr);
+    if (rc) return rc;
+    m->vvk         = std::move(v);
+    m->d_vvk_lvl   = lvl;
+    m->d_vvk_rbase = rb;
+    m->d_vvk_nbase = nb;
+    m->d_vvk_xbase = xb;
+    m->d_vvk_roff  = ro;
+    m->d_vvk_nbr   = nr;
+    m->d_vvk_xlin  = xl;
+    return RXM_OK;
+}
+
+// Steps per launch where the caller chose none (knobs 3, 4 and 8 untouched) and
+// rxm_vv_plan_build has made the plan: five while the patches are resident at
+// about once (the rings' redundant updates run on idle lanes and a launch costs
+// more than they do), three beyond. Us per ten steps with 1 / 3 / 5 steps per
+// launch: 71 patches 40 / 19 / 19 (and fewer launches to queue), 739 49 / 28 /
+// 28, 1279 62 / 42 / 44, 4249 125 / 101 / 123.
+uint32_t auto_levels(const rxm_mesh* m) { return m->h.P <= 1024u ? 5u : 3u; }
 
 // `steps` Jacobi steps in one launch over the K-level plan
 int smooth_steps(rxm_mesh* m, uint32_t steps, float lambda, const float* src, float* dst, void* stream)
@@ -523,7 +623,7 @@ int smooth_steps(rxm_mesh* m, uint32_t steps, float lambda, const float* src, fl
                                   m->d_vvk_nbase, m->d_vvk_xbase, m->d_vvk_roff, m->d_vvk_nbr, m->d_vvk_xlin, steps,
                                   lambda, src, dst);
     };
-    switch (smooth_group(m)) {
+    switch (smooth_group(m, true)) {
         case 64: return go(k_smoothk<64>, 64);
         case 256: return go(k_smoothk<256>, 256);
         case 512: return go(k_smoothk<512>, 512);
@@ -1163,7 +1263,15 @@ rxm_status rxm_vv_plan_build(rxm_mesh* m, void* stream)
 {
     if (!m) return RXM_ERR_INVALID_ARG;
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
-    return ensure_vv_plan(m, stream);
+    int rc = ensure_vv_plan(m, stream);
+    if (rc || m->vvk_tried) return rc;
+    // the multi-step plan is an option of the smoothing: patches beyond its
+    // tables or a full device leave the single-step plan in use
+    const uint32_t K = auto_levels(m);
+    rc           = (m->d_vvk_nbr && m->vvk.K >= K) ? RXM_OK : build_ring_plan(m, K, stream);
+    m->vvk_tried = rc == RXM_OK || rc == RXM_ERR_PATCH_TOO_BIG;
+    m->vvk_auto  = rc == RXM_OK;
+    return (rc == RXM_ERR_PATCH_TOO_BIG || rc == RXM_ERR_OUT_OF_MEMORY) ? RXM_OK : rc;
 }
 
 rxm_status rxm_laplacian_smooth(rxm_mesh* m, const float* pos, float* out, float* tmp, float lambda, int iters,
@@ -1172,16 +1280,19 @@ rxm_status rxm_laplacian_smooth(rxm_mesh* m, const float* pos, float* out, float
     if (!m || !pos || !out || iters < 1 || pos == out) return RXM_ERR_INVALID_ARG;
     if (iters > 1 && (!tmp || tmp == out || tmp == pos)) return RXM_ERR_INVALID_ARG;
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
-    int rc = RXM_OK;
-    if (m->smooth_steps > 0) {  // K-level plan: launches of up to smooth_steps steps
-        if ((rc = ensure_vvk_plan(m))) return rc;
-        const uint32_t S        = m->smooth_steps;
-        const int      launches = static_cast<int>((iters + S - 1) / S);
-        const float*   src      = pos;
-        int            left     = iters;
+    int        rc   = RXM_OK;
+    const bool knob = m->smooth_steps != kStepsAuto && m->smooth_steps > 0;
+    // automatic: over the plan rxm_vv_plan_build made, while knobs 3 and 4 are off
+    const bool automatic = m->smooth_steps == kStepsAuto && m->vvk_auto && iters > 1 && !m->smooth_fused && !m->smooth_aos4;
+    if (knob || automatic) {  // K-level plan: launches of up to S steps, as even as they come
+        const uint32_t S = knob ? m->smooth_steps : std::min(auto_levels(m), m->vvk.K);
+        if ((rc = ensure_vvk_plan(m, S, stream))) return rc;
+        const int    launches = static_cast<int>((iters + S - 1) / S);
+        const float* src      = pos;
+        int          left     = iters;
         for (int i = 0; i < launches; ++i) {
             float*         dst = ((launches - 1 - i) % 2 == 0) ? out : tmp;
-            const uint32_t s   = std::min<uint32_t>(S, static_cast<uint32_t>(left));
+            const uint32_t s   = static_cast<uint32_t>((left + launches - i - 1) / (launches - i));
             if ((rc = smooth_steps(m, s, lambda, src, dst, stream))) return rc;
             left -= static_cast<int>(s);
             src = dst;

@@ -541,6 +541,148 @@ __global__ __launch_bounds__(T) void k_smooth2(DevMesh m, const uint32_t* __rest
     }
 }
 
+// Build of the K-level smoothing plan on the device: one workgroup per patch
+// walks the rings around its owned vertices over the owners' rows of the VV
+// plan. Extended ids are handed out ring by ring (within a ring in the order
+// threads arrive: the order is not part of any result, a row keeps its owner's
+// neighbour order whatever the ids are), in a hash table of linear ids in LDS.
+// Run twice: with o_roff null it writes the patch's counts to lvl, then, with
+// the runs' bases, the rows, entries and ring vertices' linear ids. A patch
+// beyond the table (kRingVerts vertices or kRingEnts entries) sets *flag and
+// writes nothing. The probe loops end after a full turn of the table. About
+// 0.1 ms a pass on 4249 patches (rows and ids from L2, four dependent loads a
+// ring); the host walk it replaces, a map per patch, took hundreds.
+constexpr uint32_t kRingVerts = 2048, kRingEnts = 8192, kRingHash = 4096;
+
+struct PlanRB
+{
+    uint32_t *lin, *own, *off, *row, *key, *wave;
+    uint16_t* id;
+};
+__host__ __device__ inline PlanRB plan_rb(Bump& b)
+{
+    PlanRB p{};
+    p.lin  = b.alloc<uint32_t>(kRingVerts);  // linear id and owner patch of every extended vertex
+    p.own  = b.alloc<uint32_t>(kRingVerts);
+    p.off  = b.alloc<uint32_t>(kRingVerts + 1);
+    p.row  = b.alloc<uint32_t>(kRingEnts);   // linear ids of the rows' entries
+    p.key  = b.alloc<uint32_t>(kRingHash);
+    p.wave = b.alloc<uint32_t>(20);
+    p.id   = b.alloc<uint16_t>(kRingHash);
+    return p;
+}
+
+template <uint32_t T>
+__global__ __launch_bounds__(T) void k_ring_plan(DevMesh m, uint32_t K, const uint32_t* __restrict__ vv_rbase,
+                                                 const uint32_t* __restrict__ vv_nbase,
+                                                 const uint16_t* __restrict__ vv_roff,
+                                                 const uint16_t* __restrict__ vv_nbr, uint32_t* __restrict__ lvl,
+                                                 uint32_t* __restrict__ flag, const uint32_t* __restrict__ rbase,
+                                                 const uint32_t* __restrict__ nbase, const uint32_t* __restrict__ xbase,
+                                                 uint16_t* __restrict__ o_roff, uint16_t* __restrict__ o_nbr,
+                                                 uint32_t* __restrict__ o_xlin)
+{
+    extern __shared__ uint4 smem[];
+    __shared__ uint32_t     cnt;
+    const uint32_t  p = blockIdx.x, t = threadIdx.x;
+    const PatchDesc d = load_desc(m.patch, p);
+    Bump            b(reinterpret_cast<char*>(smem));
+    const PlanRB    L = plan_rb(b);
+    constexpr uint32_t kEmpty = 0xFFFFFFFFu, kMask = kRingHash - 1u;
+    auto hash = [](uint32_t x) { return (x * 2654435761u) >> 20; };  // Knuth's multiplicative hash, 12 bits
+    static_assert(kRingHash == 1u << 12, "hash bits");
+    uint32_t* c = lvl + size_t(p) * (2 * K + 1);
+    if (d.nvo > kRingVerts) {
+        if (t == 0) *flag = 1u;
+        return;
+    }
+    for (uint32_t i = t; i < kRingHash; i += T) L.key[i] = kEmpty;
+    if (t == 0) cnt = d.nvo;
+    __syncthreads();
+    // the slot of linear id x: claimed (*fresh) or found; kRingHash if the table is full
+    auto slot_of = [&](uint32_t x, bool* fresh) {
+        uint32_t h = hash(x);
+        for (uint32_t probe = 0; probe < kRingHash; ++probe, h = (h + 1u) & kMask) {
+            const uint32_t k = atomicCAS(&L.key[h], kEmpty, x);
+            if (k == kEmpty || k == x) {
+                *fresh = k == kEmpty;
+                return h;
+            }
+        }
+        *fresh = false;
+        return kRingHash;
+    };
+    for (uint32_t i = t; i < d.nvo; i += T) {
+        bool           fresh;
+        const uint32_t h = slot_of(d.vp + i, &fresh);
+        if (h < kRingHash) L.id[h] = static_cast<uint16_t>(i);
+        L.lin[i] = d.vp + i;
+        L.own[i] = p;
+    }
+    __syncthreads();
+    uint32_t a = 0, e = d.nvo, ent = 0;  // ring [a, e), entries so far
+    for (uint32_t k = 1; k <= K; ++k) {
+        for (uint32_t i = a + t; i < e; i += T) {
+            const uint32_t q = L.own[i], r = vv_rbase[q] + L.lin[i] - m.patch[q].vp;
+            L.off[i]         = uint32_t(vv_roff[r + 1]) - vv_roff[r];
+        }
+        const uint32_t total = scan_excl<T>(L.off + a, e - a, L.wave);
+        if (ent + total > kRingEnts) {  // uniform
+            if (t == 0) *flag = 1u;
+            return;
+        }
+        for (uint32_t i = a + t; i < e; i += T) {
+            const uint32_t q = L.own[i], qvp = m.patch[q].vp, qno = m.patch[q].nvo, qv = m.patch[q].v_off;
+            const uint32_t r = vv_rbase[q] + L.lin[i] - qvp, o = ent + L.off[i];
+            const uint32_t k0 = vv_roff[r], deg = vv_roff[r + 1] - k0;
+            const uint16_t* nb = vv_nbr + vv_nbase[q] + k0;
+            L.off[i]           = o;
+            for (uint32_t j = 0; j < deg; ++j) {
+                const uint32_t n = nb[j], x = (n < qno) ? qvp + n : m.v_lin[qv + n];
+                L.row[o + j]     = x;
+                if (*static_cast<volatile uint32_t*>(&cnt) > kRingVerts) continue;  // overflow found below
+                bool           fresh;
+                const uint32_t h = slot_of(x, &fresh);
+                if (!fresh) continue;
+                const uint32_t g = atomicAdd(&cnt, 1u);
+                if (g < kRingVerts) {
+                    L.lin[g] = x;
+                    L.own[g] = (n < qno) ? q : m.v_own[qv + n];
+                    L.id[h]  = static_cast<uint16_t>(g);
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t n = cnt;
+        __syncthreads();  // every thread has read the count before the next ring adds to it
+        if (n > kRingVerts) {  // uniform
+            if (t == 0) *flag = 1u;
+            return;
+        }
+        ent += total;
+        if (!o_roff && t == 0) {
+            if (k == 1) c[0] = d.nvo;
+            c[k]     = n;
+            c[K + k] = ent;
+        }
+        if (k < K) {
+            a = e;
+            e = n;
+        } else if (o_roff) {
+            // rows of [0, e), entries as extended ids, linear ids of the rings
+            const uint32_t rb = rbase[p], nb = nbase[p], xb = xbase[p];
+            for (uint32_t i = t; i < e; i += T) o_roff[rb + i] = static_cast<uint16_t>(L.off[i]);
+            if (t == 0) o_roff[rb + e] = static_cast<uint16_t>(ent);
+            for (uint32_t i = t; i < ent; i += T) {
+                bool           fresh;
+                const uint32_t h = slot_of(L.row[i], &fresh);
+                o_nbr[nb + i]    = L.id[h & kMask];
+            }
+            for (uint32_t i = d.nvo + t; i < n; i += T) o_xlin[xb + i - d.nvo] = L.lin[i];
+        }
+    }
+}
+
 // ---- K-step smoothing over the level plan (temporal blocking) ---------------
 // One workgroup per patch runs `steps` Jacobi steps of uniform smoothing on
 // the patch's extended vertex space (owned vertices, then the rings around
@@ -548,7 +690,9 @@ __global__ __launch_bounds__(T) void k_smooth2(DevMesh m, const uint32_t* __rest
 // previous step's values, the last step the owned vertices, which go to HBM.
 // Each vertex update lists its neighbours in the owner's canonical VV order,
 // as k_smooth_local does, so any split of the iterations into launches gives
-// bit-identical results. lvl: 2K + 1 u32 per patch (cnt[0..K], ent[0..K-1]).
+// bit-identical results. Ten iterations, 512 threads: 41k vertices (167 patches,
+// five steps per launch) 38 -> 17 us, 1.05M (three) 124 -> 101. Bound: LDS gathers
+// of the extended rows; for few patches the chain of one workgroup. lvl: 2K + 1 u32 per patch (cnt[0..K], ent[0..K-1]).
 struct PlanSK
 {
     uint16_t *ro, *nb;
@@ -588,66 +732,56 @@ __global__ __launch_bounds__(T) void k_smoothk(DevMesh m, uint32_t K, const uint
     Bump            b(reinterpret_cast<char*>(smem));
     const PlanSK    L = plan_sk(b, nin, ncomp, nent);
     {
-        // staging in two levels of global loads: (1) rows and the extended
-        // vertices' linear ids, (2) the position gathers
-        constexpr uint32_t R1 = 2, RN = 6, RV = 4;
-        const uint32_t     t   = threadIdx.x;
-        const uint32_t     nro = (ncomp + 1u + 7u) >> 3, nnb = (nent + 7u) >> 3;
-        const uint4*       rs  = reinterpret_cast<const uint4*>(roff + rbase[p]);
-        const uint4*       ns  = reinterpret_cast<const uint4*>(nbr + nbase[p]);
-        const uint32_t*    xl  = xlin + xbase[p];
-        uint4*             rd  = reinterpret_cast<uint4*>(L.ro);
-        uint4*             nd  = reinterpret_cast<uint4*>(L.nb);
-        uint4              ra[R1], na[RN];
-        uint32_t           g[RV];
+        // first round trip: rows, ring ids and owned positions; second: the
+        // rings' positions
+        constexpr uint32_t RO = (512u + T - 1u) / T, RX = (512u + T - 1u) / T;
+        const uint32_t     t = threadIdx.x, nvo = d.nvo, nx = nin - nvo;
+        const u32x4 *      rs = as_words(roff + rbase[p]), *ns = as_words(nbr + nbase[p]);
+        const uint32_t*    xl = xlin + xbase[p];
+        Held<T, RX, uint32_t>               hx;
+        Held<T, 1, u32x4>                   hro;
+        Held<T, (512u + T - 1u) / T, u32x4> hnb;
+        float                               o[RO][3], q[RX][3];
+        hx.load(xl, nx);
+        hro.load(rs, words8(ncomp + 1u));
+        hnb.load(ns, words8(nent));
 #pragma unroll
-        for (uint32_t r = 0; r < R1; ++r) ra[r] = (t + r * T < nro) ? rs[t + r * T] : uint4{};
+        for (uint32_t r = 0; r < RO; ++r)
+            if (r == 0 || r * T < nvo)
 #pragma unroll
-        for (uint32_t r = 0; r < RN; ++r) na[r] = (t + r * T < nnb) ? ns[t + r * T] : uint4{};
+                for (uint32_t k = 0; k < 3; ++k) o[r][k] = pos[size_t(k) * N + min(d.vp + t + r * T, N - 1u)];
 #pragma unroll
-        for (uint32_t r = 0; r < RV; ++r) {
-            const uint32_t l = t + r * T;
-            g[r]             = (l < d.nvo) ? d.vp + l : ((l < nin) ? xl[l - d.nvo] : 0u);
-        }
-        float x[RV], y[RV], z[RV];
+        for (uint32_t r = 0; r < RX; ++r)
+            if (r * T < nx)
 #pragma unroll
-        for (uint32_t r = 0; r < RV; ++r) {
-            if (t + r * T < nin) {
-                x[r] = pos[g[r]];
-                y[r] = pos[N + g[r]];
-                z[r] = pos[2 * N + g[r]];
-            }
-        }
+                for (uint32_t k = 0; k < 3; ++k) q[r][k] = pos[size_t(k) * N + hx.a[r]];
+        hro.store(as_words(L.ro), rs, words8(ncomp + 1u));
+        hnb.store(as_words(L.nb), ns, words8(nent));
+        auto put = [&](uint32_t l, const float (&w)[3]) {
+            L.ax[l] = w[0];
+            L.ay[l] = w[1];
+            L.az[l] = w[2];
+        };
 #pragma unroll
-        for (uint32_t r = 0; r < R1; ++r)
-            if (t + r * T < nro) rd[t + r * T] = ra[r];
+        for (uint32_t r = 0; r < RO; ++r)
+            if (t + r * T < nvo) put(t + r * T, o[r]);
 #pragma unroll
-        for (uint32_t r = 0; r < RN; ++r)
-            if (t + r * T < nnb) nd[t + r * T] = na[r];
-#pragma unroll
-        for (uint32_t r = 0; r < RV; ++r) {
-            const uint32_t l = t + r * T;
-            if (l < nin) {
-                L.ax[l] = x[r];
-                L.ay[l] = y[r];
-                L.az[l] = z[r];
-            }
-        }
-        for (uint32_t i = t + R1 * T; i < nro; i += T) rd[i] = rs[i];
-        for (uint32_t i = t + RN * T; i < nnb; i += T) nd[i] = ns[i];
-        for (uint32_t l = t + RV * T; l < nin; l += T) {
-            const uint32_t gg = (l < d.nvo) ? d.vp + l : xl[l - d.nvo];
-            L.ax[l]           = pos[gg];
-            L.ay[l]           = pos[N + gg];
-            L.az[l]           = pos[2 * N + gg];
-        }
+        for (uint32_t r = 0; r < RX; ++r)
+            if (t + r * T < nx) put(nvo + t + r * T, q[r]);
+        auto direct = [&](uint32_t l, uint32_t gg) {
+            const float w[3] = {pos[gg], pos[size_t(N) + gg], pos[2 * size_t(N) + gg]};
+            put(l, w);
+        };
+        for (uint32_t l = t + RO * T; l < nvo; l += T) direct(l, d.vp + l);
+        for (uint32_t l = t + RX * T; l < nx; l += T) direct(nvo + l, xl[l]);
     }
     __syncthreads();
     const float *sx = L.ax, *sy = L.ay, *sz = L.az;
     float *      tx = L.bx, *ty = L.by, *tz = L.bz;
+    uint32_t     n  = c[steps - 1];
     for (uint32_t i = 1; i <= steps; ++i) {
-        const uint32_t n    = c[steps - i];
         const bool     last = (i == steps);
+        const uint32_t next = last ? 0u : c[steps - i - 1];  // in flight during this step
         for (uint32_t v = threadIdx.x; v < n; v += T) {
             const uint32_t k0 = L.ro[v], k1 = L.ro[v + 1];
             float          ax = 0.f, ay = 0.f, az = 0.f;
@@ -676,6 +810,7 @@ __global__ __launch_bounds__(T) void k_smoothk(DevMesh m, uint32_t K, const uint
                 tz[v] = rz;
             }
         }
+        n = next;
         if (!last) {
             __syncthreads();
             // the buffer just read becomes the next target (its prefix is large enough)

@@ -132,3 +132,28 @@ def test_symdir3_patch_sizes(patch_size):
     ref = _dirichlet_grad64(yg, F, rest)[l2g].T
     assert np.abs(g.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
     assert torch.allclose(step, y - 1e-3 * g, rtol=1e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("shape", ["sphere", "grid", "tiny"])
+@pytest.mark.parametrize("patch_size", [16, 256, 512, 1024, 4096])
+def test_multi_step_smoothing_equals_single_steps(shape, patch_size):
+    """Smoothing over the device-built ring plan (every number of steps per
+    launch, and the automatic choice after build_vv_plan) gives the bits of
+    single steps, whose values other tests check against FP64; patches of 4096
+    faces are beyond the plan kernel's tables and take the host walk."""
+    import torch
+    V, F = {"sphere": lambda: mg.permute_mesh(*mg.icosphere(5, seed=6, sigma=0.01), seed=6),
+            "grid": lambda: mg.grid(67, seed=6), "tiny": lambda: mg.icosphere(1, seed=6, sigma=0.01)}[shape]()
+    m, x = _mesh(V, F, patch_size)
+    m.set_launch_threads(8, 0)
+    ref = {k: m.smooth(x, 0.5, k) for k in range(1, 8)}
+    n, xn = _mesh(V, F, patch_size)
+    assert torch.equal(x, xn)
+    n.build_vv_plan()
+    for k in ref:
+        assert torch.equal(n.smooth(x, 0.5, k), ref[k])
+    for steps in range(1, 7):
+        for threads in (64, 128, 256, 512):
+            m.set_launch_threads(0, threads)
+            m.set_launch_threads(8, steps)
+            assert torch.equal(m.smooth(x, 0.5, 7), ref[7])
