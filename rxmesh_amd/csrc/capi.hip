@@ -1539,12 +1539,15 @@ rxm_status rxm_mcf_explicit(rxm_mesh* m, const int32_t* row_ptr, const int32_t* 
     if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
     Bump b(nullptr);
     plan_sl(b, m->h.max_nv, m->h.max_nvo, m->vv_max_nent, false);
-    b.alloc<float>(m->vv_max_nent + m->h.max_nvo);
+    b.alloc<float>(m->vv_max_nent + m->h.max_nvo + 3u);
     const float* src = x;
     for (int it = 0; it < iters && !rc; ++it) {
         float* dst = ((iters - 1 - it) % 2 == 0) ? out : tmp;
-        rc = launch_patches_xcd(k_mcf_patch<256>, 256, b.bytes(), stream, m, m->dm, vv_base, m->d_vv_rbase,
-                                m->d_vv_nbase, m->d_vv_roff, m->d_vv_nbr, val, mass, src, dst);
+        auto go = [&](auto kernel, uint32_t T) {
+            return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
+                                      m->d_vv_roff, m->d_vv_nbr, val, mass, src, dst);
+        };
+        rc = smooth_group(m) == 512u ? go(k_mcf_patch<512>, 512) : go(k_mcf_patch<256>, 256);
         src = dst;
     }
     return rc;

@@ -845,6 +845,33 @@ __host__ __device__ inline PlanVNP plan_vnp(Bump& b, uint32_t nv, uint32_t nvo, 
     return p;
 }
 
+// Face plan and positions of a patch into LDS, every load issued before the
+// first is waited for. L: fvl, ro, vf, x, y, z.
+template <uint32_t T, typename Plan>
+__device__ __forceinline__ void stage_face_plan(const DevMesh& m, const PatchDesc& d, const uint16_t* __restrict__ fvl,
+                                                const uint16_t* __restrict__ roff, const uint16_t* __restrict__ vf,
+                                                uint32_t nent, const float* __restrict__ pos, const Plan& L)
+{
+    HeldVerts<T, 3>                     hv;
+    Held<T, (320u + T - 1u) / T, u32x4> h_fvl;
+    Held<T, (256u + T - 1u) / T, u32x4> h_vf;
+    Held<T, 1, u32x4>                   h_ro;
+    hv.ids(m, d);
+    h_fvl.load(as_words(fvl), words8(3 * d.nf));
+    h_ro.load(as_words(roff), words8(d.nvo + 1));
+    h_vf.load(as_words(vf), words8(nent));
+    hv.owned(pos, m, d);
+    hv.ribbon(pos, m, d);
+    h_fvl.store(as_words(L.fvl), as_words(fvl), words8(3 * d.nf));
+    h_ro.store(as_words(L.ro), as_words(roff), words8(d.nvo + 1));
+    h_vf.store(as_words(L.vf), as_words(vf), words8(nent));
+    hv.store(pos, m, d, [&](uint32_t l, const float (&w)[3]) {
+        L.x[l] = w[0];
+        L.y[l] = w[1];
+        L.z[l] = w[2];
+    });
+}
+
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_vertex_normals_plan(DevMesh m, int mode, const uint32_t* __restrict__ fbase,
                                                            const uint32_t* __restrict__ rbase,
@@ -862,10 +889,7 @@ __global__ __launch_bounds__(T) void k_vertex_normals_plan(DevMesh m, int mode, 
     Bump            b(reinterpret_cast<char*>(smem));
     const PlanVNP   L = plan_vnp(b, d.nv, d.nvo, d.nf, nent);
     const uint32_t  N = m.nV;
-    stage_u16x8<T>(L.fvl, fvl + fbase[p], 3 * d.nf);
-    stage_u16x8<T>(L.ro, roff + rbase[p], d.nvo + 1);
-    stage_u16x8<T>(L.vf, vf + nb0, nent);
-    stage_positions_batched<T, 512u / T, false>(L.x, L.y, L.z, nullptr, pos, N, d, m.v_lin);
+    stage_face_plan<T>(m, d, fvl + fbase[p], roff + rbase[p], vf + nb0, nent, pos, L);
     __syncthreads();
     for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
         float sx = 0.f, sy = 0.f, sz = 0.f;
@@ -974,10 +998,7 @@ __global__ __launch_bounds__(T) void k_gaussian_curvature(DevMesh m, const uint3
     Bump            b(reinterpret_cast<char*>(smem));
     const PlanGC    L = plan_gc(b, d.nv, d.nvo, d.nf, nent);
     const uint32_t  N = m.nV;
-    stage_u16x8<T>(L.fvl, fvl + fbase[p], 3 * d.nf);
-    stage_u16x8<T>(L.ro, roff + rbase[p], d.nvo + 1);
-    stage_u16x8<T>(L.vf, vf + nb0, nent);
-    stage_positions_batched<T, (512u + T - 1u) / T, false>(L.x, L.y, L.z, nullptr, pos, N, d, m.v_lin);
+    stage_face_plan<T>(m, d, fvl + fbase[p], roff + rbase[p], vf + nb0, nent, pos, L);
     __syncthreads();
     for (uint32_t f = threadIdx.x; f < d.nf; f += T) {
         float px[3], py[3], pz[3];

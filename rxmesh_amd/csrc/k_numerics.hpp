@@ -536,13 +536,34 @@ __global__ __launch_bounds__(T) void k_mcf_patch(DevMesh m, const uint32_t* __re
     const uint32_t  N    = m.nV;
     Bump            b(reinterpret_cast<char*>(smem));
     const PlanSL    L = plan_sl(b, d.nv, d.nvo, nent, false);
-    float*          w = b.alloc<float>(nent + d.nvo);
-    stage_u16x8<T>(L.ro, roff + rb, d.nvo + 1);
-    stage_u16x8<T>(L.nb, nbr + nbb, nent);
-    stage_words<T, 8>(reinterpret_cast<uint32_t*>(w), reinterpret_cast<const uint32_t*>(val) + bse, nent + d.nvo);
-    stage_positions_batched<T, 512u / T, false>(L.x, L.y, L.z, nullptr, x, N, d, m.v_lin);
+    float*          wl = b.alloc<float>(nent + d.nvo + 3u);
+    const float*    vsrc = val + bse;
+    const uint32_t  t = threadIdx.x;
+    HeldVerts<T, 3>                     hv;
+    HeldFloats<T, (512u + T - 1u) / T>  hw;
+    Held<T, (256u + T - 1u) / T, u32x4> h_nb;
+    Held<T, 1, u32x4>                   h_ro;
+    float                               M[HeldVerts<T, 3>::RO];
+    hv.ids(m, d);
+    h_ro.load(as_words(roff + rb), words8(d.nvo + 1));
+    h_nb.load(as_words(nbr + nbb), words8(nent));
+    hw.load(vsrc, nent + d.nvo);
+    hv.owned(x, m, d);
+#pragma unroll
+    for (uint32_t k = 0; k < HeldVerts<T, 3>::RO; ++k)
+        if (k == 0 || k * T < d.nvo) M[k] = mass[min(d.vp + t + k * T, N - 1u)];
+    hv.ribbon(x, m, d);
+    h_ro.store(as_words(L.ro), as_words(roff + rb), words8(d.nvo + 1));
+    h_nb.store(as_words(L.nb), as_words(nbr + nbb), words8(nent));
+    hw.store(wl, vsrc, nent + d.nvo);
+    hv.store(x, m, d, [&](uint32_t l, const float (&q)[3]) {
+        L.x[l] = q[0];
+        L.y[l] = q[1];
+        L.z[l] = q[2];
+    });
+    const float* w = wl + hw.shift(vsrc);
     __syncthreads();
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
+    auto row = [&](uint32_t v, float Mv) {
         const uint32_t k0 = L.ro[v], k1 = L.ro[v + 1];
         const float*   wr = w + k0 + v;  // diagonal, then the row's neighbours
         const float    px = L.x[v], py = L.y[v], pz = L.z[v];
@@ -555,11 +576,14 @@ __global__ __launch_bounds__(T) void k_mcf_patch(DevMesh m, const uint32_t* __re
             az += c * L.z[q];
         }
         const uint32_t g = d.vp + v;
-        const float    M = mass[g];
-        y[g]             = px + (M * px - ax) / M;
-        y[N + g]         = py + (M * py - ay) / M;
-        y[2 * N + g]     = pz + (M * pz - az) / M;
-    }
+        y[g]             = px + (Mv * px - ax) / Mv;
+        y[N + g]         = py + (Mv * py - ay) / Mv;
+        y[2 * N + g]     = pz + (Mv * pz - az) / Mv;
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < HeldVerts<T, 3>::RO; ++k)
+        if (t + k * T < d.nvo) row(t + k * T, M[k]);
+    for (uint32_t v = t + HeldVerts<T, 3>::RO * T; v < d.nvo; v += T) row(v, mass[d.vp + v]);
 }
 
 // ---- implicit MCF: conjugate gradients on the cotangent system ---------------
