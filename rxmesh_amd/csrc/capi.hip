@@ -44,6 +44,7 @@ struct rxm_mesh
     const uint32_t* d_vv_nbase = nullptr;
     uint16_t*       d_vv_roff  = nullptr;
     uint16_t*       d_vv_nbr   = nullptr;
+    uint16_t*       d_vv_ent   = nullptr;  // half-edges beside the neighbours
     uint32_t        vv_max_nent = 0;
     // two-step smoothing plan (host copy built on demand, device copy on first use)
     mutable Vv2Plan   vv2;
@@ -87,8 +88,6 @@ struct rxm_mesh
     const uint32_t* d_cot_closed = nullptr;
     const uint32_t* d_cot_plist  = nullptr;
     uint32_t        cot_nplist   = 0;
-    const uint16_t* d_cot_ent    = nullptr;  // patch-local VV edge pattern (build_vv_edge_pattern)
-    const uint32_t* d_cot_rs     = nullptr;
     uint32_t        smooth_threads = 0;        // 0: by the patch count (smooth_group)
     uint32_t        ring_threads   = 256;      // oriented VV, VE
     uint32_t        cot_threads    = 512;      // cotangent assembly
@@ -351,11 +350,16 @@ int ensure_vv_plan(rxm_mesh* m, void* stream)
     if (hipMalloc(&m->d_vv_nbr, sizeof(uint16_t) * std::max<uint32_t>(nb[h.P], 8)) != hipSuccess)
         return RXM_ERR_OUT_OF_MEMORY;
     m->allocs.push_back(m->d_vv_nbr);
-    m->device_bytes += 2ull * (rb[h.P] + nb[h.P]);
+    if (hipMalloc(&m->d_vv_ent, sizeof(uint16_t) * std::max<uint32_t>(nb[h.P], 8)) != hipSuccess) {
+        m->d_vv_nbr = nullptr;
+        return RXM_ERR_OUT_OF_MEMORY;
+    }
+    m->allocs.push_back(m->d_vv_ent);
+    m->device_bytes += 2ull * (rb[h.P] + 2ull * nb[h.P]);
     Bump b(nullptr);
     plan_vvl(b, h.max_ne, h.max_nvo);
     rc = launch_patches(k_query2_vv_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm,
-                        m->d_vv_rbase, m->d_vv_nbase, m->d_vv_roff, m->d_vv_nbr);
+                        m->d_vv_rbase, m->d_vv_nbase, m->d_vv_roff, m->d_vv_nbr, m->d_vv_ent);
     if (rc) {
         m->d_vv_nbr = nullptr;  // freed with the mesh; rebuild on the next call
         return rc;
@@ -462,46 +466,6 @@ int ensure_vv2_plan(rxm_mesh* m)
     return rc;
 }
 
-// Static part of the cotangent system, built once per mesh (the role of the
-// reference's SparseMatrix constructor): the patch-local VV edge pattern, the
-// closed-fan bitmask (per linear vertex id) and the list of patches with
-// owned vertices outside it, for the ring-row pass.
-int ensure_cot_plan(rxm_mesh* m)
-{
-    if (m->d_cot_closed) return RXM_OK;
-    const HostMesh&       h = m->h;
-    std::vector<uint16_t> ent;
-    std::vector<uint32_t> rs;
-    if (!build_vv_edge_pattern(h, op_base(m, RXM_OP_VV), ent, rs)) return RXM_ERR_PATCH_TOO_BIG;
-    int rc0 = upload(m, ent, m->d_cot_ent);
-    if (!rc0) rc0 = upload(m, rs, m->d_cot_rs);
-    if (rc0) return rc0;
-    std::vector<uint8_t> closed;
-    closed_fan_vertices(h, closed);
-    std::vector<uint32_t> bits((h.nV + 31) / 32, 0), plist;
-    for (uint32_t p = 0; p < h.P; ++p) {
-        bool ring = false;
-        for (uint32_t l = 0; l < h.nvo[p]; ++l) {
-            const uint32_t lin = h.vp[p] + l;
-            if (closed[h.ltog_v[h.v_off[p] + l]]) bits[lin >> 5] |= 1u << (lin & 31u);
-            else ring = true;
-        }
-        if (ring) plist.push_back(p);
-    }
-    const uint32_t* dl = nullptr;
-    int             rc = upload(m, plist, dl);
-    if (!rc) rc = upload(m, bits, m->d_cot_closed);  // last: marks the plan complete
-    if (rc) {
-        m->d_cot_closed = nullptr;
-        return rc;
-    }
-    m->d_cot_plist = dl;
-    m->cot_nplist  = static_cast<uint32_t>(plist.size());
-    return RXM_OK;
-}
-
-constexpr uint32_t kSmoothLevels = 6;  // rings of the K-level plan: up to 6 steps per launch
-
 // Uninitialised device array owned by the mesh.
 template <typename T>
 int device_array(rxm_mesh* m, size_t n, T** out)
@@ -514,6 +478,44 @@ int device_array(rxm_mesh* m, size_t n, T** out)
     *out = p;
     return RXM_OK;
 }
+
+// Static part of the cotangent system, built once per mesh (the role of the
+// reference's SparseMatrix constructor): the VV plan's rows and half-edges, the
+// closed-fan bitmask (per linear vertex id) and the list of patches with
+// owned vertices outside it, for the ring-row pass. Waits for the stream.
+int ensure_cot_plan(rxm_mesh* m, void* stream)
+{
+    if (m->d_cot_closed) return RXM_OK;
+    int rc = ensure_vv_plan(m, stream);
+    if (rc) return rc;
+    const HostMesh& h  = m->h;
+    const size_t    nw = (h.nV + 31u) / 32u;
+    hipStream_t     hs = static_cast<hipStream_t>(stream);
+    uint32_t*       bits = nullptr;  // bitmask, then a flag per patch
+    if ((rc = device_array(m, nw + h.P, &bits))) return rc;
+    hipLaunchKernelGGL(k_fill_u32, dim3(static_cast<uint32_t>((nw + h.P + 255) / 256)), dim3(256), 0, hs,
+                       static_cast<uint32_t>(nw + h.P), 0u, bits);
+    Bump b(nullptr);
+    b.alloc<uint32_t>(r4(h.max_ne));
+    b.alloc<uint16_t>(r4(3 * h.max_nf));
+    b.alloc<uint16_t>(2 * h.max_ne);
+    rc = launch_patches(k_closed_fans<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm, m->d_vv_rbase,
+                        m->d_vv_nbase, static_cast<const uint16_t*>(m->d_vv_roff),
+                        static_cast<const uint16_t*>(m->d_vv_nbr), static_cast<const uint16_t*>(m->d_vv_ent), bits,
+                        bits + nw);
+    if (rc) return rc;
+    std::vector<uint32_t> ring(h.P), plist;
+    RXM_HIP(hipMemcpyAsync(ring.data(), bits + nw, h.P * sizeof(uint32_t), hipMemcpyDeviceToHost, hs));
+    RXM_HIP(hipStreamSynchronize(hs));
+    for (uint32_t p = 0; p < h.P; ++p)
+        if (ring[p]) plist.push_back(p);
+    if ((rc = upload(m, plist, m->d_cot_plist))) return rc;
+    m->cot_nplist   = static_cast<uint32_t>(plist.size());
+    m->d_cot_closed = bits;  // last: marks the plan complete
+    return RXM_OK;
+}
+
+constexpr uint32_t kSmoothLevels = 6;  // rings of the K-level plan: up to 6 steps per launch
 
 // The K-level plan over K rings, built by k_ring_plan from the VV plan (waits
 // for the stream to size it): 2 launches instead of a host walk with a map per
@@ -1208,10 +1210,10 @@ rxm_status rxm_arap_weights(rxm_mesh* m, const float* pos, float* w, void* strea
 }
 
 namespace {
-// the owned rows' edges (the VV edge pattern the cotangent assembly caches)
-int arap_rows(rxm_mesh* m, const uint32_t** vv_base, uint32_t* lds, bool rot)
+// the owned rows (the VV plan) and the LDS of the kernels over them
+int arap_rows(rxm_mesh* m, const uint32_t** vv_base, uint32_t* lds, bool rot, void* stream)
 {
-    int rc = ensure_cot_plan(m);
+    int rc = ensure_vv_plan(m, stream);
     if (!rc) rc = device_base(m, RXM_OP_VV, vv_base);
     if (rc) return rc;
     Bump b(nullptr);
@@ -1228,10 +1230,11 @@ rxm_status rxm_arap_rotations(rxm_mesh* m, const float* rest, const float* x, co
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
     const uint32_t* vv_base = nullptr;
     uint32_t        lds     = 0;
-    const int       rc      = arap_rows(m, &vv_base, &lds, false);
+    const int       rc      = arap_rows(m, &vv_base, &lds, false, stream);
     if (rc) return rc;
     return launch_patches_xcd(k_arap_rotations<512>, 512, lds, stream, m, m->dm, vv_base,
-                              static_cast<const uint32_t*>(m->d_cot_rs), m->d_cot_ent,
+                              m->d_vv_rbase, m->d_vv_nbase, static_cast<const uint16_t*>(m->d_vv_roff),
+                              static_cast<const uint16_t*>(m->d_vv_nbr), static_cast<const uint16_t*>(m->d_vv_ent),
                               rest, x, w, R);
 }
 
@@ -1242,7 +1245,7 @@ rxm_status rxm_arap_energy_grad(rxm_mesh* m, const float* rest, const float* x, 
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
     const uint32_t* vv_base = nullptr;
     uint32_t        lds     = 0;
-    int             rc      = arap_rows(m, &vv_base, &lds, true);
+    int             rc      = arap_rows(m, &vv_base, &lds, true, stream);
     if (rc) return rc;
     if (!m->d_partial) {
         if (hipMalloc(&m->d_partial, sizeof(float) * m->h.P) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
@@ -1250,8 +1253,8 @@ rxm_status rxm_arap_energy_grad(rxm_mesh* m, const float* rest, const float* x, 
         m->device_bytes += sizeof(float) * m->h.P;
     }
     rc = launch_patches_xcd(k_arap_energy_grad<512>, 512, lds, stream, m, m->dm, vv_base,
-                            static_cast<const uint32_t*>(m->d_cot_rs), m->d_cot_ent,
-                            rest, x, w, R, m->d_partial, grad);
+                            m->d_vv_rbase, m->d_vv_nbase, static_cast<const uint16_t*>(m->d_vv_roff),
+                            static_cast<const uint16_t*>(m->d_vv_ent), rest, x, w, R, m->d_partial, grad);
     if (rc) return rc;
     hipLaunchKernelGGL(k_reduce_sum, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), m->h.P,
                        static_cast<const float*>(m->d_partial), total);
@@ -1456,7 +1459,8 @@ static int launch_cot_assemble(rxm_mesh* m, const uint32_t* vv_base, const float
     Bump b(nullptr);
     plan_cot(b, m->h.max_nv, m->h.max_ne, m->h.max_nvo, op_max_patch(m, RXM_OP_VV));
     auto go = [&](auto kernel, uint32_t threads) {
-        return launch_patches_xcd(kernel, threads, b.bytes(), stream, m, m->dm, vv_base, m->d_cot_rs, m->d_cot_ent,
+        return launch_patches_xcd(kernel, threads, b.bytes(), stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
+                                  static_cast<const uint16_t*>(m->d_vv_roff), static_cast<const uint16_t*>(m->d_vv_ent),
                                   pos, dt, row_ptr, col, val, mass, diag);
     };
     return (m->cot_threads == 512) ? go(k_cot_assemble<512, CSR>, 512) : go(k_cot_assemble<256, CSR>, 256);
@@ -1482,7 +1486,7 @@ rxm_status rxm_cot_csr_assemble(rxm_mesh* m, const float* pos, float dt, int32_t
     if (rc) return rc;
     const uint32_t* vv_base = nullptr;
     if ((rc = device_base(m, RXM_OP_VV, &vv_base))) return rc;
-    if ((rc = ensure_cot_plan(m))) return rc;
+    if ((rc = ensure_cot_plan(m, stream))) return rc;
     const uint32_t maxrow = op_max_patch(m, kOpCot);
     rc = launch_cot_assemble<true>(m, vv_base, pos, dt, row_ptr, col, val, mass, nullptr, stream);
     if (rc || m->cot_nplist == 0) return rc;
@@ -1677,7 +1681,7 @@ rxm_status rxm_mcf_matfree_cg(rxm_mesh* m, const float* coords, const float* x, 
     int        rc  = RXM_OK;
     if (!uni) {
         if (!(m->h.manifold && m->h.oriented)) return RXM_ERR_NON_MANIFOLD;
-        if ((rc = ensure_cot_plan(m))) return rc;
+        if ((rc = ensure_cot_plan(m, stream))) return rc;
         // the face pass gives a vertex its reference weights only when its
         // ring is one closed fan (a closed vertex-manifold mesh)
         if (m->cot_nplist != 0) return RXM_ERR_UNSUPPORTED;

@@ -190,22 +190,24 @@ __device__ inline void best_rotation(const float (&S)[3][3], float (&R)[3][3])
     R[2][2] = q0 * q0 - qx * qx - qy * qy + qz * qz;
 }
 
-// Patch-local data of the rotation and energy kernels: EV, the owned rows'
-// edges (the cached VV edge pattern, VV query order), rest and deformed
-// positions and (energy kernel) rotations of every local vertex, weights of
-// every local edge.
+// Patch-local data of the rotation and energy kernels: the VV plan's rows
+// (offsets, neighbours or half-edges), rest and deformed positions of every
+// local vertex, weights of every local edge; for the energy also EV and the
+// rotations of every local vertex, whose space then takes the residuals of the
+// local edges (three floats each).
 struct PlanAR
 {
-    uint32_t *ev, *rs;
-    uint16_t* ent;
+    uint32_t* ev;
+    uint16_t *ro, *nb, *ent;
     float *   px, *py, *pz, *xx, *xy, *xz, *w, *rot;
 };
 __host__ __device__ inline PlanAR plan_ar(Bump& b, uint32_t nv, uint32_t ne, uint32_t nvo, uint32_t nent, bool rot)
 {
     PlanAR p{};
-    p.ev  = b.alloc<uint32_t>(r4(ne));
-    p.rs  = b.alloc<uint32_t>(nvo + 1);
-    p.ent = b.alloc<uint16_t>(nent);
+    p.ev  = rot ? b.alloc<uint32_t>(r4(ne)) : nullptr;
+    p.ro  = b.alloc<uint16_t>((nvo + 1u + 7u) & ~7u);
+    p.nb  = rot ? nullptr : b.alloc<uint16_t>((nent + 7u) & ~7u);
+    p.ent = b.alloc<uint16_t>((nent + 7u) & ~7u);
     p.px  = b.alloc<float>(nv);
     p.py  = b.alloc<float>(nv);
     p.pz  = b.alloc<float>(nv);
@@ -213,36 +215,98 @@ __host__ __device__ inline PlanAR plan_ar(Bump& b, uint32_t nv, uint32_t ne, uin
     p.xy  = b.alloc<float>(nv);
     p.xz  = b.alloc<float>(nv);
     p.w   = b.alloc<float>(ne);
-    p.rot = rot ? b.alloc<float>(9 * nv) : nullptr;
+    p.rot = rot ? b.alloc<float>(9 * nv + 3u > 3 * ne ? 9 * nv + 3u : 3 * ne) : nullptr;
     return p;
 }
 
-template <uint32_t T>
-__device__ __forceinline__ void stage_arap(const DevMesh& m, const PatchDesc& d, const PlanAR& L,
-                                           const uint32_t* __restrict__ rs, const uint16_t* __restrict__ ent,
-                                           uint32_t vb, uint32_t nent, const float* __restrict__ rest,
-                                           const float* __restrict__ x, const float* __restrict__ w,
-                                           const float* __restrict__ R)
+// Stage them, every load issued before the first is waited for, in two
+// dependent round trips (the ribbon's ids, then its words).
+// ROT: L.rot is moved to the first vertex's record.
+template <uint32_t T, bool ROT>
+__device__ __forceinline__ void stage_arap(const DevMesh& m, const PatchDesc& d, PlanAR& L,
+                                           const uint16_t* __restrict__ roff, const uint16_t* __restrict__ nbr,
+                                           const uint16_t* __restrict__ ent, uint32_t nent,
+                                           const float* __restrict__ rest, const float* __restrict__ x,
+                                           const float* __restrict__ w, const float* __restrict__ R)
 {
-    constexpr uint32_t RB = (512u + T - 1u) / T;
-    stage_u32(L.ev, m.ev + d.e_off, d.ne);
-    stage_halves<T, 8>(L.ent, ent + vb, nent);
-    stage_words<T, 2>(L.rs, rs + d.vp, d.nvo + 1, vb);
-    stage_positions_batched<T, RB, false>(L.px, L.py, L.pz, nullptr, rest, m.nV, d, m.v_lin);
-    stage_positions_batched<T, RB, false>(L.xx, L.xy, L.xz, nullptr, x, m.nV, d, m.v_lin);
-    const uint32_t* el = m.e_lin + d.e_off;
-    for (uint32_t e = threadIdx.x; e < d.ne; e += T) L.w[e] = w[lin_of(e, d.neo, d.ep, el)];
-    if (R) {
-        const uint32_t* vl = m.v_lin + d.v_off;
-        for (uint32_t l = threadIdx.x; l < d.nv; l += T) {
-            const float* r = R + 9ull * lin_of(l, d.nvo, d.vp, vl);  // one 36-byte record per vertex
-            float        t[9];
+    const uint32_t     t = threadIdx.x, ner = d.ne - d.neo;
+    constexpr uint32_t RW = (768u + T - 1u) / T, RX = (512u + T - 1u) / T;  // owned / ribbon edges in registers
+    const uint32_t*    el  = m.e_lin + d.e_off;
+    const u32x4*       evs = reinterpret_cast<const u32x4*>(m.ev + d.e_off);
+    HeldVerts<T, 3>                     hp, hx;
+    Held<T, (384u + T - 1u) / T, u32x4> h_ev;
+    Held<T, (256u + T - 1u) / T, u32x4> h_nb, h_ent;
+    Held<T, 1, u32x4>                   h_ro;
+    uint32_t                            ge[RX];
+    float                               wo[RW], wr[RX];
+    // rotations: the owned vertices' records are one run of 9 nvo floats, the
+    // ribbon's are gathered word by word (record j of the ribbon at 9 (nvo + j))
+    constexpr uint32_t            RQ = (1536u + T - 1u) / T;
+    const uint32_t                nq = 9u * (d.nv - d.nvo);
+    const float*                  Ro = R + 9ull * d.vp;
+    HeldFloats<T, (768u + T - 1u) / T> h_rot;
+    uint32_t                      gq[RQ];
+    float                         rq[RQ];
+    auto rec = [&](uint32_t i) { return min(d.nvo + i / 9u, d.nv - 1u); };
+    hp.ids(m, d);
+    if constexpr (ROT)
 #pragma unroll
-            for (uint32_t c = 0; c < 9; ++c) t[c] = r[c];
+        for (uint32_t k = 0; k < RQ; ++k)
+            if (k == 0 || k * T < nq) gq[k] = m.v_lin[d.v_off + rec(t + k * T)];
 #pragma unroll
-            for (uint32_t c = 0; c < 9; ++c) L.rot[9 * l + c] = t[c];
-        }
+    for (uint32_t k = 0; k < RX; ++k)
+        if (k == 0 || k * T < ner) ge[k] = el[min(d.neo + t + k * T, d.ne - 1u)];
+    if constexpr (ROT) h_ev.load(evs, r4(d.ne) >> 2);
+    h_ro.load(as_words(roff), words8(d.nvo + 1));
+    h_ent.load(as_words(ent), words8(nent));
+    if constexpr (!ROT) h_nb.load(as_words(nbr), words8(nent));
+    if constexpr (ROT) h_rot.load(Ro, 9u * d.nvo);
+    hp.owned(rest, m, d);
+    hx.owned(x, m, d);
+#pragma unroll
+    for (uint32_t k = 0; k < RW; ++k)
+        if (k == 0 || k * T < d.neo) wo[k] = w[min(d.ep + t + k * T, m.nE - 1u)];
+#pragma unroll
+    for (uint32_t k = 0; k < HeldVerts<T, 3>::RR; ++k) hx.g[k] = hp.g[k];
+    hp.ribbon(rest, m, d);
+    hx.ribbon(x, m, d);
+#pragma unroll
+    for (uint32_t k = 0; k < RX; ++k)
+        if (k == 0 || k * T < ner) wr[k] = w[ge[k]];
+    if constexpr (ROT) {
+#pragma unroll
+        for (uint32_t k = 0; k < RQ; ++k)
+            if (k == 0 || k * T < nq) rq[k] = R[9ull * gq[k] + (t + k * T) % 9u];
+        h_rot.store(L.rot, Ro, 9u * d.nvo);
+        L.rot += h_rot.shift(Ro);
+#pragma unroll
+        for (uint32_t k = 0; k < RQ; ++k)
+            if (t + k * T < nq) L.rot[9u * d.nvo + t + k * T] = rq[k];
+        for (uint32_t i = t + RQ * T; i < nq; i += T)
+            L.rot[9u * d.nvo + i] = R[9ull * m.v_lin[d.v_off + rec(i)] + i % 9u];
+        h_ev.store(reinterpret_cast<u32x4*>(L.ev), evs, r4(d.ne) >> 2);
     }
+    h_ro.store(as_words(L.ro), as_words(roff), words8(d.nvo + 1));
+    h_ent.store(as_words(L.ent), as_words(ent), words8(nent));
+    if constexpr (!ROT) h_nb.store(as_words(L.nb), as_words(nbr), words8(nent));
+    hp.store(rest, m, d, [&](uint32_t l, const float (&q)[3]) {
+        L.px[l] = q[0];
+        L.py[l] = q[1];
+        L.pz[l] = q[2];
+    });
+    hx.store(x, m, d, [&](uint32_t l, const float (&q)[3]) {
+        L.xx[l] = q[0];
+        L.xy[l] = q[1];
+        L.xz[l] = q[2];
+    });
+#pragma unroll
+    for (uint32_t k = 0; k < RW; ++k)
+        if (t + k * T < d.neo) L.w[t + k * T] = wo[k];
+#pragma unroll
+    for (uint32_t k = 0; k < RX; ++k)
+        if (t + k * T < ner) L.w[d.neo + t + k * T] = wr[k];
+    for (uint32_t e = t + RW * T; e < d.neo; e += T) L.w[e] = w[d.ep + e];
+    for (uint32_t e = d.neo + t + RX * T; e < d.ne; e += T) L.w[e] = w[el[e]];
 }
 
 // Best rotation per owned vertex (arap_kernels.h:60-117): S = sum over the
@@ -252,7 +316,10 @@ __device__ __forceinline__ void stage_arap(const DevMesh& m, const PatchDesc& d,
 // one or two cache lines for the energy kernel's gather, not nine.
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_arap_rotations(DevMesh m, const uint32_t* __restrict__ vv_base,
-                                                      const uint32_t* __restrict__ rs,
+                                                      const uint32_t* __restrict__ rbase,
+                                                      const uint32_t* __restrict__ nbase,
+                                                      const uint16_t* __restrict__ roff,
+                                                      const uint16_t* __restrict__ nbr,
                                                       const uint16_t* __restrict__ ent,
                                                       const float* __restrict__ rest, const float* __restrict__ x,
                                                       const float* __restrict__ w, float* __restrict__ R)
@@ -260,20 +327,20 @@ __global__ __launch_bounds__(T) void k_arap_rotations(DevMesh m, const uint32_t*
     extern __shared__ uint4 smem[];
     const uint32_t p = patch_of_block(m.P);  // XCD-contiguous patch ranges
     if (p >= m.P) return;
-    const PatchDesc d  = load_desc(m.patch, p);
-    const uint32_t  vb = vv_base[p], nent = vv_base[p + 1] - vb;
+    const PatchDesc d    = load_desc(m.patch, p);
+    const uint32_t  nent = vv_base[p + 1] - vv_base[p];
     Bump            b(reinterpret_cast<char*>(smem));
-    const PlanAR    L = plan_ar(b, d.nv, d.ne, d.nvo, nent, false);
-    stage_arap<T>(m, d, L, rs, ent, vb, nent, rest, x, w, nullptr);
+    PlanAR          L = plan_ar(b, d.nv, d.ne, d.nvo, nent, false);
+    stage_arap<T, false>(m, d, L, roff + rbase[p], nbr + nbase[p], ent + nbase[p], nent, rest, x, w, nullptr);
     __syncthreads();
     for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
-        float S[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-        for (uint32_t k = L.rs[v]; k < L.rs[v + 1]; ++k) {
-            const uint32_t e = L.ent[k] >> 1, y = L.ev[e];
-            const uint32_t j = (lo16(y) == v) ? hi16(y) : lo16(y);
-            const float    wt = L.w[e];
-            const float    a[3] = {L.px[v] - L.px[j], L.py[v] - L.py[j], L.pz[v] - L.pz[j]};
-            const float    c[3] = {L.xx[v] - L.xx[j], L.xy[v] - L.xy[j], L.xz[v] - L.xz[j]};
+        float       S[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+        const float p0 = L.px[v], p1 = L.py[v], p2 = L.pz[v], x0 = L.xx[v], x1 = L.xy[v], x2 = L.xz[v];
+        for (uint32_t k = L.ro[v]; k < L.ro[v + 1]; ++k) {
+            const uint32_t j = L.nb[k];
+            const float    wt = L.w[L.ent[k] >> 1];
+            const float    a[3] = {p0 - L.px[j], p1 - L.py[j], p2 - L.pz[j]};
+            const float    c[3] = {x0 - L.xx[j], x1 - L.xy[j], x2 - L.xz[j]};
 #pragma unroll
             for (int r = 0; r < 3; ++r)
 #pragma unroll
@@ -304,37 +371,76 @@ __device__ __forceinline__ f3 arap_residual(const PlanAR& L, uint32_t i, uint32_
 // P_j)|^2 (diff_arap.cu:87-118), one partial per patch; gradient with the
 // rotations held fixed (the reference's term reads them as constants):
 // dE/dX_v = sum over v's edges of +-2 w d, + where v is the edge's i.
+// Every local edge's residual is evaluated once, into registers, and stored
+// over the rotations once all are done; the gradient gathers them per vertex
+// (patches beyond the register rounds evaluate an edge at each use). AENOTE
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_arap_energy_grad(DevMesh m, const uint32_t* __restrict__ vv_base,
-                                                        const uint32_t* __restrict__ rs,
+                                                        const uint32_t* __restrict__ rbase,
+                                                        const uint32_t* __restrict__ nbase,
+                                                        const uint16_t* __restrict__ roff,
                                                         const uint16_t* __restrict__ ent,
                                                         const float* __restrict__ rest, const float* __restrict__ x,
                                                         const float* __restrict__ w, const float* __restrict__ R,
                                                         float* __restrict__ partial, float* __restrict__ grad)
 {
+    constexpr uint32_t RE = (1536u + T - 1u) / T;  // edges in registers
     extern __shared__ uint4 smem[];
     __shared__ float red[T / 64u];
     const uint32_t   p = patch_of_block(m.P);  // XCD-contiguous patch ranges
     if (p >= m.P) return;
-    const PatchDesc d  = load_desc(m.patch, p);
-    const uint32_t  vb = vv_base[p], nent = vv_base[p + 1] - vb;
+    const PatchDesc d    = load_desc(m.patch, p);
+    const uint32_t  nent = vv_base[p + 1] - vv_base[p], t = threadIdx.x;
     Bump            b(reinterpret_cast<char*>(smem));
-    const PlanAR    L = plan_ar(b, d.nv, d.ne, d.nvo, nent, true);
-    stage_arap<T>(m, d, L, rs, ent, vb, nent, rest, x, w, R);
+    PlanAR          L = plan_ar(b, d.nv, d.ne, d.nvo, nent, true);
+    float* const    res = L.rot;  // the residuals' space
+    stage_arap<T, true>(m, d, L, roff + rbase[p], nullptr, ent + nbase[p], nent, rest, x, w, R);
     __syncthreads();
-    float acc = 0.f;
-    for (uint32_t e = threadIdx.x; e < d.neo; e += T) {
-        const uint32_t y = L.ev[e];
-        const f3       r = arap_residual(L, lo16(y), hi16(y));
-        acc += L.w[e] * dot(r, r);
+    float      acc  = 0.f;
+    const bool held = d.ne <= RE * T;
+    float *    rx = res, *ry = rx + d.ne, *rz = ry + d.ne;
+    if (held) {
+        f3 r[RE];
+#pragma unroll
+        for (uint32_t k = 0; k < RE; ++k) {
+            const uint32_t e = t + k * T;
+            if (e < d.ne) {
+                const uint32_t y = L.ev[e];
+                r[k]             = arap_residual(L, lo16(y), hi16(y));
+                if (e < d.neo) acc += L.w[e] * dot(r[k], r[k]);
+            }
+        }
+        __syncthreads();  // every rotation has been read
+#pragma unroll
+        for (uint32_t k = 0; k < RE; ++k) {
+            const uint32_t e = t + k * T;
+            if (e < d.ne) {
+                rx[e] = r[k].x;
+                ry[e] = r[k].y;
+                rz[e] = r[k].z;
+            }
+        }
+        __syncthreads();
+    } else {
+        for (uint32_t e = t; e < d.neo; e += T) {
+            const uint32_t y = L.ev[e];
+            const f3       r = arap_residual(L, lo16(y), hi16(y));
+            acc += L.w[e] * dot(r, r);
+        }
     }
     const uint32_t N = m.nV;
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
+    for (uint32_t v = t; v < d.nvo; v += T) {
         float gx = 0.f, gy = 0.f, gz = 0.f;
-        for (uint32_t k = L.rs[v]; k < L.rs[v + 1]; ++k) {
-            const uint32_t e = L.ent[k] >> 1, y = L.ev[e];
-            const f3       r = arap_residual(L, lo16(y), hi16(y));
-            const float    s = (lo16(y) == v ? 2.f : -2.f) * L.w[e];
+        for (uint32_t k = L.ro[v]; k < L.ro[v + 1]; ++k) {
+            const uint32_t u = L.ent[k], e = u >> 1;  // the half-edge leaving v: dir 0 where v is the edge's i
+            f3             r;
+            if (held) {
+                r = f3{rx[e], ry[e], rz[e]};
+            } else {
+                const uint32_t y = L.ev[e];
+                r                = arap_residual(L, lo16(y), hi16(y));
+            }
+            const float s = ((u & 1u) ? -2.f : 2.f) * L.w[e];
             gx += s * r.x;
             gy += s * r.y;
             gz += s * r.z;
@@ -346,12 +452,12 @@ __global__ __launch_bounds__(T) void k_arap_energy_grad(DevMesh m, const uint32_
     }
     // fixed-order workgroup sum of the energy
     for (uint32_t o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = acc;
+    if ((t & 63u) == 0) red[t >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (uint32_t i = 0; i < T / 64u; ++i) t += red[i];
-        partial[p] = t;
+    if (t == 0) {
+        float s = 0.f;
+        for (uint32_t i = 0; i < T / 64u; ++i) s += red[i];
+        partial[p] = s;
     }
 }
 

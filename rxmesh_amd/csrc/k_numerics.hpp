@@ -119,19 +119,18 @@ __device__ __forceinline__ FaceCot face_cot(f3 P0, f3 P1, f3 P2)
     return r;
 }
 
-// LDS carve of the assembly: float4 positions and linear ids of the patch
-// vertices, the EV slab, per-edge half-edge terms he[e] = {cot(2e), vor(2e),
-// cot(2e + 1), vor(2e + 1)} (half-edge 2e + dir starts at the edge's
-// (dir ? hi16 : lo16) endpoint; cot = the clamped cotangent of the angle
-// opposite it in its face, vor = the partial Voronoi area of its start in
-// that face; zeros where no face of the patch holds it), and the patch's
-// pattern: row starts (nvo + 1) and entries (nent).
+// LDS carve of the assembly: float4 positions of the patch vertices, the
+// ribbon's linear ids, the EV slab, per-edge half-edge terms (half-edge 2e + dir
+// starts at the edge's (dir ? hi16 : lo16) endpoint; cot = the clamped cotangent
+// of the angle opposite it in its face, vor = the partial Voronoi area of its
+// start in that face; zeros where no face of the patch holds it), and the
+// patch's pattern: row starts (nvo + 1) and half-edge entries (nent).
 struct PlanCOT
 {
     float4*   pos;
     float2 *  cot, *vor;  // per edge: the two half-edges' opposite cotangents / start Voronoi terms
-    uint32_t *lin, *ev, *rs;
-    uint16_t* ent;
+    uint32_t *rid, *ev;
+    uint16_t *ro, *ent;
 };
 __host__ __device__ inline PlanCOT plan_cot(Bump& b, uint32_t nv, uint32_t ne, uint32_t nvo, uint32_t nent)
 {
@@ -139,103 +138,21 @@ __host__ __device__ inline PlanCOT plan_cot(Bump& b, uint32_t nv, uint32_t ne, u
     p.pos = b.alloc<float4>(nv);
     p.cot = b.alloc<float2>(ne);
     p.vor = b.alloc<float2>(ne);
-    p.lin = b.alloc<uint32_t>(nv);
+    p.rid = b.alloc<uint32_t>(nv);
     p.ev  = b.alloc<uint32_t>(r4(ne));
-    p.rs  = b.alloc<uint32_t>(nvo + 1);
-    p.ent = b.alloc<uint16_t>(nent);
+    p.ro  = b.alloc<uint16_t>((nvo + 1u + 7u) & ~7u);
+    p.ent = b.alloc<uint16_t>((nent + 7u) & ~7u);
     return p;
-}
-
-// Copy n u32 global -> LDS (any alignment), R loads of a thread in flight
-// before its stores; dst[i] = src[i] - sub.
-template <uint32_t T, uint32_t R>
-__device__ __forceinline__ void stage_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
-                                            uint32_t n, uint32_t sub = 0)
-{
-    for (uint32_t b0 = 0; b0 < n; b0 += R * T) {
-        uint32_t x[R];
-#pragma unroll
-        for (uint32_t r = 0; r < R; ++r) {
-            const uint32_t i = b0 + r * T + threadIdx.x;
-            x[r]             = (i < n) ? src[i] : 0u;
-        }
-#pragma unroll
-        for (uint32_t r = 0; r < R; ++r) {
-            const uint32_t i = b0 + r * T + threadIdx.x;
-            if (i < n) dst[i] = x[r] - sub;
-        }
-    }
-}
-
-// Copy n u16 global -> LDS (any alignment), R loads of a thread in flight
-// before its stores.
-template <uint32_t T, uint32_t R>
-__device__ __forceinline__ void stage_halves(uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, uint32_t n)
-{
-    for (uint32_t b0 = 0; b0 < n; b0 += R * T) {
-        uint16_t x[R];
-#pragma unroll
-        for (uint32_t r = 0; r < R; ++r) {
-            const uint32_t i = b0 + r * T + threadIdx.x;
-            x[r]             = (i < n) ? src[i] : uint16_t(0);
-        }
-#pragma unroll
-        for (uint32_t r = 0; r < R; ++r) {
-            const uint32_t i = b0 + r * T + threadIdx.x;
-            if (i < n) dst[i] = x[r];
-        }
-    }
-}
-
-// Stage, per patch vertex, its linear id (owned by prefix, ribbon from the
-// owner table) and position; all global loads of a thread are issued before
-// its LDS stores.
-template <uint32_t T>
-__device__ __forceinline__ void stage_vertices(const DevMesh& m, const PatchDesc& d, const float* __restrict__ pos,
-                                               float4* s_pos, uint32_t* s_lin)
-{
-    constexpr uint32_t R  = 2;
-    const uint32_t     N  = m.nV;
-    const uint32_t*    vl = m.v_lin + d.v_off;
-    uint32_t           g[R];
-    float              x[R], y[R], z[R];
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        const uint32_t l = threadIdx.x + r * T;
-        g[r]             = (l < d.nvo) ? d.vp + l : ((l < d.nv) ? vl[l] : 0u);
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        if (threadIdx.x + r * T < d.nv) {
-            x[r] = pos[g[r]];
-            y[r] = pos[N + g[r]];
-            z[r] = pos[2 * N + g[r]];
-        }
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        const uint32_t l = threadIdx.x + r * T;
-        if (l < d.nv) {
-            s_pos[l] = make_float4(x[r], y[r], z[r], 0.f);
-            s_lin[l] = g[r];
-        }
-    }
-    for (uint32_t l = threadIdx.x + R * T; l < d.nv; l += T) {
-        const uint32_t gg = lin_of(l, d.nvo, d.vp, vl);
-        s_pos[l]          = make_float4(pos[gg], pos[N + gg], pos[2 * N + gg], 0.f);
-        s_lin[l]          = gg;
-    }
 }
 
 // Rows of A = M + dt L over linear ids (apps/MCF/mcf_kernels.cuh:354-426,
 // mcf_A_setup): the diagonal, then the neighbours in VV query order
 // (ascending local id of the connecting edge), the column order SparseMatrix
 // fills (sparse_matrix_kernels.cuh:75-140); mass[v] = 1 / v_weight.
-// The pattern is static, like the reference's SparseMatrix: `ent` holds, in
-// VV query order, each owned row's entries of the patch as (local edge) |
-// (local row << 16), `rs` each linear vertex's first entry (patch-relative
-// offsets come from vv_base, the VV query's per-patch base; the system's
-// base is vv_base + the vertex prefix, one diagonal per owned row).
+// The pattern is static, like the reference's SparseMatrix: the VV plan's rows
+// (roff) and half-edge entries (ent); the patch's run of the system starts at
+// vv_base (the VV query's per-patch base) + the vertex prefix, one diagonal
+// per owned row.
 // Every face of the patch is evaluated once and stores, for each of its
 // half-edges, the cotangent opposite it and the Voronoi term of its start
 // (plain stores: a half-edge has one face on a consistently oriented
@@ -248,9 +165,13 @@ __device__ __forceinline__ void stage_vertices(const DevMesh& m, const PatchDesc
 // does, and are rewritten afterwards by k_cot_ring_rows.
 // CSR false: values, mass and, by vertex, the diagonal only (the weights of the
 // matrix-free solve); row_ptr and col are not written.
+// All loads of the staging are issued before the first is waited for, with
+// 16-byte loads of the pattern. COTNOTE
 template <uint32_t T, bool CSR = true>
 __global__ __launch_bounds__(T) void k_cot_assemble(DevMesh m, const uint32_t* __restrict__ vv_base,
-                                                    const uint32_t* __restrict__ rs,
+                                                    const uint32_t* __restrict__ rbase,
+                                                    const uint32_t* __restrict__ nbase,
+                                                    const uint16_t* __restrict__ roff,
                                                     const uint16_t* __restrict__ ent, const float* __restrict__ pos,
                                                     float dt, int32_t* __restrict__ row_ptr,
                                                     int32_t* __restrict__ col, float* __restrict__ val,
@@ -259,27 +180,45 @@ __global__ __launch_bounds__(T) void k_cot_assemble(DevMesh m, const uint32_t* _
     extern __shared__ uint4 smem[];
     const uint32_t p = patch_of_block(m.P);  // XCD-contiguous patch ranges
     if (p >= m.P) return;
-    const PatchDesc d    = load_desc(m.patch, p);
-    const uint32_t  vb   = vv_base[p], nent = vv_base[p + 1] - vb;
-    const uint32_t  bse  = vb + d.vp;  // first entry of the patch's rows
+    const PatchDesc d   = load_desc(m.patch, p);
+    const uint32_t  vb  = vv_base[p], nent = vv_base[p + 1] - vb;
+    const uint32_t  bse = vb + d.vp;  // first entry of the patch's rows
     Bump            b(reinterpret_cast<char*>(smem));
     const PlanCOT   L = plan_cot(b, d.nv, d.ne, d.nvo, nent);
+    const uint32_t  t = threadIdx.x;
     // the FE words of this thread's faces, loaded with the staging's loads
     constexpr uint32_t RF = (1024u + T - 1u) / T;
     const uint16_t*    fe = m.fe + 3u * d.f_off;
-    uint32_t           fw[RF][3];
+    const u32x4 *      evs = reinterpret_cast<const u32x4*>(m.ev + d.e_off), *ros = as_words(roff + rbase[p]),
+                *ens = as_words(ent + nbase[p]);
+    FaceWords                           fw[RF];
+    HeldVerts<T, 3>                     hv_;
+    Held<T, (384u + T - 1u) / T, u32x4> h_ev;
+    Held<T, (256u + T - 1u) / T, u32x4> h_ent;
+    Held<T, 1, u32x4>                   h_ro;
+    hv_.ids(m, d);
 #pragma unroll
     for (uint32_t r = 0; r < RF; ++r)
-#pragma unroll
-        for (uint32_t j = 0; j < 3; ++j) fw[r][j] = (threadIdx.x + r * T < d.nf) ? fe[3 * (threadIdx.x + r * T) + j] : 0u;
-    stage_u32(L.ev, m.ev + d.e_off, d.ne);
-    stage_halves<T, 8>(L.ent, ent + vb, nent);
-    stage_words<T, 2>(L.rs, rs + d.vp, d.nvo + 1, vb);
-    stage_vertices<T>(m, d, pos, L.pos, L.lin);
-    for (uint32_t i = threadIdx.x; i < d.ne; i += T) {
+        if (r == 0 || r * T < d.nf) fw[r].load(fe, min(t + r * T, d.nf - 1u));
+    h_ev.load(evs, r4(d.ne) >> 2);
+    h_ro.load(ros, words8(d.nvo + 1));
+    h_ent.load(ens, words8(nent));
+    hv_.owned(pos, m, d);
+    hv_.ribbon(pos, m, d);
+    for (uint32_t i = t; i < d.ne; i += T) {
         L.cot[i] = make_float2(0.f, 0.f);
         L.vor[i] = make_float2(0.f, 0.f);
     }
+    if constexpr (CSR) {
+#pragma unroll
+        for (uint32_t k = 0; k < HeldVerts<T, 3>::RR; ++k)
+            if (d.nvo + t + k * T < d.nv) L.rid[t + k * T] = hv_.g[k];
+        for (uint32_t l = d.nvo + t + HeldVerts<T, 3>::RR * T; l < d.nv; l += T) L.rid[l - d.nvo] = m.v_lin[d.v_off + l];
+    }
+    h_ev.store(reinterpret_cast<u32x4*>(L.ev), evs, r4(d.ne) >> 2);
+    h_ro.store(as_words(L.ro), ros, words8(d.nvo + 1));
+    h_ent.store(as_words(L.ent), ens, words8(nent));
+    hv_.store(pos, m, d, [&](uint32_t l, const float (&w)[3]) { L.pos[l] = make_float4(w[0], w[1], w[2], 0.f); });
     __syncthreads();
     // per face: the terms of its half-edges, stored at the half-edge's FE
     // word 2 e + dir (float half dir of edge e's pair)
@@ -303,15 +242,19 @@ __global__ __launch_bounds__(T) void k_cot_assemble(DevMesh m, const uint32_t* _
     };
 #pragma unroll
     for (uint32_t r = 0; r < RF; ++r)
-        if (threadIdx.x + r * T < d.nf) face(fw[r]);
-    for (uint32_t f = threadIdx.x + RF * T; f < d.nf; f += T) {
+        if (t + r * T < d.nf) {
+            uint32_t x[3];
+            fw[r].get(x);
+            face(x);
+        }
+    for (uint32_t f = t + RF * T; f < d.nf; f += T) {
         const uint32_t x[3] = {fe[3 * f], fe[3 * f + 1], fe[3 * f + 2]};
         face(x);
     }
     __syncthreads();
     // rows: diagonal and mass (entries in pattern order)
     for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
-        const uint32_t k0 = L.rs[v], k1 = L.rs[v + 1];
+        const uint32_t k0 = L.ro[v], k1 = L.ro[v + 1];
         float          sum_w = 0.f, vw = 0.f;
         for (uint32_t k = k0; k < k1; ++k) {
             const uint32_t u = L.ent[k];  // the half-edge leaving v
@@ -338,8 +281,59 @@ __global__ __launch_bounds__(T) void k_cot_assemble(DevMesh m, const uint32_t* _
         const float2   c = L.cot[e];
         const float    w = c.x + c.y;
         const uint32_t o = bse + k + v + 1;
-        if constexpr (CSR) col[o] = static_cast<int32_t>(L.lin[(u & 1u) ? lo16(x) : hi16(x)]);
+        if constexpr (CSR) {
+            const uint32_t q = (u & 1u) ? lo16(x) : hi16(x), r = L.rid[max(q, d.nvo) - d.nvo];
+            col[o]           = static_cast<int32_t>((q < d.nvo) ? d.vp + q : r);
+        }
         val[o] = -(((w >= 0.f) ? w : 0.f) * dt);
+    }
+}
+
+// Which owned vertices have a ring of one closed fan (host definition: the
+// successor map of the vertex's faces -- half-edge v -> a of face (v, a, b) is
+// followed by b -- is one cycle through all its neighbours): bit per linear
+// vertex into `closed` (cleared before), ring[patch] = 1 where one has not.
+template <uint32_t T>
+__global__ __launch_bounds__(T) void k_closed_fans(DevMesh m, const uint32_t* __restrict__ rbase,
+                                                   const uint32_t* __restrict__ nbase,
+                                                   const uint16_t* __restrict__ roff, const uint16_t* __restrict__ nbr,
+                                                   const uint16_t* __restrict__ ent, uint32_t* __restrict__ closed,
+                                                   uint32_t* __restrict__ ring)
+{
+    extern __shared__ uint4 smem[];
+    const uint32_t  p = blockIdx.x;
+    const PatchDesc d = load_desc(m.patch, p);
+    Bump            b(reinterpret_cast<char*>(smem));
+    uint32_t*       ev = b.alloc<uint32_t>(r4(d.ne));
+    uint16_t*       fe = b.alloc<uint16_t>(r4(3 * d.nf));
+    uint16_t*       hn = b.alloc<uint16_t>(2 * d.ne);
+    stage_u32(ev, m.ev + d.e_off, d.ne);
+    stage_fe(fe, m.fe + 3u * d.f_off, d.nf);
+    for (uint32_t i = threadIdx.x; i < d.ne; i += T) reinterpret_cast<uint32_t*>(hn)[i] = 0xFFFFFFFFu;
+    __syncthreads();
+    build_half_next(fe, ev, d.nf, hn);
+    __syncthreads();
+    const uint16_t* ro = roff + rbase[p];
+    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
+        const uint32_t  k0 = ro[v], K = ro[v + 1] - k0;
+        const uint16_t *nb = nbr + nbase[p] + k0, *he = ent + nbase[p] + k0;
+        uint32_t        cur = 0, steps = 0;
+        bool            ok = K > 0;
+        for (; ok && steps < K; ++steps) {  // at most K steps
+            const uint32_t q = hn[he[cur]];
+            uint32_t       j = 0;
+            while (j < K && nb[j] != q) ++j;
+            ok  = q != kInv16 && j < K;
+            cur = j;
+            if (cur == 0) {
+                ++steps;
+                break;
+            }
+        }
+        ok = ok && cur == 0 && steps == K;
+        const uint32_t lv = d.vp + v;
+        if (ok) atomicOr(&closed[lv >> 5], 1u << (lv & 31u));
+        else ring[p] = 1u;
     }
 }
 
@@ -1340,6 +1334,11 @@ __device__ __forceinline__ float symdir3_face(const f3 a, const f3 b, const f3 c
 
 // Work-queue counter reset (a kernel, so graphs hold no memset nodes).
 __global__ void k_reset_counter(uint32_t* c) { c[0] = 0u; }
+__global__ __launch_bounds__(256) void k_fill_u32(uint32_t n, uint32_t v, uint32_t* __restrict__ dst)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) dst[i] = v;
+}
 
 // Corner gradients (9 values: da, db, dc) of one face; zero for a degenerate
 // face.

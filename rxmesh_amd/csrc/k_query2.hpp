@@ -172,7 +172,9 @@ __global__ __launch_bounds__(T) void k_query2_vx(DevMesh m, const uint32_t* __re
 
 // VV in patch-local form: per patch, u16 row offsets of the owned vertices
 // (nvo + 1, relative to the patch's entry base) at roff + rbase[p], and u16
-// local neighbour ids at nbr + nbase[p], rows in ascending local-edge order.
+// local neighbour ids at nbr + nbase[p], rows in ascending local-edge order;
+// beside each neighbour, at ent + nbase[p], the half-edge 2 e + dir that leaves
+// the row's vertex (it starts at the edge's (dir ? hi16 : lo16) endpoint).
 // This is the query engine's native (RXMesh-style) encoding of the relation;
 // iterative kernels consume it with half the index bytes of an int32 CSR.
 // Slots are u16, EV's index of the row's other endpoint (2 e + 1 - end: sorts
@@ -195,7 +197,8 @@ __host__ __device__ inline PlanVVL plan_vvl(Bump& b, uint32_t ne, uint32_t nvo)
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_query2_vv_local(DevMesh m, const uint32_t* __restrict__ rbase,
                                                        const uint32_t* __restrict__ nbase,
-                                                       uint16_t* __restrict__ roff, uint16_t* __restrict__ nbr)
+                                                       uint16_t* __restrict__ roff, uint16_t* __restrict__ nbr,
+                                                       uint16_t* __restrict__ ent)
 {
     extern __shared__ uint4 smem[];
     const uint32_t  p = blockIdx.x;
@@ -211,10 +214,14 @@ __global__ __launch_bounds__(T) void k_query2_vv_local(DevMesh m, const uint32_t
         L.off, L.slots, L.wave);
     uint16_t* ro = roff + rbase[p];
     uint16_t* nb = nbr + nbase[p];
+    uint16_t* he = ent + nbase[p];
     for (uint32_t v = threadIdx.x; v <= d.nvo; v += T) ro[v] = static_cast<uint16_t>(L.off[v]);
     for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
         const uint32_t o = L.off[v], k = L.off[v + 1] - o;
-        sort_row(L.slots + o, k, [&](uint32_t j, uint32_t s) { nb[o + j] = ev16[s]; });
+        sort_row(L.slots + o, k, [&](uint32_t j, uint32_t s) {
+            nb[o + j] = ev16[s];
+            he[o + j] = static_cast<uint16_t>(s ^ 1u);
+        });
     }
 }
 

@@ -148,6 +148,27 @@ struct HeldFloats
     }
 };
 
+// The three FE words of a local face from HBM in two 4-byte loads (a face's six
+// bytes start at an even u16, so they lie in two words of the slab, which is
+// padded to four faces), split into halves when they are used.
+struct FaceWords
+{
+    uint32_t w0, w1, odd;
+    __device__ __forceinline__ void load(const uint16_t* __restrict__ fe, uint32_t f)
+    {
+        const uint32_t* q = reinterpret_cast<const uint32_t*>(fe) + ((3u * f) >> 1);
+        w0  = q[0];
+        w1  = q[1];
+        odd = f & 1u;
+    }
+    __device__ __forceinline__ void get(uint32_t (&x)[3]) const
+    {
+        x[0] = odd ? w0 >> 16 : w0 & 0xFFFFu;
+        x[1] = odd ? w1 & 0xFFFFu : w0 >> 16;
+        x[2] = odd ? w1 >> 16 : w1 & 0xFFFFu;
+    }
+};
+
 // Copy 3*nf u16 of a face row (8-byte aligned, padded to 4 faces) into LDS.
 __device__ __forceinline__ void stage_fe(uint16_t* __restrict__ dst, const uint16_t* __restrict__ src,
                                          uint32_t nf)
