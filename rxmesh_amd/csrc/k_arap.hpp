@@ -19,16 +19,13 @@ __device__ __forceinline__ float arap_cot(f3 a, f3 b, f3 c)
 // ---- edge weights ------------------------------------------------------------
 struct PlanAW
 {
-    uint32_t* ev;
-    uint16_t* fe;
-    uint32_t* opp;
+    uint32_t *ev, *opp;
     float *   x, *y, *z;
 };
-__host__ __device__ inline PlanAW plan_aw(Bump& b, uint32_t nv, uint32_t ne, uint32_t nf, uint32_t neo)
+__host__ __device__ inline PlanAW plan_aw(Bump& b, uint32_t nv, uint32_t ne, uint32_t neo)
 {
     PlanAW p{};
     p.ev  = b.alloc<uint32_t>(r4(ne));
-    p.fe  = b.alloc<uint16_t>(r4(3 * nf));
     p.opp = b.alloc<uint32_t>(2 * neo);
     p.x   = b.alloc<float>(nv);
     p.y   = b.alloc<float>(nv);
@@ -36,6 +33,8 @@ __host__ __device__ inline PlanAW plan_aw(Bump& b, uint32_t nv, uint32_t ne, uin
     return p;
 }
 
+// 654k vertices 18.2 -> 14.3 us, 2.6M 52 -> 40 (loads issued together, faces in
+// registers; 512 threads 15.5 and 49).
 // Per owned edge p-r with EVDiamond opposite vertices q and s (the slots of
 // k_query_evd): w = max(0, (cot_q + cot_s) / 2) (arap_kernels.h:8-54); 0 for
 // an edge that lacks a side, which the reference skips, leaving the weight at
@@ -48,17 +47,26 @@ __global__ __launch_bounds__(T) void k_arap_weights(DevMesh m, const float* __re
     if (p >= m.P) return;
     const PatchDesc d = load_desc(m.patch, p);
     Bump            b(reinterpret_cast<char*>(smem));
-    const PlanAW    L = plan_aw(b, d.nv, d.ne, d.nf, d.neo);
+    const PlanAW    L = plan_aw(b, d.nv, d.ne, d.neo);
+    const uint16_t* fe  = m.fe + 3u * d.f_off;
+    const u32x4*    evs = reinterpret_cast<const u32x4*>(m.ev + d.e_off);
+    FaceWords                           fw[(768u + T - 1u) / T];
+    Held<T, (384u + T - 1u) / T, u32x4> h_ev;
+    HeldVerts<T, 3>                     hv;
+    hv.ids(m, d);
+    h_ev.load(evs, r4(d.ne) >> 2);
+    load_faces<T>(fw, fe, d.nf);
+    hv.owned(pos, m, d);
+    hv.ribbon(pos, m, d);
     for (uint32_t i = threadIdx.x; i < 2 * d.neo; i += T) L.opp[i] = 0u;
-    stage_u32(L.ev, m.ev + d.e_off, d.ne);
-    stage_fe(L.fe, m.fe + 3u * d.f_off, d.nf);
-    stage_positions_batched<T, (512u + T - 1u) / T, false>(L.x, L.y, L.z, nullptr, pos, m.nV, d, m.v_lin);
+    h_ev.store(reinterpret_cast<u32x4*>(L.ev), evs, r4(d.ne) >> 2);
+    hv.store(pos, m, d, [&](uint32_t l, const float (&q)[3]) {
+        L.x[l] = q[0];
+        L.y[l] = q[1];
+        L.z[l] = q[2];
+    });
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < 3 * d.nf; i += T) {
-        const uint32_t f = i / 3u, k = i - 3u * f;
-        const uint32_t y = L.fe[3u * f + (k == 2u ? 0u : k + 1u)];
-        if ((y >> 1) < d.neo) atomicMax(&L.opp[y], ((f + 1u) << 16) | face_vertex(L.fe, L.ev, f, k));
-    }
+    edge_opposites<T>(fw, fe, L.ev, d, L.opp);
     __syncthreads();
     for (uint32_t e = threadIdx.x; e < d.neo; e += T) {
         const uint32_t qa = L.opp[2 * e], sa = L.opp[2 * e + 1];
@@ -188,6 +196,100 @@ __device__ inline void best_rotation(const float (&S)[3][3], float (&R)[3][3])
     R[2][0] = 2.f * (qz * qx - q0 * qy);
     R[2][1] = 2.f * (qz * qy + q0 * qx);
     R[2][2] = q0 * q0 - qx * qx - qy * qy + qz * qz;
+}
+
+// The same rotation without the sweeps, in FP64 (which runs at the rate of plain
+// FP32 here): the largest eigenvalue of N(S) is the largest root of its
+// characteristic polynomial, whose coefficients are S's invariants
+// (l^4 - 2 |S|^2 l^2 - 8 det(S) l + |S|^4 - 4 |cof(S)|^2), found by Newton's
+// method from the bound sqrt(3) |S| (monotone from above); its eigenvector is
+// the largest column of the adjugate of N - l I (Theobald, Acta Cryst. A 61:478,
+// 2005, takes the same two steps). Returns false, R unset, where the gap to the
+// next eigenvalue leaves the adjugate fewer than about nine digits, or the root
+// has not settled: the sweeps decide there. About 300 instructions a vertex
+// against 2,000 and more of the sweeps, which bound the kernel
+// (654k vertices 41 -> 30 us with the records written as one run and 256 threads,
+// 2.6M 129 -> 90; now the staging). Its error against FP64 is not larger: R is
+// rounded once (energy and gradient that use R: 6.9e-7 -> 3.3e-7 off).
+__device__ inline bool best_rotation_direct(const float (&Sf)[3][3], float (&R)[3][3])
+{
+    double S[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) S[i][j] = static_cast<double>(Sf[i][j]);
+    double f = 0.0, cf = 0.0, det = 0.0;  // |S|^2, |cof(S)|^2, det(S)
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int    i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
+            const double c = S[i1][j1] * S[i2][j2] - S[i1][j2] * S[i2][j1];
+            f += S[i][j] * S[i][j];
+            cf += c * c;
+            if (i == 0) det += S[0][j] * c;
+        }
+    const double c2 = -2.0 * f, c1 = -8.0 * det, c0 = f * f - 4.0 * cf;
+    double       l = sqrt(3.0 * f);
+    bool         settled = false;
+    for (int it = 0; it < 24 && !settled; ++it) {
+        const double l2 = l * l;
+        const double p = ((l2 + c2) * l + c1) * l + c0, dp = (4.0 * l2 + 2.0 * c2) * l + c1;
+        const double step = p * __builtin_amdgcn_rcp(dp);  // an approximate step only slows the last digits
+        l -= step;
+        settled = fabs(step) <= 1e-12 * l;
+    }
+    // B = N(S) - l I, upper triangle
+    const double b00 = S[0][0] + S[1][1] + S[2][2] - l, b11 = S[0][0] - S[1][1] - S[2][2] - l;
+    const double b22 = -S[0][0] + S[1][1] - S[2][2] - l, b33 = -S[0][0] - S[1][1] + S[2][2] - l;
+    const double b01 = S[1][2] - S[2][1], b02 = S[2][0] - S[0][2], b03 = S[0][1] - S[1][0];
+    const double b12 = S[0][1] + S[1][0], b13 = S[2][0] + S[0][2], b23 = S[1][2] + S[2][1];
+    // 2 x 2 minors of rows (2, 3) and of rows (0, 1), columns as named
+    const double m01 = b02 * b13 - b12 * b03, m02 = b02 * b23 - b22 * b03, m03 = b02 * b33 - b23 * b03;
+    const double m12 = b12 * b23 - b22 * b13, m13 = b12 * b33 - b23 * b13, m23 = b22 * b33 - b23 * b23;
+    const double n01 = b00 * b11 - b01 * b01, n02 = b00 * b12 - b02 * b01, n03 = b00 * b13 - b03 * b01;
+    const double n12 = b01 * b12 - b02 * b11, n13 = b01 * b13 - b03 * b11;
+    // cofactors (symmetric)
+    const double a00 = b11 * m23 - b12 * m13 + b13 * m12, a01 = -(b01 * m23 - b12 * m03 + b13 * m02);
+    const double a02 = b01 * m13 - b11 * m03 + b13 * m01, a03 = -(b01 * m12 - b11 * m02 + b12 * m01);
+    const double a11 = b00 * m23 - b02 * m03 + b03 * m02, a12 = -(b00 * m13 - b01 * m03 + b03 * m01);
+    const double a13 = b00 * m12 - b01 * m02 + b02 * m01;
+    const double a22 = b33 * n01 - b13 * n03 + b03 * n13, a23 = -(b23 * n01 - b13 * n02 + b03 * n12);
+    const double a33 = b22 * n01 - b12 * n02 + b02 * n12;
+    double       dg = fabs(a00), q0 = a00, qx = a01, qy = a02, qz = a03;
+    auto         take = [&](double d, double e0, double ex, double ey, double ez) {
+        const bool up = fabs(d) > dg;
+        dg = up ? fabs(d) : dg;
+        q0 = up ? e0 : q0;
+        qx = up ? ex : qx;
+        qy = up ? ey : qy;
+        qz = up ? ez : qz;
+    };
+    take(a11, a01, a11, a12, a13);
+    take(a22, a02, a12, a22, a23);
+    take(a33, a03, a13, a23, a33);
+    // a degenerate S (l = 0) or a NaN fails the comparison
+    if (!(settled && dg >= 1e-7 * l * l * l && l > 0.0)) return false;
+    // unit scale: the components squared neither over- nor underflow
+    const double u  = __builtin_amdgcn_rcp(dg);
+    q0 *= u;
+    qx *= u;
+    qy *= u;
+    qz *= u;
+    const double n = q0 * q0 + qx * qx + qy * qy + qz * qz;
+    double       v = __builtin_amdgcn_rcp(n);
+    v              = v * (2.0 - n * v);
+    v              = v * (2.0 - n * v);
+    R[0][0] = static_cast<float>(v * (q0 * q0 + qx * qx - qy * qy - qz * qz));
+    R[0][1] = static_cast<float>(2.0 * v * (qx * qy - q0 * qz));
+    R[0][2] = static_cast<float>(2.0 * v * (qx * qz + q0 * qy));
+    R[1][0] = static_cast<float>(2.0 * v * (qy * qx + q0 * qz));
+    R[1][1] = static_cast<float>(v * (q0 * q0 - qx * qx + qy * qy - qz * qz));
+    R[1][2] = static_cast<float>(2.0 * v * (qy * qz - q0 * qx));
+    R[2][0] = static_cast<float>(2.0 * v * (qz * qx - q0 * qy));
+    R[2][1] = static_cast<float>(2.0 * v * (qz * qy + q0 * qx));
+    R[2][2] = static_cast<float>(v * (q0 * q0 - qx * qx - qy * qy + qz * qz));
+    return true;
 }
 
 // Patch-local data of the rotation and energy kernels: the VV plan's rows
@@ -332,27 +434,34 @@ __global__ __launch_bounds__(T) void k_arap_rotations(DevMesh m, const uint32_t*
     Bump            b(reinterpret_cast<char*>(smem));
     PlanAR          L = plan_ar(b, d.nv, d.ne, d.nvo, nent, false);
     stage_arap<T, false>(m, d, L, roff + rbase[p], nbr + nbase[p], ent + nbase[p], nent, rest, x, w, nullptr);
+    float* const out = b.alloc<float>(9u * T);  // this round's records, written as one run
     __syncthreads();
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
-        float       S[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-        const float p0 = L.px[v], p1 = L.py[v], p2 = L.pz[v], x0 = L.xx[v], x1 = L.xy[v], x2 = L.xz[v];
-        for (uint32_t k = L.ro[v]; k < L.ro[v + 1]; ++k) {
-            const uint32_t j = L.nb[k];
-            const float    wt = L.w[L.ent[k] >> 1];
-            const float    a[3] = {p0 - L.px[j], p1 - L.py[j], p2 - L.pz[j]};
-            const float    c[3] = {x0 - L.xx[j], x1 - L.xy[j], x2 - L.xz[j]};
+    for (uint32_t v0 = 0; v0 < d.nvo; v0 += T) {
+        const uint32_t v = v0 + threadIdx.x, nr = min(T, d.nvo - v0);
+        if (v < d.nvo) {
+            float       S[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+            const float p0 = L.px[v], p1 = L.py[v], p2 = L.pz[v], x0 = L.xx[v], x1 = L.xy[v], x2 = L.xz[v];
+            for (uint32_t k = L.ro[v]; k < L.ro[v + 1]; ++k) {
+                const uint32_t j = L.nb[k];
+                const float    wt = L.w[L.ent[k] >> 1];
+                const float    a[3] = {p0 - L.px[j], p1 - L.py[j], p2 - L.pz[j]};
+                const float    c[3] = {x0 - L.xx[j], x1 - L.xy[j], x2 - L.xz[j]};
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+#pragma unroll
+                    for (int s = 0; s < 3; ++s) S[r][s] += wt * a[r] * c[s];
+            }
+            float Rv[3][3];
+            if (!best_rotation_direct(S, Rv)) best_rotation(S, Rv);
 #pragma unroll
             for (int r = 0; r < 3; ++r)
 #pragma unroll
-                for (int s = 0; s < 3; ++s) S[r][s] += wt * a[r] * c[s];
+                for (int s = 0; s < 3; ++s) out[9u * threadIdx.x + 3u * r + s] = Rv[r][s];
         }
-        float Rv[3][3];
-        best_rotation(S, Rv);
-        float* out = R + 9ull * (d.vp + v);
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int s = 0; s < 3; ++s) out[3 * r + s] = Rv[r][s];
+        __syncthreads();
+        float* dst = R + 9ull * (d.vp + v0);
+        for (uint32_t i = threadIdx.x; i < 9u * nr; i += T) dst[i] = out[i];
+        __syncthreads();
     }
 }
 
@@ -373,7 +482,9 @@ __device__ __forceinline__ f3 arap_residual(const PlanAR& L, uint32_t i, uint32_
 // dE/dX_v = sum over v's edges of +-2 w d, + where v is the edge's i.
 // Every local edge's residual is evaluated once, into registers, and stored
 // over the rotations once all are done; the gradient gathers them per vertex
-// (patches beyond the register rounds evaluate an edge at each use). AENOTE
+// (patches beyond the register rounds evaluate an edge at each use). 654k
+// vertices 42.8 -> 33 us, 2.6M 142 -> 112. Bound: the gathers of the ribbon's
+// rotations and the residuals' LDS reads.
 template <uint32_t T>
 __global__ __launch_bounds__(T) void k_arap_energy_grad(DevMesh m, const uint32_t* __restrict__ vv_base,
                                                         const uint32_t* __restrict__ rbase,

@@ -157,3 +157,92 @@ def test_multi_step_smoothing_equals_single_steps(shape, patch_size):
             m.set_launch_threads(0, threads)
             m.set_launch_threads(8, steps)
             assert torch.equal(m.smooth(x, 0.5, 7), ref[7])
+
+
+def _arap64(V, F, P, X, w):
+    """Covariances, best proper rotations (SVD), energy and gradient; w per (i, j) pair with i the larger id."""
+    e = np.unique(np.sort(np.concatenate([F[:, [0, 1]], F[:, [1, 2]], F[:, [2, 0]]]).astype(np.int64), 1), axis=0)
+    i, j = e[:, 1], e[:, 0]
+    dp, dx = P[i] - P[j], X[i] - X[j]
+    wt = np.array([w[(a, b)] for a, b in zip(i, j)])
+    S = np.zeros((len(V), 3, 3))
+    t = wt[:, None, None] * dp[:, :, None] * dx[:, None, :]
+    np.add.at(S, i, t)
+    np.add.at(S, j, t)
+    u, s, vt = np.linalg.svd(S)
+    sign = np.sign(np.linalg.det(np.swapaxes(vt, 1, 2) @ np.swapaxes(u, 1, 2)))
+    gap = s[:, 1] + sign * s[:, 2]
+    u[:, :, 2] *= sign[:, None]
+    R = np.swapaxes(vt, 1, 2) @ np.swapaxes(u, 1, 2)
+    return R, gap > 1e-2 * s[:, 0], (i, j, wt, dp, dx)
+
+
+@pytest.mark.parametrize("patch_size", [16, 512, 2048])
+@pytest.mark.parametrize("mirror", [False, True])
+def test_arap_patch_sizes(patch_size, mirror):
+    """Rotations, energy and gradient against FP64 over patches from a few
+    faces to more than the register rounds; mirrored poses have negative
+    determinants everywhere. Tolerances of the other ARAP tests: 1e-4 per
+    entry where the covariance fixes R, 1e-5 of the energy, 1e-4 of the
+    largest gradient entry."""
+    import torch
+    V, F = mg.permute_mesh(*mg.icosphere(4, seed=7, sigma=0.02), seed=7)
+    m, x = _mesh(V, F, patch_size)
+    pose = (x + 0.3 * torch.sin(2.0 * x.flip(0))).contiguous()
+    if mirror:
+        pose[0] = -pose[0]
+    w = m.arap_weights(x)
+    R = m.arap_rotations(x, pose, w)
+    E, g = m.arap_energy_grad(x, pose, w, R)
+    l2g, e_l2g = m.array("v_l2g"), m.array("e_l2g")
+    P, X = np.empty((m.nV, 3)), np.empty((m.nV, 3))
+    P[l2g], X[l2g] = x.cpu().numpy().T, pose.cpu().numpy().T
+    ev = m.array("ev").reshape(-1, 2).astype(np.int64)[e_l2g]
+    wd = {(max(a, b), min(a, b)): v for (a, b), v in zip(ev.tolist(), w.cpu().numpy().astype(np.float64))}
+    R64, fixed, (i, j, wt, dp, dx) = _arap64(V, F, P, X, wd)
+    Rg = np.empty((m.nV, 9))
+    Rg[l2g] = R.cpu().numpy()
+    assert np.abs(Rg.reshape(-1, 3, 3) - R64)[fixed].max() <= 1e-4
+    assert np.abs(Rg.reshape(-1, 3, 3) @ np.swapaxes(Rg.reshape(-1, 3, 3), 1, 2) - np.eye(3)).max() <= 1e-5
+    d = dx - np.einsum("nij,nj->ni", Rg.reshape(-1, 3, 3)[i], dp)
+    grad = np.zeros((m.nV, 3))
+    np.add.at(grad, i, 2 * wt[:, None] * d)
+    np.add.at(grad, j, -2 * wt[:, None] * d)
+    e64 = (wt * (d * d).sum(1)).sum()
+    assert abs(float(E[0]) - e64) <= 1e-5 * e64
+    assert np.abs(g.cpu().numpy().T - grad[l2g]).max() <= 1e-4 * np.abs(grad).max()
+
+
+def test_arap_rotations_of_undetermined_covariances():
+    """No weight at all gives the identity; an unmoved pose the identity; a
+    pose squeezed to a line or a point, where the covariance does not fix R, a
+    proper rotation."""
+    import torch
+    V, F = mg.icosphere(3, seed=8, sigma=0.02)
+    m, x = _mesh(V, F, 64)
+    eye = torch.eye(3, device="cuda").reshape(1, 9)
+    w = m.arap_weights(x)
+    assert torch.equal(m.arap_rotations(x, x.flip(0).contiguous(), torch.zeros_like(w)), eye.expand(m.nV, 9))
+    assert (m.arap_rotations(x, x, w) - eye).abs().max() <= 1e-5
+    for keep in (1, 0):
+        pose = x.clone()
+        pose[keep:] = 0.0
+        R = m.arap_rotations(x, pose, w).reshape(-1, 3, 3).double()
+        assert (R @ R.transpose(1, 2).contiguous() - torch.eye(3, device="cuda")).abs().max() <= 1e-5
+        assert (torch.linalg.det(R.cpu()) - 1.0).abs().max() <= 1e-5
+
+
+@pytest.mark.parametrize("patch_size", [16, 512, 2048])
+def test_evd_rows_at_any_alignment(patch_size):
+    """The EVDiamond columns leave as 16-byte stores where the array allows:
+    the same rows from an array that starts at every word of a line."""
+    import torch
+    V, F = mg.grid(37, seed=9)
+    m, _ = _mesh(V, F, patch_size)
+    n = m.query_nnz("EVD")
+    rp, col = m.query("EVD")
+    for mis in (1, 2, 3):
+        c = torch.full((n + 8,), -7, dtype=torch.int32, device="cuda")
+        r2, _ = m.query("EVD", col=c[mis:mis + n])
+        assert torch.equal(r2, rp) and torch.equal(c[mis:mis + n], col[:n])
+        assert (c[:mis] == -7).all() and (c[mis + n:] == -7).all()
