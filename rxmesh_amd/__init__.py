@@ -134,27 +134,54 @@ def _check(rc, what):
         raise RXMError(rc, what)
 
 
+_torch = _DTYPES = _raw_stream = None
+
+
+def _load_torch():
+    """The torch objects every call needs, looked up once."""
+    global _torch, _DTYPES, _raw_stream
+    import torch
+    _torch = torch
+    _DTYPES = {"float32": torch.float32, "int32": torch.int32}
+    raw, dev = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+    if raw is None or dev is None:
+        _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    else:
+        _raw_stream = lambda: raw(dev())  # noqa: E731  (the handle of torch.cuda.current_stream() without its object)
+
+
 def _stream(stream):
     if stream is None:
-        import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        if _torch is None:
+            _load_torch()
+        return _raw_stream()
     if hasattr(stream, "cuda_stream"):
-        return ctypes.c_void_p(stream.cuda_stream)
-    return ctypes.c_void_p(stream)
+        return stream.cuda_stream
+    return stream
 
 
 def _dev(t, name, shape=None, dtype="float32", min_numel=None):
-    """ctypes pointer to a tensor the C-ABI reads or writes, after checking
+    """Device address of a tensor the C-ABI reads or writes, after checking
     what the C-ABI cannot see through a raw pointer: the dtype, the exact
-    shape (or, for buffers sized by a count, a minimum element count),
-    contiguity and that the tensor lives on the GPU. Raises ValueError before
-    anything is launched, so a transposed view, a (V, 3) array where (3, V)
-    SoA is expected, an undersized buffer or a float16 tensor never reaches a
-    kernel."""
-    import torch
-    if not isinstance(t, torch.Tensor):
+    shape (a tuple of ints; or, for buffers sized by a count, a minimum element
+    count), contiguity and that the tensor lives on the GPU. Raises ValueError
+    before anything is launched, so a transposed view, a (V, 3) array where
+    (3, V) SoA is expected, an undersized buffer or a float16 tensor never
+    reaches a kernel. The checks of a good tensor come to a handful of
+    attribute reads (the wrapper's time is what bounds calls on small meshes);
+    the messages are made only for one that fails."""
+    if _torch is None:
+        _load_torch()
+    if (isinstance(t, _torch.Tensor) and t.dtype is _DTYPES[dtype] and (shape is None or t.shape == shape)
+            and (min_numel is None or (t.dim() == 1 and t.numel() >= min_numel)) and t.is_contiguous() and t.is_cuda):
+        return t.data_ptr()
+    return _refuse(t, name, shape, dtype, min_numel)
+
+
+def _refuse(t, name, shape, dtype, min_numel):
+    if not isinstance(t, _torch.Tensor):
         raise ValueError("%s: expected a torch tensor, got %s" % (name, type(t).__name__))
-    want = {"float32": torch.float32, "int32": torch.int32}[dtype]
+    want = _DTYPES[dtype]
     if t.dtype != want:
         raise ValueError("%s: expected dtype %s, got %s" % (name, want, t.dtype))
     if shape is not None and tuple(t.shape) != tuple(int(n) for n in shape):
@@ -166,7 +193,7 @@ def _dev(t, name, shape=None, dtype="float32", min_numel=None):
         raise ValueError("%s: tensor must be contiguous (call .contiguous())" % name)
     if not t.is_cuda:
         raise ValueError("%s: tensor must be on the GPU" % name)
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()  # e.g. a shape given as a list of the same numbers
 
 
 def _opt(t, *args, **kw):
@@ -239,6 +266,9 @@ class Mesh:
         self.nE = self.info["num_edges"]
         self.nF = self.info["num_faces"]
         self.P = self.info["num_patches"]
+        self._shape_v3, self._shape_mr, self._shape_rp = (3, self.nV), (4, self.nF), (self.nV + 1,)
+        self._counts = {}  # entries per query: fixed by the connectivity
+        self._nsrc = {"V": self.nV, "E": self.nE, "F": self.nF}
 
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:
@@ -271,17 +301,20 @@ class Mesh:
     # -- argument shapes ------------------------------------------------
     def _v3(self, t, name):
         """(3, V) float32 SoA positions / vertex vectors over linear ids."""
-        return _dev(t, name, (3, self.nV))
+        return _dev(t, name, self._shape_v3)
 
     def _mr(self, Mr):
         """(4, F) float32 rest shapes (rxm_symdir_rest)."""
-        return _dev(Mr, "Mr", (4, self.nF))
+        return _dev(Mr, "Mr", self._shape_mr)
 
     # -- queries --------------------------------------------------------
     def query_nnz(self, op):
-        n = ctypes.c_int64()
-        _check(lib().rxm_query_nnz(self._h, OP[op], ctypes.byref(n)), "rxm_query_nnz")
-        return n.value
+        n = self._counts.get(op)
+        if n is None:
+            c = ctypes.c_int64()
+            _check(lib().rxm_query_nnz(self._h, OP[op], ctypes.byref(c)), "rxm_query_nnz")
+            n = self._counts[op] = c.value
+        return n
 
     def query_vv_vf(self, vv=None, vf=None, stream=None):
         """VV and VF CSRs (same as query("VV") and query("VF")) from one launch."""
@@ -293,13 +326,13 @@ class Mesh:
         if vf is None:
             vf = (torch.empty(self.nV + 1, dtype=torch.int32, device="cuda"),
                   torch.empty(max(nvf, 1), dtype=torch.int32, device="cuda"))
-        args = (_dev(vv[0], "vv row_ptr", (self.nV + 1,), "int32"), _dev(vv[1], "vv col", None, "int32", nvv),
-                _dev(vf[0], "vf row_ptr", (self.nV + 1,), "int32"), _dev(vf[1], "vf col", None, "int32", nvf))
+        args = (_dev(vv[0], "vv row_ptr", self._shape_rp, "int32"), _dev(vv[1], "vv col", None, "int32", nvv),
+                _dev(vf[0], "vf row_ptr", self._shape_rp, "int32"), _dev(vf[1], "vf col", None, "int32", nvf))
         _check(lib().rxm_query_vv_vf(self._h, *args, _stream(stream)), "rxm_query_vv_vf")
         return vv, vf
 
     def num_src(self, op):
-        return {"V": self.nV, "E": self.nE, "F": self.nF}[op[0]]
+        return self._nsrc[op[0]]
 
     def query(self, op, oriented=False, row_ptr=None, col=None, stream=None):
         """CSR (row_ptr, col) of `op` over linear ids, as int32 device tensors."""
@@ -468,9 +501,12 @@ class Mesh:
 
     # -- cotangent system / explicit MCF ------------------------------
     def cot_nnz(self):
-        n = ctypes.c_int64()
-        _check(lib().rxm_cot_nnz(self._h, ctypes.byref(n)), "rxm_cot_nnz")
-        return n.value
+        n = self._counts.get("cot")
+        if n is None:
+            c = ctypes.c_int64()
+            _check(lib().rxm_cot_nnz(self._h, ctypes.byref(c)), "rxm_cot_nnz")
+            n = self._counts["cot"] = c.value
+        return n
 
     def _system(self, A):
         """Pointers of a cotangent system (row_ptr, col, val, mass) as
@@ -641,7 +677,7 @@ def smooth_symdir_steps_each(meshes, Mrs, xs, tmps, lam, eta, steps, stream=None
     n = len(meshes)
     if not (len(Mrs) == len(xs) == len(tmps) == n):
         raise ValueError("smooth_symdir_steps_each: one Mr, x and tmp per mesh")
-    arr = lambda items: (ctypes.c_void_p * n)(*[p.value for p in items])  # noqa: E731
+    arr = lambda items: (ctypes.c_void_p * n)(*items)  # noqa: E731
     _check(lib().rxm_smooth_symdir_steps_each((ctypes.c_void_p * n)(*[m._h.value for m in meshes]),
                                               arr([m._mr(t) for m, t in zip(meshes, Mrs)]),
                                               arr([m._v3(t, "x") for m, t in zip(meshes, xs)]),
@@ -656,7 +692,7 @@ def query_smooth_symdir_steps_each(meshes, Mrs, xs, tmps, bufs, lam, eta, steps,
     n = len(meshes)
     if not (len(Mrs) == len(xs) == len(tmps) == len(bufs) == n):
         raise ValueError("query_smooth_symdir_steps_each: one Mr, x, tmp and buffer set per mesh")
-    arr = lambda items: (ctypes.c_void_p * n)(*[p.value for p in items])  # noqa: E731
+    arr = lambda items: (ctypes.c_void_p * n)(*items)  # noqa: E731
     ptrs = [m._vv_vf_ptrs(*b) for m, b in zip(meshes, bufs)]
     _check(lib().rxm_query_smooth_symdir_steps_each((ctypes.c_void_p * n)(*[m._h.value for m in meshes]),
                                                     arr([m._mr(t) for m, t in zip(meshes, Mrs)]),
@@ -695,7 +731,10 @@ class SymmetricDirichlet:
                 @staticmethod
                 def backward(ctx, g):
                     (uv_,) = ctx.saved_tensors
-                    g = g.detach().to(torch.float32).contiguous()
+                    g = g.detach()
+                    if g.dtype is not torch.float32:
+                        g = g.to(torch.float32)
+                    g = g.contiguous()
                     return ctx.mesh.symdir_grad(ctx.Mr, uv_, scale=g), None, None
 
             cls._fn = _SymDir

@@ -246,3 +246,21 @@ def test_evd_rows_at_any_alignment(patch_size):
         r2, _ = m.query("EVD", col=c[mis:mis + n])
         assert torch.equal(r2, rp) and torch.equal(c[mis:mis + n], col[:n])
         assert (c[:mis] == -7).all() and (c[mis + n:] == -7).all()
+
+
+def test_calls_go_to_the_current_stream():
+    """A call without a stream argument is queued on torch's current stream,
+    also inside a stream context and in another thread."""
+    import threading
+    import rxmesh_amd as rx
+    import torch
+    side = torch.cuda.Stream()
+    assert rx._stream(None) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert rx._stream(None) == side.cuda_stream == rx._stream(side)
+        got = []
+        th = threading.Thread(target=lambda: got.append((rx._stream(None), torch.cuda.current_stream().cuda_stream)))
+        th.start()
+        th.join()
+    assert got[0][0] == got[0][1]
+    assert rx._stream(None) == torch.cuda.current_stream().cuda_stream
