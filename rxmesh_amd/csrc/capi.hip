@@ -98,6 +98,7 @@ struct rxm_mesh
     bool            system_runs_ok = false;    // check_system_runs passed
     uint32_t        query_stable   = 2;        // transposes: 0 LDS atomics + row sort, 1 atomic-free stable sort, 2 as 0 with the fused VV + VF launch in one pass
     uint32_t        vvf_nslots     = 0;        // largest VV + VF entry count of a patch (0: not computed yet)
+    uint32_t        max_row        = 0;        // largest VV or VF row of a vertex
     uint32_t        max_nrv = 0, max_nre = 0, max_nrf = 0;  // largest ribbon vertex / edge / face count of a patch
     int             num_cus        = 0;
     // batch (disjoint union of meshes): per-mesh id / patch offsets
@@ -258,8 +259,15 @@ void vvf_slots(rxm_mesh* m)
         m->max_nre    = std::max(m->max_nre, m->h.ne[p] - m->h.neo[p]);
         m->max_nrf    = std::max(m->max_nrf, m->h.nf[p] - m->h.nfo[p]);
     }
+    const HostMesh& h = m->h;
+    // on an edge-manifold mesh a vertex has no more faces than edges
+    m->max_row = h.max_valence;
+    if (!h.manifold)
+        for (uint32_t v = 0; v < h.nV; ++v) m->max_row = std::max(m->max_row, h.vf_off[v + 1] - h.vf_off[v]);
     m->vvf_nslots = std::max(m->vvf_nslots, 1u);
 }
+
+
 
 // The patch-local MCF and CG kernels stage patch p's run of the cotangent
 // system's values as [vv_base[p] + vp[p], vv_base[p + 1] + vp[p + 1]): the
@@ -324,6 +332,63 @@ template <typename K, typename... Args>
 int launch_patches_xcd(K kernel, uint32_t threads, uint32_t lds, void* stream, const rxm_mesh* m, Args... args)
 {
     return launch_grid(kernel, patch_grid(m->h.P), threads, lds, stream, args...);
+}
+
+// The query of REL (k_query_rows) on the fixed-width-slot kernel, or false if
+// the mesh does not fit it.
+template <uint32_t REL>
+bool launch_rows(rxm_mesh* m, const uint32_t* v_base, const uint32_t* f_base, int32_t* v_row, int32_t* v_col,
+                 int32_t* f_row, int32_t* f_col, void* stream, int* rc)
+{
+    vvf_slots(m);
+    const HostMesh& h = m->h;
+    if (m->query_stable != 2 || m->max_row > kRowMax || 2u * h.max_ne > 0x10000u) return false;
+    constexpr uint32_t nrel = (REL & (kRowsVV | kRowsVE) ? 1u : 0u) + (REL & kRowsVF ? 1u : 0u);
+    const uint32_t     nl = (REL & kRowsVV) ? h.max_nv : ((REL & kRowsVE) ? h.max_ne : 0u);
+    Bump               b(nullptr);
+    plan_rows(b, h.max_nvo, h.max_ne, nrel, nl, (REL & kRowsVF) ? h.max_nf : 0u);
+    if (b.bytes() > kMaxLdsBytes) return false;
+    auto fits = [&](uint32_t T, uint32_t RF, uint32_t RQ, uint32_t RV) {
+        return h.max_nf <= RF * T && h.max_ne <= 4u * RQ * T && h.max_nvo <= RV * T;
+    };
+    auto go = [&](auto kernel, uint32_t T) {
+        *rc = launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, v_base, f_base, v_row, v_col, f_row, f_col);
+        return true;
+    };
+    // Few patches: one workgroup's chain is the launch, and more threads shorten
+    // it; many: small workgroups overlap more. VV + VF with 1024 / 512 / 256
+    // threads: 10 patches 5.2 / 5.5 / 7.1 us, 167 5.6 / 6.0 / 7.8, 491 7.8 / 7.5 /
+    // 8.9, 2687 29.7 / 22.2 / 21.8, 10677 97.7 / 70.0 / 58.8 (k_query2_vv_vf1,
+    // 256 threads: 8.4, 8.6, 9.4, 25.3, 67.6).
+    if (h.P <= 256u && fits(1024, 1, 1, 1)) return go(k_query_rows<1024, 1, 1, 1, REL>, 1024);
+    if (h.P > 1500u && fits(256, 3, 2, 2)) return go(k_query_rows<256, 3, 2, 2, REL>, 256);
+    if (fits(512, 3, 2, 2)) return go(k_query_rows<512, 3, 2, 2, REL>, 512);
+    return false;
+}
+
+// EF or FF on the direct-slot kernel (k_query_dir), or false if the mesh does
+// not fit it.
+template <bool FF>
+bool launch_dir(rxm_mesh* m, const uint32_t* base, int32_t* row_ptr, int32_t* col, void* stream, int* rc)
+{
+    const HostMesh& h = m->h;
+    if (m->query_stable != 2 || !h.manifold || !h.oriented || 2u * h.max_ne > 0x10000u) return false;
+    const uint32_t nout = std::max(op_max_patch(m, FF ? RXM_OP_FF : RXM_OP_EF), 1u);
+    Bump           b(nullptr);
+    plan_dir(b, h.max_ne, h.max_nf, nout);
+    if (b.bytes() > kMaxLdsBytes) return false;
+    const uint32_t ns   = FF ? h.max_nfo : h.max_neo;
+    auto           fits = [&](uint32_t T, uint32_t RF, uint32_t RS) { return h.max_nf <= RF * T && ns <= RS * T; };
+    auto           go   = [&](auto kernel, uint32_t T) {
+        *rc = launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, nout, base, row_ptr, col);
+        return true;
+    };
+    // workgroup sizes as launch_rows chooses them
+    constexpr uint32_t RS = FF ? 3 : 4;
+    if (h.P <= 256u && fits(1024, 1, 1)) return go(k_query_dir<1024, 1, 1, FF>, 1024);
+    if (h.P > 1500u && fits(256, 3, RS)) return go(k_query_dir<256, 3, RS, FF>, 256);
+    if (fits(512, 3, RS)) return go(k_query_dir<512, 3, RS, FF>, 512);
+    return false;
 }
 
 int ensure_vv_plan(rxm_mesh* m, void* stream)
@@ -1051,16 +1116,23 @@ rxm_status rxm_query_csr(rxm_mesh* m, int op, int oriented, int32_t* row_ptr, in
     if (rc) return rc;
     Bump b(nullptr);
     constexpr uint32_t T = kQueryThreads;
-    if (oriented) {  // oriented VV / VE: owned transpose columns + canonical CCW walk
-        plan_vxo(b, h.max_nv, h.max_ne, h.max_nf, h.max_nv, op_max_patch(m, op));
+    if (oriented) {  // oriented VV / VE: canonical CCW rings along half-edge successors
+        vvf_slots(m);
+        const uint32_t nrid = (op == RXM_OP_VV) ? m->max_nrv : m->max_nre;
+        plan_vxo(b, h.max_nv, h.max_ne, h.max_nvo, op_max_patch(m, op), nrid);
         auto go = [&](auto kernel, uint32_t threads) {
-            return launch_patches_xcd(kernel, threads, b.bytes(), stream, m, m->dm, base, row_ptr, col);
+            return launch_patches_xcd(kernel, threads, b.bytes(), stream, m, m->dm, nrid, base, row_ptr, col);
         };
         if (m->ring_threads == 512)
             return (op == RXM_OP_VV) ? go(k_query_vx_oriented<512, true>, 512)
                                      : go(k_query_vx_oriented<512, false>, 512);
         return (op == RXM_OP_VV) ? go(k_query_vx_oriented<256, true>, 256) : go(k_query_vx_oriented<256, false>, 256);
     }
+    if (op == RXM_OP_VV && launch_rows<kRowsVV>(m, base, nullptr, row_ptr, col, nullptr, nullptr, stream, &rc)) return rc;
+    if (op == RXM_OP_VE && launch_rows<kRowsVE>(m, base, nullptr, row_ptr, col, nullptr, nullptr, stream, &rc)) return rc;
+    if (op == RXM_OP_VF && launch_rows<kRowsVF>(m, nullptr, base, nullptr, nullptr, row_ptr, col, stream, &rc)) return rc;
+    if (op == RXM_OP_EF && launch_dir<false>(m, base, row_ptr, col, stream, &rc)) return rc;
+    if (op == RXM_OP_FF && launch_dir<true>(m, base, row_ptr, col, stream, &rc)) return rc;
     // VV / VE / VF / EF in the one-pass form (knob 10 = 2, the default) where
     // the patches fit its carve (VV / VE slots are EV's u16 indices 2 e + 1 -
     // end, 16 bits)
@@ -1138,6 +1210,7 @@ static int query_vv_vf_launch(rxm_mesh* m, int32_t* vv_row_ptr, int32_t* vv_col,
     if (!rc) rc = device_base(m, RXM_OP_VF, &vf_base);
     if (rc) return rc;
     constexpr uint32_t T = kQueryThreads;
+    if (launch_rows<kRowsVV | kRowsVF>(m, vv_base, vf_base, vv_row_ptr, vv_col, vf_row_ptr, vf_col, stream, &rc)) return rc;
     if (m->query_stable == 2) {  // one counting sort for both relations
         vvf_slots(m);
         Bump b1(nullptr);

@@ -13,26 +13,38 @@ namespace rxm {
 
 constexpr uint32_t kQueryThreads = 256;
 
-// ---- LDS plans (same carve on host for sizing and on device) -------------
-// Oriented VV / VE: EV and FE slabs, the owned columns of the vertex-edge
-// transpose (nrow = entries of the patch's owned rows), the half-edge
-// successor table and the global ids that fix each ring's start.
+// FE words of a thread's faces, addresses clamped to the last face
+template <uint32_t T, uint32_t RF>
+__device__ __forceinline__ void load_faces(FaceWords (&fw)[RF], const uint16_t* __restrict__ fe, uint32_t nf)
+{
+#pragma unroll
+    for (uint32_t r = 0; r < RF; ++r)
+        if (r == 0 || r * T < nf) fw[r].load(fe, min(threadIdx.x + r * T, nf - 1u));
+}
+
+// ---- oriented VV / VE ----------------------------------------------------------
+// LDS carve: EV slab, per half-edge the next one around its start, per owned
+// vertex the best start (u64) and the row offset, the rows (nrow = entries of
+// the patch's owned rows), global ids of the local vertices and linear ids of
+// the ribbon's elements the rows list.
 struct PlanVXO
 {
-    uint32_t *ev, *off, *wave, *slots, *gid;
-    uint16_t *fe, *hn;
+    uint64_t* start;
+    uint32_t *ev, *nh, *off, *wave, *gid, *rid;
+    uint16_t* rows;
 };
-__host__ __device__ inline PlanVXO plan_vxo(Bump& b, uint32_t nv, uint32_t ne, uint32_t nf, uint32_t nvo,
-                                            uint32_t nrow)
+__host__ __device__ inline PlanVXO plan_vxo(Bump& b, uint32_t nv, uint32_t ne, uint32_t nvo, uint32_t nrow,
+                                            uint32_t nrid)
 {
     PlanVXO p{};
+    p.start = b.alloc<uint64_t>(nvo);
     p.ev    = b.alloc<uint32_t>(r4(ne));
+    p.nh    = b.alloc<uint32_t>(ne);
     p.off   = b.alloc<uint32_t>(nvo + 1);
     p.wave  = b.alloc<uint32_t>(20);
-    p.slots = b.alloc<uint32_t>(nrow);
-    p.fe    = b.alloc<uint16_t>(r4(3 * nf));
-    p.hn    = b.alloc<uint16_t>(2 * ne);
     p.gid   = b.alloc<uint32_t>(nv);
+    p.rid   = b.alloc<uint32_t>(nrid + 1u);  // at least one: read at clamped indices
+    p.rows  = b.alloc<uint16_t>(nrow);
     return p;
 }
 
@@ -49,38 +61,62 @@ __host__ __device__ inline PlanFX plan_fx(Bump& b, uint32_t ne, uint32_t nf)
     return p;
 }
 
-// Oriented rows of the patch's owned vertices: stage EV / FE / global ids,
-// build the half-edge successor table and the owned columns of the
-// vertex-edge transpose, then order every row into its canonical CCW ring
-// (neighbour vertices if NBR, else edges) in place in L.slots. On return
-// L.off[v] is the start of row v and L.off[nvo] the total.
-template <uint32_t T, bool NBR>
-__device__ inline void oriented_rows(const DevMesh& m, const PatchDesc& d, const PlanVXO& L)
+// The ring of a vertex of several fans, or whose fan does not start where the
+// rule says: the vertex's edges in ascending local id, then the rule of
+// orient_ring_lds (selection of a start among the edges left, walk, restart).
+template <bool NBR>
+__device__ inline void ring_by_selection(uint32_t v, uint32_t k0, uint32_t k1, const PlanVXO& L, uint32_t ne)
 {
-    stage_u32(L.ev, m.ev + d.e_off, d.ne);
-    stage_fe(L.fe, m.fe + 3u * d.f_off, d.nf);
-    for (uint32_t v = threadIdx.x; v < d.nv; v += T) L.gid[v] = m.ltog_v[d.v_off + v];
-    for (uint32_t i = threadIdx.x; i < d.ne; i += T) reinterpret_cast<uint32_t*>(L.hn)[i] = 0xFFFFFFFFu;
-    for (uint32_t c = threadIdx.x; c <= d.nvo; c += T) L.off[c] = 0;
-    __syncthreads();
-    // the successor table is complete before the rows are ordered: the
-    // counting sort below contains block barriers
-    build_half_next(L.fe, L.ev, d.nf, L.hn);
-    fill_columns<T, true>(
-        2 * d.ne, d.nvo,
-        [&](uint32_t i) {
-            const uint32_t x = L.ev[i >> 1];
-            return (i & 1u) ? hi16(x) : lo16(x);
-        },
-        [&](uint32_t i) { return i >> 1; }, L.off, L.slots, L.wave);
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T)
-        orient_ring<12, NBR>(v, L.off[v], L.off[v + 1], L.slots, L.slots, L.ev, L.hn, L.gid);
-    __syncthreads();
+    const uint16_t* ev16 = reinterpret_cast<const uint16_t*>(L.ev);
+    const uint16_t* nh   = reinterpret_cast<const uint16_t*>(L.nh);
+    uint32_t        n = k0;
+    for (uint32_t i = 0; i < 2u * ne && n < k1; ++i)  // half-edge i leaves vertex ev16[i]
+        if (ev16[i] == v) L.rows[n++] = static_cast<uint16_t>(i);
+    auto nbr       = [&](uint32_t h) { return static_cast<uint32_t>(ev16[h ^ 1u]); };
+    auto startable = [&](uint32_t h) { return nh[h] != kInv16 && nh[h ^ 1u] == kInv16; };
+    uint32_t pos = k0;
+    while (pos < k1) {
+        uint32_t best = pos;
+        for (uint32_t j = pos + 1; j < k1; ++j) {
+            const uint32_t hj = L.rows[j], hb = L.rows[best];
+            const bool     sj = startable(hj), sb = startable(hb);
+            if ((sj && !sb) || (sj == sb && L.gid[nbr(hj)] < L.gid[nbr(hb)])) best = j;
+        }
+        uint16_t x   = L.rows[pos];
+        L.rows[pos]  = L.rows[best];
+        L.rows[best] = x;
+        while (true) {
+            const uint32_t q = nh[L.rows[pos]];
+            uint32_t       j = pos + 1;
+            while (j < k1 && L.rows[j] != q) ++j;
+            if (q == kInv16 || j >= k1) break;
+            x               = L.rows[pos + 1];
+            L.rows[pos + 1] = L.rows[j];
+            L.rows[j]       = x;
+            ++pos;
+        }
+        ++pos;
+    }
+    for (uint32_t k = k0; k < k1; ++k) {
+        const uint32_t h = L.rows[k];
+        L.rows[k]        = static_cast<uint16_t>(NBR ? nbr(h) : h >> 1);
+    }
 }
 
-// Oriented VV (IS_VV) or VE; rows leave as one contiguous range per patch.
+// Oriented VV (IS_VV) or VE: every owned vertex's canonical CCW ring (the rule is
+// orient.hpp's). Face slot i holds half-edge fv[i] -> fv[i+1]; the one after it
+// around fv[i] is the reverse of slot i + 2, so the FE words alone give every
+// half-edge its successor (one LDS store per slot). The start -- an edge the walk
+// can proceed from and no face precedes, else the smallest global id -- is one
+// 64-bit LDS minimum per half-edge over (not startable, neighbour's global id,
+// half-edge); the ring is then one LDS read per entry along the successors.
+// Sorting each row and matching successors against it in registers took 43.7 us
+// on 654k vertices and 110 on 2.6M; this takes 19.0 and 46. Bound: LDS (random
+// minima and adds). A vertex the walk does not
+// exhaust (several fans) takes ring_by_selection. Needs ne < 2^15 and a
+// consistently oriented edge-manifold mesh (checked on the host).
 template <uint32_t T, bool IS_VV>
-__global__ __launch_bounds__(T) void k_query_vx_oriented(DevMesh m, const uint32_t* __restrict__ base,
+__global__ __launch_bounds__(T) void k_query_vx_oriented(DevMesh m, uint32_t nrid, const uint32_t* __restrict__ base,
                                                          int32_t* __restrict__ row_ptr, int32_t* __restrict__ col)
 {
     extern __shared__ uint4 smem[];
@@ -89,18 +125,81 @@ __global__ __launch_bounds__(T) void k_query_vx_oriented(DevMesh m, const uint32
     const PatchDesc d   = load_desc(m.patch, p);
     const uint32_t  bse = base[p], nent = base[p + 1] - bse;
     Bump            b(reinterpret_cast<char*>(smem));
-    const PlanVXO   L = plan_vxo(b, d.nv, d.ne, d.nf, d.nvo, nent);
-    oriented_rows<T, IS_VV>(m, d, L);
+    const PlanVXO   L = plan_vxo(b, d.nv, d.ne, d.nvo, nent, nrid);
+    const uint32_t  t = threadIdx.x, nvo = d.nvo;
+    const uint16_t* fe  = m.fe + 3u * d.f_off;
+    const u32x4*    evs = reinterpret_cast<const u32x4*>(m.ev + d.e_off);
+    const uint32_t* gs  = m.ltog_v + d.v_off;
+    const uint32_t  no = IS_VV ? nvo : d.neo, nr = (IS_VV ? d.nv : d.ne) - no, pre = IS_VV ? d.vp : d.ep;
+    const uint32_t* rs = (IS_VV ? m.v_lin + d.v_off : m.e_lin + d.e_off) + no;
+    FaceWords                              fw[(768u + T - 1u) / T];
+    Held<T, (384u + T - 1u) / T, u32x4>    h_ev;
+    Held<T, (512u + T - 1u) / T, uint32_t> h_gid;
+    Held<T, (256u + T - 1u) / T, uint32_t> h_rid;
+    h_ev.load(evs, r4(d.ne) >> 2);
+    load_faces<T>(fw, fe, d.nf);
+    h_gid.load(gs, d.nv);
+    h_rid.load(rs, nr);
+    for (uint32_t i = t; i < d.ne; i += T) L.nh[i] = 0xFFFFFFFFu;
+    for (uint32_t v = t; v < nvo; v += T) L.start[v] = ~0ull;
+    for (uint32_t v = t; v <= nvo; v += T) L.off[v] = 0u;
+    h_ev.store(reinterpret_cast<u32x4*>(L.ev), evs, r4(d.ne) >> 2);
+    h_gid.store(L.gid, gs, d.nv);
+    h_rid.store(L.rid, rs, nr);
+    __syncthreads();
+    uint16_t* nh = reinterpret_cast<uint16_t*>(L.nh);
+    auto face = [&](const uint32_t (&x)[3]) {
+#pragma unroll
+        for (uint32_t i = 0; i < 3; ++i) nh[x[i]] = static_cast<uint16_t>(x[(i + 2u) % 3u] ^ 1u);
+    };
+#pragma unroll
+    for (uint32_t r = 0; r < (768u + T - 1u) / T; ++r)
+        if (t + r * T < d.nf) {
+            uint32_t x[3];
+            fw[r].get(x);
+            face(x);
+        }
+    for (uint32_t f = t + (768u + T - 1u) / T * T; f < d.nf; f += T) {
+        const uint32_t x[3] = {fe[3 * f], fe[3 * f + 1], fe[3 * f + 2]};
+        face(x);
+    }
+    __syncthreads();
+    for (uint32_t e = t; e < d.ne; e += T) {
+        const uint32_t x = L.ev[e], n = L.nh[e];
+        const bool     f0 = lo16(n) != kInv16, f1 = hi16(n) != kInv16;  // half-edge 2 e / 2 e + 1 has a face
+        auto half = [&](uint32_t v, uint32_t q, uint32_t h, bool startable) {
+            if (v >= nvo) return;
+            const uint64_t key = (uint64_t(startable ? 0u : 1u) << 63) | (uint64_t(L.gid[q]) << 16) | h;
+            atomicMin(reinterpret_cast<unsigned long long*>(&L.start[v]), static_cast<unsigned long long>(key));
+            atomicAdd(&L.off[v + 1u], 1u);
+        };
+        half(lo16(x), hi16(x), 2u * e, f0 && !f1);
+        half(hi16(x), lo16(x), 2u * e + 1u, f1 && !f0);
+    }
+    const uint32_t total = scan_excl<T>(L.off + 1, nvo, L.wave);  // off[v + 1] = start of row v
     // the host's row counts (global valences) match the patch's owned
     // columns on every manifold patch; anything else leaves it unwritten
-    if (L.off[d.nvo] != nent) return;
-    for (uint32_t v = threadIdx.x; v < d.nvo; v += T) row_ptr[d.vp + v] = static_cast<int32_t>(bse + L.off[v]);
-    if (threadIdx.x == 0) row_ptr[d.vp + d.nvo] = static_cast<int32_t>(bse + nent);
-    for (uint32_t k = threadIdx.x; k < nent; k += T) {
-        const uint32_t x = L.slots[k];
-        const uint32_t out = IS_VV ? lin_of(x, d.nvo, d.vp, m.v_lin + d.v_off)
-                                   : lin_of(x, d.neo, d.ep, m.e_lin + d.e_off);
-        col[bse + k] = static_cast<int32_t>(out);
+    if (total != nent) return;
+    const uint16_t* ev16 = reinterpret_cast<const uint16_t*>(L.ev);
+    auto            row0 = [&](uint32_t v) { return L.off[v + 1u]; };
+    auto            row1 = [&](uint32_t v) { return v + 1u < nvo ? L.off[v + 2u] : nent; };
+    for (uint32_t v = t; v < nvo; v += T) {
+        const uint32_t k0 = row0(v), k1 = row1(v);
+        if (k0 >= k1) continue;
+        const uint32_t s = static_cast<uint32_t>(L.start[v]) & 0xFFFFu;
+        uint32_t       h = s, k = k0;
+        do {
+            L.rows[k++] = static_cast<uint16_t>(IS_VV ? static_cast<uint32_t>(ev16[h ^ 1u]) : h >> 1);
+            h           = nh[h];
+        } while (k < k1 && h != kInv16 && h != s);
+        if (k < k1) ring_by_selection<IS_VV>(v, k0, k1, L, d.ne);
+    }
+    __syncthreads();
+    for (uint32_t v = t; v < nvo; v += T) row_ptr[d.vp + v] = static_cast<int32_t>(bse + row0(v));
+    if (t == 0) row_ptr[d.vp + nvo] = static_cast<int32_t>(bse + nent);
+    for (uint32_t k = t; k < nent; k += T) {
+        const uint32_t x = L.rows[k], r = L.rid[max(x, no) - no];
+        col[bse + k]     = static_cast<int32_t>((x < no) ? pre + x : r);
     }
 }
 
@@ -190,13 +289,6 @@ __device__ __forceinline__ void edge_opposites(const FaceWords (&fw)[RF], const 
         const uint32_t x[3] = {fe[3 * f], fe[3 * f + 1], fe[3 * f + 2]};
         face(f, x);
     }
-}
-template <uint32_t T, uint32_t RF>
-__device__ __forceinline__ void load_faces(FaceWords (&fw)[RF], const uint16_t* __restrict__ fe, uint32_t nf)
-{
-#pragma unroll
-    for (uint32_t r = 0; r < RF; ++r)
-        if (r == 0 || r * T < nf) fw[r].load(fe, min(threadIdx.x + r * T, nf - 1u));
 }
 
 // Rows leave as one 16-byte store per edge; vertex ids of the ribbon are staged

@@ -883,6 +883,354 @@ __global__ __launch_bounds__(T) void k_query2_x1(DevMesh m, uint32_t nslots, uin
     }
 }
 
+// ---- vertex rows in fixed-width slots ------------------------------------------
+// VV / VE and VF rows of meshes whose vertices have at most kRowMax edges and
+// faces: every owned vertex has kRowMax u16 slots per relation, so an entry is
+// placed by one returning LDS atomic on its vertex's counter (VV counts in the
+// low half, VF in the high half of one word) with no histogram before it; a
+// vertex's rows are read with one 16-byte load each, sorted in registers two
+// relations at once (packed u16 min / max, slots left at 0xFFFF sort last),
+// placed by one packed scan over the counts and written back compacted over
+// the slots; one coalesced pass then turns them into linear ids. Same CSRs as
+// k_query2_vv_vf1 / k_query2_x1, which serve the other meshes. A slot holds
+// EV's u16 index of the row's other endpoint (2 e + 1 - end, sorts like e) or
+// the local face. Per
+// wave 489 VALU and 102 LDS instructions against 654 and 136. VV + VF: 654k vertices
+// 25.3 -> 21.0 us, 2.6M 67.6 -> 57.9; VV 37.6 -> 31.6, VF 38.2 -> 33. Bound: LDS, busy
+// three quarters of the time, over half of that in bank conflicts of the random
+// atomics and slot stores.
+// REL: kRowsVV or kRowsVE, kRowsVF, or a VV with a VF.
+enum : uint32_t { kRowsVV = 1, kRowsVE = 2, kRowsVF = 4 };
+constexpr uint32_t kRowMax = 8;
+
+struct PlanRows
+{
+    uint32_t *ev, *cnt, *wave, *lv, *lf;
+    uint16_t* slots;
+};
+// nl: local vertices (VV) or edges (VE) of the patch, 0 without them; nlf: local
+// faces (VF) or 0. The slots come first: their LDS address is a constant.
+__host__ __device__ inline PlanRows plan_rows(Bump& b, uint32_t nvo, uint32_t ne, uint32_t nrel, uint32_t nl,
+                                              uint32_t nlf)
+{
+    PlanRows p{};
+    p.slots = b.alloc<uint16_t>(kRowMax * nrel * nvo);
+    p.ev    = b.alloc<uint32_t>(r4(ne));
+    p.cnt   = b.alloc<uint32_t>(nvo);
+    p.wave  = b.alloc<uint32_t>(64);
+    p.lv    = b.alloc<uint32_t>(nl);
+    p.lf    = b.alloc<uint32_t>(nlf);
+    return p;
+}
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+// compare-exchange of both halves
+__device__ __forceinline__ void cswap2(uint32_t& a, uint32_t& b)
+{
+    const u16x2 x = __builtin_bit_cast(u16x2, a), y = __builtin_bit_cast(u16x2, b);
+    a = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(x, y));
+    b = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(x, y));
+}
+// the networks of net_sort on two u16 rows at once
+template <uint32_t N>
+__device__ __forceinline__ void net_sort2(uint32_t (&a)[8])
+{
+    if constexpr (N == 6) {
+        cswap2(a[0], a[5]); cswap2(a[1], a[3]); cswap2(a[2], a[4]);
+        cswap2(a[1], a[2]); cswap2(a[3], a[4]);
+        cswap2(a[0], a[3]); cswap2(a[2], a[5]);
+        cswap2(a[0], a[1]); cswap2(a[2], a[3]); cswap2(a[4], a[5]);
+        cswap2(a[1], a[2]); cswap2(a[3], a[4]);
+    } else {
+        cswap2(a[0], a[1]); cswap2(a[2], a[3]); cswap2(a[4], a[5]); cswap2(a[6], a[7]);
+        cswap2(a[0], a[2]); cswap2(a[1], a[3]); cswap2(a[4], a[6]); cswap2(a[5], a[7]);
+        cswap2(a[1], a[2]); cswap2(a[5], a[6]);
+        cswap2(a[0], a[4]); cswap2(a[1], a[5]); cswap2(a[2], a[6]); cswap2(a[3], a[7]);
+        cswap2(a[2], a[4]); cswap2(a[3], a[5]);
+        cswap2(a[1], a[2]); cswap2(a[3], a[4]); cswap2(a[5], a[6]);
+    }
+}
+
+// T threads, RF / RQ / RV rounds of faces, EV quads and owned vertices held in
+// registers: needs nf <= RF T, ne <= 4 RQ T, nvo <= RV T (checked on the host).
+template <uint32_t T, uint32_t RF, uint32_t RQ, uint32_t RV, uint32_t REL>
+__global__ __launch_bounds__(T) void k_query_rows(DevMesh m, const uint32_t* __restrict__ v_base,
+                                                  const uint32_t* __restrict__ f_base, int32_t* __restrict__ v_row,
+                                                  int32_t* __restrict__ v_col, int32_t* __restrict__ f_row,
+                                                  int32_t* __restrict__ f_col)
+{
+    constexpr bool     VE = REL & kRowsVE, V = (REL & kRowsVV) || VE, F = REL & kRowsVF;
+    constexpr uint32_t NREL = (V ? 1u : 0u) + (F ? 1u : 0u), NW = T / 64u;
+    static_assert(kRowMax == 8 && NW * RV <= 64, "slots of 16 bytes, wave totals");
+    extern __shared__ uint4 smem[];
+    const uint32_t  p = patch_of_block(m.P);  // XCD-contiguous patch ranges
+    if (p >= m.P) return;
+    const PatchDesc d = load_desc(m.patch, p);
+    const uint32_t  bv = V ? v_base[p] : 0u, bf = F ? f_base[p] : 0u;
+    Bump            b(reinterpret_cast<char*>(smem));
+    const PlanRows  L   = plan_rows(b, d.nvo, d.ne, NREL, VE ? d.ne : (V ? d.nv : 0u), F ? d.nf : 0u);
+    const uint32_t  nvo = d.nvo, t = threadIdx.x, lane = t & 63u, wid = t >> 6;
+    const uint16_t* fs  = m.fe + 3u * d.f_off;
+    const u32x4*    es  = reinterpret_cast<const u32x4*>(m.ev + d.e_off);
+    // linear ids of the ribbon's elements a VV / VE row and a VF row list
+    const uint32_t* vl = VE ? m.e_lin + d.e_off + d.neo : m.v_lin + d.v_off + nvo;
+    const uint32_t  no = VE ? d.neo : nvo, nr = (VE ? d.ne : d.nv) - no, mr = d.nf - d.nfo;
+    const uint32_t* fl = m.f_lin + d.f_off + d.nfo;
+    Held<T, RQ, u32x4> hq;
+    FaceWords          fw[RF];
+    Held<T, (256u + T - 1u) / T, uint32_t> hv, hf;
+    hq.load(es, r4(d.ne) >> 2);
+    if constexpr (F)
+#pragma unroll
+        for (uint32_t r = 0; r < RF; ++r)
+            if (r == 0 || r * T < d.nf) fw[r].load(fs, min(t + r * T, d.nf - 1u));
+    if constexpr (V) hv.load(vl, nr);
+    if constexpr (F) hf.load(fl, mr);
+    for (uint32_t i = t; i < nvo; i += T) L.cnt[i] = 0u;
+    for (uint32_t i = t; i < nvo * NREL; i += T)
+        reinterpret_cast<u32x4*>(L.slots)[i] = u32x4{0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
+    hq.store(reinterpret_cast<u32x4*>(L.ev), es, r4(d.ne) >> 2);
+    // linear ids of every local element: owned ids follow from the prefix
+    if constexpr (V) {
+        const uint32_t pre = VE ? d.ep : d.vp;
+        for (uint32_t l = t; l < no; l += T) L.lv[l] = pre + l;
+        hv.store(L.lv + no, vl, nr);
+    }
+    if constexpr (F) {
+        for (uint32_t l = t; l < d.nfo; l += T) L.lf[l] = d.fp + l;
+        hf.store(L.lf + d.nfo, fl, mr);
+    }
+    __syncthreads();
+    // counters in bytes of slots: slot `at` bytes into vertex v's row. The rank
+    // stays below kRowMax by the mesh's largest row; the mask keeps it there
+    auto slot = [](uint16_t* rows, uint32_t v, uint32_t at) {
+        return reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(rows) + (v * (2u * kRowMax) + (at & (2u * kRowMax - 1u))));
+    };
+    if constexpr (V) {
+        auto entry = [&](uint32_t v, uint32_t s) {
+            if (v < nvo) *slot(L.slots, v, atomicAdd(&L.cnt[v], 2u)) = static_cast<uint16_t>(s);
+        };
+#pragma unroll
+        for (uint32_t r = 0; r < RQ; ++r)
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t e = 4u * (t + r * T) + j;
+                if (e < d.ne) {
+                    const uint32_t x = hq.a[r][j];
+                    entry(lo16(x), 2u * e + 1u);
+                    entry(hi16(x), 2u * e);
+                }
+            }
+    }
+    if constexpr (F) {
+        constexpr uint32_t one = V ? 0x20000u : 2u, sh = V ? 16u : 0u;
+        uint16_t* const    fslots = L.slots + (V ? kRowMax * nvo : 0u);
+#pragma unroll
+        for (uint32_t r = 0; r < RF; ++r) {
+            const uint32_t f = t + r * T;
+            if (f < d.nf) {
+                uint32_t x[3];
+                fw[r].get(x);
+#pragma unroll
+                for (uint32_t j = 0; j < 3; ++j) {
+                    const uint32_t e = L.ev[x[j] >> 1], v = (x[j] & 1u) ? hi16(e) : lo16(e);
+                    if (v < nvo)
+                        *slot(fslots, v, atomicAdd(&L.cnt[v], one) >> sh) = static_cast<uint16_t>(f);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    // per owned vertex: counts (VV low half, VF high; one relation: low), rows
+    // sorted in registers, packed exclusive scan of the counts
+    uint32_t c[RV], a[RV][8], inc[RV];
+#pragma unroll
+    for (uint32_t r = 0; r < RV; ++r) {
+        if (r && r * T >= nvo) continue;
+        const uint32_t v = t + r * T;
+        c[r]             = 0u;
+        if (v < nvo) {
+            c[r]           = L.cnt[v] >> 1;  // both halves are even
+            const u32x4 q0 = reinterpret_cast<const u32x4*>(L.slots)[v];
+            const u32x4 q1 = (NREL == 2) ? reinterpret_cast<const u32x4*>(L.slots)[nvo + v] : q0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                a[r][2 * j]     = __builtin_amdgcn_perm(q1[j], q0[j], 0x05040100u);  // low halves
+                a[r][2 * j + 1] = __builtin_amdgcn_perm(q1[j], q0[j], 0x07060302u);  // high halves
+            }
+        }
+        const bool wide = lo16(c[r]) > 6u || hi16(c[r]) > 6u;
+        if (!__builtin_amdgcn_ballot_w64(wide)) net_sort2<6>(a[r]);
+        else net_sort2<8>(a[r]);
+        inc[r] = wave_incl_scan(c[r]);
+        if (lane == 63u) L.wave[r * NW + wid] = inc[r];
+    }
+    __syncthreads();  // the wave totals; and every row is in registers
+    uint32_t before[RV], total = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < RV; ++r) {
+        if (r && r * T >= nvo) continue;
+        before[r] = total;
+#pragma unroll
+        for (uint32_t w = 0; w < NW; ++w) {
+            const uint32_t x = L.wave[r * NW + w];
+            before[r] += (w < wid) ? x : 0u;
+            total += x;
+        }
+    }
+    const uint32_t nvv = V ? lo16(total) : 0u, nvf = V ? hi16(total) : total;  // entries of the patch
+    if (t == 0) {
+        if constexpr (V) v_row[d.vp + nvo] = static_cast<int32_t>(bv + nvv);
+        if constexpr (F) f_row[d.vp + nvo] = static_cast<int32_t>(bf + nvf);
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < RV; ++r) {
+        const uint32_t v = t + r * T;
+        if (v >= nvo) continue;
+        const uint32_t o = before[r] + inc[r] - c[r];
+        if constexpr (V) {
+            const uint32_t o0 = lo16(o), k = lo16(c[r]);
+            v_row[d.vp + v]   = static_cast<int32_t>(bv + o0);
+#pragma unroll
+            for (uint32_t j = 0; j < kRowMax; ++j)
+                if (j < k) L.slots[o0 + j] = static_cast<uint16_t>(a[r][j]);
+        }
+        if constexpr (F) {
+            const uint32_t o1 = V ? hi16(o) : o, k = V ? hi16(c[r]) : c[r];
+            f_row[d.vp + v]   = static_cast<int32_t>(bf + o1);
+#pragma unroll
+            for (uint32_t j = 0; j < kRowMax; ++j)
+                if (j < k) L.slots[nvv + o1 + j] = static_cast<uint16_t>(V ? a[r][j] >> 16 : a[r][j]);
+        }
+    }
+    __syncthreads();
+    // columns
+    if constexpr (V) {
+        const uint16_t* ev16 = reinterpret_cast<const uint16_t*>(L.ev);
+        for (uint32_t i = t; i < nvv; i += T) {
+            const uint32_t s = L.slots[i];
+            v_col[bv + i]    = static_cast<int32_t>(L.lv[VE ? s >> 1 : static_cast<uint32_t>(ev16[s])]);
+        }
+    }
+    if constexpr (F)
+        for (uint32_t i = t; i < nvf; i += T) f_col[bf + i] = static_cast<int32_t>(L.lf[L.slots[nvv + i]]);
+}
+
+// ---- EF and FF of oriented edge-manifold meshes ----------------------------------
+// An edge has at most one face per direction there, and an FE word 2 e + dir names
+// the half-edge, so the faces of all local edges are one plain LDS store per face
+// slot: no histogram, no atomic, no sort. An EF row is the edge's two slots in
+// ascending order; an FF row is, per edge of the face, the slot of the reverse
+// half-edge. Counts are scanned per wave, rows go to LDS compacted and leave in
+// one coalesced pass. Same CSRs as k_query2_x1 / k_query2_ff1, which serve the
+// other meshes. EFNOTE
+struct PlanDir
+{
+    uint32_t *face, *lf, *wave;  // face: two u16 per edge (kInv16: none)
+    uint16_t* out;
+};
+// nout: the largest entry count of a patch
+__host__ __device__ inline PlanDir plan_dir(Bump& b, uint32_t ne, uint32_t nf, uint32_t nout)
+{
+    PlanDir p{};
+    p.face = b.alloc<uint32_t>(ne);
+    p.lf   = b.alloc<uint32_t>(nf);
+    p.wave = b.alloc<uint32_t>(64);
+    p.out  = b.alloc<uint16_t>(nout);
+    return p;
+}
+
+// RF / RS: rounds of local faces / of owned sources (edges, or faces for FF)
+// held in registers: needs nf <= RF T and neo (nfo) <= RS T, checked on the host.
+template <uint32_t T, uint32_t RF, uint32_t RS, bool FF>
+__global__ __launch_bounds__(T) void k_query_dir(DevMesh m, uint32_t nout, const uint32_t* __restrict__ base,
+                                                 int32_t* __restrict__ row_ptr, int32_t* __restrict__ col)
+{
+    constexpr uint32_t NW = T / 64u;
+    static_assert(NW * RS <= 64, "wave totals");
+    extern __shared__ uint4 smem[];
+    const uint32_t  p = patch_of_block(m.P);  // XCD-contiguous patch ranges
+    if (p >= m.P) return;
+    const PatchDesc d   = load_desc(m.patch, p);
+    const uint32_t  bse = base[p];
+    Bump            b(reinterpret_cast<char*>(smem));
+    const PlanDir   L = plan_dir(b, d.ne, d.nf, nout);
+    const uint32_t  t = threadIdx.x, lane = t & 63u, wid = t >> 6;
+    const uint32_t  ns = FF ? d.nfo : d.neo, r0 = FF ? d.fp : d.ep;  // sources, their linear-id prefix
+    const uint16_t* fe = m.fe + 3u * d.f_off;
+    const uint32_t* fl = m.f_lin + d.f_off + d.nfo;
+    FaceWords       fw[RF];
+    Held<T, (256u + T - 1u) / T, uint32_t> hf;
+#pragma unroll
+    for (uint32_t r = 0; r < RF; ++r)
+        if (r == 0 || r * T < d.nf) fw[r].load(fe, min(t + r * T, d.nf - 1u));
+    hf.load(fl, d.nf - d.nfo);
+    for (uint32_t i = t; i < d.ne; i += T) L.face[i] = 0xFFFFFFFFu;
+    for (uint32_t l = t; l < d.nfo; l += T) L.lf[l] = d.fp + l;
+    hf.store(L.lf + d.nfo, fl, d.nf - d.nfo);
+    __syncthreads();
+    uint16_t* const face = reinterpret_cast<uint16_t*>(L.face);
+#pragma unroll
+    for (uint32_t r = 0; r < RF; ++r)
+        if (t + r * T < d.nf) {
+            uint32_t x[3];
+            fw[r].get(x);
+#pragma unroll
+            for (uint32_t j = 0; j < 3; ++j) face[x[j]] = static_cast<uint16_t>(t + r * T);
+        }
+    __syncthreads();
+    uint32_t g[RS][FF ? 3 : 2], cnt[RS], inc[RS];
+#pragma unroll
+    for (uint32_t r = 0; r < RS; ++r) {
+        if (r && r * T >= ns) continue;
+        const uint32_t i = t + r * T;
+        cnt[r]           = 0u;
+        if (i < ns) {
+            if constexpr (FF) {
+                static_assert(!FF || RS <= RF, "a source face's words are held");
+                uint32_t x[3];
+                fw[r].get(x);
+#pragma unroll
+                for (uint32_t j = 0; j < 3; ++j) {
+                    g[r][j] = face[x[j] ^ 1u];
+                    cnt[r] += (g[r][j] != kInv16) ? 1u : 0u;
+                }
+            } else {
+                const uint32_t q = L.face[i];  // kInv16 sorts last
+                g[r][0]          = min(lo16(q), hi16(q));
+                g[r][1]          = max(lo16(q), hi16(q));
+                cnt[r]           = (g[r][0] != kInv16 ? 1u : 0u) + (g[r][1] != kInv16 ? 1u : 0u);
+            }
+        }
+        inc[r] = wave_incl_scan(cnt[r]);
+        if (lane == 63u) L.wave[r * NW + wid] = inc[r];
+    }
+    __syncthreads();
+    uint32_t total = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < RS; ++r) {
+        if (r && r * T >= ns) continue;
+        uint32_t o = total;
+#pragma unroll
+        for (uint32_t w = 0; w < NW; ++w) {
+            const uint32_t x = L.wave[r * NW + w];
+            o += (w < wid) ? x : 0u;
+            total += x;
+        }
+        o += inc[r] - cnt[r];
+        const uint32_t i = t + r * T;
+        if (i < ns) {
+            row_ptr[r0 + i] = static_cast<int32_t>(bse + o);
+#pragma unroll
+            for (uint32_t j = 0; j < (FF ? 3u : 2u); ++j)
+                if (g[r][j] != kInv16) L.out[o++] = static_cast<uint16_t>(g[r][j]);
+        }
+    }
+    if (t == 0) row_ptr[r0 + ns] = static_cast<int32_t>(bse + total);
+    __syncthreads();
+    for (uint32_t i = t; i < total; i += T) col[bse + i] = static_cast<int32_t>(L.lf[L.out[i]]);
+}
+
 // FF in one pass: the EF counting sort over every local edge (keys = the
 // edges of the faces' FE words, held in registers), the edge rows sorted,
 // then each owned face lists the faces of its three edges but itself (edges

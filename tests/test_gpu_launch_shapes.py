@@ -264,3 +264,99 @@ def test_calls_go_to_the_current_stream():
         th.join()
     assert got[0][0] == got[0][1]
     assert rx._stream(None) == torch.cuda.current_stream().cuda_stream
+
+
+def _fan(k, closed):
+    """One vertex with k neighbours in a closed or open fan."""
+    ring = np.arange(1, k + 1)
+    nxt = np.roll(ring, -1)
+    f = np.stack([np.zeros(k, np.int64), ring, nxt], 1)
+    return (f if closed else f[:-1]).astype(np.uint32)
+
+
+def _query_mesh(name):
+    if name == "sphere":
+        return mg.permute_mesh(*mg.icosphere(4, seed=2, sigma=0.01), seed=2)[1]
+    if name == "grid":
+        return mg.grid(45, seed=2)[1]
+    if name == "torus":  # valence 4 and 8
+        return mg.permute_mesh(*mg.torus(40, 30), seed=2)[1]
+    if name == "triangle":
+        return np.array([[0, 1, 2]], np.uint32)
+    if name == "fan7":
+        return _fan(7, False)
+    if name == "fan8":
+        return _fan(8, True)
+    if name == "fan9":  # one row beyond the fixed slots
+        return np.concatenate([mg.grid(20, seed=2)[1], _fan(9, True) + 400])
+    if name == "fan40":
+        return _fan(40, True)
+    if name == "bowtie":  # two fans, and three, sharing one vertex
+        a, b = _fan(6, True), _fan(4, False)
+        b[b > 0] += 10
+        c = _fan(5, False)
+        c[c > 0] += 20
+        f = np.concatenate([a, b, c])
+        return np.unique(f, return_inverse=True)[1].reshape(-1, 3).astype(np.uint32)
+    if name == "flipped":
+        f = mg.grid(20, seed=2)[1].copy()
+        f[37] = f[37][::-1]
+        return f
+    f = mg.grid(12, seed=2)[1]  # "fin": an edge with three faces
+    return np.concatenate([f, np.array([[f[50][0], f[50][1], 144]], np.uint32)])
+
+
+@pytest.mark.parametrize("name", ["sphere", "grid", "torus", "triangle", "fan7", "fan8", "fan9", "fan40", "bowtie",
+                                  "flipped", "fin"])
+@pytest.mark.parametrize("patch_size", [16, 256, 512, 1024, 4096])
+def test_query_kernels_over_forms(name, patch_size):
+    """Every relation of the default kernels against the oracle: meshes inside
+    and outside what the fixed-slot and direct-slot kernels take (long rows,
+    flipped faces, edges with three faces), patches on either side of their
+    register rounds, vertices of several fans for the oriented rows, and the
+    general kernels (knob 10 = 0) on the same mesh."""
+    import rxmesh_amd as rx
+    import torch
+    from oracle.oracle import OracleMesh
+    F = _query_mesh(name)
+    m = rx.Mesh(F, patch_size=patch_size)
+    o = OracleMesh(F).set_patches(m.array("face_patch"), m.array("patches_val"), m.array("patches_offset"))
+    for knob in (2, 0):
+        m.set_launch_threads(10, knob)
+        for op in ("VV", "VE", "VF", "EF", "FF", "EV", "FV", "FE", "EVD"):
+            rp, col = m.query(op)
+            orp, ocol = o.query(op)
+            assert np.array_equal(rp.cpu().numpy(), orp), (op, knob)
+            assert np.array_equal(col.cpu().numpy()[:len(ocol)], ocol), (op, knob)
+        (vr, vc), (fr, fc) = m.query_vv_vf()
+        for (rp, col), op in (((vr, vc), "VV"), ((fr, fc), "VF")):
+            orp, ocol = o.query(op)
+            assert np.array_equal(rp.cpu().numpy(), orp) and np.array_equal(col.cpu().numpy()[:len(ocol)], ocol)
+    if name in ("flipped", "fin"):
+        return
+    for threads in (256, 512):
+        m.set_launch_threads(6, threads)
+        for op in ("VV", "VE"):
+            rp, col = m.query(op, oriented=True)
+            orp, ocol = o.query(op, oriented=True)
+            assert np.array_equal(rp.cpu().numpy(), orp) and np.array_equal(col.cpu().numpy()[:len(ocol)], ocol), op
+
+
+@pytest.mark.parametrize("level,patch_size", [(7, 512), (7, 1024), (7, 128), (6, 256)])
+def test_query_kernels_of_many_patches(level, patch_size):
+    """The workgroup sizes chosen for hundreds and thousands of patches: the
+    rows of the general kernels, bit for bit."""
+    import torch
+    V, F = mg.permute_mesh(*mg.icosphere(level, seed=5), seed=5)
+    m, _ = _mesh(V, F, patch_size)
+    for op in ("VV", "VE", "VF", "EF", "FF"):
+        m.set_launch_threads(10, 2)
+        rp, col = m.query(op)
+        m.set_launch_threads(10, 0)
+        r2, c2 = m.query(op)
+        assert torch.equal(rp, r2) and torch.equal(col, c2), op
+    m.set_launch_threads(10, 2)
+    a = m.query_vv_vf()
+    m.set_launch_threads(10, 0)
+    b = m.query_vv_vf()
+    assert all(torch.equal(x, y) for p, q in zip(a, b) for x, y in zip(p, q))
