@@ -478,10 +478,14 @@ int ensure_face_plan(rxm_mesh* m, void* stream)
 // latency. Ten single steps with 512 / 256 threads: 71 patches 35.4 / 43.5 us,
 // 491 42.6 / 48.1, 1279 61.8 / 64.3, 2015 80.9 / 78.6, 4249 143 / 124.
 // Several steps per launch have more to spread: three steps, ten iterations,
-// 2015 patches 55.1 / 57.2, 4249 102.8 / 100.7.
+// 2015 patches 55.1 / 57.2, 4249 102.8 / 100.7; with 1024 / 512 threads, ten
+// steps five a launch, 10 patches 14.1 / 15.2, 167 14.8 / 16.1, 491 22.0 / 22.2,
+// 1037 (three a launch) 55 / 38.
 uint32_t smooth_group(const rxm_mesh* m, bool multi = false)
 {
-    return m->smooth_threads ? m->smooth_threads : (m->h.P <= (multi ? 3000u : 1500u) ? 512u : 256u);
+    if (m->smooth_threads) return m->smooth_threads;
+    if (multi) return m->h.P <= 256u ? 1024u : m->h.P <= 3000u ? 512u : 256u;
+    return m->h.P <= 1500u ? 512u : 256u;
 }
 
 template <bool AOS4>
@@ -694,6 +698,7 @@ int smooth_steps(rxm_mesh* m, uint32_t steps, float lambda, const float* src, fl
         case 64: return go(k_smoothk<64>, 64);
         case 256: return go(k_smoothk<256>, 256);
         case 512: return go(k_smoothk<512>, 512);
+        case 1024: return go(k_smoothk<1024>, 1024);
         default: return go(k_smoothk<128>, 128);
     }
 }
@@ -1250,8 +1255,13 @@ rxm_status rxm_vertex_normals(rxm_mesh* m, int mode, const float* pos, float* no
     if (prc == RXM_OK) {
         Bump b(nullptr);
         plan_vnp(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
-        return launch_patches_xcd(k_vertex_normals_plan<256>, 256, b.bytes(), stream, m, m->dm, mode, m->d_fp_fbase,
-                              m->d_fp_rbase, m->d_fp_nbase, m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, normals);
+        auto go = [&](auto kernel, uint32_t T) {
+            return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, mode, m->d_fp_fbase, m->d_fp_rbase,
+                                      m->d_fp_nbase, m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, normals);
+        };
+        // us with 512 / 256 threads: 10 patches 4.0 / 4.6, 491 5.4 / 6.0, 2687
+        // 18.2 / 18.5, 10677 55 / 50
+        return m->h.P <= 4096u ? go(k_vertex_normals_plan<512>, 512) : go(k_vertex_normals_plan<256>, 256);
     }
     if (prc != RXM_ERR_PATCH_TOO_BIG) return prc;
     Bump b(nullptr);
@@ -1279,7 +1289,10 @@ rxm_status rxm_arap_weights(rxm_mesh* m, const float* pos, float* w, void* strea
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
     Bump b(nullptr);
     plan_aw(b, m->h.max_nv, m->h.max_ne, m->h.max_neo);
-    return launch_patches_xcd(k_arap_weights<256>, 256, b.bytes(), stream, m, m->dm, pos, w);
+    auto go = [&](auto kernel, uint32_t T) { return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, pos, w); };
+    // us with 1024 / 256 threads: 10 patches 3.7 / 4.6, 491 4.9 / 5.6, 1037 8.6 /
+    // 8.0, 2687 17.8 / 14.5 (512 lies between: 3.8, 5.0, 7.8, 14.8)
+    return m->h.P <= 512u ? go(k_arap_weights<1024>, 1024) : go(k_arap_weights<256>, 256);
 }
 
 namespace {

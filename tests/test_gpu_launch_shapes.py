@@ -360,3 +360,33 @@ def test_query_kernels_of_many_patches(level, patch_size):
     m.set_launch_threads(10, 0)
     b = m.query_vv_vf()
     assert all(torch.equal(x, y) for p, q in zip(a, b) for x, y in zip(p, q))
+
+
+@pytest.mark.parametrize("level,patch_size", [(1, 512), (4, 16), (4, 512), (5, 2048), (5, 16), (6, 16)])
+def test_normals_and_edge_weights_of_few_and_many_patches(level, patch_size):
+    """Every workgroup size that the patch count chooses, patches from a few
+    faces to more than the register rounds. FP32 sums of a few exact-input
+    terms: 1e-5 of the largest value."""
+    V, F = mg.permute_mesh(*mg.icosphere(level, seed=8, sigma=0.002), seed=8)
+    m, x = _mesh(V, F, patch_size)
+    l2g = m.array("v_l2g")
+    X = np.empty((m.nV, 3))
+    X[l2g] = x.cpu().numpy().T
+    c = X[F]
+    n = np.cross(c[:, 1] - c[:, 0], c[:, 2] - c[:, 0])
+    l = ((c - np.roll(c, -1, 1)) ** 2).sum(2)  # corner j to j + 1
+    for mode, wt in (("max", 1.0 / (l + np.roll(l, 1, 1))), ("area", np.full(l.shape, 0.5))):
+        ref = np.zeros((m.nV, 3))
+        np.add.at(ref, F.reshape(-1), (n[:, None, :] * wt[:, :, None]).reshape(-1, 3))
+        got = m.vertex_normals(x, mode).cpu().numpy().T
+        assert np.abs(got - ref[l2g]).max() <= 1e-5 * np.abs(ref).max()
+    cot = {}
+    for j in range(3):
+        a, b = c[:, (j + 1) % 3] - c[:, j], c[:, (j + 2) % 3] - c[:, j]
+        k = (a * b).sum(1) / np.linalg.norm(np.cross(a, b), axis=1)
+        for p, q, v in zip(F[:, (j + 1) % 3].tolist(), F[:, (j + 2) % 3].tolist(), k):
+            cot[(min(p, q), max(p, q))] = cot.get((min(p, q), max(p, q)), 0.0) + v
+    ev = np.sort(m.array("ev").reshape(-1, 2).astype(np.int64)[m.array("e_l2g")], 1)
+    w = m.arap_weights(x).cpu().numpy()
+    ref = np.array([cot[(a, b)] for a, b in ev.tolist()])
+    assert np.abs(w - np.maximum(0.0, 0.5 * ref)).max() <= 1e-5 * np.abs(ref).max()
