@@ -1283,72 +1283,6 @@ int build_patches(HostMesh& m)
 }
 
 // ---------------------------------------------------------------------------
-// Closed-fan vertices (host_build.h).
-void closed_fan_vertices(const HostMesh& m, std::vector<uint8_t>& closed)
-{
-    std::vector<uint32_t> valence(m.nV, 0);
-    for (uint32_t e = 0; e < m.nE; ++e) {
-        valence[m.ev[2ull * e]]++;
-        valence[m.ev[2ull * e + 1]]++;
-    }
-    closed.assign(m.nV, 0);
-    parallel_for(m.nV, [&](size_t v) {
-        const uint32_t b = m.vf_off[v], k = m.vf_off[v + 1] - b;
-        if (k == 0 || k != valence[v]) return;
-        std::vector<uint32_t> key(k), nxt(k);
-        for (uint32_t i = 0; i < k; ++i) {
-            const uint32_t f = m.vf_val[b + i];
-            uint32_t       j = 0;
-            while (j < 3 && m.fv[3ull * f + j] != v) ++j;
-            if (j == 3) return;
-            key[i] = m.fv[3ull * f + (j + 1) % 3];
-            nxt[i] = m.fv[3ull * f + (j + 2) % 3];
-        }
-        // follow the successor map from key[0]; a single cycle visits k keys
-        uint32_t cur = 0, steps = 0;
-        do {
-            uint32_t i = 0;
-            while (i < k && key[i] != nxt[cur]) ++i;
-            if (i == k) return;
-            cur = i;
-            ++steps;
-        } while (cur != 0 && steps <= k);
-        if (cur == 0 && steps == k) closed[v] = 1;
-    }, 4096);
-}
-
-// ---------------------------------------------------------------------------
-// Patch-local VV edge pattern (host_build.h).
-bool build_vv_edge_pattern(const HostMesh& m, const std::vector<uint32_t>& vv_base, std::vector<uint16_t>& ent,
-                           std::vector<uint32_t>& rs)
-{
-    for (uint32_t p = 0; p < m.P; ++p)
-        if (m.ne[p] >= 0x8000u) return false;
-    ent.assign(vv_base[m.P], 0);
-    rs.assign(m.nV + 1, 0);
-    rs[m.nV] = vv_base[m.P];
-    parallel_for(m.P, [&](size_t p) {
-        const uint32_t        nvo = m.nvo[p], ne = m.ne[p], vp = m.vp[p];
-        std::vector<uint32_t> cnt(nvo + 1, 0);
-        const uint32_t*       ev = m.ev_local.data() + m.e_off[p];
-        for (uint32_t e = 0; e < ne; ++e) {
-            const uint32_t a = ev[e] & 0xFFFFu, b = ev[e] >> 16;
-            if (a < nvo) cnt[a + 1]++;
-            if (b < nvo) cnt[b + 1]++;
-        }
-        for (uint32_t l = 0; l < nvo; ++l) cnt[l + 1] += cnt[l];
-        for (uint32_t l = 0; l < nvo; ++l) rs[vp + l] = vv_base[p] + cnt[l];
-        uint16_t* out = ent.data() + vv_base[p];
-        for (uint32_t e = 0; e < ne; ++e) {
-            const uint32_t a = ev[e] & 0xFFFFu, b = ev[e] >> 16;
-            if (a < nvo) out[cnt[a]++] = static_cast<uint16_t>(2u * e);
-            if (b < nvo) out[cnt[b]++] = static_cast<uint16_t>(2u * e + 1u);
-        }
-    }, 16);
-    return true;
-}
-
-// ---------------------------------------------------------------------------
 // Two-step smoothing plan (host_build.h).
 int build_vv2_plan(const HostMesh& m, Vv2Plan& out)
 {

@@ -159,24 +159,6 @@ struct VvkPlan
 };
 int build_vvk_plan(const HostMesh& m, uint32_t K, VvkPlan& out);
 
-// Vertices whose one-ring is one closed fan: the successor map of its faces
-// (half-edge v -> a of face (v, a, b) is followed by b) is a single cycle
-// through all its neighbours. The canonical ring of such a vertex has a real
-// face between every two consecutive neighbours, so its cotangent row can be
-// built from per-face quantities. Needs a consistently oriented mesh.
-// closed[g] = 1 for such vertices (global ids).
-void closed_fan_vertices(const HostMesh& m, std::vector<uint8_t>& closed);
-
-// Patch-local pattern of the VV query: for every patch p and owned vertex l,
-// the patch's local edges incident to l in ascending local edge id (the VV
-// query's row order), as ent[vv_base[p] + k] = 2 edge + (l is the edge's
-// second endpoint): the index, in FE's encoding, of the half-edge leaving l.
-// rs[lin] is the first entry of linear vertex lin, rs[nV] the total. vv_base
-// is the VV query's per-patch entry base (P + 1). Returns false when a patch
-// has 2^15 edges or more (the entries hold 16 bits).
-bool build_vv_edge_pattern(const HostMesh& m, const std::vector<uint32_t>& vv_base, std::vector<uint16_t>& ent,
-                           std::vector<uint32_t>& rs);
-
 // Host threads a build may use: RXM_NUM_THREADS or the hardware's count,
 // capped on the calling thread by a ThreadLimit in scope (k = 0 keeps the
 // current cap; threads a build spawns inherit the cap).

@@ -26,56 +26,6 @@ __device__ __forceinline__ void stage_positions(float* sx, float* sy, float* sz,
     }
 }
 
-// Same staging with all of a thread's loads issued before any LDS store:
-// R rounds of T vertices are unrolled, so a thread's owner-table loads go out
-// together, then its position gathers, instead of one dependent load chain
-// per loop iteration. Vertices past R * T (larger patches) take the loop.
-template <uint32_t T, uint32_t R, bool AOS4>
-__device__ __forceinline__ void stage_positions_batched(float* sx, float* sy, float* sz, float4* s4,
-                                                        const float* __restrict__ pos, uint32_t N,
-                                                        const PatchDesc& d, const uint32_t* __restrict__ v_lin)
-{
-    uint32_t g[R];
-    float    x[R], y[R], z[R];
-    const uint32_t* lin = v_lin + d.v_off;
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        const uint32_t l = threadIdx.x + r * T;
-        g[r]             = (l < d.nvo) ? d.vp + l : ((l < d.nv) ? lin[l] : 0u);
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        if (threadIdx.x + r * T < d.nv) {
-            x[r] = pos[g[r]];
-            y[r] = pos[N + g[r]];
-            z[r] = pos[2 * N + g[r]];
-        }
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < R; ++r) {
-        const uint32_t l = threadIdx.x + r * T;
-        if (l < d.nv) {
-            if constexpr (AOS4) {
-                s4[l] = make_float4(x[r], y[r], z[r], 0.f);
-            } else {
-                sx[l] = x[r];
-                sy[l] = y[r];
-                sz[l] = z[r];
-            }
-        }
-    }
-    for (uint32_t l = threadIdx.x + R * T; l < d.nv; l += T) {
-        const uint32_t gg = lin_of(l, d.nvo, d.vp, lin);
-        if constexpr (AOS4) {
-            s4[l] = make_float4(pos[gg], pos[N + gg], pos[2 * N + gg], 0.f);
-        } else {
-            sx[l] = pos[gg];
-            sy[l] = pos[N + gg];
-            sz[l] = pos[2 * N + gg];
-        }
-    }
-}
-
 // C-component SoA vertex attribute of a patch (component stride N) on its way
 // into LDS, in the two halves of Held: ids() and owned() issue the loads that
 // depend on the descriptor alone, ribbon() those that need the ribbon's owner
@@ -249,16 +199,6 @@ __host__ __device__ inline PlanSL plan_sl(Bump& b, uint32_t nv, uint32_t nvo, ui
         p.z = b.alloc<float>(nv);
     }
     return p;
-}
-
-// copy n u16 from a 16-byte aligned, 8-element padded run into LDS
-template <uint32_t T>
-__device__ __forceinline__ void stage_u16x8(uint16_t* dst, const uint16_t* __restrict__ src, uint32_t n)
-{
-    const uint32_t n8 = (n + 7u) >> 3;
-    const uint4*   s  = reinterpret_cast<const uint4*>(src);
-    uint4*         d  = reinterpret_cast<uint4*>(dst);
-    for (uint32_t i = threadIdx.x; i < n8; i += T) d[i] = s[i];
 }
 
 template <uint32_t T, bool AOS4>
