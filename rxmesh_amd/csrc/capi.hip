@@ -1255,10 +1255,14 @@ rxm_status rxm_vertex_normals(rxm_mesh* m, int mode, const float* pos, float* no
     if (prc == RXM_OK) {
         Bump b(nullptr);
         plan_vnp(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
+        const bool lean = b.bytes() > kMaxLdsBytes;
+        Bump       bl(nullptr);
+        plan_vnp(bl, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent, true);
         auto go = [&](auto kernel, uint32_t T) {
-            return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, mode, m->d_fp_fbase, m->d_fp_rbase,
+            return launch_patches_xcd(kernel, T, lean ? bl.bytes() : b.bytes(), stream, m, m->dm, mode, m->d_fp_fbase, m->d_fp_rbase,
                                       m->d_fp_nbase, m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, normals);
         };
+        if (lean) return go(k_vertex_normals_plan<256, true>, 256);
         // us with 512 / 256 threads: 10 patches 4.0 / 4.6, 491 5.4 / 6.0, 2687
         // 18.2 / 18.5, 10677 55 / 50
         return m->h.P <= 4096u ? go(k_vertex_normals_plan<512>, 512) : go(k_vertex_normals_plan<256>, 256);
@@ -1297,14 +1301,13 @@ rxm_status rxm_arap_weights(rxm_mesh* m, const float* pos, float* w, void* strea
 
 namespace {
 // the owned rows (the VV plan) and the LDS of the kernels over them
-int arap_rows(rxm_mesh* m, const uint32_t** vv_base, uint32_t* lds, bool rot, uint32_t threads, void* stream)
+int arap_rows(rxm_mesh* m, const uint32_t** vv_base, uint32_t* lds, bool rot, void* stream)
 {
     int rc = ensure_vv_plan(m, stream);
     if (!rc) rc = device_base(m, RXM_OP_VV, vv_base);
     if (rc) return rc;
     Bump b(nullptr);
     plan_ar(b, m->h.max_nv, m->h.max_ne, m->h.max_nvo, op_max_patch(m, RXM_OP_VV), rot);
-    if (!rot) b.alloc<float>(9u * threads);
     *lds = b.bytes();
     return RXM_OK;
 }
@@ -1321,13 +1324,16 @@ rxm_status rxm_arap_rotations(rxm_mesh* m, const float* rest, const float* x, co
     const uint32_t RT = m->h.P <= 512u ? 512u : 256u;
     const uint32_t* vv_base = nullptr;
     uint32_t        lds     = 0;
-    const int       rc      = arap_rows(m, &vv_base, &lds, false, RT, stream);
+    const int       rc      = arap_rows(m, &vv_base, &lds, false, stream);
     if (rc) return rc;
+    const bool run = lds + 36u * RT <= kMaxLdsBytes;  // room for a round's records
+    if (run) lds += 36u * RT;
     auto go = [&](auto kernel, uint32_t T) {
         return launch_patches_xcd(kernel, T, lds, stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
                                   static_cast<const uint16_t*>(m->d_vv_roff), static_cast<const uint16_t*>(m->d_vv_nbr),
                                   static_cast<const uint16_t*>(m->d_vv_ent), rest, x, w, R);
     };
+    if (!run) return go(k_arap_rotations<256, false>, 256);
     return RT == 512 ? go(k_arap_rotations<512>, 512) : go(k_arap_rotations<256>, 256);
 }
 
@@ -1339,7 +1345,7 @@ rxm_status rxm_arap_energy_grad(rxm_mesh* m, const float* rest, const float* x, 
     constexpr uint32_t RT = 512;
     const uint32_t* vv_base = nullptr;
     uint32_t        lds     = 0;
-    int             rc      = arap_rows(m, &vv_base, &lds, true, RT, stream);
+    int             rc      = arap_rows(m, &vv_base, &lds, true, stream);
     if (rc) return rc;
     if (!m->d_partial) {
         if (hipMalloc(&m->d_partial, sizeof(float) * m->h.P) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
@@ -1778,6 +1784,7 @@ rxm_status rxm_mcf_matfree_cg(rxm_mesh* m, const float* coords, const float* x, 
     int        rc  = RXM_OK;
     if (!uni) {
         if (!(m->h.manifold && m->h.oriented)) return RXM_ERR_NON_MANIFOLD;
+        if (!m->h.closed) return RXM_ERR_UNSUPPORTED;
         if ((rc = ensure_cot_plan(m, stream))) return rc;
         // the face pass gives a vertex its reference weights only when its
         // ring is one closed fan (a closed vertex-manifold mesh)

@@ -416,7 +416,9 @@ __device__ __forceinline__ void stage_arap(const DevMesh& m, const PatchDesc& d,
 // holds one row-major 3 x 3 record per vertex, R[9 v + 3 i + j] = R_v(i, j)
 // (the reference's rotations(v, i * 3 + j)): a ribbon vertex's rotation is
 // one or two cache lines for the energy kernel's gather, not nine.
-template <uint32_t T>
+// RUN: a round's records pass through LDS and leave as one run; without, each
+// lane stores its own, for patches that leave no LDS for them.
+template <uint32_t T, bool RUN = true>
 __global__ __launch_bounds__(T) void k_arap_rotations(DevMesh m, const uint32_t* __restrict__ vv_base,
                                                       const uint32_t* __restrict__ rbase,
                                                       const uint32_t* __restrict__ nbase,
@@ -434,10 +436,11 @@ __global__ __launch_bounds__(T) void k_arap_rotations(DevMesh m, const uint32_t*
     Bump            b(reinterpret_cast<char*>(smem));
     PlanAR          L = plan_ar(b, d.nv, d.ne, d.nvo, nent, false);
     stage_arap<T, false>(m, d, L, roff + rbase[p], nbr + nbase[p], ent + nbase[p], nent, rest, x, w, nullptr);
-    float* const out = b.alloc<float>(9u * T);  // this round's records, written as one run
+    float* const out = RUN ? b.alloc<float>(9u * T) : nullptr;  // this round's records, written as one run
     __syncthreads();
     for (uint32_t v0 = 0; v0 < d.nvo; v0 += T) {
         const uint32_t v = v0 + threadIdx.x, nr = min(T, d.nvo - v0);
+        float* const   dst = R + 9ull * (d.vp + v0);
         if (v < d.nvo) {
             float       S[3][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
             const float p0 = L.px[v], p1 = L.py[v], p2 = L.pz[v], x0 = L.xx[v], x1 = L.xy[v], x2 = L.xz[v];
@@ -453,15 +456,17 @@ __global__ __launch_bounds__(T) void k_arap_rotations(DevMesh m, const uint32_t*
             }
             float Rv[3][3];
             if (!best_rotation_direct(S, Rv)) best_rotation(S, Rv);
+            float* const rec = RUN ? out + 9u * threadIdx.x : dst + 9u * threadIdx.x;
 #pragma unroll
             for (int r = 0; r < 3; ++r)
 #pragma unroll
-                for (int s = 0; s < 3; ++s) out[9u * threadIdx.x + 3u * r + s] = Rv[r][s];
+                for (int s = 0; s < 3; ++s) rec[3u * r + s] = Rv[r][s];
         }
-        __syncthreads();
-        float* dst = R + 9ull * (d.vp + v0);
-        for (uint32_t i = threadIdx.x; i < 9u * nr; i += T) dst[i] = out[i];
-        __syncthreads();
+        if constexpr (RUN) {
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < 9u * nr; i += T) dst[i] = out[i];
+            __syncthreads();
+        }
     }
 }
 

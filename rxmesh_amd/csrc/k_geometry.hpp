@@ -773,12 +773,15 @@ __global__ __launch_bounds__(T) void k_smoothk(DevMesh m, uint32_t K, const uint
 // nine of its corners and their indexes, and computes nothing: the normals of a
 // torus of 1.3M faces took 20.4 us with the face evaluated anew in each of its
 // three rows, 18.2 so; 10 patches 6.2 -> 4.0, 491 8.3 -> 5.4.
+// LEAN: no face pass; every (vertex, face) pair evaluates the face, for patches
+// whose face terms (24 bytes a face) do not fit LDS. Same results.
 struct PlanVNP
 {
     uint16_t *fvl, *ro, *vf;
     float *   x, *y, *z, *n[3], *cw;
 };
-__host__ __device__ inline PlanVNP plan_vnp(Bump& b, uint32_t nv, uint32_t nvo, uint32_t nf, uint32_t nent)
+__host__ __device__ inline PlanVNP plan_vnp(Bump& b, uint32_t nv, uint32_t nvo, uint32_t nf, uint32_t nent,
+                                            bool lean = false)
 {
     PlanVNP p{};
     p.fvl = b.alloc<uint16_t>((3 * nf + 7u) & ~7u);
@@ -787,8 +790,8 @@ __host__ __device__ inline PlanVNP plan_vnp(Bump& b, uint32_t nv, uint32_t nvo, 
     p.x   = b.alloc<float>(nv);
     p.y   = b.alloc<float>(nv);
     p.z   = b.alloc<float>(nv);
-    for (int c = 0; c < 3; ++c) p.n[c] = b.alloc<float>(nf);
-    p.cw = b.alloc<float>(3 * nf);
+    for (int c = 0; c < 3; ++c) p.n[c] = lean ? nullptr : b.alloc<float>(nf);
+    p.cw = lean ? nullptr : b.alloc<float>(3 * nf);
     return p;
 }
 
@@ -819,7 +822,7 @@ __device__ __forceinline__ void stage_face_plan(const DevMesh& m, const PatchDes
     });
 }
 
-template <uint32_t T>
+template <uint32_t T, bool LEAN = false>
 __global__ __launch_bounds__(T) void k_vertex_normals_plan(DevMesh m, int mode, const uint32_t* __restrict__ fbase,
                                                            const uint32_t* __restrict__ rbase,
                                                            const uint32_t* __restrict__ nbase,
@@ -834,18 +837,18 @@ __global__ __launch_bounds__(T) void k_vertex_normals_plan(DevMesh m, int mode, 
     const PatchDesc d = load_desc(m.patch, p);
     const uint32_t  nb0 = nbase[p], nent = nbase[p + 1] - nb0;
     Bump            b(reinterpret_cast<char*>(smem));
-    const PlanVNP   L = plan_vnp(b, d.nv, d.nvo, d.nf, nent);
+    const PlanVNP   L = plan_vnp(b, d.nv, d.nvo, d.nf, nent, LEAN);
     const uint32_t  N = m.nV;
     stage_face_plan<T>(m, d, fvl + fbase[p], roff + rbase[p], vf + nb0, nent, pos, L);
     __syncthreads();
-    for (uint32_t f = threadIdx.x; f < d.nf; f += T) {
+    auto face = [&](uint32_t f, float (&n)[3], float (&w)[3]) {
         const uint32_t a = L.fvl[3 * f], bb = L.fvl[3 * f + 1], cc = L.fvl[3 * f + 2];
         const float    ux = L.x[bb] - L.x[a], uy = L.y[bb] - L.y[a], uz = L.z[bb] - L.z[a];
         const float    wx = L.x[cc] - L.x[a], wy = L.y[cc] - L.y[a], wz = L.z[cc] - L.z[a];
-        L.n[0][f] = uy * wz - uz * wy;
-        L.n[1][f] = uz * wx - ux * wz;
-        L.n[2][f] = ux * wy - uy * wx;
-        float w[3] = {0.5f, 0.5f, 0.5f};
+        n[0] = uy * wz - uz * wy;
+        n[1] = uz * wx - ux * wz;
+        n[2] = ux * wy - uy * wx;
+        w[0] = w[1] = w[2] = 0.5f;
         if (mode == 0) {
             const float vx = L.x[cc] - L.x[bb], vy = L.y[cc] - L.y[bb], vz = L.z[cc] - L.z[bb];
             const float l0 = ux * ux + uy * uy + uz * uz;  // a-b
@@ -855,18 +858,36 @@ __global__ __launch_bounds__(T) void k_vertex_normals_plan(DevMesh m, int mode, 
             w[1] = __builtin_amdgcn_rcpf(l1 + l0);
             w[2] = __builtin_amdgcn_rcpf(l2 + l1);
         }
+    };
+    if constexpr (!LEAN) {
+        for (uint32_t f = threadIdx.x; f < d.nf; f += T) {
+            float n[3], w[3];
+            face(f, n, w);
 #pragma unroll
-        for (uint32_t j = 0; j < 3; ++j) L.cw[3 * f + j] = w[j];
+            for (uint32_t j = 0; j < 3; ++j) {
+                L.n[j][f]       = n[j];
+                L.cw[3 * f + j] = w[j];
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
     for (uint32_t v = threadIdx.x; v < d.nvo; v += T) {
         float sx = 0.f, sy = 0.f, sz = 0.f;
         for (uint32_t k = L.ro[v]; k < L.ro[v + 1]; ++k) {
             const uint32_t s = L.vf[k], f = s >> 2;
-            const float    w = L.cw[3u * f + (s & 3u)];
-            sx += L.n[0][f] * w;
-            sy += L.n[1][f] * w;
-            sz += L.n[2][f] * w;
+            float          n[3], w;
+            if constexpr (LEAN) {
+                float cw[3];
+                face(f, n, cw);
+                w = (s & 3u) == 0u ? cw[0] : (s & 3u) == 1u ? cw[1] : cw[2];
+            } else {
+                w = L.cw[3u * f + (s & 3u)];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) n[j] = L.n[j][f];
+            }
+            sx += n[0] * w;
+            sy += n[1] * w;
+            sz += n[2] * w;
         }
         const uint32_t g = d.vp + v;
         nrm[g]           = sx;

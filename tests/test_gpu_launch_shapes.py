@@ -390,3 +390,43 @@ def test_normals_and_edge_weights_of_few_and_many_patches(level, patch_size):
     w = m.arap_weights(x).cpu().numpy()
     ref = np.array([cot[(a, b)] for a, b in ev.tolist()])
     assert np.abs(w - np.maximum(0.0, 0.5 * ref)).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("name,a,b", [("normals", 40, 64), ("rotations", 28, 85), ("smooth", 50, 100), ("weights", 40, 80),
+                                      ("step", 43, 60)])
+def test_patches_near_the_lds_limit(name, a, b):
+    """One patch that holds a whole torus of 2 a b faces and takes the form
+    that needs least LDS, against patches of 512 faces. The row orders differ:
+    twice the 1e-5 (rotations 1e-4) of each against FP64."""
+    import torch
+    V, F = mg.permute_mesh(*mg.torus(a, b), seed=9)
+    out = []
+    for patch_size in (16384, 512):
+        m, x = _mesh(V, F, patch_size)
+        assert (m.P == 1) == (patch_size == 16384)
+        pose = (x + 0.3 * torch.sin(2.0 * x.flip(0))).contiguous()
+        ids = m.array("v_l2g")
+        if name == "normals":
+            y = m.vertex_normals(x).T
+        elif name == "smooth":
+            y = m.smooth(x, 0.5, 3).T
+        elif name == "weights":
+            y, ids = m.arap_weights(x)[:, None], m.array("e_l2g")
+        elif name == "step":
+            y = m.symdir3_grad_step(m.symdir_rest(x), pose, 1e-3).T
+        else:
+            y = m.arap_rotations(x, pose, m.arap_weights(x))
+        r = np.empty(y.shape)
+        r[ids] = y.cpu().numpy()
+        out.append(r)
+    assert np.abs(out[0] - out[1]).max() <= (2e-4 if name == "rotations" else 2e-5) * np.abs(out[1]).max()
+
+
+def test_matrix_free_solve_refuses_open_meshes_of_any_patch_size():
+    import rxmesh_amd as rx
+    V, F = mg.grid(80)
+    for patch_size in (512, 32768):
+        m, x = _mesh(V, F, patch_size)
+        with pytest.raises(rx.RXMError) as e:
+            m.mcf_matfree_cg(x, x, 1e-3, max_iter=3)
+        assert e.value.code == 6
