@@ -267,9 +267,11 @@ rxm_status rxm_vv_plan_build(rxm_mesh* mesh, void* stream);
  *             counting sort (wave ballots + mbcnt ranks + one block scan;
  *             rows come out in order, no row sort); 2 (default) = one pass
  *             per launch for VV / VE / VF / EF / FF and for rxm_query_vv_vf
- *             (both relations in one counting sort): keys per edge or per
- *             face held in registers, rows sorted in registers, one
- *             coalesced write.
+ *             (both relations together): keys per edge or per face held in
+ *             registers, rows of at most 8 entries in fixed-width LDS slots
+ *             (EF / FF of an oriented manifold: one plain store per
+ *             half-edge), else one counting sort; rows sorted in registers,
+ *             one coalesced write.
  * Settings of kernels 0-4 and 6-10 give bit-identical results; kernel 5 changes
  * the summation order of a row (fp32 results within rounding). */
 rxm_status rxm_set_launch_threads(rxm_mesh* mesh, int kernel, int threads);

@@ -96,7 +96,7 @@ struct rxm_mesh
     uint32_t        grad_queue     = 0;        // 1: persistent work-queue launch
     uint32_t*       d_queue        = nullptr;  // work-queue ticket counter
     bool            system_runs_ok = false;    // check_system_runs passed
-    uint32_t        query_stable   = 2;        // transposes: 0 LDS atomics + row sort, 1 atomic-free stable sort, 2 as 0 with the fused VV + VF launch in one pass
+    uint32_t        query_stable   = 2;        // transposes: 0 LDS atomics + row sort, 1 atomic-free stable sort, 2 one pass (slots, else one counting sort)
     uint32_t        vvf_nslots     = 0;        // largest VV + VF entry count of a patch (0: not computed yet)
     uint32_t        max_row        = 0;        // largest VV or VF row of a vertex
     uint32_t        max_nrv = 0, max_nre = 0, max_nrf = 0;  // largest ribbon vertex / edge / face count of a patch
@@ -361,7 +361,7 @@ bool launch_rows(rxm_mesh* m, const uint32_t* v_base, const uint32_t* f_base, in
     // 8.9, 2687 29.7 / 22.2 / 21.8, 10677 97.7 / 70.0 / 58.8 (k_query2_vv_vf1,
     // 256 threads: 8.4, 8.6, 9.4, 25.3, 67.6).
     if (h.P <= 256u && fits(1024, 1, 1, 1)) return go(k_query_rows<1024, 1, 1, 1, REL>, 1024);
-    if (h.P > 1500u && fits(256, 3, 2, 2)) return go(k_query_rows<256, 3, 2, 2, REL>, 256);
+    if (h.P > 1500u && fits(256, 4, 2, 2)) return go(k_query_rows<256, 4, 2, 2, REL>, 256);
     if (fits(512, 3, 2, 2)) return go(k_query_rows<512, 3, 2, 2, REL>, 512);
     return false;
 }
@@ -386,7 +386,7 @@ bool launch_dir(rxm_mesh* m, const uint32_t* base, int32_t* row_ptr, int32_t* co
     // workgroup sizes as launch_rows chooses them
     constexpr uint32_t RS = FF ? 3 : 4;
     if (h.P <= 256u && fits(1024, 1, 1)) return go(k_query_dir<1024, 1, 1, FF>, 1024);
-    if (h.P > 1500u && fits(256, 3, RS)) return go(k_query_dir<256, 3, RS, FF>, 256);
+    if (h.P > 1500u && fits(256, 4, RS)) return go(k_query_dir<256, 4, RS, FF>, 256);
     if (fits(512, 3, RS)) return go(k_query_dir<512, 3, RS, FF>, 512);
     return false;
 }
@@ -429,6 +429,10 @@ int ensure_vv_plan(rxm_mesh* m, void* stream)
         m->d_vv_nbr = nullptr;  // freed with the mesh; rebuild on the next call
         return rc;
     }
+    // complete before a call on another stream can read it
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    RXM_HIP(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap));
+    if (cap == hipStreamCaptureStatusNone) RXM_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
     return RXM_OK;
 }
 

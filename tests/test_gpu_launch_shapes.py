@@ -342,7 +342,7 @@ def test_query_kernels_over_forms(name, patch_size):
             assert np.array_equal(rp.cpu().numpy(), orp) and np.array_equal(col.cpu().numpy()[:len(ocol)], ocol), op
 
 
-@pytest.mark.parametrize("level,patch_size", [(7, 512), (7, 1024), (7, 128), (6, 256)])
+@pytest.mark.parametrize("level,patch_size", [(7, 512), (7, 1024), (7, 128), (6, 256), (8, 700)])
 def test_query_kernels_of_many_patches(level, patch_size):
     """The workgroup sizes chosen for hundreds and thousands of patches: the
     rows of the general kernels, bit for bit."""
