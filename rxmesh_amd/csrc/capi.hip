@@ -391,6 +391,18 @@ bool launch_dir(rxm_mesh* m, const uint32_t* base, int32_t* row_ptr, int32_t* co
     return false;
 }
 
+// Waits for a plan's build, before the plan is published: calls on other streams
+// read it from then on. Not while the stream is capturing, where the build is a
+// node of the graph.
+int plan_complete(void* stream)
+{
+    hipStream_t            hs  = static_cast<hipStream_t>(stream);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    RXM_HIP(hipStreamIsCapturing(hs, &cap));
+    if (cap == hipStreamCaptureStatusNone) RXM_HIP(hipStreamSynchronize(hs));
+    return RXM_OK;
+}
+
 int ensure_vv_plan(rxm_mesh* m, void* stream)
 {
     if (m->d_vv_nbr) return RXM_OK;
@@ -429,11 +441,7 @@ int ensure_vv_plan(rxm_mesh* m, void* stream)
         m->d_vv_nbr = nullptr;  // freed with the mesh; rebuild on the next call
         return rc;
     }
-    // complete before a call on another stream can read it
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    RXM_HIP(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap));
-    if (cap == hipStreamCaptureStatusNone) RXM_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
-    return RXM_OK;
+    return plan_complete(stream);
 }
 
 int ensure_face_plan(rxm_mesh* m, void* stream)
@@ -635,7 +643,7 @@ int build_ring_plan(rxm_mesh* m, uint32_t K, void* stream)
         (rc = device_array(m, xb[P], &xl)))
         return rc;
     const uint32_t *drb = d_base, *dnb = d_base + P + 1, *dxb = d_base + 2 * (P + 1);
-    if ((rc = go(drb, dnb, dxb, ro, nr, xl))) return rc;
+    if ((rc = go(drb, dnb, dxb, ro, nr, xl)) || (rc = plan_complete(stream))) return rc;
     v.lvl.clear();
     m->vvk         = std::move(v);
     m->d_vvk_lvl   = lvl;

@@ -430,3 +430,34 @@ def test_matrix_free_solve_refuses_open_meshes_of_any_patch_size():
         with pytest.raises(rx.RXMError) as e:
             m.mcf_matfree_cg(x, x, 1e-3, max_iter=3)
         assert e.value.code == 6
+
+
+def _two_streams(V, F):
+    """A mesh, its positions and two streams that wait for neither the default stream nor each other."""
+    import torch
+    m, x = _mesh(V, F, 512)
+    torch.cuda.synchronize()
+    return m, x, torch.cuda.Stream(), torch.cuda.Stream()
+
+
+@pytest.mark.parametrize("steps", [0, 4])
+def test_ring_plan_built_on_another_stream(steps):
+    """A call on one stream builds the multi-step plan (build_vv_plan, or a
+    smoothing with `steps` per launch), the next on another smooths over it:
+    the bits of single steps."""
+    import torch
+    V, F = mg.icosphere(7, seed=11, sigma=0.01)
+    m, x, a, b = _two_streams(V, F)
+    m.set_launch_threads(8, 0)
+    ref = m.smooth(x, 0.5, 7)
+    n, _, _, _ = _two_streams(V, F)
+    out, tmp, out_a, tmp_a = (torch.empty_like(x) for _ in range(4))
+    torch.cuda.synchronize()
+    if steps:
+        n.set_launch_threads(8, steps)
+        n.smooth(x, 0.5, 4, out=out_a, tmp=tmp_a, stream=a)
+    else:
+        n.build_vv_plan(stream=a)
+    n.smooth(x, 0.5, 7, out=out, tmp=tmp, stream=b)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)

@@ -1,0 +1,107 @@
+"""What the C-ABI asks of the HIP runtime, and in which order, without a GPU:
+plans that calls on any stream read are complete before they are used or the
+call that builds them returns, nothing that a capturing stream forbids is
+asked of one, and a failed allocation leaves nothing behind. Each case runs in
+a process of its own with tests/cpp/hip_recorder.cpp in front of the runtime:
+kernels are recorded, not run."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+SRC = os.path.join(HERE, "cpp", "hip_recorder.cpp")
+LIB = os.path.join(HERE, "cpp", "_build", "libhip_recorder.so")
+A, B = 0x10, 0x20  # stream handles: the recorder only tells them apart
+PTR = 0x1000       # stands for a caller's device array; no kernel runs
+PLANS = ("k_query2_vv_local", "k_query2_vf_local", "k_ring_plan", "k_closed_fans")  # kernels that write plans
+
+
+class Recorder:
+    """A mesh on the recorder's device and its log."""
+
+    def __init__(self, fv, patch_size=64):
+        sys.path.insert(0, ROOT)
+        sys.modules["torch"] = None  # the wrapper starts torch's own HIP runtime where it finds torch
+        import rxmesh_amd as rx
+        self.rec = ctypes.CDLL(LIB)
+        self.rec.rec_log.restype = ctypes.c_char_p
+        self.rec.rec_live_bytes.restype = self.rec.rec_live_count.restype = ctypes.c_size_t
+        self.host = rx.Mesh(fv, patch_size=patch_size, host_only=True)  # the build itself runs on the host
+        self.mesh = rx.Mesh(None, parts=[self.host])
+        self.h, self.lib, self.log = self.mesh._h, rx.lib(), []
+        self.events()
+
+    def events(self):
+        """(what, kernel or "", stream) since the last call."""
+        out = []
+        for line in self.rec.rec_log().decode().splitlines():
+            what, _, rest = line.partition(" ")
+            name, _, stream = rest.rpartition("@")
+            out.append((what, name.strip(), int(stream) if stream.isdigit() else rest))
+        return out
+
+    def __call__(self, name, *args):
+        return getattr(self.lib, name)(self.h, *args)
+
+    def smooth(self, iters, stream):
+        return self("rxm_laplacian_smooth", PTR, 2 * PTR, 3 * PTR, 0.5, iters, stream)
+
+
+def check_plans_waited_for(events):
+    """Every plan kernel is followed by a wait for its stream before any kernel
+    that does not build plans, and before the end."""
+    pending = {}
+    for what, name, stream in events:
+        if what == "launch" and any(p in name for p in PLANS):
+            pending[stream] = name
+        elif what == "wait":
+            pending.pop(stream, None)
+        elif what == "launch" and "k_fill" not in name and "k_reset" not in name:
+            assert not pending, "%s launched while %s may still run" % (name, pending)
+    assert not pending, "returned while %s may still run" % pending
+
+
+def sphere():
+    sys.path.insert(0, ROOT)
+    from rxmesh_amd import meshgen as mg
+    return mg.icosphere(3, seed=0)[1]
+
+
+def case_ring_plan():
+    """rxm_vv_plan_build, and the smoothing that builds its own ring plan."""
+    r = Recorder(sphere())
+    assert r("rxm_vv_plan_build", A) == 0
+    e = r.events()
+    assert any("k_ring_plan" in n for _, n, _ in e)
+    check_plans_waited_for(e)
+    assert r.smooth(4, B) == 0
+    assert [n for w, n, _ in r.events() if w == "launch" and "k_smoothk" not in n] == []
+    r = Recorder(sphere())
+    assert r("rxm_set_launch_threads", 8, 4) == 0
+    assert r.smooth(4, A) == 0
+    e = r.events()
+    assert any("k_ring_plan" in n for _, n, _ in e) and any("k_smoothk" in n for _, n, _ in e)
+    check_plans_waited_for(e)
+
+
+def case_names():
+    return [n[5:] for n in globals() if n.startswith("case_") and n != "case_names"]
+
+
+@pytest.mark.parametrize("case", case_names())
+def test_host_calls(case):
+    if not os.path.exists(LIB) or os.path.getmtime(LIB) < os.path.getmtime(SRC):
+        os.makedirs(os.path.dirname(LIB), exist_ok=True)
+        subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", SRC, "-o", LIB + ".tmp"])
+        os.replace(LIB + ".tmp", LIB)
+    q = subprocess.run([sys.executable, os.path.abspath(__file__), case], env=dict(os.environ, LD_PRELOAD=LIB),
+                       capture_output=True, text=True, timeout=120)
+    assert q.returncode == 0, q.stdout + q.stderr
+
+
+if __name__ == "__main__":
+    globals()["case_" + sys.argv[1]]()
