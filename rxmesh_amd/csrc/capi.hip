@@ -475,7 +475,7 @@ int ensure_face_plan(rxm_mesh* m, void* stream)
     plan_q2(b, 1, h.max_nv, h.max_ne, h.max_nf);
     rc = launch_patches(k_query2_vf_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm, m->d_fp_fbase,
                         m->d_fp_rbase, m->d_fp_nbase, bufs[0], bufs[1], bufs[2]);
-    if (rc) return rc;
+    if (rc || (rc = plan_complete(stream))) return rc;
     m->d_fp_fvl = bufs[0];
     m->d_fp_roff = bufs[1];
     m->d_fp_vf = bufs[2];

@@ -461,3 +461,27 @@ def test_ring_plan_built_on_another_stream(steps):
     n.smooth(x, 0.5, 7, out=out, tmp=tmp, stream=b)
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
+
+
+def test_face_plan_built_on_another_stream():
+    """Normals on one stream build the face plan, curvature, gradient and step
+    on another use it: the bits of the same calls in order."""
+    import torch
+    V, F = mg.icosphere(7, seed=12, sigma=0.01)
+    m, x, a, b = _two_streams(V, F)
+    Mr = m.symdir_rest(x)
+    y = (x * 1.1).contiguous()
+    torch.cuda.synchronize()
+    calls = (lambda q, s: q.gaussian_curvature(y, stream=s), lambda q, s: q.symdir3_grad(Mr, y, stream=s),
+             lambda q, s: q.symdir3_grad_step(Mr, y, 1e-3, stream=s))
+    for call in calls:
+        n, _, _, _ = _two_streams(V, F)
+        with torch.cuda.stream(a):
+            n.vertex_normals(y, "max")
+        with torch.cuda.stream(b):
+            got = call(n, None)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(b):
+            want = call(n, None)
+        torch.cuda.synchronize()
+        assert torch.equal(got[0] if isinstance(got, tuple) else got, want[0] if isinstance(want, tuple) else want)

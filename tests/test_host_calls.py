@@ -88,6 +88,21 @@ def case_ring_plan():
     check_plans_waited_for(e)
 
 
+def case_face_plan():
+    """Each entry point that builds the face plan on its first call."""
+    for name, args in (("rxm_vertex_normals", (0, PTR, 2 * PTR)), ("rxm_gaussian_curvature", (PTR, 2 * PTR, 3 * PTR)),
+                       ("rxm_symdir3_grad", (PTR, 2 * PTR, 3 * PTR)),
+                       ("rxm_symdir3_grad_step", (PTR, 2 * PTR, 0.1, 3 * PTR)),
+                       ("rxm_smooth_symdir_steps", (PTR, 2 * PTR, 3 * PTR, 0.5, 0.1, 1))):
+        r = Recorder(sphere())
+        assert r(name, *args, A) == 0
+        e = r.events()
+        assert any("k_query2_vf_local" in n for _, n, _ in e)
+        check_plans_waited_for(e)
+        assert r(name, *args, B) == 0
+        assert not any(p in n for _, n, _ in r.events() for p in PLANS)
+
+
 def case_names():
     return [n[5:] for n in globals() if n.startswith("case_") and n != "case_names"]
 
