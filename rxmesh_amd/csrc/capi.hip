@@ -121,19 +121,57 @@ constexpr int kOpCot = 100;  // rows of the cotangent system: VV + diagonal
         if (e_ != hipSuccess) return RXM_ERR_DEVICE;  \
     } while (0)
 
+// Uninitialised device array owned by the mesh. A refused allocation is reported
+// here, not again by the error check of the next launch.
+template <typename T>
+int device_array(rxm_mesh* m, size_t n, T** out)
+{
+    const size_t bytes = std::max<size_t>(n * sizeof(T), 16);
+    T*           p     = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return RXM_ERR_OUT_OF_MEMORY;
+    }
+    m->allocs.push_back(p);
+    m->device_bytes += bytes;
+    *out = p;
+    return RXM_OK;
+}
+
 template <typename T>
 int upload(rxm_mesh* m, const std::vector<T>& v, const T*& dst)
 {
-    T*     p     = nullptr;
-    size_t bytes = std::max<size_t>(v.size() * sizeof(T), 16);
-    if (hipMalloc(&p, bytes) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-    m->allocs.push_back(p);
-    m->device_bytes += bytes;
+    T*  p  = nullptr;
+    int rc = device_array(m, v.size(), &p);
+    if (rc) return rc;
     if (!v.empty() && hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess)
         return RXM_ERR_DEVICE;
     dst = p;
     return RXM_OK;
 }
+
+// The mesh's arrays made since, until keep(): a plan that is not finished frees
+// what it had (hipFree waits for kernels that write it).
+class Unfinished
+{
+    rxm_mesh* m;
+    size_t    n;
+    uint64_t  bytes;
+
+   public:
+    explicit Unfinished(rxm_mesh* mesh) : m(mesh), n(mesh->allocs.size()), bytes(mesh->device_bytes) {}
+    Unfinished(const Unfinished&) = delete;
+    void keep() { m = nullptr; }
+    ~Unfinished()
+    {
+        if (!m) return;
+        while (m->allocs.size() > n) {
+            if (hipFree(m->allocs.back()) != hipSuccess) (void)hipGetLastError();
+            m->allocs.pop_back();
+        }
+        m->device_bytes = bytes;
+    }
+};
 
 int upload_mesh(rxm_mesh* m)
 {
@@ -417,31 +455,29 @@ int ensure_vv_plan(rxm_mesh* m, void* stream)
         rb[p + 1] = rb[p] + ((h.nvo[p] + 1u + 7u) & ~7u);
         nb[p + 1] = nb[p] + ((nent + 7u) & ~7u);
     }
-    m->vv_max_nent = maxn;
-    int rc = upload(m, rb, m->d_vv_rbase);
-    if (!rc) rc = upload(m, nb, m->d_vv_nbase);
-    if (rc) return rc;
-    if (hipMalloc(&m->d_vv_roff, sizeof(uint16_t) * std::max<uint32_t>(rb[h.P], 8)) != hipSuccess)
-        return RXM_ERR_OUT_OF_MEMORY;
-    m->allocs.push_back(m->d_vv_roff);
-    if (hipMalloc(&m->d_vv_nbr, sizeof(uint16_t) * std::max<uint32_t>(nb[h.P], 8)) != hipSuccess)
-        return RXM_ERR_OUT_OF_MEMORY;
-    m->allocs.push_back(m->d_vv_nbr);
-    if (hipMalloc(&m->d_vv_ent, sizeof(uint16_t) * std::max<uint32_t>(nb[h.P], 8)) != hipSuccess) {
-        m->d_vv_nbr = nullptr;
-        return RXM_ERR_OUT_OF_MEMORY;
-    }
-    m->allocs.push_back(m->d_vv_ent);
-    m->device_bytes += 2ull * (rb[h.P] + 2ull * nb[h.P]);
+    Unfinished      arrays(m);
+    const uint32_t *rbase = nullptr, *nbase = nullptr;
+    uint16_t *      roff = nullptr, *nbr = nullptr, *ent = nullptr;
+    int             rc = upload(m, rb, rbase);
+    if (!rc) rc = upload(m, nb, nbase);
+    if (!rc) rc = device_array(m, rb[h.P], &roff);
+    if (!rc) rc = device_array(m, nb[h.P], &nbr);
+    if (!rc) rc = device_array(m, nb[h.P], &ent);
     Bump b(nullptr);
     plan_vvl(b, h.max_ne, h.max_nvo);
-    rc = launch_patches(k_query2_vv_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm,
-                        m->d_vv_rbase, m->d_vv_nbase, m->d_vv_roff, m->d_vv_nbr, m->d_vv_ent);
-    if (rc) {
-        m->d_vv_nbr = nullptr;  // freed with the mesh; rebuild on the next call
-        return rc;
-    }
-    return plan_complete(stream);
+    if (!rc)
+        rc = launch_patches(k_query2_vv_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm, rbase, nbase,
+                            roff, nbr, ent);
+    if (!rc) rc = plan_complete(stream);
+    if (rc) return rc;
+    arrays.keep();
+    m->vv_max_nent = maxn;
+    m->d_vv_rbase  = rbase;
+    m->d_vv_nbase  = nbase;
+    m->d_vv_roff   = roff;
+    m->d_vv_ent    = ent;
+    m->d_vv_nbr    = nbr;  // last: marks the plan complete
+    return RXM_OK;
 }
 
 int ensure_face_plan(rxm_mesh* m, void* stream)
@@ -459,27 +495,30 @@ int ensure_face_plan(rxm_mesh* m, void* stream)
         rb[p + 1] = rb[p] + ((h.nvo[p] + 1u + 7u) & ~7u);
         nb[p + 1] = nb[p] + ((nent + 7u) & ~7u);
     }
-    int rc = upload(m, fb, m->d_fp_fbase);
-    if (!rc) rc = upload(m, rb, m->d_fp_rbase);
-    if (!rc) rc = upload(m, nb, m->d_fp_nbase);
-    if (rc) return rc;
-    uint16_t* bufs[3] = {nullptr, nullptr, nullptr};
-    const uint32_t sizes[3] = {fb[h.P], rb[h.P], nb[h.P]};
-    for (int i = 0; i < 3; ++i) {
-        if (hipMalloc(&bufs[i], sizeof(uint16_t) * std::max<uint32_t>(sizes[i], 8)) != hipSuccess)
-            return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(bufs[i]);
-        m->device_bytes += 2ull * sizes[i];
-    }
+    Unfinished      arrays(m);
+    const uint32_t *fbase = nullptr, *rbase = nullptr, *nbase = nullptr;
+    uint16_t *      fvl = nullptr, *roff = nullptr, *vf = nullptr;
+    int             rc = upload(m, fb, fbase);
+    if (!rc) rc = upload(m, rb, rbase);
+    if (!rc) rc = upload(m, nb, nbase);
+    if (!rc) rc = device_array(m, fb[h.P], &fvl);
+    if (!rc) rc = device_array(m, rb[h.P], &roff);
+    if (!rc) rc = device_array(m, nb[h.P], &vf);
     Bump b(nullptr);
     plan_q2(b, 1, h.max_nv, h.max_ne, h.max_nf);
-    rc = launch_patches(k_query2_vf_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm, m->d_fp_fbase,
-                        m->d_fp_rbase, m->d_fp_nbase, bufs[0], bufs[1], bufs[2]);
-    if (rc || (rc = plan_complete(stream))) return rc;
-    m->d_fp_fvl = bufs[0];
-    m->d_fp_roff = bufs[1];
-    m->d_fp_vf = bufs[2];
+    if (!rc)
+        rc = launch_patches(k_query2_vf_local<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm, fbase, rbase,
+                            nbase, fvl, roff, vf);
+    if (!rc) rc = plan_complete(stream);
+    if (rc) return rc;
+    arrays.keep();
     m->fp_max_nent = maxn;
+    m->d_fp_fbase  = fbase;
+    m->d_fp_rbase  = rbase;
+    m->d_fp_nbase  = nbase;
+    m->d_fp_fvl    = fvl;
+    m->d_fp_roff   = roff;
+    m->d_fp_vf     = vf;  // last: marks the plan complete
     return RXM_OK;
 }
 
@@ -536,6 +575,7 @@ int ensure_vv2_plan(rxm_mesh* m)
     if (m->d_vv2_nbr) return RXM_OK;
     int rc = host_vv2_plan(m);
     const Vv2Plan& v = m->vv2;
+    Unfinished     arrays(m);
     if (!rc) rc = upload(m, v.rbase, m->d_vv2_rbase);
     if (!rc) rc = upload(m, v.nbase, m->d_vv2_nbase);
     if (!rc) rc = upload(m, v.xbase, m->d_vv2_xbase);
@@ -544,20 +584,8 @@ int ensure_vv2_plan(rxm_mesh* m)
     if (!rc) rc = upload(m, v.xlin, m->d_vv2_xlin);
     if (!rc) rc = upload(m, v.nbr, m->d_vv2_nbr);  // last: marks the plan complete
     if (rc) m->d_vv2_nbr = nullptr;
+    else arrays.keep();
     return rc;
-}
-
-// Uninitialised device array owned by the mesh.
-template <typename T>
-int device_array(rxm_mesh* m, size_t n, T** out)
-{
-    const size_t bytes = std::max<size_t>(n * sizeof(T), 16);
-    T*           p     = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-    m->allocs.push_back(p);
-    m->device_bytes += bytes;
-    *out = p;
-    return RXM_OK;
 }
 
 // Static part of the cotangent system, built once per mesh (the role of the
@@ -572,6 +600,7 @@ int ensure_cot_plan(rxm_mesh* m, void* stream)
     const HostMesh& h  = m->h;
     const size_t    nw = (h.nV + 31u) / 32u;
     hipStream_t     hs = static_cast<hipStream_t>(stream);
+    Unfinished      arrays(m);
     uint32_t*       bits = nullptr;  // bitmask, then a flag per patch
     if ((rc = device_array(m, nw + h.P, &bits))) return rc;
     hipLaunchKernelGGL(k_fill_u32, dim3(static_cast<uint32_t>((nw + h.P + 255) / 256)), dim3(256), 0, hs,
@@ -591,6 +620,7 @@ int ensure_cot_plan(rxm_mesh* m, void* stream)
     for (uint32_t p = 0; p < h.P; ++p)
         if (ring[p]) plist.push_back(p);
     if ((rc = upload(m, plist, m->d_cot_plist))) return rc;
+    arrays.keep();
     m->cot_nplist   = static_cast<uint32_t>(plist.size());
     m->d_cot_closed = bits;  // last: marks the plan complete
     return RXM_OK;
@@ -607,8 +637,9 @@ int build_ring_plan(rxm_mesh* m, uint32_t K, void* stream)
     hipStream_t    hs = static_cast<hipStream_t>(stream);
     Bump           b(nullptr);
     plan_rb(b);
-    uint32_t* lvl  = nullptr;  // counts, then the overflow flag
-    int       rc = device_array(m, size_t(P) * W + 1, &lvl);
+    Unfinished arrays(m);
+    uint32_t*  lvl = nullptr;  // counts, then the overflow flag
+    int        rc  = device_array(m, size_t(P) * W + 1, &lvl);
     if (rc) return rc;
     uint32_t* flag = lvl + size_t(P) * W;
     hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, hs, flag);
@@ -644,6 +675,7 @@ int build_ring_plan(rxm_mesh* m, uint32_t K, void* stream)
         return rc;
     const uint32_t *drb = d_base, *dnb = d_base + P + 1, *dxb = d_base + 2 * (P + 1);
     if ((rc = go(drb, dnb, dxb, ro, nr, xl)) || (rc = plan_complete(stream))) return rc;
+    arrays.keep();
     v.lvl.clear();
     m->vvk         = std::move(v);
     m->d_vvk_lvl   = lvl;
@@ -664,7 +696,8 @@ int ensure_vvk_plan(rxm_mesh* m, uint32_t K, void* stream)
     int rc = ensure_vv_plan(m, stream);
     if (!rc) rc = build_ring_plan(m, K, stream);
     if (rc != RXM_ERR_PATCH_TOO_BIG) return rc;
-    VvkPlan v;
+    VvkPlan    v;
+    Unfinished arrays(m);
     rc = build_vvk_plan(m->h, K, v);
     const uint32_t *lvl = nullptr, *rb = nullptr, *nb = nullptr, *xb = nullptr, *xl = nullptr;
     const uint16_t *ro = nullptr, *nr = nullptr;
@@ -676,6 +709,7 @@ int ensure_vvk_plan(rxm_mesh* m, uint32_t K, void* stream)
     if (!rc) rc = upload(m, v.xlin, xl);
     if (!rc) rc = upload(m, v.nbr, nr);
     if (rc) return rc;
+    arrays.keep();
     m->vvk         = std::move(v);
     m->d_vvk_lvl   = lvl;
     m->d_vvk_rbase = rb;
@@ -1359,11 +1393,7 @@ rxm_status rxm_arap_energy_grad(rxm_mesh* m, const float* rest, const float* x, 
     uint32_t        lds     = 0;
     int             rc      = arap_rows(m, &vv_base, &lds, true, stream);
     if (rc) return rc;
-    if (!m->d_partial) {
-        if (hipMalloc(&m->d_partial, sizeof(float) * m->h.P) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(m->d_partial);
-        m->device_bytes += sizeof(float) * m->h.P;
-    }
+    if (!m->d_partial && (rc = device_array(m, m->h.P, &m->d_partial))) return rc;
     auto go = [&](auto kernel, uint32_t T) {
         return launch_patches_xcd(kernel, T, lds, stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
                                   static_cast<const uint16_t*>(m->d_vv_roff), static_cast<const uint16_t*>(m->d_vv_ent),
@@ -1424,13 +1454,7 @@ rxm_status rxm_laplacian_smooth(rxm_mesh* m, const float* pos, float* out, float
         // an odd step first (SoA -> SoA), then pairs whose iterates between
         // launches are float4 rows in two mesh-owned buffers
         const size_t n = m->h.nV;
-        if (!m->d_iter4) {
-            float* p = nullptr;
-            if (hipMalloc(&p, 8 * n * sizeof(float)) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-            m->allocs.push_back(p);
-            m->device_bytes += 8 * n * sizeof(float);
-            m->d_iter4 = p;
-        }
+        if (!m->d_iter4 && (rc = device_array(m, 8 * n, &m->d_iter4))) return rc;
         const float* src = pos;
         if (iters % 2) {
             if ((rc = smooth_once(m, lambda, pos, tmp, stream))) return rc;
@@ -1689,13 +1713,9 @@ int cg_work(rxm_mesh* m, CgWork& w)
 {
     const size_t   v3 = 3 * cg_stride(m->h.nV), np = (size_t(m->h.P) + 63u) & ~size_t(63);
     const size_t   nd = kCgUpdateGroups * sizeof(double) + 2 * sizeof(CgState), bytes = (4 * v3 + np) * sizeof(float) + nd;
-    if (!m->d_cg) {
-        float* p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(p);
-        m->device_bytes += bytes;
-        m->d_cg = p;
-    }
+    static_assert(sizeof(CgState) % sizeof(float) == 0, "counted in floats");
+    int rc = RXM_OK;
+    if (!m->d_cg && (rc = device_array(m, bytes / sizeof(float), &m->d_cg))) return rc;
     w.r    = m->d_cg;
     w.p[0] = w.r + v3;
     w.p[1] = w.p[0] + v3;
@@ -1807,11 +1827,7 @@ rxm_status rxm_mcf_matfree_cg(rxm_mesh* m, const float* coords, const float* x, 
     // mass and diagonal per vertex; the weights, one float per row entry
     const size_t n = cg_stride(m->h.nV), cnt = 2 * n + (uni ? 0 : size_t(op_base(m, kOpCot).back()));
     if (cnt > m->mf_floats) {
-        float* p = nullptr;
-        if (hipMalloc(&p, cnt * sizeof(float)) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(p);
-        m->device_bytes += cnt * sizeof(float);
-        m->d_mf      = p;
+        if ((rc = device_array(m, cnt, &m->d_mf))) return rc;
         m->mf_floats = cnt;
     }
     float *mass = m->d_mf, *diag = mass + n, *val = diag + n;
@@ -1868,11 +1884,8 @@ rxm_status rxm_symdir_energy(rxm_mesh* m, const float* Mr, const float* uv, floa
 {
     if (!m || !Mr || !uv || !energy || !total) return RXM_ERR_INVALID_ARG;
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
-    if (!m->d_partial) {
-        if (hipMalloc(&m->d_partial, sizeof(float) * m->h.P) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(m->d_partial);
-        m->device_bytes += sizeof(float) * m->h.P;
-    }
+    int rc = RXM_OK;
+    if (!m->d_partial && (rc = device_array(m, m->h.P, &m->d_partial))) return rc;
     return symdir_energy_launch(m, Mr, uv, energy, total, m->d_partial, stream);
 }
 
@@ -1997,10 +2010,7 @@ static int prepare_steps(rxm_mesh* m, void* stream)
 {
     int rc = ensure_vv_plan(m, stream);
     if (!rc) rc = ensure_face_plan(m, stream);
-    if (!rc && !m->d_queue) {
-        if (hipMalloc(&m->d_queue, 256) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
-        m->allocs.push_back(m->d_queue);
-    }
+    if (!rc && !m->d_queue) rc = device_array(m, 64, &m->d_queue);
     if (!rc && m->num_cus == 0)
         RXM_HIP(hipDeviceGetAttribute(&m->num_cus, hipDeviceAttributeMultiprocessorCount, m->device));
     return rc;

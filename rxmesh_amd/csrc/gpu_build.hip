@@ -143,6 +143,7 @@ int build_supporting_device(const uint32_t* fv, uint32_t nF, uint32_t nV, std::v
     const size_t o_tmp = o_off + up(4 * (size_t(std::max(nV, nH)) + 1)), total = o_tmp + up(sort_bytes);
     char*        base = nullptr;
     if (hipMalloc(&base, total) != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch's check
         (void)hipStreamDestroy(s);
         return RXM_ERR_OUT_OF_MEMORY;
     }
@@ -228,7 +229,10 @@ extern "C" rxm_status rxm_build_edges_device(const uint32_t* fv, uint32_t num_fa
     const size_t o_rank = o_flag + up(4 * n), o_hpos = o_rank + up(4 * n), o_head = o_hpos + up(4 * n);
     const size_t o_bad = o_head + up(4 * n), o_tmp = o_bad + 256, total = o_tmp + up(tmp_bytes);
     char*        base      = nullptr;
-    if (hipMalloc(&base, total) != hipSuccess) return RXM_ERR_OUT_OF_MEMORY;
+    if (hipMalloc(&base, total) != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch's check
+        return RXM_ERR_OUT_OF_MEMORY;
+    }
     uint64_t* k0   = reinterpret_cast<uint64_t*>(base);
     uint64_t* k1   = reinterpret_cast<uint64_t*>(base + o_k1);
     uint32_t* v0   = reinterpret_cast<uint32_t*>(base + o_v0);

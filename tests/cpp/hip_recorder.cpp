@@ -16,13 +16,13 @@ struct dim3
 {
     uint32_t x, y, z;
 };
-enum { kOk = 0, kInvalid = 1, kNoMemory = 2, kCaptureUnsupported = 900 };
+enum { kOk = 0, kInvalid = 1, kNoMemory = 2, kCaptureUnsupported = 900, kUnknown = 999 };
 struct Rec
 {
     std::map<const void*, std::string> names;  // host handle -> kernel
     std::map<void*, size_t>            live;
     std::vector<std::string>           log;
-    int  fail_in = 0;  // > 0: that allocation from now fails
+    int  fail_in = 0, wait_fail_in = 0;  // > 0: that allocation / wait from now fails
     bool capturing = false;
     int  last_error = kOk;  // sticky until hipGetLastError reads it
     dim3 grid{}, block{};
@@ -39,6 +39,7 @@ int fail(int e)
 
 extern "C" {
 void   rec_fail_malloc(int n) { r.fail_in = n; }
+void   rec_fail_wait(int n) { r.wait_fail_in = n; }
 void   rec_capturing(int on) { r.capturing = on != 0; }
 size_t rec_live_count() { return r.live.size(); }
 size_t rec_live_bytes()
@@ -131,6 +132,7 @@ int hipMemcpyAsync(void* d, const void* s, size_t n, int, void* stream)
 int hipStreamSynchronize(void* s)
 {
     if (r.capturing) return r.log.push_back("illegal wait"), fail(kCaptureUnsupported);
+    if (r.wait_fail_in > 0 && --r.wait_fail_in == 0) return fail(kUnknown);
     r.log.push_back("wait" + at(s));
     return kOk;
 }

@@ -103,6 +103,76 @@ def case_face_plan():
         assert not any(p in n for _, n, _ in r.events() for p in PLANS)
 
 
+def first_calls():
+    """name -> calls of which each builds plans or work arrays on first use."""
+    cg = (PTR,) * 7 + (3, 0.0, 0.0, None, None, None)
+    return {
+        "plan": [("rxm_vv_plan_build",)],
+        "smooth": [("rxm_laplacian_smooth", PTR, 2 * PTR, 3 * PTR, 0.5, 4)],
+        "smooth, four steps a launch": [("rxm_set_launch_threads", 8, 4),
+                                        ("rxm_laplacian_smooth", PTR, 2 * PTR, 3 * PTR, 0.5, 4)],
+        "smooth, two steps a launch": [("rxm_set_launch_threads", 4, 1),
+                                       ("rxm_laplacian_smooth", PTR, 2 * PTR, 3 * PTR, 0.5, 5)],
+        "normals": [("rxm_vertex_normals", 0, PTR, 2 * PTR)],
+        "gradient step": [("rxm_symdir3_grad_step", PTR, 2 * PTR, 0.1, 3 * PTR)],
+        "rotations": [("rxm_arap_rotations", PTR, 2 * PTR, 3 * PTR, 4 * PTR)],
+        "energy": [("rxm_arap_energy_grad", PTR, PTR, PTR, PTR, 2 * PTR, 3 * PTR)],
+        "assembly": [("rxm_cot_csr_assemble", PTR, 0.1, 2 * PTR, 3 * PTR, 4 * PTR, 5 * PTR)],
+        "cg": [("rxm_mcf_implicit_cg", *cg[:5], 6 * PTR, *cg[7:])],
+        "matrix-free cg": [("rxm_mcf_matfree_cg", PTR, PTR, 2 * PTR, 0.1, 0, 0, 3, 0.0, 0.0, None, None, None)],
+        "query": [("rxm_query_vv_vf", PTR, 2 * PTR, 3 * PTR, 4 * PTR)],
+    }
+
+
+def last_call(r, calls, stream):
+    for c in calls[:-1]:
+        assert r(*c) == 0
+    r.events()
+    return r(*calls[-1], stream)
+
+
+def case_failed_allocation():
+    """Any one allocation of a first call fails: the call says so (or, where
+    the plan is an option, does without), leaves no array of the unfinished
+    plan behind and no error for the next call, which builds it whole."""
+    for what, calls in first_calls().items():
+        r = Recorder(sphere())
+        assert last_call(r, calls, A) == 0, what
+        whole, n = r.rec.rec_live_bytes(), 0
+        while True:
+            n += 1
+            r = Recorder(sphere())
+            before = r.rec.rec_live_bytes()
+            r.rec.rec_fail_malloc(n)
+            rc = last_call(r, calls, A)
+            r.rec.rec_fail_malloc(0)
+            if rc == 0 and r.rec.rec_live_bytes() == whole:
+                break  # fewer than n allocations: none failed
+            assert rc in (0, 7), (what, n, rc)
+            check_plans_waited_for(r.events())
+            kept = r.rec.rec_live_bytes() - before
+            assert last_call(r, calls, A) == 0, (what, n, "the call after a failed allocation")
+            assert r.rec.rec_live_bytes() == whole, (what, n, kept, r.rec.rec_live_bytes(), whole)
+        assert n > 1, what
+
+
+def case_failed_wait():
+    """A plan whose build could not be waited for is not published: the call
+    fails, and the next one builds the plan anew."""
+    for name, kernel, args in (("rxm_arap_rotations", "k_query2_vv_local", (PTR, 2 * PTR, 3 * PTR, 4 * PTR)),
+                               ("rxm_vertex_normals", "k_query2_vf_local", (0, PTR, 2 * PTR))):
+        r = Recorder(sphere())
+        before = r.rec.rec_live_count()
+        r.rec.rec_fail_wait(1)
+        assert r(name, *args, A) == 5
+        assert r.rec.rec_live_count() == before
+        r.rec.rec_fail_wait(0)
+        r.rec.hipGetLastError()  # a caller that goes on after such an error has read it
+        r.events()
+        assert r(name, *args, A) == 0
+        assert any(kernel in n for _, n, _ in r.events())
+
+
 def case_names():
     return [n[5:] for n in globals() if n.startswith("case_") and n != "case_names"]
 
