@@ -237,7 +237,9 @@ rxm_status rxm_build_edges_device(const uint32_t* fv, uint32_t num_faces, uint32
  * builds it on first use; call this to keep the build out of a timed loop.
  * It also builds the multi-step smoothing plan (patch + rings of neighbours,
  * three or five levels by the number of patches), which rxm_laplacian_smooth
- * then uses for iters > 1; waits for the stream. */
+ * then uses for iters > 1 (without this call it takes one step per launch).
+ * Waits for the stream; on a capturing stream, where it cannot, it leaves the
+ * multi-step plan to a later call. */
 rxm_status rxm_vv_plan_build(rxm_mesh* mesh, void* stream);
 /* Launch configuration knobs (used by the autotuner):
  *   kernel 0: smoothing workgroup size 64 / 128 / 256 / 512 (default: by the

@@ -429,15 +429,23 @@ bool launch_dir(rxm_mesh* m, const uint32_t* base, int32_t* row_ptr, int32_t* co
     return false;
 }
 
+int is_capturing(void* stream, bool* yes)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    RXM_HIP(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap));
+    *yes = cap != hipStreamCaptureStatusNone;
+    return RXM_OK;
+}
+
 // Waits for a plan's build, before the plan is published: calls on other streams
 // read it from then on. Not while the stream is capturing, where the build is a
 // node of the graph.
 int plan_complete(void* stream)
 {
-    hipStream_t            hs  = static_cast<hipStream_t>(stream);
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    RXM_HIP(hipStreamIsCapturing(hs, &cap));
-    if (cap == hipStreamCaptureStatusNone) RXM_HIP(hipStreamSynchronize(hs));
+    bool      capturing = false;
+    const int rc        = is_capturing(stream, &capturing);
+    if (rc) return rc;
+    if (!capturing) RXM_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
     return RXM_OK;
 }
 
@@ -1414,7 +1422,10 @@ rxm_status rxm_vv_plan_build(rxm_mesh* m, void* stream)
     int rc = ensure_vv_plan(m, stream);
     if (rc || m->vvk_tried) return rc;
     // the multi-step plan is an option of the smoothing: patches beyond its
-    // tables or a full device leave the single-step plan in use
+    // tables or a full device leave the single-step plan in use, and so does a
+    // capturing stream, which its build could not wait for
+    bool capturing = false;
+    if ((rc = is_capturing(stream, &capturing)) || capturing) return rc;
     const uint32_t K = auto_levels(m);
     rc           = (m->d_vvk_nbr && m->vvk.K >= K) ? RXM_OK : build_ring_plan(m, K, stream);
     m->vvk_tried = rc == RXM_OK || rc == RXM_ERR_PATCH_TOO_BIG;

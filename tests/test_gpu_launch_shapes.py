@@ -485,3 +485,32 @@ def test_face_plan_built_on_another_stream():
             want = call(n, None)
         torch.cuda.synchronize()
         assert torch.equal(got[0] if isinstance(got, tuple) else got, want[0] if isinstance(want, tuple) else want)
+
+
+@pytest.mark.parametrize("planned", [False, True])
+def test_smoothing_in_a_captured_graph(planned):
+    """Capture with build_vv_plan inside, of a mesh whose VV plan exists
+    already (and, `planned`, its multi-step plan): three replays, eager work
+    between them, each the bits of the eager smoothing."""
+    import torch
+    V, F = mg.icosphere(5, seed=13, sigma=0.01)
+    m, x = _mesh(V, F, 256)
+    ref, tmp = m.smooth(x, 0.5, 4), torch.empty_like(x)  # builds the VV plan
+    if planned:
+        m.build_vv_plan()
+    src, out = x.clone(), torch.empty_like(x)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        m.build_vv_plan()
+        m.smooth(src, 0.5, 4, out=out, tmp=tmp)
+    for k in (1.0, 2.0, 0.5):  # powers of two: the smoothing scales exactly
+        src.copy_(x * k)
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref * k)
+        assert torch.equal(m.smooth(src, 0.5, 4), ref * k)
+        torch.cuda.synchronize()
+    m.build_vv_plan()
+    assert torch.equal(m.smooth(x, 0.5, 4), ref)

@@ -173,6 +173,28 @@ def case_failed_wait():
         assert any(kernel in n for _, n, _ in r.events())
 
 
+def case_capture():
+    """Once a smoothing has built the VV plan, rxm_vv_plan_build and smoothing
+    ask nothing of a capturing stream that it forbids; the multi-step plan is
+    made by the first call outside."""
+    r = Recorder(sphere())
+    assert r.smooth(1, A) == 0
+    r.events()
+    r.rec.rec_capturing(1)
+    assert r("rxm_vv_plan_build", A) == 0
+    assert r.smooth(4, A) == 0
+    e = r.events()
+    assert not [x for x in e if x[0] == "illegal"], e
+    assert sum("k_smooth_local" in n for _, n, _ in e) == 4
+    r.rec.rec_capturing(0)
+    assert r("rxm_vv_plan_build", A) == 0
+    check_plans_waited_for(r.events())
+    r.rec.rec_capturing(1)
+    assert r.smooth(4, A) == 0
+    e = r.events()
+    assert [w for w, _, _ in e] == ["launch"] and "k_smoothk" in e[0][1], e
+
+
 def case_names():
     return [n[5:] for n in globals() if n.startswith("case_") and n != "case_names"]
 
