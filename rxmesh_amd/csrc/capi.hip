@@ -1307,19 +1307,26 @@ rxm_status rxm_vertex_normals(rxm_mesh* m, int mode, const float* pos, float* no
     // patches exceed its u16 encoding use the self-contained kernel
     const int prc = ensure_face_plan(m, stream);
     if (prc == RXM_OK) {
-        Bump b(nullptr);
-        plan_vnp(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
-        const bool lean = b.bytes() > kMaxLdsBytes;
+        const HostMesh& h = m->h;
+        Bump            b(nullptr);
+        plan_vnp(b, h.max_nv, h.max_nvo, h.max_nf, m->fp_max_nent);
+        const bool lean = b.bytes() > kMaxLdsBytes || h.max_nf > kFaceRounds * 1024u;
         Bump       bl(nullptr);
-        plan_vnp(bl, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent, true);
+        plan_vnp(bl, h.max_nv, h.max_nvo, h.max_nf, m->fp_max_nent, true);
         auto go = [&](auto kernel, uint32_t T) {
-            return launch_patches_xcd(kernel, T, lean ? bl.bytes() : b.bytes(), stream, m, m->dm, mode, m->d_fp_fbase, m->d_fp_rbase,
-                                      m->d_fp_nbase, m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, normals);
+            return launch_patches_xcd(kernel, T, lean ? bl.bytes() : b.bytes(), stream, m, m->dm, mode, m->d_fp_fbase,
+                                      m->d_fp_rbase, m->d_fp_nbase, m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, normals);
         };
-        if (lean) return go(k_vertex_normals_plan<256, true>, 256);
-        // us with 512 / 256 threads: 10 patches 4.0 / 4.6, 491 5.4 / 6.0, 2687
-        // 18.2 / 18.5, 10677 55 / 50
-        return m->h.P <= 4096u ? go(k_vertex_normals_plan<512>, 512) : go(k_vertex_normals_plan<256>, 256);
+        if (lean) return go(k_vertex_normals_plan<512, true>, 512);
+        // Two rounds of a patch's faces or less while the patches are few (one
+        // workgroup's chain is the launch), four once others hide it, from one
+        // patch a CU where a patch has a round of 512 and from eight where it has
+        // two. us with 256 / 512 / 1024 threads, patch size 256: 23 patches 3.8 /
+        // 3.7 / -, 336 4.1 / 4.3, 1330 6.0 / 7.1, 21324 44 / 67; 512: 10 4.7 / 3.9 /
+        // 4.2, 670 6.3 / 6.0 / 7.9, 1111 8.9 / 8.6, 2675 15.1 / 15.4, 10630 41 / 46 /
+        // 77; 1024 (512 / 1024): 134 5.5 / 5.2, 335 6.7 / 7.1, 4274 40 / 45.
+        if (h.max_nf <= 1024u && h.P > (h.max_nf <= 512u ? 256u : 2048u)) return go(k_vertex_normals_plan<256>, 256);
+        return h.max_nf <= 2048u ? go(k_vertex_normals_plan<512>, 512) : go(k_vertex_normals_plan<1024>, 1024);
     }
     if (prc != RXM_ERR_PATCH_TOO_BIG) return prc;
     Bump b(nullptr);

@@ -766,15 +766,19 @@ __global__ __launch_bounds__(T) void k_smoothk(DevMesh m, uint32_t K, const uint
 // ---- vertex normals over the patch-local face plan ----------------------------
 // Same weights and summation order as k_vertex_normals (incident faces in
 // ascending local order), but the VF rows come precomputed from the face
-// plan. Face pass: every local face's normal and three corner weights into LDS;
-// vertex pass: each owned vertex sums its rows. Bound by
-// LDS gathers (its LDS was busy 64% of the time, half of that conflicts of the
-// random reads), so a row reads four words of a finished face rather than the
-// nine of its corners and their indexes, and computes nothing: the normals of a
-// torus of 1.3M faces took 20.4 us with the face evaluated anew in each of its
-// three rows, 18.2 so; 10 patches 6.2 -> 4.0, 491 8.3 -> 5.4.
+// plan. Face pass: every local face's normal and three corner weights, in registers
+// until all are done, then into LDS over the corners and positions they came
+// from; vertex pass: each owned vertex sums its rows, four words of a finished face
+// an entry. Bound: LDS gathers of both passes, and for large meshes how many
+// workgroups a CU holds, so the terms share the space of what they replace: beside
+// it (33 KB a patch of 512 faces, four workgroups instead of six) 10630 patches
+// of a sphere took 48 us, 46 with the face evaluated anew in each of its three
+// rows, and 41 so; 8638 patches of a torus 43, 45 and 37; 2675 15.2, 17.9, 15.1;
+// 10 3.8, 6.1 and 3.9.
 // LEAN: no face pass; every (vertex, face) pair evaluates the face, for patches
-// whose face terms (24 bytes a face) do not fit LDS. Same results.
+// whose face terms (24 bytes a face) do not fit LDS or the rounds in registers.
+// Same results.
+constexpr uint32_t kFaceRounds = 4;
 struct PlanVNP
 {
     uint16_t *fvl, *ro, *vf;
@@ -784,14 +788,19 @@ __host__ __device__ inline PlanVNP plan_vnp(Bump& b, uint32_t nv, uint32_t nvo, 
                                             bool lean = false)
 {
     PlanVNP p{};
+    p.ro = b.alloc<uint16_t>((nvo + 1u + 7u) & ~7u);
+    p.vf = b.alloc<uint16_t>((nent + 7u) & ~7u);
+    const uint32_t start = b.off;
     p.fvl = b.alloc<uint16_t>((3 * nf + 7u) & ~7u);
-    p.ro  = b.alloc<uint16_t>((nvo + 1u + 7u) & ~7u);
-    p.vf  = b.alloc<uint16_t>((nent + 7u) & ~7u);
     p.x   = b.alloc<float>(nv);
     p.y   = b.alloc<float>(nv);
     p.z   = b.alloc<float>(nv);
-    for (int c = 0; c < 3; ++c) p.n[c] = lean ? nullptr : b.alloc<float>(nf);
-    p.cw = lean ? nullptr : b.alloc<float>(3 * nf);
+    if (lean) return p;
+    const uint32_t end = b.off;  // the face terms take the same space
+    b.off = start;
+    for (int c = 0; c < 3; ++c) p.n[c] = b.alloc<float>(nf);
+    p.cw  = b.alloc<float>(3 * nf);
+    b.off = b.off > end ? b.off : end;
     return p;
 }
 
@@ -860,14 +869,20 @@ __global__ __launch_bounds__(T) void k_vertex_normals_plan(DevMesh m, int mode, 
         }
     };
     if constexpr (!LEAN) {
-        for (uint32_t f = threadIdx.x; f < d.nf; f += T) {
-            float n[3], w[3];
-            face(f, n, w);
+        float n[kFaceRounds][3], w[kFaceRounds][3];
 #pragma unroll
-            for (uint32_t j = 0; j < 3; ++j) {
-                L.n[j][f]       = n[j];
-                L.cw[3 * f + j] = w[j];
-            }
+        for (uint32_t r = 0; r < kFaceRounds; ++r)
+            if (threadIdx.x + r * T < d.nf) face(threadIdx.x + r * T, n[r], w[r]);
+        __syncthreads();  // every corner has been read
+#pragma unroll
+        for (uint32_t r = 0; r < kFaceRounds; ++r) {
+            const uint32_t f = threadIdx.x + r * T;
+            if (f < d.nf)
+#pragma unroll
+                for (uint32_t j = 0; j < 3; ++j) {
+                    L.n[j][f]       = n[r][j];
+                    L.cw[3 * f + j] = w[r][j];
+                }
         }
         __syncthreads();
     }

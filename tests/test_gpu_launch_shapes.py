@@ -514,3 +514,32 @@ def test_smoothing_in_a_captured_graph(planned):
         torch.cuda.synchronize()
     m.build_vv_plan()
     assert torch.equal(m.smooth(x, 0.5, 4), ref)
+
+
+@pytest.mark.parametrize("nu,nw,patch_size", [(16, 16, 8192), (16, 32, 8192), (32, 32, 8192), (25, 41, 8192),
+                                              (32, 64, 8192), (3, 683, 8192), (1200, 460, 512), (97, 53, 256)])
+def test_vertex_normals_at_the_rounds_of_each_workgroup(nu, nw, patch_size):
+    """One patch of 512, 1024, 2048, 2050, 4096 and 4098 faces (a round more or
+    less for 256, 512 and 1024 threads, and the form without a face pass), and
+    many patches, against FP64. Bound per vertex, from the fp32 evaluation (u the
+    unit roundoff): a normal's component is off by at most 4 u |e1| |e2| (two
+    products of rounded differences, one subtraction), a weight by 6 u (two
+    squared lengths of three terms, a reciprocal of 1 ulp) and a sum of k terms
+    by k u: (10 + k) u times the sum of weight |e1| |e2| over its faces."""
+    V, F = mg.permute_mesh(*mg.torus(nu, nw), seed=14)
+    m, x = _mesh(V, F, patch_size)
+    assert (m.P == 1) == (patch_size == 8192) and (patch_size != 512 or m.P > 2048)
+    l2g = m.array("v_l2g")
+    X = np.empty((m.nV, 3))
+    X[l2g] = x.cpu().numpy().T
+    c = X[F]
+    n = np.cross(c[:, 1] - c[:, 0], c[:, 2] - c[:, 0])
+    l = ((c - np.roll(c, -1, 1)) ** 2).sum(2)
+    size = np.sqrt(l[:, 0] * l[:, 2])  # |e1| |e2|: edges 0 -> 1 and 2 -> 0
+    gather = lambda t: np.bincount(F.reshape(-1), t.reshape(-1), m.nV)  # noqa: E731
+    k = gather(np.ones(F.shape))
+    for mode, wt in (("max", 1.0 / (l + np.roll(l, 1, 1))), ("area", np.full(l.shape, 0.5))):
+        ref = np.stack([gather(n[:, None, j] * wt) for j in range(3)], 1)
+        bound = (10 + k) * 2.0 ** -24 * gather(size[:, None] * wt)
+        got = m.vertex_normals(x, mode).cpu().numpy().T
+        assert (np.abs(got - ref[l2g]) <= bound[l2g][:, None]).all()
