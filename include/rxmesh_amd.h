@@ -242,8 +242,9 @@ rxm_status rxm_build_edges_device(const uint32_t* fv, uint32_t num_faces, uint32
  * multi-step plan to a later call. */
 rxm_status rxm_vv_plan_build(rxm_mesh* mesh, void* stream);
 /* Launch configuration knobs (used by the autotuner):
- *   kernel 0: smoothing workgroup size 64 / 128 / 256 / 512 (default: by the
- *             number of patches);
+ *   kernel 0: smoothing workgroup size 64 / 128 / 256 / 512, or 0 (default) =
+ *             by the number of patches (then also 1024 for several steps per
+ *             launch);
  *   kernel 1: symmetric-Dirichlet step workgroup size 128 / 256 / 512;
  *   kernel 2: symmetric-Dirichlet step launch, 0 = one workgroup per patch,
  *             1 = persistent grid over a global patch work queue;
@@ -256,8 +257,8 @@ rxm_status rxm_vv_plan_build(rxm_mesh* mesh, void* stream);
  *   kernel 7: cotangent assembly workgroup size 256 / 512;
  *   kernel 8: smoothing, 1-6 = that many Jacobi steps per launch over the
  *             K-level plan (patch + rings of neighbours kept in LDS; overrides
- *             kernels 3 and 4), 0 = off; until it is set, and while kernels 3
- *             and 4 are 0, the steps rxm_vv_plan_build planned for;
+ *             kernels 3 and 4), 0 = off, -1 (default) = while kernels 3 and 4
+ *             are 0, the steps rxm_vv_plan_build planned for;
  *   kernel 9: smoothing with two steps per launch (kernel 4 = 1, float
  *             arrays in LDS) and >= 4 iterations: 1 = the iterates between
  *             launches are one float4 per vertex in two buffers the mesh

@@ -65,6 +65,7 @@ SMOOTH_STEPS_THREADS = (128, 256, 512)
 
 
 def smooth_configs():
+    yield {"smooth_threads": 0, "smooth_layout": 0, "smooth_fused": 0, "smooth_steps": -1}  # the library's own choice
     for fused in SMOOTH_FUSED:
         for st in SMOOTH_THREADS:
             for lay in SMOOTH_LAYOUTS:
@@ -77,6 +78,8 @@ def smooth_configs():
 
 
 def config_name(cfg):
+    if cfg.get("smooth_steps", 0) < 0:
+        return "auto"
     if cfg.get("smooth_steps", 0):
         return "t%d/k%d" % (cfg["smooth_threads"], cfg["smooth_steps"])
     return "t%d/l%d/f%d%s" % (cfg["smooth_threads"], cfg["smooth_layout"], cfg["smooth_fused"],
@@ -94,8 +97,8 @@ def apply(mesh, cfg):
         mesh.set_launch_threads(3, cfg["smooth_layout"])
     if "smooth_fused" in cfg:
         mesh.set_launch_threads(4, cfg["smooth_fused"])
-    if "smooth_threads" in cfg:
-        mesh.set_launch_threads(8, cfg.get("smooth_steps", 0))
+    if "smooth_steps" in cfg:  # a config of the step loop, which smooths by single steps, has none
+        mesh.set_launch_threads(8, cfg["smooth_steps"])
         mesh.set_launch_threads(9, cfg.get("smooth_g4", 0))
 
 

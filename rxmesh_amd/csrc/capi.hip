@@ -1506,7 +1506,7 @@ rxm_status rxm_laplacian_smooth(rxm_mesh* m, const float* pos, float* out, float
 rxm_status rxm_set_launch_threads(rxm_mesh* m, int kernel, int threads)
 {
     if (!m) return RXM_ERR_INVALID_ARG;
-    if (kernel == 0 && (threads == 64 || threads == 128 || threads == 256 || threads == 512)) {
+    if (kernel == 0 && (threads == 0 || threads == 64 || threads == 128 || threads == 256 || threads == 512)) {
         m->smooth_threads = static_cast<uint32_t>(threads);
         return RXM_OK;
     }
@@ -1549,8 +1549,8 @@ rxm_status rxm_set_launch_threads(rxm_mesh* m, int kernel, int threads)
         m->smooth_g4 = static_cast<uint32_t>(threads);
         return RXM_OK;
     }
-    if (kernel == 8 && threads >= 0 && threads <= static_cast<int>(kSmoothLevels)) {
-        m->smooth_steps = static_cast<uint32_t>(threads);
+    if (kernel == 8 && threads >= -1 && threads <= static_cast<int>(kSmoothLevels)) {
+        m->smooth_steps = static_cast<uint32_t>(threads);  // -1: kStepsAuto
         return RXM_OK;
     }
     return RXM_ERR_INVALID_ARG;

@@ -195,6 +195,33 @@ def case_capture():
     assert [w for w, _, _ in e] == ["launch"] and "k_smoothk" in e[0][1], e
 
 
+def case_automatic_smoothing():
+    """Tuning the gradient step loop leaves the steps per launch of the
+    smoothing alone, and knobs 0 and 8 have a value that means the automatic
+    choice."""
+    r = Recorder(sphere())
+    from rxmesh_amd import autotune
+    assert r("rxm_vv_plan_build", A) == 0
+
+    def kernels():
+        r.events()
+        assert r.smooth(4, A) == 0
+        return [n for _, n, _ in r.events()]
+    default = kernels()
+    assert len(default) == 1 and "k_smoothkILj1024" in default[0]
+    autotune.apply(r.mesh, {"smooth_threads": 256, "grad_threads": 256, "grad_queue": 0})
+    tuned = kernels()
+    assert len(tuned) == 1 and "k_smoothkILj256" in tuned[0], tuned
+    for cfg in autotune.smooth_configs():
+        autotune.apply(r.mesh, cfg)
+        assert (kernels() == default) == (cfg["smooth_steps"] == -1), cfg
+    assert r("rxm_set_launch_threads", 8, 0) == 0 and len(kernels()) == 4
+    assert r("rxm_set_launch_threads", 0, 0) == 0 and r("rxm_set_launch_threads", 8, -1) == 0
+    assert kernels() == default
+    for knob, value in ((0, -1), (0, 1), (0, 1024), (8, -2), (8, 7)):
+        assert r("rxm_set_launch_threads", knob, value) == 1
+
+
 def case_names():
     return [n[5:] for n in globals() if n.startswith("case_") and n != "case_names"]
 
