@@ -634,7 +634,7 @@ int ensure_cot_plan(rxm_mesh* m, void* stream)
     return RXM_OK;
 }
 
-constexpr uint32_t kSmoothLevels = 6;  // rings of the K-level plan: up to 6 steps per launch
+constexpr uint32_t kSmoothLevels = 6;  // largest number of steps per launch that knob 8 takes
 
 // The K-level plan over K rings, built by k_ring_plan from the VV plan (waits
 // for the stream to size it): 2 launches instead of a host walk with a map per
@@ -696,11 +696,15 @@ int build_ring_plan(rxm_mesh* m, uint32_t K, void* stream)
     return RXM_OK;
 }
 
-// A K-level plan of at least K rings: on the device, or, for patches beyond
-// that kernel's tables, by the host walk.
-int ensure_vvk_plan(rxm_mesh* m, uint32_t K, void* stream)
+// A K-level plan of at least `steps` rings: on the device, or, for patches beyond
+// that kernel's tables, by the host walk. One that has to be built gets every
+// ring that knob 8 can ask for: the arrays of a plan it replaces stay with the
+// mesh (launches and graphs may hold them), so a mesh has at most the automatic
+// plan and this one.
+int ensure_vvk_plan(rxm_mesh* m, uint32_t steps, void* stream)
 {
-    if (m->d_vvk_nbr && m->vvk.K >= K) return RXM_OK;
+    if (m->d_vvk_nbr && m->vvk.K >= steps) return RXM_OK;
+    constexpr uint32_t K = kSmoothLevels;
     int rc = ensure_vv_plan(m, stream);
     if (!rc) rc = build_ring_plan(m, K, stream);
     if (rc != RXM_ERR_PATCH_TOO_BIG) return rc;
@@ -1436,7 +1440,8 @@ rxm_status rxm_vv_plan_build(rxm_mesh* m, void* stream)
     const uint32_t K = auto_levels(m);
     rc           = (m->d_vvk_nbr && m->vvk.K >= K) ? RXM_OK : build_ring_plan(m, K, stream);
     m->vvk_tried = rc == RXM_OK || rc == RXM_ERR_PATCH_TOO_BIG;
-    m->vvk_auto  = rc == RXM_OK;
+    // a plan that the host built before may hold larger patches
+    m->vvk_auto = rc == RXM_OK && m->vvk.max_cnt[K] <= kRingVerts && m->vvk.max_ent[K - 1] <= kRingEnts;
     return (rc == RXM_ERR_PATCH_TOO_BIG || rc == RXM_ERR_OUT_OF_MEMORY) ? RXM_OK : rc;
 }
 

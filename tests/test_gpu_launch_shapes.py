@@ -543,3 +543,23 @@ def test_vertex_normals_at_the_rounds_of_each_workgroup(nu, nw, patch_size):
         bound = (10 + k) * 2.0 ** -24 * gather(size[:, None] * wt)
         got = m.vertex_normals(x, mode).cpu().numpy().T
         assert (np.abs(got - ref[l2g]) <= bound[l2g][:, None]).all()
+
+
+def test_automatic_smoothing_of_patches_beyond_several_steps():
+    """Two patches of 8000 faces, beyond the plan kernel's tables: one step per
+    launch goes over the host-built plan, five do not fit LDS. The automatic
+    choice stays with single steps whatever plan was made before."""
+    import torch
+    import rxmesh_amd as rx
+    V, F = mg.torus(80, 100)
+    m = rx.Mesh(F, face_patch=(F.min(1) // 100 >= 40).astype(np.uint32))
+    assert m.P == 2 and m.info["max_owned_faces"] < 8500
+    x = torch.from_numpy(np.ascontiguousarray(V[m.array("v_l2g")].T.astype(np.float32))).cuda()
+    m.set_launch_threads(8, 0)
+    ref = m.smooth(x, 0.5, 6)
+    one = m.smooth(x, 0.5, 1)
+    m.set_launch_threads(8, 6)
+    assert torch.equal(m.smooth(x, 0.5, 1), one)
+    m.build_vv_plan()
+    m.set_launch_threads(8, -1)
+    assert torch.equal(m.smooth(x, 0.5, 6), ref)

@@ -222,6 +222,24 @@ def case_automatic_smoothing():
         assert r("rxm_set_launch_threads", knob, value) == 1
 
 
+def case_one_plan_for_every_steps():
+    """Walking the steps per launch upwards (as the tuner does) makes one plan
+    that holds them all, beside the automatic one where that was made."""
+    for planned in (0, 1):
+        r = Recorder(sphere())
+        if planned:
+            assert r("rxm_vv_plan_build", A) == 0
+        assert r.smooth(1, A) == 0
+        sizes = []
+        r.events()
+        for steps in (2, 3, 4, 5, 6, 1, 6):
+            assert r("rxm_set_launch_threads", 8, steps) == 0
+            assert r.smooth(12, A) == 0
+            sizes.append(r.rec.rec_live_bytes())
+        assert sum("k_ring_plan" in n for _, n, _ in r.events()) == 2  # its two passes
+        assert sizes[-1] == sizes[4] and (planned or len(set(sizes)) == 1)
+
+
 def case_names():
     return [n[5:] for n in globals() if n.startswith("case_") and n != "case_names"]
 
