@@ -267,13 +267,15 @@ class Mesh:
         self.nF = self.info["num_faces"]
         self.P = self.info["num_patches"]
         self._shape_v3, self._shape_mr, self._shape_rp = (3, self.nV), (4, self.nF), (self.nV + 1,)
-        self._counts = {}  # entries per query: fixed by the connectivity
+        self._counts = {}  # entries per query: fixed by the connectivity, kept while the mesh is open
+        self._cot_nnz = None
         self._nsrc = {"V": self.nV, "E": self.nE, "F": self.nF}
 
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:
             _check(lib().rxm_mesh_destroy(self._h), "rxm_mesh_destroy")
         self._h = None
+        self._counts, self._cot_nnz = {}, None
 
     def __del__(self):
         try:
@@ -501,11 +503,11 @@ class Mesh:
 
     # -- cotangent system / explicit MCF ------------------------------
     def cot_nnz(self):
-        n = self._counts.get("cot")
+        n = self._cot_nnz
         if n is None:
             c = ctypes.c_int64()
             _check(lib().rxm_cot_nnz(self._h, ctypes.byref(c)), "rxm_cot_nnz")
-            n = self._counts["cot"] = c.value
+            n = self._cot_nnz = c.value
         return n
 
     def _system(self, A):

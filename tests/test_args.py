@@ -100,3 +100,15 @@ def test_host_memory_refused(mesh):
         rx.build_edges_device(torch.zeros(5, 3, dtype=torch.int32), 3)
     with pytest.raises(ValueError, match=r"\(F, 3\)"):
         rx.build_edges_device(torch.zeros(15, dtype=torch.int32), 3)
+
+
+def test_counts_of_a_closed_mesh_and_of_unknown_queries_refused():
+    """Kept counts answer for a live mesh and its queries only."""
+    m = rx.Mesh(mg.icosphere(2, seed=0)[1], patch_size=64, host_only=True)
+    assert m.query_nnz("VV") == 2 * m.nE and m.cot_nnz() == 2 * m.nE + m.nV
+    with pytest.raises(KeyError):
+        m.query_nnz("cot")
+    m.close()
+    for count in (lambda: m.query_nnz("VV"), m.cot_nnz):
+        with pytest.raises(rx.RXMError):
+            count()
