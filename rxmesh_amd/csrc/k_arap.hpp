@@ -205,8 +205,12 @@ __device__ inline void best_rotation(const float (&S)[3][3], float (&R)[3][3])
 // method from the bound sqrt(3) |S| (monotone from above); its eigenvector is
 // the largest column of the adjugate of N - l I (Theobald, Acta Cryst. A 61:478,
 // 2005, takes the same two steps). Returns false, R unset, where the gap to the
-// next eigenvalue leaves the adjugate fewer than about nine digits, or the root
-// has not settled: the sweeps decide there. About 300 instructions a vertex
+// next eigenvalue all but cancels the adjugate (below 1e-7 of l^3), or the root
+// has not settled: the sweeps decide there. What it accepts loses digits with the
+// gap, but far fewer than the sweeps do in FP32: over random mirrored covariances
+// the eigenvector is off by at most 8e-13, 6e-10, 1e-7, 2e-6 and 8e-6 at gaps of
+// 1e-1 to 1e-5 of l, an FP32 eigenvector by 8e-7, 7e-6, 7e-5, 8e-4 and 7e-3, and
+// S's own FP32 rounding moves it by 6e-8 over the gap. About 300 instructions a vertex
 // against 2,000 and more of the sweeps, which bound the kernel
 // (654k vertices 41 -> 30 us with the records written as one run and 256 threads,
 // 2.6M 129 -> 90; now the staging). Its error against FP64 is not larger: R is

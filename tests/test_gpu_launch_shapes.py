@@ -563,3 +563,59 @@ def test_automatic_smoothing_of_patches_beyond_several_steps():
     m.build_vv_plan()
     m.set_launch_threads(8, -1)
     assert torch.equal(m.smooth(x, 0.5, 6), ref)
+
+
+def test_arap_rotations_of_nearly_undecided_covariances():
+    """Covariances whose best rotation leads the next one by a gap of 1e-1 to
+    1e-5 of the largest singular value (mirrored ones, and such of nearly one
+    direction), where the closed form and the sweeps it falls back on meet. R
+    against FP64 of the same fp32 input. Bound, u the fp32 unit roundoff: k
+    products summed leave S off by (k + 3) u sum w |a| |c|, the 4 x 4 matrix by
+    sqrt(3) of that, its eigenvector by that over the gap of its eigenvalues, R
+    by 4 times that; the sweeps add 64 u |S| over the gap, the closed form at
+    most 1e-5."""
+    import torch
+    V, F = mg.permute_mesh(*mg.icosphere(5, seed=15), seed=15)
+    m, _ = _mesh(V, F, 512)
+    l2g, e_l2g = m.array("v_l2g"), m.array("e_l2g")
+    ev = m.array("ev").reshape(-1, 2).astype(np.int64)[e_l2g]  # global endpoints by linear edge
+    rng = np.random.default_rng(15)
+    w = rng.uniform(0.5, 1.5, m.nE).astype(np.float32)
+    ring = [[] for _ in range(m.nV)]
+    for k, (i, j) in enumerate(ev.tolist()):
+        ring[i].append((j, k))
+        ring[j].append((i, k))
+    P, X = (rng.normal(size=(m.nV, 3)).astype(np.float32) for _ in range(2))
+    free, chosen = np.ones(m.nV, bool), []
+    for v in range(m.nV):  # vertices whose rings are disjoint
+        ids = [v] + [j for j, _ in ring[v]]
+        if free[ids].all():
+            free[ids] = False
+            chosen.append(v)
+    rot = lambda: np.linalg.qr(rng.normal(size=(3, 3)))[0]  # noqa: E731
+    for n, v in enumerate(chosen):
+        gap, s2 = 10.0 ** -rng.uniform(1, 5), rng.uniform(0.2, 0.9)
+        U, W = rot(), rot()
+        mirrored = n % 4 != 0
+        U[:, 2] *= np.sign(np.linalg.det(U @ W)) * (-1.0 if mirrored else 1.0)
+        T = U @ np.diag([1.0, s2, s2 - gap / 2] if mirrored else [1.0, gap / 4, gap / 4]) @ W
+        P[v] = X[v] = 0.0
+        nb, wt = [j for j, _ in ring[v]], np.array([w[k] for _, k in ring[v]], np.float64)
+        a = -P[nb].astype(np.float64)
+        X[nb] = -(a @ np.linalg.solve((wt[:, None] * a).T @ a, T))  # sum w a c^T = T
+    Pd, Xd = (torch.from_numpy(np.ascontiguousarray(q[l2g].T)).cuda() for q in (P, X))
+    R = np.empty((m.nV, 3, 3))
+    R[l2g] = m.arap_rotations(Pd, Xd, torch.from_numpy(w).cuda()).cpu().numpy().reshape(-1, 3, 3)
+    u, decades = 2.0 ** -24, set()
+    for v in chosen:
+        nb, wt = [j for j, _ in ring[v]], np.array([w[k] for _, k in ring[v]], np.float64)
+        a, c = -P[nb].astype(np.float64), -X[nb].astype(np.float64)
+        U, s, Wt = np.linalg.svd((wt[:, None] * a).T @ c)
+        sign = np.sign(np.linalg.det(U @ Wt))
+        U[:, 2] *= sign
+        gap = 2.0 * (s[1] + sign * s[2])
+        off = np.sqrt(3.0) * (len(nb) + 3) * (wt * np.linalg.norm(a, axis=1) * np.linalg.norm(c, axis=1)).sum()
+        bound = 1e-5 + 4.0 * u * (off + 64.0 * s[0]) / gap
+        assert np.abs(R[v] - Wt.T @ U.T).max() <= bound, (v, gap / s[0], bound)
+        decades.add(int(np.floor(np.log10(gap / s[0]))))
+    assert {-2, -3, -4, -5} <= decades
