@@ -360,8 +360,9 @@ rxm_status rxm_symdir_grad(rxm_mesh* mesh, const float* Mr, const float* uv, con
  * synchronisation; when any of iters / start_residual / final_residual is
  * non-NULL the call waits for the stream and reports the iterations taken and
  * the squared residual norms, as the reference's solver does. Work vectors
- * (4 x 3V floats, shared by the solves of the mesh) are allocated by the mesh
- * on first use. */
+ * and scalars (4 x 3V floats) are allocated by the mesh on first use and shared
+ * by every solve on it, this one and rxm_mcf_matfree_cg: solves of one mesh
+ * on different streams have to be ordered by the caller. */
 rxm_status rxm_mcf_implicit_cg(rxm_mesh* mesh, const int32_t* row_ptr, const int32_t* col,
                                const float* val, const float* mass, const float* x, float* out,
                                int max_iter, float abs_tol, float rel_tol, int* iters,
@@ -370,8 +371,9 @@ rxm_status rxm_mcf_implicit_cg(rxm_mesh* mesh, const int32_t* row_ptr, const int
 /* Implicit MCF step without a system from the caller: CG (precond = 0) or
  * Jacobi-preconditioned CG (precond = 1) on A X = B with the weights of the
  * fixed input coordinates `coords` (3 x V SoA), evaluated once per call into
- * mesh-owned scratch (cotangent weights: rxm_cot_nnz floats; no CSR): A = M + dt L with cotangent weights max(0, cot + cot) and Voronoi
- * mass (uniform = 0), or unit weights and mass = valence (uniform = 1); B =
+ * mesh-owned scratch (cotangent weights: rxm_cot_nnz floats; no CSR), which the
+ * solves of the mesh share as they share their work vectors: A = M + dt L with
+ * cotangent weights max(0, cot + cot) and Voronoi mass (uniform = 0), or unit weights and mass = valence (uniform = 1); B =
  * M x (the reference's init_B). x is the initial X (3 x V SoA; the reference
  * starts from the input coordinates), the solution goes to `out`. Stopping
  * rules, residuals (|r|^2, or <r, r / diag> with the preconditioner) and
