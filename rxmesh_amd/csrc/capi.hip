@@ -421,10 +421,15 @@ bool launch_dir(rxm_mesh* m, const uint32_t* base, int32_t* row_ptr, int32_t* co
         *rc = launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, nout, base, row_ptr, col);
         return true;
     };
-    // workgroup sizes as launch_rows chooses them
+    // Small workgroups overlap each other's chains from fewer patches on than in
+    // launch_rows, there being less to do per thread. us with 256 / 512 / 1024
+    // threads, EF and FF: 166 patches 4.3 / 3.7 / 3.5 and 3.7 / 3.4 / 3.3, 267
+    // 4.5 / 4.0 / 4.2 and 3.9 / 3.7 / 3.9, 670 5.2 / 5.0 / 5.9 and 4.6 / 4.7 / 5.5,
+    // 1111 6.4 / 6.9 / 8.4 and 5.8 / 6.2 / 7.7, 2675 10.6 / 11.8 / 15.7 and
+    // 9.7 / 10.3 / 14.5, 10630 26 / 33 / 51 and 25 / 29 / 46.
     constexpr uint32_t RS = FF ? 3 : 4;
     if (h.P <= 256u && fits(1024, 1, 1)) return go(k_query_dir<1024, 1, 1, FF>, 1024);
-    if (h.P > 1500u && fits(256, 4, RS)) return go(k_query_dir<256, 4, RS, FF>, 256);
+    if (h.P > 700u && fits(256, 4, RS)) return go(k_query_dir<256, 4, RS, FF>, 256);
     if (fits(512, 3, RS)) return go(k_query_dir<512, 3, RS, FF>, 512);
     return false;
 }
@@ -1713,6 +1718,9 @@ rxm_status rxm_mcf_explicit(rxm_mesh* m, const int32_t* row_ptr, const int32_t* 
             return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
                                       m->d_vv_roff, m->d_vv_nbr, val, mass, src, dst);
         };
+        // the smoothing's sizes: us with 512 / 256 threads, 166 patches 3.8 / 4.4,
+        // 670 5.3 / 5.6, 1111 7.0 / 7.5, 1961 10.1 / 10.1, 2675 12.6 / 12.0, 10630
+        // 35 / 31
         rc = smooth_group(m) == 512u ? go(k_mcf_patch<512>, 512) : go(k_mcf_patch<256>, 256);
         src = dst;
     }
