@@ -27,6 +27,7 @@ __device__ __forceinline__ void load_faces(FaceWords (&fw)[RF], const uint16_t* 
 // vertex the best start (u64) and the row offset, the rows (nrow = entries of
 // the patch's owned rows), global ids of the local vertices and linear ids of
 // the ribbon's elements the rows list.
+constexpr uint32_t kSeveralFans = 19;  // word of PlanVXO::wave past what the scan uses: some vertex has several fans
 struct PlanVXO
 {
     uint64_t* start;
@@ -62,16 +63,14 @@ __host__ __device__ inline PlanFX plan_fx(Bump& b, uint32_t ne, uint32_t nf)
 }
 
 // The ring of a vertex of several fans, or whose fan does not start where the
-// rule says: the vertex's edges in ascending local id, then the rule of
-// orient_ring_lds (selection of a start among the edges left, walk, restart).
+// rule says: L.rows holds the half-edges leaving it, in any order; the rule of
+// orient_ring_lds (selection of a start among the edges left, walk, restart),
+// whose result does not depend on theirs.
 template <bool NBR>
-__device__ inline void ring_by_selection(uint32_t v, uint32_t k0, uint32_t k1, const PlanVXO& L, uint32_t ne)
+__device__ inline void ring_by_selection(uint32_t k0, uint32_t k1, const PlanVXO& L)
 {
     const uint16_t* ev16 = reinterpret_cast<const uint16_t*>(L.ev);
     const uint16_t* nh   = reinterpret_cast<const uint16_t*>(L.nh);
-    uint32_t        n = k0;
-    for (uint32_t i = 0; i < 2u * ne && n < k1; ++i)  // half-edge i leaves vertex ev16[i]
-        if (ev16[i] == v) L.rows[n++] = static_cast<uint16_t>(i);
     auto nbr       = [&](uint32_t h) { return static_cast<uint32_t>(ev16[h ^ 1u]); };
     auto startable = [&](uint32_t h) { return nh[h] != kInv16 && nh[h ^ 1u] == kInv16; };
     uint32_t pos = k0;
@@ -113,8 +112,11 @@ __device__ inline void ring_by_selection(uint32_t v, uint32_t k0, uint32_t k1, c
 // Sorting each row and matching successors against it in registers took 43.7 us
 // on 654k vertices and 110 on 2.6M; this takes 19.0 and 46. Bound: LDS (random
 // minima and adds). A vertex the walk does not
-// exhaust (several fans) takes ring_by_selection. Needs ne < 2^15 and a
-// consistently oriented edge-manifold mesh (checked on the host).
+// exhaust (several fans) takes ring_by_selection; where a patch has any, the
+// workgroup first collects their half-edges in one pass (a thread that looked for
+// its row's by itself held up the launch: two tori glued at one vertex, 358
+// patches, 29 us with rows matched in registers, 199 so, 23 now). Needs ne < 2^15
+// and a consistently oriented edge-manifold mesh (checked on the host).
 template <uint32_t T, bool IS_VV>
 __global__ __launch_bounds__(T) void k_query_vx_oriented(DevMesh m, uint32_t nrid, const uint32_t* __restrict__ base,
                                                          int32_t* __restrict__ row_ptr, int32_t* __restrict__ col)
@@ -143,6 +145,7 @@ __global__ __launch_bounds__(T) void k_query_vx_oriented(DevMesh m, uint32_t nri
     for (uint32_t i = t; i < d.ne; i += T) L.nh[i] = 0xFFFFFFFFu;
     for (uint32_t v = t; v < nvo; v += T) L.start[v] = ~0ull;
     for (uint32_t v = t; v <= nvo; v += T) L.off[v] = 0u;
+    if (t == 0) L.wave[kSeveralFans] = 0u;
     h_ev.store(reinterpret_cast<u32x4*>(L.ev), evs, r4(d.ne) >> 2);
     h_gid.store(L.gid, gs, d.nv);
     h_rid.store(L.rid, rs, nr);
@@ -185,16 +188,34 @@ __global__ __launch_bounds__(T) void k_query_vx_oriented(DevMesh m, uint32_t nri
     auto            row1 = [&](uint32_t v) { return v + 1u < nvo ? L.off[v + 2u] : nent; };
     for (uint32_t v = t; v < nvo; v += T) {
         const uint32_t k0 = row0(v), k1 = row1(v);
-        if (k0 >= k1) continue;
         const uint32_t s = static_cast<uint32_t>(L.start[v]) & 0xFFFFu;
         uint32_t       h = s, k = k0;
+        L.start[v] = ~0ull;
+        if (k0 >= k1) continue;
         do {
             L.rows[k++] = static_cast<uint16_t>(IS_VV ? static_cast<uint32_t>(ev16[h ^ 1u]) : h >> 1);
             h           = nh[h];
         } while (k < k1 && h != kInv16 && h != s);
-        if (k < k1) ring_by_selection<IS_VV>(v, k0, k1, L, d.ne);
+        if (k < k1) {  // several fans: a cursor into the row (no other value is that small)
+            L.start[v]           = 0ull;
+            L.wave[kSeveralFans] = 1u;
+        }
     }
     __syncthreads();
+    if (L.wave[kSeveralFans]) {  // uniform
+        auto several = [&](uint32_t v) { return L.start[v] != ~0ull; };
+        for (uint32_t i = t; i < 2u * d.ne; i += T) {  // half-edge i leaves vertex ev16[i]
+            const uint32_t v = ev16[i];
+            if (v < nvo && several(v))
+                L.rows[row0(v) + static_cast<uint32_t>(
+                                     atomicAdd(reinterpret_cast<unsigned long long*>(&L.start[v]), 1ull))] =
+                    static_cast<uint16_t>(i);
+        }
+        __syncthreads();
+        for (uint32_t v = t; v < nvo; v += T)
+            if (several(v)) ring_by_selection<IS_VV>(row0(v), row1(v), L);
+        __syncthreads();
+    }
     for (uint32_t v = t; v < nvo; v += T) row_ptr[d.vp + v] = static_cast<int32_t>(bse + row0(v));
     if (t == 0) row_ptr[d.vp + nvo] = static_cast<int32_t>(bse + nent);
     for (uint32_t k = t; k < nent; k += T) {

@@ -619,3 +619,30 @@ def test_arap_rotations_of_nearly_undecided_covariances():
         assert np.abs(R[v] - Wt.T @ U.T).max() <= bound, (v, gap / s[0], bound)
         decades.add(int(np.floor(np.log10(gap / s[0]))))
     assert {-2, -3, -4, -5} <= decades
+
+
+@pytest.mark.parametrize("share", [1, 7, 900])
+@pytest.mark.parametrize("patch_size", [64, 512, 4096])
+def test_oriented_rows_of_many_vertices_with_several_fans(share, patch_size):
+    """Two closed surfaces and a sheet glued vertex to vertex (two and three
+    fans, closed and open, one to most vertices of a patch): oriented VV and
+    VE against the oracle, unoriented too."""
+    import rxmesh_amd as rx
+    from oracle.oracle import OracleMesh
+    parts = [mg.torus(60, 40)[1], mg.torus(60, 40)[1] + 2400, mg.grid(60, seed=3)[1] + 4800]
+    n = 4800 + int(parts[2].max()) - 4799
+    spots = np.random.default_rng(16).permutation((np.arange(0, 58, 2)[:, None] * 40 + np.arange(0, 38, 2)).ravel())[:share]
+    glue = np.arange(n)
+    glue[spots + 2400] = spots
+    third = spots[::3]
+    glue[4800 + (third // 40) * 60 + third % 40] = third  # vertices of the sheet, two apart in both directions
+    F = np.unique(glue[np.concatenate(parts)], return_inverse=True)[1].reshape(-1, 3).astype(np.uint32)
+    F = mg.permute_mesh(np.zeros((int(F.max()) + 1, 3)), F, seed=16)[1]
+    m = rx.Mesh(F, patch_size=patch_size)
+    assert m.info["is_edge_manifold"] and m.info["is_consistently_oriented"]
+    o = OracleMesh(F).set_patches(m.array("face_patch"), m.array("patches_val"), m.array("patches_offset"))
+    for op in ("VV", "VE"):
+        for oriented in (True, False):
+            rp, col = m.query(op, oriented=oriented)
+            orp, ocol = o.query(op, oriented=oriented)
+            assert np.array_equal(rp.cpu().numpy(), orp) and np.array_equal(col.cpu().numpy()[:len(ocol)], ocol)
