@@ -619,13 +619,10 @@ int ensure_cot_plan(rxm_mesh* m, void* stream)
     hipLaunchKernelGGL(k_fill_u32, dim3(static_cast<uint32_t>((nw + h.P + 255) / 256)), dim3(256), 0, hs,
                        static_cast<uint32_t>(nw + h.P), 0u, bits);
     Bump b(nullptr);
-    b.alloc<uint32_t>(r4(h.max_ne));
-    b.alloc<uint16_t>(r4(3 * h.max_nf));
     b.alloc<uint16_t>(2 * h.max_ne);
     rc = launch_patches(k_closed_fans<kQueryThreads>, kQueryThreads, b.bytes(), stream, m, m->dm, m->d_vv_rbase,
                         m->d_vv_nbase, static_cast<const uint16_t*>(m->d_vv_roff),
-                        static_cast<const uint16_t*>(m->d_vv_nbr), static_cast<const uint16_t*>(m->d_vv_ent), bits,
-                        bits + nw);
+                        static_cast<const uint16_t*>(m->d_vv_ent), bits, bits + nw);
     if (rc) return rc;
     std::vector<uint32_t> ring(h.P), plist;
     RXM_HIP(hipMemcpyAsync(ring.data(), bits + nw, h.P * sizeof(uint32_t), hipMemcpyDeviceToHost, hs));

@@ -646,3 +646,75 @@ def test_oriented_rows_of_many_vertices_with_several_fans(share, patch_size):
             rp, col = m.query(op, oriented=oriented)
             orp, ocol = o.query(op, oriented=oriented)
             assert np.array_equal(rp.cpu().numpy(), orp) and np.array_equal(col.cpu().numpy()[:len(ocol)], ocol)
+
+
+@pytest.mark.parametrize("shape", ["cones", "glued", "grid", "sphere"])
+@pytest.mark.parametrize("patch_size", [16, 512, 4096])
+def test_closed_fans_of_any_valence(shape, patch_size):
+    """Which vertices the assembly takes from the face pass: the diagonal and
+    mass of the assembled system against FP64 sums over the faces for vertices
+    of one closed fan, among them such of 700 faces, boundaries and glued
+    vertices. 1e-5 of the largest value, the assembly's bound elsewhere, on
+    the vertices of closed fans."""
+    import torch
+    if shape == "cones":  # closed fans of 700, 30 and 3 faces; the rims are boundaries
+        F = np.concatenate([_fan(700, True), _fan(30, True) + 701, _fan(3, True) + 732])
+    elif shape == "glued":
+        F = np.concatenate([mg.torus(20, 12)[1], mg.torus(20, 12)[1] + 240])
+        F = np.unique(np.where(F == 245, 7, F), return_inverse=True)[1].reshape(-1, 3)
+    else:
+        F = mg.grid(25, seed=4)[1] if shape == "grid" else mg.icosphere(3, seed=4)[1]
+    F = F.astype(np.uint32)
+    rng = np.random.default_rng(17)
+    V = rng.normal(size=(int(F.max()) + 1, 3))
+    m, x = _mesh(V, F, patch_size)
+    X = np.empty((m.nV, 3))
+    X[m.array("v_l2g")] = x.cpu().numpy().T
+    rp, col, val, mass = (t.cpu().numpy() for t in m.cot_assemble(x, 0.1))
+    nxt = {}  # successor around v, by (v, neighbour)
+    for a, b, c in F.tolist():
+        for v, p, q in ((a, b, c), (b, c, a), (c, a, b)):
+            nxt.setdefault(v, {})[p] = q
+    closed = np.zeros(m.nV, bool)
+    for v, succ in nxt.items():
+        nb = set(succ) | set(succ.values())
+        p = s = next(iter(succ))
+        n = 0
+        while p in succ and n < len(nb):
+            p, n = succ[p], n + 1
+            if p == s:
+                break
+        closed[v] = p == s and n == len(nb)
+    if shape in ("glued", "sphere"):  # closed surfaces: the matrix-free solve wants every vertex of one closed fan
+        import rxmesh_amd as rx
+        if shape == "sphere":
+            m.mcf_matfree_cg(x, x, 1e-3, max_iter=1)
+        else:
+            with pytest.raises(rx.RXMError) as e:
+                m.mcf_matfree_cg(x, x, 1e-3, max_iter=1)
+            assert e.value.code == 6
+    assert closed.any() and closed.sum() == {"cones": 3, "glued": 478, "grid": 23 * 23, "sphere": m.nV}[shape]
+    c = X[F]
+    area = 0.5 * np.linalg.norm(np.cross(c[:, 1] - c[:, 0], c[:, 2] - c[:, 0]), axis=1)
+    w, vor = {}, np.zeros(m.nV)
+    clamp = lambda t: np.clip(t, -19.1, 19.1)  # noqa: E731
+    for j in range(3):
+        i0, i1, i2 = j, (j + 1) % 3, (j + 2) % 3
+        e1, e2 = c[:, i1] - c[:, i0], c[:, i2] - c[:, i0]
+        d0 = (e1 * e2).sum(1)
+        d1 = -(e1 * (c[:, i2] - c[:, i1])).sum(1)
+        d2 = (e2 * (c[:, i2] - c[:, i1])).sum(1)
+        for p, q, t in zip(F[:, i1].tolist(), F[:, i2].tolist(), clamp(d0 / area)):
+            w[(min(p, q), max(p, q))] = w.get((min(p, q), max(p, q)), 0.0) + t
+        t = np.maximum(0.125 * ((e2 * e2).sum(1) * clamp(d1 / area) + (e1 * e1).sum(1) * clamp(d2 / area)), 0.0)
+        t = np.where(d0 < 0, 0.25 * area, np.where((d1 < 0) | (d2 < 0), 0.125 * area, t))
+        np.add.at(vor, F[:, i0], t)
+    ms = vor / 0.5
+    diag = ms.copy()
+    for (p, q), t in w.items():
+        diag[p] += 0.1 * max(t, 0.0)
+        diag[q] += 0.1 * max(t, 0.0)
+    l2g = m.array("v_l2g")
+    ok = closed[l2g]
+    for got, ref in ((mass, ms), (val[rp[:-1]], diag)):
+        assert np.abs(got - ref[l2g])[ok].max() <= 1e-5 * np.abs(ref[l2g][ok]).max()
