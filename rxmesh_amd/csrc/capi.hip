@@ -372,6 +372,24 @@ int launch_patches_xcd(K kernel, uint32_t threads, uint32_t lds, void* stream, c
     return launch_grid(kernel, patch_grid(m->h.P), threads, lds, stream, args...);
 }
 
+// Workgroup size for patches of at most `nf` local faces, P of them. A patch of up
+// to 256 faces is one round of 256 threads, and more only idle; up to 512 faces,
+// 512 threads shorten one workgroup's chain while the patches are few enough for it
+// to be the launch, and 256 leave room for more workgroups a CU once they are
+// many; larger patches take 512. us with 256 / 512 threads (face lists' largest:
+// 160, 250, 400-450 and 720-780 faces):
+//   EVDiamond  3993 patches 6.4 / 8.6; 669 3.7 / 4.0; 83 3.7 / 3.3, 430 4.1 / 3.8,
+//              1006 4.9 / 5.0, 5356 14.0 / 15.6; 670 6.0 / 5.5, 8638 32 / 31
+//   curvature  3993 8.8 / 12.9; 669 4.7 / 5.1; 83 4.5 / 4.3, 430 5.2 / 5.2, 1006
+//              6.2 / 6.5, 5356 18 / 23; 670 7.1 / 6.6, 8638 49 / 43
+//   ARAP energy and gradient  3993 20 / 28; 669 8.8 / 9.3; 83 8.2 / 7.7, 430 9.3 /
+//              9.3, 1006 11.3 / 13.4, 5356 33 / 44; 670 13.3 / 12.6, 8638 103 / 89
+uint32_t patch_group(const rxm_mesh* m)
+{
+    const uint32_t nf = m->h.max_nf;
+    return nf <= 256u || (nf <= 512u && m->h.P > 512u) ? 256u : 512u;
+}
+
 // The query of REL (k_query_rows) on the fixed-width-slot kernel, or false if
 // the mesh does not fit it.
 template <uint32_t REL>
@@ -393,13 +411,16 @@ bool launch_rows(rxm_mesh* m, const uint32_t* v_base, const uint32_t* f_base, in
         *rc = launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, v_base, f_base, v_row, v_col, f_row, f_col);
         return true;
     };
-    // Few patches: one workgroup's chain is the launch, and more threads shorten
-    // it; many: small workgroups overlap more. VV + VF with 1024 / 512 / 256
-    // threads: 10 patches 5.2 / 5.5 / 7.1 us, 167 5.6 / 6.0 / 7.8, 491 7.8 / 7.5 /
-    // 8.9, 2687 29.7 / 22.2 / 21.8, 10677 97.7 / 70.0 / 58.8 (k_query2_vv_vf1,
-    // 256 threads: 8.4, 8.6, 9.4, 25.3, 67.6).
-    if (h.P <= 256u && fits(1024, 1, 1, 1)) return go(k_query_rows<1024, 1, 1, 1, REL>, 1024);
-    if (h.P > 1500u && fits(256, 4, 2, 2)) return go(k_query_rows<256, 4, 2, 2, REL>, 256);
+    // Patches above 512 faces: few, one workgroup's chain is the launch and more
+    // threads shorten it; many, small workgroups overlap more. VV + VF with 1024 /
+    // 512 / 256 threads: 10 patches 5.2 / 5.5 / 7.1 us, 166 5.7 / 6.1 / 7.7, 503
+    // 7.9 / 7.5 / 8.9, 1111 15.2 / 12.8 / 12.2, 2754 31 / 23 / 23, 10677 98 / 70 /
+    // 59 (k_query2_vv_vf1, 256 threads: 8.4, 8.6, 9.4, 25.3 at 2687, 67.6). Smaller
+    // ones as patch_group: up to 450 faces, 512 / 256 threads, 83 patches 5.1 / 5.5,
+    // 430 6.1 / 6.3, 1006 8.3 / 7.4, 5356 29 / 22; 250 faces, 669 6.5 / 5.6.
+    const uint32_t W = h.max_nf <= 512u ? patch_group(m) : h.P <= 256u ? 1024u : h.P <= 1000u ? 512u : 256u;
+    if (W == 1024u && fits(1024, 1, 1, 1)) return go(k_query_rows<1024, 1, 1, 1, REL>, 1024);
+    if (W == 256u && fits(256, 4, 2, 2)) return go(k_query_rows<256, 4, 2, 2, REL>, 256);
     if (fits(512, 3, 2, 2)) return go(k_query_rows<512, 3, 2, 2, REL>, 512);
     return false;
 }
@@ -426,10 +447,13 @@ bool launch_dir(rxm_mesh* m, const uint32_t* base, int32_t* row_ptr, int32_t* co
     // threads, EF and FF: 166 patches 4.3 / 3.7 / 3.5 and 3.7 / 3.4 / 3.3, 267
     // 4.5 / 4.0 / 4.2 and 3.9 / 3.7 / 3.9, 670 5.2 / 5.0 / 5.9 and 4.6 / 4.7 / 5.5,
     // 1111 6.4 / 6.9 / 8.4 and 5.8 / 6.2 / 7.7, 2675 10.6 / 11.8 / 15.7 and
-    // 9.7 / 10.3 / 14.5, 10630 26 / 33 / 51 and 25 / 29 / 46.
+    // 9.7 / 10.3 / 14.5, 10630 26 / 33 / 51 and 25 / 29 / 46. Patches up to 512
+    // faces as patch_group: EF with 256 / 512, up to 450 faces, 83 patches 3.8 /
+    // 3.5, 430 4.1 / 3.9, 1006 4.6 / 5.0, 5356 13 / 16; 250 faces, 669 3.6 / 4.0.
     constexpr uint32_t RS = FF ? 3 : 4;
-    if (h.P <= 256u && fits(1024, 1, 1)) return go(k_query_dir<1024, 1, 1, FF>, 1024);
-    if (h.P > 700u && fits(256, 4, RS)) return go(k_query_dir<256, 4, RS, FF>, 256);
+    const uint32_t W = h.max_nf <= 512u ? patch_group(m) : h.P <= 256u ? 1024u : h.P <= 700u ? 512u : 256u;
+    if (W == 1024u && fits(1024, 1, 1)) return go(k_query_dir<1024, 1, 1, FF>, 1024);
+    if (W == 256u && fits(256, 4, RS)) return go(k_query_dir<256, 4, RS, FF>, 256);
     if (fits(512, 3, RS)) return go(k_query_dir<512, 3, RS, FF>, 512);
     return false;
 }
@@ -536,20 +560,33 @@ int ensure_face_plan(rxm_mesh* m, void* stream)
 }
 
 // Workgroup size of the smoothing kernels where the caller chose none. While
-// the patches are resident at about once (4 workgroups of 512 threads on each
-// of 256 CUs) a launch lasts as long as one workgroup's chain, which more
-// threads shorten; beyond that more, smaller workgroups hide each other's
-// latency. Ten single steps with 512 / 256 threads: 71 patches 35.4 / 43.5 us,
-// 491 42.6 / 48.1, 1279 61.8 / 64.3, 2015 80.9 / 78.6, 4249 143 / 124.
-// Several steps per launch have more to spread: three steps, ten iterations,
-// 2015 patches 55.1 / 57.2, 4249 102.8 / 100.7; with 1024 / 512 threads, ten
-// steps five a launch, 10 patches 14.1 / 15.2, 167 14.8 / 16.1, 491 22.0 / 22.2,
-// 1037 (three a launch) 55 / 38.
+// patches above 512 faces are resident at about once (4 workgroups of 512 threads on
+// each of 256 CUs) a launch lasts as long as one workgroup's chain, which more
+// threads shorten; beyond that, and with the vertices of smaller patches, which
+// 256 threads hold in one round, smaller workgroups hide each other's latency. One
+// step with 512 / 256 threads, up to 780 faces: 166 patches 3.7 / 4.2 us, 503 4.3 /
+// 4.8, 1111 5.6 / 6.0, 2754 11.0 / 10.4, 8638 27 / 22; up to 450: 83 3.5 / 3.5, 430
+// 4.0 / 3.8, 1330 5.3 / 4.4, 5356 13.9 / 10.4. With 256 / 128 threads, up to 450:
+// 3386 6.9 / 7.3, 5356 10.4 / 10.1, 17184 26 / 22; up to 250: 164 3.4 / 3.5, 669 3.7 /
+// 3.7, 2021 4.7 / 4.4, 10780 14.4 / 11.9; up to 160: 329 3.5 / 3.6, 3993 6.0 / 5.1.
+// Several steps per launch have more to spread. Ten, with 1024 / 512 / 256 threads,
+// up to 780 faces: 10 patches 14.1 / 15.2 / -, 166 15.5 / 16.5 / 23, 503 - / 24 / 30,
+// 1111 - / 41 / 43, 2754 - / 78 / 80, 8638 - / 197 / 181; above 1024 faces: 22 18 / 22,
+// 4274 - / 185 / 207; up to 450: 83 14.0 / 13.3 / 17, 430 - / 18.8 / 23, 1006 - / 25 /
+// 27, 1330 - / 34 / 27, 5356 - / 96 / 68; up to 250: 164 13.8 / 13.1 / 14.5, 669 - /
+// 16.0 / 16.6, 2021 - / 42 / 29 (128: 31), 10780 256 / 128 106 / 92; up to 160, 3993
+// 42 / 33.
 uint32_t smooth_group(const rxm_mesh* m, bool multi = false)
 {
     if (m->smooth_threads) return m->smooth_threads;
-    if (multi) return m->h.P <= 256u ? 1024u : m->h.P <= 3000u ? 512u : 256u;
-    return m->h.P <= 1500u ? 512u : 256u;
+    const uint32_t nf = m->h.max_nf, P = m->h.P;
+    if (!multi) {
+        if (nf > 512u) return P <= 1500u ? 512u : 256u;
+        return P <= (nf <= 256u ? 512u : 5000u) ? 256u : 128u;
+    }
+    if (nf <= 256u) return P <= 256u ? 512u : P <= 3000u ? 256u : 128u;
+    if (nf <= 512u) return P <= 1024u ? 512u : 256u;
+    return P <= 256u ? 1024u : P <= 3000u || nf > 1024u ? 512u : 256u;
 }
 
 template <bool AOS4>
@@ -1259,7 +1296,9 @@ rxm_status rxm_query_csr(rxm_mesh* m, int op, int oriented, int32_t* row_ptr, in
             return launch_patches(k_query_fixed<7>, T, b.bytes(), stream, m, m->dm, row_ptr, col);
         case RXM_OP_EVD:
             plan_evd(b, h.max_nv, h.max_ne, 0, h.max_neo);
-            return launch_patches_xcd(k_query_evd<512>, 512, b.bytes(), stream, m, m->dm, row_ptr, col);
+            return patch_group(m) == 512u
+                       ? launch_patches_xcd(k_query_evd<512>, 512, b.bytes(), stream, m, m->dm, row_ptr, col)
+                       : launch_patches_xcd(k_query_evd<256>, 256, b.bytes(), stream, m, m->dm, row_ptr, col);
         default: return RXM_ERR_INVALID_ARG;
     }
 }
@@ -1348,9 +1387,11 @@ rxm_status rxm_gaussian_curvature(rxm_mesh* m, const float* pos, float* gc, floa
     if (rc) return rc;
     Bump b(nullptr);
     plan_gc(b, m->h.max_nv, m->h.max_nvo, m->h.max_nf, m->fp_max_nent);
-    return launch_patches_xcd(k_gaussian_curvature<512>, 512, b.bytes(), stream, m, m->dm, m->d_fp_fbase,
-                              m->d_fp_rbase, m->d_fp_nbase, m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, gc,
-                              area_mixed);
+    auto go = [&](auto kernel, uint32_t T) {
+        return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, m->d_fp_fbase, m->d_fp_rbase, m->d_fp_nbase,
+                                  m->d_fp_fvl, m->d_fp_roff, m->d_fp_vf, pos, gc, area_mixed);
+    };
+    return patch_group(m) == 512u ? go(k_gaussian_curvature<512>, 512) : go(k_gaussian_curvature<256>, 256);
 }
 
 // ---- ARAP-style deformation -------------------------------------------------
@@ -1409,7 +1450,6 @@ rxm_status rxm_arap_energy_grad(rxm_mesh* m, const float* rest, const float* x, 
 {
     if (!m || !rest || !x || !w || !R || !total || !grad) return RXM_ERR_INVALID_ARG;
     if (!m->on_device) return RXM_ERR_UNSUPPORTED;
-    constexpr uint32_t RT = 512;
     const uint32_t* vv_base = nullptr;
     uint32_t        lds     = 0;
     int             rc      = arap_rows(m, &vv_base, &lds, true, stream);
@@ -1420,7 +1460,10 @@ rxm_status rxm_arap_energy_grad(rxm_mesh* m, const float* rest, const float* x, 
                                   static_cast<const uint16_t*>(m->d_vv_roff), static_cast<const uint16_t*>(m->d_vv_ent),
                                   rest, x, w, R, m->d_partial, grad);
     };
-    rc = go(k_arap_energy_grad<RT>, RT);
+    // patches above 1024 faces: us with 1024 / 512 threads, 22 patches 9.8 / 12.5, 335
+    // 17.1 / 18.2, 541 25 / 28, 1374 50 / 51, 4274 136 / 128
+    if (m->h.max_nf > 1024u && m->h.P <= 1400u) rc = go(k_arap_energy_grad<1024>, 1024);
+    else rc = patch_group(m) == 512u ? go(k_arap_energy_grad<512>, 512) : go(k_arap_energy_grad<256>, 256);
     if (rc) return rc;
     hipLaunchKernelGGL(k_reduce_sum, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), m->h.P,
                        static_cast<const float*>(m->d_partial), total);
@@ -1715,10 +1758,12 @@ rxm_status rxm_mcf_explicit(rxm_mesh* m, const int32_t* row_ptr, const int32_t* 
             return launch_patches_xcd(kernel, T, b.bytes(), stream, m, m->dm, vv_base, m->d_vv_rbase, m->d_vv_nbase,
                                       m->d_vv_roff, m->d_vv_nbr, val, mass, src, dst);
         };
-        // the smoothing's sizes: us with 512 / 256 threads, 166 patches 3.8 / 4.4,
-        // 670 5.3 / 5.6, 1111 7.0 / 7.5, 1961 10.1 / 10.1, 2675 12.6 / 12.0, 10630
-        // 35 / 31
-        rc = smooth_group(m) == 512u ? go(k_mcf_patch<512>, 512) : go(k_mcf_patch<256>, 256);
+        // the smoothing's sizes (us with 512 / 256 threads, up to 780 faces: 166
+        // patches 3.8 / 4.4, 670 5.3 / 5.6, 1111 7.0 / 7.5, 1961 10.1 / 10.1, 2675
+        // 12.6 / 12.0, 10630 35 / 31; up to 450: 83 3.5 / 3.4, 430 4.2 / 4.0, 1330
+        // 6.4 / 5.1, 5356 17 / 12), but for patches above 1024 faces, whose values
+        // 512 threads hold in two rounds (1374 14.7 / 17.7, 4274 30 / 36)
+        rc = smooth_group(m) == 512u || (!m->smooth_threads && m->h.max_nf > 1024u) ? go(k_mcf_patch<512>, 512) : go(k_mcf_patch<256>, 256);
         src = dst;
     }
     return rc;

@@ -718,3 +718,39 @@ def test_closed_fans_of_any_valence(shape, patch_size):
     ok = closed[l2g]
     for got, ref in ((mass, ms), (val[rp[:-1]], diag)):
         assert np.abs(got - ref[l2g])[ok].max() <= 1e-5 * np.abs(ref[l2g][ok]).max()
+
+
+@pytest.mark.parametrize("level,patch_size", [(3, 16), (6, 64), (4, 256), (6, 256), (7, 256), (4, 512), (5, 1024)])
+def test_workgroup_sizes_of_small_patches(level, patch_size):
+    """Curvature, explicit step and single smoothing steps where the size of the
+    patches and their number choose the workgroup: curvature against FP64
+    (1e-5 of the angle sums, the angles' 1.4e-7 rad times the valence well
+    inside), the others the bits of the general CSR kernels or of every
+    workgroup size."""
+    import torch
+    V, F = mg.permute_mesh(*mg.icosphere(level, seed=18, sigma=0.002), seed=18)
+    m, x = _mesh(V, F, patch_size)
+    l2g = m.array("v_l2g")
+    X = np.empty((m.nV, 3))
+    X[l2g] = x.cpu().numpy().T
+    c = X[F]
+    ang, mix = np.zeros(m.nV), np.zeros(m.nV)
+    dots, s = [], np.linalg.norm(np.cross(c[:, 1] - c[:, 0], c[:, 2] - c[:, 0]), axis=1)
+    for j in range(3):
+        dots.append(((c[:, (j + 1) % 3] - c[:, j]) * (c[:, (j + 2) % 3] - c[:, j])).sum(1))
+    obtuse = (dots[0] < 0) | (dots[1] < 0) | (dots[2] < 0)
+    length = [((c[:, j] - c[:, (j + 1) % 3]) ** 2).sum(1) for j in range(3)]
+    for j in range(3):
+        a = (length[(j + 2) % 3] * dots[(j + 1) % 3] + length[j] * dots[(j + 2) % 3]) / (8 * s)
+        ang += np.bincount(F[:, j], np.arctan2(s, dots[j]), m.nV)
+        mix += np.bincount(F[:, j], np.where(obtuse, np.where(dots[j] < 0, s / 4, s / 8), a), m.nV)
+    gc, am = (t.cpu().numpy().astype(np.float64) for t in m.gaussian_curvature(x))
+    assert np.abs(am - mix[l2g]).max() <= 1e-5 * mix.max()
+    assert np.abs(gc * am - (2 * np.pi - ang)[l2g]).max() <= 1e-5 * 2 * np.pi
+    m.set_launch_threads(8, 0)
+    assert torch.equal(m.smooth(x, 0.5, 3), m.smooth_csr(m.query("VV"), x, 0.5, 3))
+    A = m.cot_assemble(x, 1e-4)
+    y = m.mcf_explicit(A, x, 2)
+    for threads in (256, 512):
+        m.set_launch_threads(0, threads)
+        assert torch.equal(m.mcf_explicit(A, x, 2), y)

@@ -199,7 +199,7 @@ def case_automatic_smoothing():
     """Tuning the gradient step loop leaves the steps per launch of the
     smoothing alone, and knobs 0 and 8 have a value that means the automatic
     choice."""
-    r = Recorder(sphere())
+    r = Recorder(sphere(), patch_size=1024)
     from rxmesh_amd import autotune
     assert r("rxm_vv_plan_build", A) == 0
 
