@@ -897,8 +897,8 @@ __global__ __launch_bounds__(T) void k_query2_x1(DevMesh m, uint32_t nslots, uin
 // the local face. Per
 // wave 489 VALU and 102 LDS instructions against 654 and 136. VV + VF: 654k vertices
 // 25.3 -> 21.0 us, 2.6M 67.6 -> 57.9; VV 37.6 -> 31.6, VF 38.2 -> 33. Bound: LDS, busy
-// three quarters of the time, over half of that in bank conflicts of the random
-// atomics and slot stores.
+// 56% of the time, half of that in bank conflicts of the random atomics and slot
+// stores, and VALU (55%), each in its own phase between barriers.
 // REL: kRowsVV or kRowsVE, kRowsVF, or a VV with a VF.
 enum : uint32_t { kRowsVV = 1, kRowsVE = 2, kRowsVF = 4 };
 constexpr uint32_t kRowMax = 8;
