@@ -404,6 +404,9 @@ class Mesh:
         return total, grad
 
     def smooth(self, pos, lam=0.5, iters=1, out=None, tmp=None, stream=None):
+        """`iters` uniform smoothing steps of (3, V) positions: one step per
+        launch, or three to five once build_vv_plan() has been called (same
+        bits; set_launch_threads(8, k) chooses)."""
         import torch
         if out is None:
             out = torch.empty_like(pos)
@@ -415,6 +418,7 @@ class Mesh:
         return out
 
     def build_vv_plan(self, stream=None):
+        """Build the smoothing's plans now, once per mesh (waits for the stream)."""
         _check(lib().rxm_vv_plan_build(self._h, _stream(stream)), "rxm_vv_plan_build")
 
     def set_launch_threads(self, kernel, threads):
